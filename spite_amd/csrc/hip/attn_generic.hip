@@ -1,5 +1,6 @@
 // Attention over the paged cache, one wave per (token, query head): the plain kernel of the
-// true 32-bit path, and of bf16 for head sizes that the MFMA kernels refuse.
+// true 32-bit path for head and page sizes that attn_f32.hip refuses, and of bf16 for head sizes
+// that the MFMA kernels refuse.
 //
 // The query at position p of its request reads the keys at [first_visible(p), p] through
 // the request's block table.  Keys are walked in tiles of 64 that start at first_visible(p),
@@ -8,6 +9,10 @@
 // output are fp32; exp is the accurate one.  Options: a smooth cap on the scaled scores, and
 // per-head slopes of a bias slope * (key position - query position) added before the cap.
 #include "common.h"
+
+int sp_attn_f32(const float* q, const float* k_pages, const float* v_pages, float* out, const int* positions,
+                const int* seq_of_token, const int* block_table, int max_blocks, int T, int H, int G, int hd, int page_size,
+                int vis, int span, float scale, float softcap, const float* slopes, hipStream_t st);   // attn_f32.hip; 1: not its shape
 
 #define ATT_MAX_D 8   // head sizes up to 512
 
@@ -103,6 +108,11 @@ extern "C" int spite_attn_generic(const void* q, const void* k_pages, const void
     SP_REQUIRE(!kv_tiled || (dtype == SP_BF16 && hd % 32 == 0 && page_size % 32 == 0),
                "attention: pages in operand order are bfloat16 with head size %d and page size %d multiples of 32", hd, page_size);
     if (T == 0) return 0;
+    if (dtype == SP_F32) {
+        const int rc = sp_attn_f32((const float*)q, (const float*)k_pages, (const float*)v_pages, (float*)out, positions, seq_of_token,
+                                   block_table, max_blocks, T, H, G, hd, page_size, vis, span, scale, softcap, slopes, st);
+        if (rc <= 0) return rc;
+    }
     dim3 grid(T, H);
     const size_t sh = (size_t)(hd + 64) * sizeof(float) + 64 * sizeof(long long) + 64 * sizeof(int) + 8;
     if (dtype == SP_F32)

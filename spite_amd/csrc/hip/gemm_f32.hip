@@ -1,0 +1,257 @@
+// fp32 matrix product Y = A . W^T on the matrix units (v_mfma_f32_16x16x4_f32: fp32 operands, fp32 FMAs, no narrower
+// step anywhere), the true 32-bit path of every projection whose rows can be read 16 bytes at a time.
+//
+// The order of every sum depends on K alone.  k is cut into eight runs of `seg` (K / 8 rounded up to 32); inside a
+// run the products are added in steps of 16 k, four MFMAs a step (MFMA e takes k0 + 4q + e of its four rows of lanes
+// q); the runs' sums are then added in their order, ((0 + s0) + s1) + ... + s7.  Both kernels below keep this order, so
+// a row has the same bits whether it comes alone or among many, and shorter chains round less than one ascending
+// chain over K.
+//
+//  gemm_f32_rows: few rows.  Bound by the stream of W (one row of X makes 0.5 FLOP a byte).  A workgroup takes 16
+//    rows of W (GLU: 16 of each half) and gives one run of k to each of its eight waves, so that a product with
+//    2,048 output rows has 1,024 waves in flight; the runs' sums meet in LDS.
+//  gemm_f32_tile: many rows, bound by the MFMAs (256 FLOP a clock and compute unit).  64 rows of X times 64 rows of W a
+//    workgroup: X through double-buffered LDS, read by all four waves; a wave's 16 rows of W straight into registers, a
+//    step ahead.  The smaller tile than a large product would want is for the sizes at hand: 301 tokens times 2,048
+//    columns are 160 workgroups.
+//
+// SP_F32_ROWS_MAX: up to 64 rows the first one reads each byte of W once, beyond it would read W again for every
+// further 64 rows.
+#include "common.h"
+
+#define SP_F32_ROWS_MAX 64
+
+// sum of one step of 16 k: the lane's four k of each operand
+__device__ __forceinline__ void f32_step(f32x4& acc, f32x4 w, f32x4 x) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[0], x[0], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[1], x[1], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[2], x[2], acc, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[3], x[3], acc, 0, 0, 0);
+}
+
+__device__ __forceinline__ int f32_seg(int K) { return (K + 255) / 256 * 32; }
+
+// A lane of a result tile holds W rows n0 + 4q .. + 3 of X row `s`.
+__device__ __forceinline__ void f32_store(float* __restrict__ Y, size_t row, int ldy, int n, int N, f32x4 v, bool vec) {
+    float* y = Y + row * ldy + n;
+    if (vec && n + 3 < N) *(f32x4*)y = v;
+    else
+#pragma unroll
+        for (int r = 0; r < 4; ++r) if (n + r < N) y[r] = v[r];
+}
+
+template <int MT, int GLU>
+__global__ __launch_bounds__(512)
+void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, long w_group_stride,
+                          float* __restrict__ Y, int ldy, int M, int N, int K, const int* __restrict__ offsets, int n_groups,
+                          const int* __restrict__ a_rows, const float* __restrict__ a_scale, const int* __restrict__ y_rows,
+                          int act, float act_limit, int vec_y) {
+    constexpr int NB = GLU ? 2 : 1;
+    __shared__ f32x4 red[8][MT * NB][64];
+    int g = 0, row0 = 0, row_end = M;
+    if (offsets) {
+        if (!sp_find_tile(offsets, n_groups, MT * 16, blockIdx.y, g, row0, row_end)) return;
+    } else {
+        row0 = blockIdx.y * (MT * 16);
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int n0 = blockIdx.x * 16;
+    const float* Wg = W + (size_t)g * w_group_stride;
+    const int wn = n0 + r < N ? n0 + r : N - 1;
+    const float* wp[NB];
+    wp[0] = Wg + (size_t)wn * K;
+    if (GLU) wp[NB - 1] = Wg + (size_t)(N + wn) * K;
+    const float* xp[MT];
+    float sc[MT];
+    bool live[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int s = row0 + m * 16 + r;
+        live[m] = s < row_end;
+        const int ss = live[m] ? s : row0;             // a row that exists: its products are not stored
+        xp[m] = A + (size_t)(a_rows ? a_rows[ss] : ss) * lda;
+        sc[m] = a_scale ? a_scale[ss] : 1.0f;
+    }
+    const int seg = f32_seg(K);
+    const int k_lo = wave * seg, k_hi = k_lo + seg < K ? k_lo + seg : K;
+    f32x4 acc[MT][NB];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[m][b] = {0.f, 0.f, 0.f, 0.f};
+    constexpr int U = MT == 4 ? 4 : 8;                  // steps of 16 k whose loads are in flight together (registers)
+    for (int k0 = k_lo; k0 < k_hi; k0 += 16 * U) {
+        f32x4 w[U][NB], x[U][MT];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k0 + u * 16 + q * 4;
+            const bool in = k < k_hi;                  // K is a multiple of 4, a run's end of 4
+#pragma unroll
+            for (int b = 0; b < NB; ++b) w[u][b] = in ? __builtin_nontemporal_load((const f32x4*)(wp[b] + k)) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int m = 0; m < MT; ++m) x[u][m] = in ? *(const f32x4*)(xp[m] + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u)
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                const f32x4 xs = x[u][m] * sc[m];
+#pragma unroll
+                for (int b = 0; b < NB; ++b) f32_step(acc[m][b], w[u][b], xs);
+            }
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) red[wave][m * NB + b][lane] = acc[m][b];
+    __syncthreads();
+    if (wave >= MT) return;
+    const int m = wave, s = row0 + m * 16 + r;
+    f32x4 t[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        t[b] = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 8; ++i) t[b] += red[i][m * NB + b][lane];
+    }
+    if (s >= row_end) return;
+    if (GLU)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[0][e] = sp_gated(t[0][e], t[NB - 1][e], act, act_limit, false);
+    f32_store(Y, y_rows ? (size_t)y_rows[s] : (size_t)s, ldy, n0 + q * 4, N, t[0], vec_y);
+}
+
+#define F32_TM 64                 // rows of X a workgroup
+#define F32_TK 32                 // k a step through LDS
+#define F32_LD (F32_TK + 4)       // LDS row: 16 bytes more than a step, so that 16 rows' reads spread over the banks
+
+template <int GLU>
+__global__ __launch_bounds__(256)
+void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, long w_group_stride,
+                          float* __restrict__ Y, int ldy, int M, int N, int K, const int* __restrict__ offsets, int n_groups,
+                          const int* __restrict__ a_rows, const float* __restrict__ a_scale, const int* __restrict__ y_rows,
+                          int act, float act_limit, int vec_y) {
+    constexpr int NB = GLU ? 2 : 1, MT = F32_TM / 16;
+    __shared__ __align__(16) float xs[2][F32_TM * F32_LD];
+    int g = 0, row0 = 0, row_end = M;
+    if (offsets) {
+        if (!sp_find_tile(offsets, n_groups, F32_TM, blockIdx.y, g, row0, row_end)) return;
+    } else {
+        row0 = blockIdx.y * F32_TM;
+    }
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const int n0 = blockIdx.x * 64 + wave * 16;
+    const float* Wg = W + (size_t)g * w_group_stride;
+    const int wn = n0 + r < N ? n0 + r : N - 1;
+    const float* wp[NB];
+    wp[0] = Wg + (size_t)wn * K;
+    if (GLU) wp[NB - 1] = Wg + (size_t)(N + wn) * K;
+    // the loader: a thread brings 4 k of rows lr and lr + 32
+    const int lk = (threadIdx.x & 7) * 4, lr = threadIdx.x >> 3;
+    const float* xp[2];
+    float sc[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int s = row0 + lr + i * 32, ss = s < row_end ? s : row0;
+        xp[i] = A + (size_t)(a_rows ? a_rows[ss] : ss) * lda;
+        sc[i] = a_scale ? a_scale[ss] : 1.0f;
+    }
+    const int seg = f32_seg(K);
+    const int live = __builtin_amdgcn_readfirstlane((row_end - row0 + 15) / 16 < MT ? (row_end - row0 + 15) / 16 : MT);   // 16-row tiles with rows
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[MT][NB], tot[MT][NB], w[2][NB], xv[2];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[m][b] = tot[m][b] = zero;
+
+    auto fetch = [&](int k0) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int k = k0 + u * 16 + q * 4;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) w[u][b] = k < K ? *(const f32x4*)(wp[b] + k) : zero;
+        }
+        const int k = k0 + lk;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) xv[i] = k < K ? *(const f32x4*)(xp[i] + k) * sc[i] : zero;
+    };
+    auto put = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < 2; ++i) *(f32x4*)(&xs[buf][(lr + i * 32) * F32_LD + lk]) = xv[i];
+    };
+    fetch(0);
+    put(0);
+    int buf = 0;
+    for (int k0 = 0; k0 < K; k0 += F32_TK, buf ^= 1) {
+        __syncthreads();                               // this step's rows are in LDS, the other buffer is free
+        f32x4 wc[2][NB];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) wc[u][b] = w[u][b];
+        const bool more = k0 + F32_TK < K;
+        if (more) fetch(k0 + F32_TK);
+        if (k0 && k0 % seg == 0) {                     // a run of k ends
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) { tot[m][b] += acc[m][b]; acc[m][b] = zero; }
+        }
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m) {
+                if (m < live) {
+                    const f32x4 x = *(const f32x4*)(&xs[buf][(m * 16 + r) * F32_LD + u * 16 + q * 4]);
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) f32_step(acc[m][b], wc[u][b], x);
+                }
+            }
+        }
+        if (more) put(buf ^ 1);
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int s = row0 + m * 16 + r;
+        if (s >= row_end) continue;
+        f32x4 t = tot[m][0] + acc[m][0];
+        if (GLU) {
+            const f32x4 u = tot[m][NB - 1] + acc[m][NB - 1];
+#pragma unroll
+            for (int e = 0; e < 4; ++e) t[e] = sp_gated(t[e], u[e], act, act_limit, false);
+        }
+        f32_store(Y, y_rows ? (size_t)y_rows[s] : (size_t)s, ldy, n0 + q * 4, N, t, vec_y);
+    }
+}
+
+// The product if its rows can be read 16 bytes at a time (returns 0, or an error), else 1: the plain kernel's.
+int sp_gemm_f32(const float* A, int lda, const float* W, long w_group_stride, float* Y, int ldy, int M, int N, int K,
+                const int* offsets, int n_groups, const int* a_rows, const float* a_scale, const int* y_rows, int glu,
+                float act_limit, hipStream_t st) {
+    if (K % 4 || lda % 4 || w_group_stride % 4 || ((uintptr_t)A | (uintptr_t)W) % 16) return 1;
+    const int vec_y = ldy % 4 == 0 && (uintptr_t)Y % 16 == 0;
+    const int tile = M > SP_F32_ROWS_MAX ? F32_TM : M > 32 ? 64 : M > 16 ? 32 : 16;
+    const int m_tiles = offsets ? M / tile + (n_groups < M ? n_groups : M) : (M + tile - 1) / tile;
+    SP_REQUIRE(m_tiles <= 65535, "gemm: too many row tiles (%d)", m_tiles);
+#define SP_F32_ARGS A, lda, W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, act_limit, vec_y
+    if (M > SP_F32_ROWS_MAX) {
+        dim3 grid((N + 63) / 64, m_tiles);
+        if (glu) gemm_f32_tile_kernel<1><<<grid, 256, 0, st>>>(SP_F32_ARGS);
+        else gemm_f32_tile_kernel<0><<<grid, 256, 0, st>>>(SP_F32_ARGS);
+        SP_LAUNCH_CHECK("gemm_f32_tile");
+        return 0;
+    }
+    dim3 grid((N + 15) / 16, m_tiles);
+#define SP_F32_ROWS(MT) do { if (glu) gemm_f32_rows_kernel<MT, 1><<<grid, 512, 0, st>>>(SP_F32_ARGS); \
+                             else gemm_f32_rows_kernel<MT, 0><<<grid, 512, 0, st>>>(SP_F32_ARGS); } while (0)
+    if (tile == 16) SP_F32_ROWS(1);
+    else if (tile == 32) SP_F32_ROWS(2);
+    else SP_F32_ROWS(4);
+#undef SP_F32_ROWS
+#undef SP_F32_ARGS
+    SP_LAUNCH_CHECK("gemm_f32_rows");
+    return 0;
+}

@@ -1,5 +1,6 @@
 // Plain tiled matrix product, Y = A . W^T, fp32 FMA with fp32 accumulation in ascending k:
-// the true 32-bit path of every projection, and the bf16 path for shapes that the MFMA
+// the 32-bit path of shapes that the fp32 MFMA kernels refuse (gemm_f32.hip: rows that are no
+// multiple of 16 bytes, or not aligned to them), and the bf16 path for shapes that the bf16 MFMA
 // kernels refuse.  Each output element is one thread's private sum, so a row's result does
 // not depend on which other rows share the call.
 //
@@ -9,6 +10,10 @@
 // y_rows[s] of Y.  With `glu` the group's W holds 2N rows, gate rows first, and the kernel
 // writes act(gate) * up (`glu`: the activation's code, `act_limit` its bound where it has one; see sp_gated).
 #include "common.h"
+
+int sp_gemm_f32(const float* A, int lda, const float* W, long w_group_stride, float* Y, int ldy, int M, int N, int K,
+                const int* offsets, int n_groups, const int* a_rows, const float* a_scale, const int* y_rows, int glu,
+                float act_limit, hipStream_t st);      // gemm_f32.hip; 1: not its shape
 
 #define GBM 64
 #define GBN 64
@@ -103,6 +108,11 @@ extern "C" int spite_gemm_generic(const void* A, int lda, const void* W, long w_
     SP_REQUIRE(!offsets || n_groups > 0, "gemm: grouped call without groups");
     SP_REQUIRE(glu >= 0 && glu <= SP_ACT_LAST && (glu != SP_ACT_CLAMPED || act_limit > 0.f), "gemm: activation code %d with bound %g", glu, act_limit);
     if (M == 0) return 0;
+    if (dtype == SP_F32 && y_dtype == SP_F32) {
+        const int rc = sp_gemm_f32((const float*)A, lda, (const float*)W, w_group_stride, (float*)Y, ldy, M, N, K, offsets, n_groups,
+                                   a_rows, a_scale, y_rows, glu, act_limit, st);
+        if (rc <= 0) return rc;
+    }
     // row tiles: a group with rows has 1 + (rows - 1) / tile of them, so groups with rows + M / tile bounds them
     const int m_tiles = offsets ? M / GBM + (n_groups < M ? n_groups : M) : (M + GBM - 1) / GBM;
     SP_REQUIRE(m_tiles <= 65535, "gemm: too many row tiles (%d)", m_tiles);
