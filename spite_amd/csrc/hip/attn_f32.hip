@@ -1,18 +1,19 @@
 // fp32 attention over row-major pages (head sizes in multiples of 16 up to 128, pages in multiples of 4 keys): the true
 // 32-bit path at the sizes that models have; attn_generic.hip keeps the others.
 //
-// A workgroup of four waves per (token, query head).  Keys are walked in tiles of 64 that start at multiples of 64
-// positions, tile t by wave t % 4, each wave with its own running maximum, sum and output; the four meet in LDS at the
+// A workgroup of eight waves per (token, query head).  Keys are walked in tiles of 32 that start at multiples of 32
+// positions, tile t by wave t % 8, each wave with its own running maximum, sum and output; the eight meet in LDS at the
 // end, in their order.  So the order of every sum depends on the query's position alone, as in the plain kernel: a token
 // gives the same bits whether it comes in a whole prompt, a portion or alone.
 //
-// Bound by latency (decode: a chain of loads over few workgroups) or by the loads' path (prompts).  Hence 16-byte loads
-// over whole runs: for the scores a key's row is read by four lanes, 64 bytes a load and key, all loads of 16 keys
-// in flight; for the output 16 lanes read 64 consecutive keys of a value row, and a lane keeps the partial sums of its
-// four keys until the end instead of summing across lanes in every tile.
+// Bound by latency (decode: a chain of loads, table entry - keys - values, over few workgroups) or by the loads' path
+// (prompts).  Hence tiles of 32 over eight waves, so that 256 keys are one such chain; 16-byte loads over whole lines,
+// for the scores a key's row by four lanes, for the output 32 consecutive keys of a value row by eight; a lane keeps the
+// partial sums of its four keys until the end instead of summing across lanes in every tile.
 #include "common.h"
 
-#define AF_WAVES 4
+#define AF_WAVES 8
+#define AF_KEYS 32
 
 template <int NI>     // the head size in units of 16, at most
 __global__ __launch_bounds__(64 * AF_WAVES)
@@ -20,7 +21,7 @@ void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pa
                      float* __restrict__ out, const int* __restrict__ positions, const int* __restrict__ seq_of_token,
                      const int* __restrict__ block_table, int max_blocks, int H, int G, int hd, int ps, int vis, int span,
                      float scale, float softcap, const float* __restrict__ slopes) {
-    __shared__ __align__(16) float p_sh[AF_WAVES][64];
+    __shared__ __align__(16) float p_sh[AF_WAVES][AF_KEYS];
     __shared__ float o_sh[AF_WAVES][NI * 16];
     __shared__ float ml_sh[AF_WAVES][2];
     const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
@@ -32,83 +33,96 @@ void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pa
     const float slope = slopes ? slopes[h] : 0.f;
     const float* qr = q + ((size_t)t * H + h) * hd;
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    // scores: lane (kr, cq) takes elements 16 i + 4 cq .. + 3 of keys kr, kr + 16, ... of a tile
+    // scores: lane (kr, cq) takes elements 16 i + 4 cq .. + 3 of keys kr and kr + 16 of a tile
     const int kr = lane >> 2, cq = (lane & 3) * 4;
     f32x4 qv[NI];
 #pragma unroll
     for (int i = 0; i < NI; ++i) qv[i] = i < ni ? *(const f32x4*)(qr + i * 16 + cq) : zero;
-    // output: lane (cr, kq) takes elements 4 i + cr of keys 4 kq .. + 3
-    const int cr = lane >> 4, kq = (lane & 15) * 4;
-    float o[NI * 4];
+    // output: lane (cr, kq) takes elements 8 i + cr of keys 4 kq .. + 3
+    const int cr = lane >> 3, kq = (lane & 7) * 4;
+    float o[NI * 2];
 #pragma unroll
-    for (int i = 0; i < NI * 4; ++i) o[i] = 0.f;
+    for (int i = 0; i < NI * 2; ++i) o[i] = 0.f;
     float m = -INFINITY, l = 0.f;
 
-    for (int j0 = (lo & ~63) + wave * 64; j0 <= p; j0 += 64 * AF_WAVES) {
-        float s[4];
+    for (int j0 = (lo & ~(AF_KEYS - 1)) + wave * AF_KEYS; j0 <= p; j0 += AF_KEYS * AF_WAVES) {
+        // the table entries of this tile's keys and values, then every row of keys, before anything waits for them
+        int page[2];
+        bool seen[2];
 #pragma unroll
-        for (int n = 0; n < 4; ++n) {
+        for (int n = 0; n < 2; ++n) {
             const int j = j0 + n * 16 + kr;
-            const bool seen = j >= lo && j <= p;
-            const int page = seen ? bt[j / ps] : -1;
-            const float* row = page >= 0 ? k_pages + ((size_t)page * G + g) * hd * ps + (size_t)(j % ps) * hd : qr;
+            seen[n] = j >= lo && j <= p;
+            page[n] = seen[n] ? bt[j / ps] : -1;
+        }
+        const int jv = j0 + kq;
+        const int vpage = jv + 3 >= lo && jv <= p ? bt[jv / ps] : -1;
+        f32x4 kv[2][NI];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
+            const float* row = page[n] >= 0 ? k_pages + ((size_t)page[n] * G + g) * hd * ps + (size_t)((j0 + n * 16 + kr) % ps) * hd : qr;
+#pragma unroll
+            for (int i = 0; i < NI; ++i) kv[n][i] = *(const f32x4*)(row + (i < ni ? i : 0) * 16 + cq);
+        }
+        float s[2];
+#pragma unroll
+        for (int n = 0; n < 2; ++n) {
             f32x4 a = zero;
 #pragma unroll
-            for (int i = 0; i < NI; ++i)
-                if (i < ni) {
-                    const f32x4 kv = *(const f32x4*)(row + i * 16 + cq);
+            for (int i = 0; i < NI; ++i)               // (qv is zero beyond the head)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) a[e] = fmaf(qv[i][e], kv[e], a[e]);
-                }
+                for (int e = 0; e < 4; ++e) a[e] = fmaf(qv[i][e], kv[n][i][e], a[e]);
             float x = (a[0] + a[1]) + (a[2] + a[3]);
             x += __shfl_xor(x, 1, 64);
             x += __shfl_xor(x, 2, 64);
-            x = x * scale + slope * (float)(j - p);
+            x = x * scale + slope * (float)(j0 + n * 16 + kr - p);
             if (softcap > 0.f) x = softcap * tanhf(x / softcap);
-            s[n] = !seen ? -INFINITY : page >= 0 ? x : NAN;    // a page that was given back is asked for: poison the result
+            s[n] = !seen[n] ? -INFINITY : page[n] >= 0 ? x : NAN;    // a page that was given back is asked for: poison the result
         }
-        float mx = fmaxf(fmaxf(s[0], s[1]), fmaxf(s[2], s[3]));
+        const float* vp = vpage >= 0 ? v_pages + ((size_t)vpage * G + g) * hd * ps + (jv % ps) : nullptr;
+        f32x4 v[NI * 2];
+#pragma unroll
+        for (int i = 0; i < NI * 2; ++i) v[i] = vp ? *(const f32x4*)(vp + (size_t)((i < ni * 2 ? i : 0) * 8 + cr) * ps) : zero;
+        float mx = fmaxf(s[0], s[1]);
 #pragma unroll
         for (int d = 4; d < 64; d <<= 1) mx = fmaxf(mx, __shfl_xor(mx, d, 64));
         const float m_new = fmaxf(m, mx), alpha = expf(m - m_new);
-        float ps_ = 0.f;
+        float sum = 0.f;
 #pragma unroll
-        for (int n = 0; n < 4; ++n) {
+        for (int n = 0; n < 2; ++n) {
             s[n] = expf(s[n] - m_new);                 // 0 where the key is not seen
-            ps_ += s[n];
+            sum += s[n];
             if ((lane & 3) == n) p_sh[wave][n * 16 + kr] = s[n];
         }
 #pragma unroll
-        for (int d = 4; d < 64; d <<= 1) ps_ += __shfl_xor(ps_, d, 64);
-        l = l * alpha + ps_;
+        for (int d = 4; d < 64; d <<= 1) sum += __shfl_xor(sum, d, 64);
+        l = l * alpha + sum;
         m = m_new;
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         const f32x4 pv = *(const f32x4*)&p_sh[wave][kq];
-        const int jv = j0 + kq;
-        const int page = jv + 3 >= lo && jv <= p ? bt[jv / ps] : -1;
-        const bool edge = j0 < lo || j0 + 63 > p;      // some keys of the tile are not seen: what their places hold must not count
-        const float* vp = page >= 0 ? v_pages + ((size_t)page * G + g) * hd * ps + (jv % ps) : nullptr;
+        if (j0 < lo || j0 + AF_KEYS - 1 > p) {         // some keys of the tile are not seen: what their places hold must not count
 #pragma unroll
-        for (int i = 0; i < NI * 4; ++i)
-            if (i < ni * 4) {
-                f32x4 v = vp ? *(const f32x4*)(vp + (size_t)(i * 4 + cr) * ps) : zero;
-                if (edge) {
+            for (int i = 0; i < NI * 2; ++i)
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) v[e] = jv + e >= lo && jv + e <= p ? v[e] : 0.f;
-                }
-                float a = o[i] * alpha;
+                for (int e = 0; e < 4; ++e) v[i][e] = jv + e >= lo && jv + e <= p ? v[i][e] : 0.f;
+        }
 #pragma unroll
-                for (int e = 0; e < 4; ++e) a = fmaf(pv[e], v[e], a);
-                o[i] = a;
-            }
+        for (int i = 0; i < NI * 2; ++i) {
+            float a = o[i] * alpha;
+#pragma unroll
+            for (int e = 0; e < 4; ++e) a = fmaf(pv[e], v[i][e], a);
+            o[i] = a;
+        }
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     }
 #pragma unroll
-    for (int i = 0; i < NI * 4; ++i)
-        if (i < ni * 4) {
-            const float a = row16_sum(o[i]);
-            if ((lane & 15) == (i & 15)) o_sh[wave][i * 4 + cr] = a;
-        }
+    for (int i = 0; i < NI * 2; ++i) {
+        float a = o[i];
+        a += __shfl_xor(a, 1, 64);
+        a += __shfl_xor(a, 2, 64);
+        a += __shfl_xor(a, 4, 64);
+        if ((lane & 7) == (i & 7)) o_sh[wave][i * 8 + cr] = a;
+    }
     if (lane == 0) { ml_sh[wave][0] = m; ml_sh[wave][1] = l; }
     __syncthreads();
     const int c = threadIdx.x;

@@ -126,14 +126,75 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
 #define F32_TK 32                 // k a step through LDS
 #define F32_LD (F32_TK + 4)       // LDS row: 16 bytes more than a step, so that 16 rows' reads spread over the banks
 
+// The loop over k for a tile whose first LIVE groups of 16 rows hold rows (an expert's last tile is seldom full).  Loads
+// are unconditional, a step ahead of their use, and scaled only when they go to LDS, so that nothing waits for them
+// before the step's MFMAs; a chain of four MFMAs is spread over the accumulators.
+template <int NB, int LIVE>
+__device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp, const float* const* xp, const float* sc, int K,
+                                              int seg, int lr, int lk, int r, int q, f32x4 (&tot)[4][NB]) {
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[LIVE][NB], w[2][NB], xv[2];
+#pragma unroll
+    for (int m = 0; m < LIVE; ++m)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[m][b] = zero;
+    // k past the end: the last four's address, and zeros instead
+#define F32_FETCH(k0) do { \
+    _Pragma("unroll") for (int u = 0; u < 2; ++u) { \
+        const int k = (k0) + u * 16 + q * 4, kc = k < K ? k : K - 4; \
+        _Pragma("unroll") for (int b = 0; b < NB; ++b) w[u][b] = *(const f32x4*)(wp[b] + kc); } \
+    const int kx = (k0) + lk < K ? (k0) + lk : K - 4; \
+    _Pragma("unroll") for (int i = 0; i < 2; ++i) xv[i] = *(const f32x4*)(xp[i] + kx); } while (0)
+#define F32_PUT(buf, k0) do { \
+    _Pragma("unroll") for (int i = 0; i < 2; ++i) \
+        *(f32x4*)(xs + (buf) * (F32_TM * F32_LD) + (lr + i * 32) * F32_LD + lk) = (k0) + lk < K ? xv[i] * sc[i] : zero; } while (0)
+    F32_FETCH(0);
+    F32_PUT(0, 0);
+    int buf = 0;
+    for (int run = 0; run < K; run += seg) {
+        const int end = run + seg < K ? run + seg : K;
+        for (int k0 = run; k0 < end; k0 += F32_TK, buf ^= 1) {
+            __syncthreads();                           // this step's rows are in LDS, the other buffer is free
+            f32x4 wc[2][NB];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) wc[u][b] = k0 + u * 16 + q * 4 < K ? w[u][b] : zero;
+            F32_FETCH(k0 + F32_TK);
+            f32x4 x[2][LIVE];
+            const float* xb = xs + buf * (F32_TM * F32_LD);
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int m = 0; m < LIVE; ++m) x[u][m] = *(const f32x4*)(xb + (m * 16 + r) * F32_LD + u * 16 + q * 4);
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+#pragma unroll
+                for (int e = 0; e < 4; ++e)
+#pragma unroll
+                    for (int m = 0; m < LIVE; ++m)
+#pragma unroll
+                        for (int b = 0; b < NB; ++b)
+                            acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[u][b][e], x[u][m][e], acc[m][b], 0, 0, 0);
+            F32_PUT(buf ^ 1, k0 + F32_TK);
+        }
+#pragma unroll
+        for (int m = 0; m < LIVE; ++m)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) { tot[m][b] += acc[m][b]; acc[m][b] = zero; }
+    }
+#undef F32_FETCH
+#undef F32_PUT
+}
+
 template <int GLU>
 __global__ __launch_bounds__(256)
 void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, long w_group_stride,
                           float* __restrict__ Y, int ldy, int M, int N, int K, const int* __restrict__ offsets, int n_groups,
                           const int* __restrict__ a_rows, const float* __restrict__ a_scale, const int* __restrict__ y_rows,
                           int act, float act_limit, int vec_y) {
-    constexpr int NB = GLU ? 2 : 1, MT = F32_TM / 16;
-    __shared__ __align__(16) float xs[2][F32_TM * F32_LD];
+    constexpr int NB = GLU ? 2 : 1;
+    __shared__ __align__(16) float xs[2 * F32_TM * F32_LD];
     int g = 0, row0 = 0, row_end = M;
     if (offsets) {
         if (!sp_find_tile(offsets, n_groups, F32_TM, blockIdx.y, g, row0, row_end)) return;
@@ -158,71 +219,24 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
         xp[i] = A + (size_t)(a_rows ? a_rows[ss] : ss) * lda;
         sc[i] = a_scale ? a_scale[ss] : 1.0f;
     }
-    const int seg = f32_seg(K);
-    const int live = __builtin_amdgcn_readfirstlane((row_end - row0 + 15) / 16 < MT ? (row_end - row0 + 15) / 16 : MT);   // 16-row tiles with rows
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 acc[MT][NB], tot[MT][NB], w[2][NB], xv[2];
+    f32x4 tot[4][NB];
 #pragma unroll
-    for (int m = 0; m < MT; ++m)
+    for (int m = 0; m < 4; ++m)
 #pragma unroll
-        for (int b = 0; b < NB; ++b) acc[m][b] = tot[m][b] = zero;
-
-    auto fetch = [&](int k0) {
+        for (int b = 0; b < NB; ++b) tot[m][b] = {0.f, 0.f, 0.f, 0.f};
+    const int rows = row_end - row0, seg = f32_seg(K);
+    if (rows > 48) f32_tile_loop<NB, 4>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+    else if (rows > 32) f32_tile_loop<NB, 3>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+    else if (rows > 16) f32_tile_loop<NB, 2>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+    else f32_tile_loop<NB, 1>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
 #pragma unroll
-        for (int u = 0; u < 2; ++u) {
-            const int k = k0 + u * 16 + q * 4;
-#pragma unroll
-            for (int b = 0; b < NB; ++b) w[u][b] = k < K ? *(const f32x4*)(wp[b] + k) : zero;
-        }
-        const int k = k0 + lk;
-#pragma unroll
-        for (int i = 0; i < 2; ++i) xv[i] = k < K ? *(const f32x4*)(xp[i] + k) * sc[i] : zero;
-    };
-    auto put = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < 2; ++i) *(f32x4*)(&xs[buf][(lr + i * 32) * F32_LD + lk]) = xv[i];
-    };
-    fetch(0);
-    put(0);
-    int buf = 0;
-    for (int k0 = 0; k0 < K; k0 += F32_TK, buf ^= 1) {
-        __syncthreads();                               // this step's rows are in LDS, the other buffer is free
-        f32x4 wc[2][NB];
-#pragma unroll
-        for (int u = 0; u < 2; ++u)
-#pragma unroll
-            for (int b = 0; b < NB; ++b) wc[u][b] = w[u][b];
-        const bool more = k0 + F32_TK < K;
-        if (more) fetch(k0 + F32_TK);
-        if (k0 && k0 % seg == 0) {                     // a run of k ends
-#pragma unroll
-            for (int m = 0; m < MT; ++m)
-#pragma unroll
-                for (int b = 0; b < NB; ++b) { tot[m][b] += acc[m][b]; acc[m][b] = zero; }
-        }
-#pragma unroll
-        for (int u = 0; u < 2; ++u) {
-#pragma unroll
-            for (int m = 0; m < MT; ++m) {
-                if (m < live) {
-                    const f32x4 x = *(const f32x4*)(&xs[buf][(m * 16 + r) * F32_LD + u * 16 + q * 4]);
-#pragma unroll
-                    for (int b = 0; b < NB; ++b) f32_step(acc[m][b], wc[u][b], x);
-                }
-            }
-        }
-        if (more) put(buf ^ 1);
-    }
-#pragma unroll
-    for (int m = 0; m < MT; ++m) {
+    for (int m = 0; m < 4; ++m) {
         const int s = row0 + m * 16 + r;
         if (s >= row_end) continue;
-        f32x4 t = tot[m][0] + acc[m][0];
-        if (GLU) {
-            const f32x4 u = tot[m][NB - 1] + acc[m][NB - 1];
+        f32x4 t = tot[m][0];
+        if (GLU)
 #pragma unroll
-            for (int e = 0; e < 4; ++e) t[e] = sp_gated(t[e], u[e], act, act_limit, false);
-        }
+            for (int e = 0; e < 4; ++e) t[e] = sp_gated(t[e], tot[m][NB - 1][e], act, act_limit, false);
         f32_store(Y, y_rows ? (size_t)y_rows[s] : (size_t)s, ldy, n0 + q * 4, N, t, vec_y);
     }
 }

@@ -45,7 +45,7 @@ def test_the_sum_is_no_less_exact_than_an_ascending_chain():
 
 @pytest.mark.parametrize("H,G,hd,ps,vis,span", [(4, 2, 16, 4, "full", 0), (6, 3, 48, 8, "window", 70), (8, 2, 128, 64, "chunk", 128),
                                                 (3, 1, 64, 32, "window", 1), (4, 4, 128, 64, "window", 300)])
-def test_attention_over_tiles_of_64_keys(H, G, hd, ps, vis, span):
+def test_attention_over_tiles_of_32_keys(H, G, hd, ps, vis, span):
     lens = [330, 64, 1]
     queries = [(0, 329), (0, 63), (0, 64), (0, 127), (0, 128), (0, 255), (0, 256), (0, 300), (1, 63), (1, 0), (2, 0)]
     kv = PagedKV(lens, G, hd, ps, torch.float32)
