@@ -216,22 +216,31 @@ extern "C" int spite_gemm_skinny(const void* X, int ldx, const void* W, long w_g
     SP_REQUIRE(!w_tiled || (K % 32 == 0 && N % 16 == 0), "gemm_skinny: operand order needs K=%d a multiple of 32 and N=%d of 16", K, N);
     if (M == 0) return 0;
 #define SP_ARGS X, ldx, W, w_group_stride, Y, y_dtype, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, w_tiled, live_groups, st
-    // measured on MI355X (GB/s of W at Llama 4 Scout's shapes): one row tile per workgroup for
-    // the experts' grouped stream, two for the dense projections, four for the output matrix
+    // Measured on an MI355X, launches in a row over weights that the caches do not hold.  Up to 16 rows the time is the
+    // stream of W, so what counts is workgroups enough to keep it busy, and no more of the fixed part of each than that
+    // takes: 16 rows of W a workgroup (variant 6) where 32 (variant 8) would leave half of the compute units without one
+    // (2,048 x 2,048: 4.4 against 5.1 us, 2 groups of 2,048 x 3,072: 7.0 against 8.7) and for the experts' plain products,
+    // 32 where there are enough (5,120 x 5,120: 10.6 against 12.5, 2 groups of 2 x 3,072 x 2,048 gated: 10.7 against
+    // 11.8); for the output matrix more columns of X or longer blocks.
     if (variant == 0) {
-        // (with one or two tokens only a few groups have rows at all: more rows of W a workgroup)
         if (max_rows <= 16) {
-            if (offsets) variant = glu ? 8 : (max_rows <= 2 ? 7 : 6);
+            const long groups = !offsets ? 1 : (live_groups > 0 && live_groups < n_groups ? live_groups : n_groups);
+            const bool few = (long)((N + 31) / 32) * (groups < M ? groups : M) < sp_cu_count() / 2;
+            if (offsets) variant = glu && !few ? 8 : 6;
             else if ((size_t)N * K >= ((size_t)1 << 28)) variant = max_rows <= 8 ? 4 : 7;
-            else variant = 8;
+            else variant = few ? 6 : 8;
         }
-        else if (max_rows <= 32) variant = !offsets && (size_t)N * K >= ((size_t)1 << 28) ? 10 : 2;
+        // (the output matrix's stream outweighs the second read of its rows by two row tiles: 59 against 71 us at
+        // 32 rows of 32,768 x 5,120)
+        else if (max_rows <= 32) variant = !offsets && (size_t)N * K >= ((size_t)1 << 27) ? 10 : 2;
         // (groups of experts at 33 to 64 tokens hold a few rows each, only the shared one all:
         // 32 columns a workgroup and a second row tile for that group beat 64 columns for all)
         else if (offsets) variant = glu ? 2 : 10;
         // (a plain product's time grows with the tokens, whose rows every workgroup reads from
         // L2 beside its rows of W: from about 50 tokens on, 64 rows of W a workgroup with two row
-        // tiles of 32 columns beat 32 rows of W with all 64 columns)
+        // tiles of 32 columns beat 32 rows of W with all 64 columns; where 64 rows of W would leave
+        // the chip half empty, 32 with two row tiles: 3,072 x 2,048 8.4 against 11.1 us)
+        else if ((N + 63) / 64 * 2 < sp_cu_count() / 2) variant = 2;
         else variant = max_rows > 48 ? 10 : 9;
     }
     switch (variant) {
