@@ -299,13 +299,20 @@ void attn_latent_join_kernel(const float* __restrict__ part, bf16* __restrict__ 
     if (lane == 0) red[4 + wave] = L;
     __syncthreads();
     const float inv = 1.0f / fmaxf(red[4] + red[5] + red[6] + red[7], 1e-30f);
-    for (int c = tid; c < R; c += 256) {
-        float acc = 0.f;
+    // (a split without keys left zeros and the weight 0: its record is read like the others', so that the loads follow
+    // each other without waiting; two columns a thread, R is a multiple of 8)
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    for (int c = tid * 2; c < R; c += 512) {
+        f32x2 acc = {0.f, 0.f};
+#pragma unroll 8
         for (int s = 0; s < n_splits; ++s) {
-            const float w = wsh[s];
-            if (w != 0.f) acc += w * rec[(size_t)s * (R + 2) + c];
+            const f32x2 v = *(const f32x2*)(rec + (size_t)s * (R + 2) + c);
+            acc[0] += wsh[s] * v[0];
+            acc[1] += wsh[s] * v[1];
         }
-        out[row * R + c] = (bf16)(acc * inv);
+        bf16* o = out + row * R + c;
+        o[0] = (bf16)(acc[0] * inv);
+        o[1] = (bf16)(acc[1] * inv);
     }
 }
 

@@ -835,12 +835,17 @@ def latent_workgroups(counts, cu_seqlens, H):
 
 def latent_splits(n_wg: int, longest: int) -> int:
     """Into how many workgroups the keys of every work item are best dealt, for ``n_wg`` items whose
-    queries read at most ``longest`` keys: about one workgroup a compute unit, each with at least eight
-    blocks of 32 keys (a workgroup's record is as large as what it reads of two or three such blocks)."""
+    queries read at most ``longest`` keys.  A block of 32 keys takes a workgroup 4.6 us and its start
+    about 8, the records of a split as much as two blocks' rows: shares of two blocks, fewer than eight
+    splits only where there are fewer blocks, at most 32 splits and about one workgroup a compute unit.
+    (40 heads on an MI355X, 1,024 keys: 1 to 8 items 50 us with four splits, 31 to 35 with 16; 4,096
+    keys: 57 to 62 us with 16, 49 to 56 with 32; 16 items 64 with 16, 85 with 32.)"""
     if n_wg <= 0:
         return 1
+    blocks = -(-longest // 32)
+    share = min(max(-(-blocks // 2), min(blocks, 8)), 32, max(1, cu_count() // n_wg))
     # (no fewer than keep a share within the 4,096 keys whose cache rows the staging waves look up ahead)
-    return max(1, min(-(-cu_count() // n_wg), -(-longest // 256), 256), min(-(-longest // 4096), 256))
+    return max(1, share, min(-(-longest // 4096), 256))
 
 
 def attn_latent_mfma(q, kv_pages, out, positions, seq_of_token, block_table, wg, n_wg, max_rows, T, H, Dk, R, vis, span, scale,
