@@ -1,7 +1,7 @@
 // fp32 matrix product Y = A . W^T on the matrix units (v_mfma_f32_16x16x4_f32: fp32 operands, fp32 FMAs, no narrower
 // step anywhere), the true 32-bit path of every projection whose rows can be read 16 bytes at a time.
 //
-// The order of every sum depends on K alone.  k is cut into eight runs of `seg` (K / 8 rounded up to 32); inside a
+// The order of every sum depends on K alone.  k is cut into eight runs of `seg` (K / 8 rounded up to 64); inside a
 // run the products are added in steps of 16 k, four MFMAs a step (MFMA e takes k0 + 4q + e of its four rows of lanes
 // q); the runs' sums are then added in their order, ((0 + s0) + s1) + ... + s7.  Both kernels below keep this order, so
 // a row has the same bits whether it comes alone or among many, and shorter chains round less than one ascending
@@ -29,7 +29,7 @@ __device__ __forceinline__ void f32_step(f32x4& acc, f32x4 w, f32x4 x) {
     acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[3], x[3], acc, 0, 0, 0);
 }
 
-__device__ __forceinline__ int f32_seg(int K) { return (K + 255) / 256 * 32; }
+__device__ __forceinline__ int f32_seg(int K) { return (K + 511) / 512 * 64; }
 
 // A lane of a result tile holds W rows n0 + 4q .. + 3 of X row `s`.
 __device__ __forceinline__ void f32_store(float* __restrict__ Y, size_t row, int ldy, int n, int N, f32x4 v, bool vec) {
@@ -88,7 +88,7 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
             const int k = k0 + u * 16 + q * 4;
             const bool in = k < k_hi;                  // K is a multiple of 4, a run's end of 4
 #pragma unroll
-            for (int b = 0; b < NB; ++b) w[u][b] = in ? __builtin_nontemporal_load((const f32x4*)(wp[b] + k)) : f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int b = 0; b < NB; ++b) w[u][b] = in ? *(const f32x4*)(wp[b] + k) : f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
             for (int m = 0; m < MT; ++m) x[u][m] = in ? *(const f32x4*)(xp[m] + k) : f32x4{0.f, 0.f, 0.f, 0.f};
         }
@@ -123,7 +123,7 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
 }
 
 #define F32_TM 64                 // rows of X a workgroup
-#define F32_TK 32                 // k a step through LDS
+#define F32_TK 64                 // k a step through LDS
 #define F32_LD (F32_TK + 4)       // LDS row: 16 bytes more than a step, so that 16 rows' reads spread over the banks
 
 // The loop over k for a tile whose first LIVE groups of 16 rows hold rows (an expert's last tile is seldom full).  Loads
@@ -133,57 +133,67 @@ template <int NB, int LIVE>
 __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp, const float* const* xp, const float* sc, int K,
                                               int seg, int lr, int lk, int r, int q, f32x4 (&tot)[4][NB]) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    f32x4 acc[LIVE][NB], w[2][NB], xv[2];
+    constexpr int U = F32_TK / 16, XL = F32_TM * F32_TK / 1024;      // steps of 16 k, 16-byte pieces of X a thread
+    f32x4 acc[LIVE][NB], w0[U][NB], w1[U][NB], w2[U][NB], xv[XL];
 #pragma unroll
     for (int m = 0; m < LIVE; ++m)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[m][b] = zero;
     // k past the end: the last four's address, and zeros instead
-#define F32_FETCH(k0) do { \
-    _Pragma("unroll") for (int u = 0; u < 2; ++u) { \
+#define F32_W(w, k0) do { \
+    _Pragma("unroll") for (int u = 0; u < U; ++u) { \
         const int k = (k0) + u * 16 + q * 4, kc = k < K ? k : K - 4; \
-        _Pragma("unroll") for (int b = 0; b < NB; ++b) w[u][b] = *(const f32x4*)(wp[b] + kc); } \
+        _Pragma("unroll") for (int b = 0; b < NB; ++b) w[u][b] = *(const f32x4*)(wp[b] + kc); } } while (0)
+#define F32_X(k0) do { \
     const int kx = (k0) + lk < K ? (k0) + lk : K - 4; \
-    _Pragma("unroll") for (int i = 0; i < 2; ++i) xv[i] = *(const f32x4*)(xp[i] + kx); } while (0)
+    _Pragma("unroll") for (int i = 0; i < XL; ++i) xv[i] = *(const f32x4*)(xp[i] + kx); } while (0)
 #define F32_PUT(buf, k0) do { \
-    _Pragma("unroll") for (int i = 0; i < 2; ++i) \
-        *(f32x4*)(xs + (buf) * (F32_TM * F32_LD) + (lr + i * 32) * F32_LD + lk) = (k0) + lk < K ? xv[i] * sc[i] : zero; } while (0)
-    F32_FETCH(0);
+    _Pragma("unroll") for (int i = 0; i < XL; ++i) \
+        *(f32x4*)(xs + (buf) * (F32_TM * F32_LD) + (lr + i * (F32_TM / XL)) * F32_LD + lk) = (k0) + lk < K ? xv[i] * sc[i] : zero; } while (0)
+    // Step k0 multiplies the set wa with the rows in buffer `buf`; the rows of the next step and W of the step after the
+    // next are asked for first, in this order: waiting for the rows leaves W on its way.
+#define F32_STEP(wa, wc) do { \
+    __syncthreads();                                   /* this step's rows are in LDS, the other buffer is free */ \
+    if (k0 == flush) { \
+        _Pragma("unroll") for (int m = 0; m < LIVE; ++m) \
+        _Pragma("unroll") for (int b = 0; b < NB; ++b) { tot[m][b] += acc[m][b]; acc[m][b] = zero; } \
+        flush += seg; } \
+    F32_X(k0 + F32_TK); \
+    F32_W(wc, k0 + 2 * F32_TK); \
+    __builtin_amdgcn_sched_barrier(0); \
+    const float* xb = xs + buf * (F32_TM * F32_LD); \
+    _Pragma("unroll") for (int u = 0; u < U; ++u) { \
+        if (k0 + u * 16 + 16 > K) { \
+            const bool in = k0 + u * 16 + q * 4 < K; \
+            _Pragma("unroll") for (int b = 0; b < NB; ++b) wa[u][b] = in ? wa[u][b] : zero; } \
+        f32x4 x[LIVE]; \
+        _Pragma("unroll") for (int m = 0; m < LIVE; ++m) x[m] = *(const f32x4*)(xb + (m * 16 + r) * F32_LD + u * 16 + q * 4); \
+        _Pragma("unroll") for (int e = 0; e < 4; ++e) \
+        _Pragma("unroll") for (int m = 0; m < LIVE; ++m) \
+        _Pragma("unroll") for (int b = 0; b < NB; ++b) \
+            acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[u][b][e], x[m][e], acc[m][b], 0, 0, 0); } \
+    F32_PUT(buf ^ 1, k0 + F32_TK); \
+    buf ^= 1; \
+    k0 += F32_TK; } while (0)
+    F32_X(0);
+    F32_W(w0, 0);
+    F32_W(w1, F32_TK);
     F32_PUT(0, 0);
-    int buf = 0;
-    for (int run = 0; run < K; run += seg) {
-        const int end = run + seg < K ? run + seg : K;
-        for (int k0 = run; k0 < end; k0 += F32_TK, buf ^= 1) {
-            __syncthreads();                           // this step's rows are in LDS, the other buffer is free
-            f32x4 wc[2][NB];
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int b = 0; b < NB; ++b) wc[u][b] = k0 + u * 16 + q * 4 < K ? w[u][b] : zero;
-            F32_FETCH(k0 + F32_TK);
-            f32x4 x[2][LIVE];
-            const float* xb = xs + buf * (F32_TM * F32_LD);
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int m = 0; m < LIVE; ++m) x[u][m] = *(const f32x4*)(xb + (m * 16 + r) * F32_LD + u * 16 + q * 4);
-#pragma unroll
-            for (int u = 0; u < 2; ++u)
-#pragma unroll
-                for (int e = 0; e < 4; ++e)
-#pragma unroll
-                    for (int m = 0; m < LIVE; ++m)
-#pragma unroll
-                        for (int b = 0; b < NB; ++b)
-                            acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wc[u][b][e], x[u][m][e], acc[m][b], 0, 0, 0);
-            F32_PUT(buf ^ 1, k0 + F32_TK);
-        }
-#pragma unroll
-        for (int m = 0; m < LIVE; ++m)
-#pragma unroll
-            for (int b = 0; b < NB; ++b) { tot[m][b] += acc[m][b]; acc[m][b] = zero; }
+    int buf = 0, k0 = 0, flush = seg;
+    while (k0 + 2 * F32_TK < K) {
+        F32_STEP(w0, w2);
+        F32_STEP(w1, w0);
+        F32_STEP(w2, w1);
     }
-#undef F32_FETCH
+    if (k0 < K) F32_STEP(w0, w2);
+    if (k0 < K) F32_STEP(w1, w0);
+#pragma unroll
+    for (int m = 0; m < LIVE; ++m)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) tot[m][b] += acc[m][b];
+#undef F32_STEP
+#undef F32_W
+#undef F32_X
 #undef F32_PUT
 }
 
@@ -209,13 +219,14 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
     const float* wp[NB];
     wp[0] = Wg + (size_t)wn * K;
     if (GLU) wp[NB - 1] = Wg + (size_t)(N + wn) * K;
-    // the loader: a thread brings 4 k of rows lr and lr + 32
-    const int lk = (threadIdx.x & 7) * 4, lr = threadIdx.x >> 3;
-    const float* xp[2];
-    float sc[2];
+    // the loader: a thread brings 4 k of every XL-th part of the rows
+    constexpr int XL = F32_TM * F32_TK / 1024, PIECES = F32_TK / 4;
+    const int lk = (threadIdx.x % PIECES) * 4, lr = threadIdx.x / PIECES;
+    const float* xp[XL];
+    float sc[XL];
 #pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int s = row0 + lr + i * 32, ss = s < row_end ? s : row0;
+    for (int i = 0; i < XL; ++i) {
+        const int s = row0 + lr + i * (F32_TM / XL), ss = s < row_end ? s : row0;
         xp[i] = A + (size_t)(a_rows ? a_rows[ss] : ss) * lda;
         sc[i] = a_scale ? a_scale[ss] : 1.0f;
     }
