@@ -584,9 +584,8 @@ extern "C" int spite_router_top1(const float* x, const float* wr, int* expert, f
 // From expert[t], weight[t] build the row list that the grouped products walk:
 //   slots [0,T): tokens in order of expert (stable), src[s] = token, scale[s] = its weight,
 //                dst[s] = token;
-//   slots [T,2T) (if shared): src = dst-T = token, scale 1, dst[s] = T + token  (the group E
-//                that every token visits);
-//   offsets[g] = first slot of group g, g in [0, E+1] (+1 with the shared group).
+//   the slots behind them, `shared` groups E, E + 1, ... that every token visits: src = token, scale 1, dst[s] = s;
+//   offsets[g] = first slot of group g, g in [0, E + shared + 1).
 // With `logits` ([T, E] fp32) the kernels make the router's choice themselves and write it to
 // expert[] and weight[]: the largest logit, the lowest index among equals, weight =
 // 1/(1+exp(-logit)).
@@ -634,7 +633,11 @@ __global__ void moe_plan_kernel(int* __restrict__ expert, float* __restrict__ we
             rank += (ej < me) || (ej == me && j < t);
         }
         src[rank] = t / fan; scale[rank] = wt; dst[rank] = t;
-        if (shared) { src[T + t] = t; scale[T + t] = 1.0f; dst[T + t] = T + t; }
+        const int tokens = T / fan;
+        for (int g = 0; g < shared && t < tokens; ++g) {
+            const int j = T + g * tokens + t;
+            src[j] = t; scale[j] = 1.0f; dst[j] = j;
+        }
     }
     if (blockIdx.x == 0) {
         for (int g = threadIdx.x; g <= E; g += blockDim.x) {
@@ -642,7 +645,7 @@ __global__ void moe_plan_kernel(int* __restrict__ expert, float* __restrict__ we
             for (int j = 0; j < T; ++j) c += e_of[j] < g;
             offsets[g] = c;
         }
-        if (shared && threadIdx.x == 0) offsets[E + 1] = 2 * T;
+        if (threadIdx.x < shared) offsets[E + 1 + threadIdx.x] = T + (threadIdx.x + 1) * (T / fan);
     }
 }
 
@@ -692,11 +695,15 @@ void moe_plan_hist_kernel(int* __restrict__ expert, float* __restrict__ weight,
         int rank = first[me] + before[me];
         for (int j = 0; j < (int)threadIdx.x; ++j) rank += mine[j] == me;
         src[rank] = t / fan; scale[rank] = wt; dst[rank] = t;
-        if (shared) { src[T + t] = t; scale[T + t] = 1.0f; dst[T + t] = T + t; }
+        const int tokens = T / fan;
+        for (int g = 0; g < shared && t < tokens; ++g) {
+            const int j = T + g * tokens + t;
+            src[j] = t; scale[j] = 1.0f; dst[j] = j;
+        }
     }
     if (blockIdx.x == 0) {
         for (int g = threadIdx.x; g <= E; g += 256) offsets[g] = first[g];
-        if (shared && threadIdx.x == 0) offsets[E + 1] = 2 * T;
+        if (threadIdx.x < shared) offsets[E + 1 + threadIdx.x] = T + (threadIdx.x + 1) * (T / fan);
     }
 }
 
@@ -707,7 +714,8 @@ void moe_plan_hist_kernel(int* __restrict__ expert, float* __restrict__ weight,
 extern "C" int spite_moe_plan(int* expert, float* weight, const float* logits, int* src, float* scale, int* dst,
                               int* offsets, int T, int E, int shared, int fan, hipStream_t st) {
     SP_REQUIRE(T >= 0 && E > 0 && E < 65535, "moe_plan: bad sizes T=%d E=%d", T, E);
-    SP_REQUIRE(fan >= 1 && (fan == 1 || (!shared && !logits)), "moe_plan: a fan of %d goes with given experts and no shared group", fan);
+    SP_REQUIRE(fan >= 1 && T % fan == 0 && (fan == 1 || !logits), "moe_plan: a fan of %d goes with given experts, T=%d a multiple of it", fan, T);
+    SP_REQUIRE(shared >= 0 && shared <= 64, "moe_plan: %d shared groups", shared);
     SP_REQUIRE(T <= ((T > 256 && E <= PLAN_MAX_E) ? (1 << 22) : 32768), "moe_plan: %d entries in one step are too many", T);
     const int grid = T > 0 ? (T + 255) / 256 : 1;
     if (T > 256 && E <= PLAN_MAX_E)

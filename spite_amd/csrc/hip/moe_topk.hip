@@ -12,24 +12,22 @@
 // With `n_groups` > 1 the experts form equal groups of neighbours and only those of the `keep_groups` groups whose
 // largest choice value is largest can be taken (the lowest group among equals).  The logits' rows may lie `ld` apart.
 // Outputs expert[t*top + j] and weight[t*top + j] in the order of choice:
-// "virtual tokens" t*top + j that the expert plan (moe_plan with its fan) sorts by expert.
+// "virtual tokens" t*top + j that the expert plan (moe_plan with its fan) sorts by expert.  router_plan: both at once.
 // moe_combine: out[t] = sum_j weight[t*top + j] * y[t*top + j] (+ extra[t]) in fp32, j in order (no weights: all 1);
-// with `gate` the extra row is multiplied by sigmoid(gate[t*ldg]).
+// the extra row may come in `n_extra` parts, T rows apart, that are added first; with `gate` it is multiplied by
+// sigmoid(gate[t*ldg]).
 // gated_rows: g[t] = gelu_tanh(a[t]) * table[ids[t]][col0 .. col0 + n): a gate on a per-token row
 // of a table (a second, small embedding that a layer mixes into the stream).
 #include "common.h"
 
 #define TOPK_MAX_PER_LANE 8      // up to 512 experts
 
-// NU: experts a lane, so that 64 * NU >= E.
+// One token's choice by one wave: lane j < min(top, 64) gets the j-th taken expert and its weight, and everything is
+// written to expert[] and weight[].  NU: experts a lane, so that 64 * NU >= E.
 template <int NU>
-__global__ __launch_bounds__(256)
-void router_topk_kernel(const float* __restrict__ logits, const float* __restrict__ bias, int* __restrict__ expert,
-                        float* __restrict__ weight, int T, int E, int ld, int top, int renorm, int mode,
-                        int n_groups, int keep_groups) {
-    const int lane = threadIdx.x & 63;
-    const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
-    if (t >= T) return;
+__device__ __forceinline__ int topk_of_token(const float* __restrict__ logits, const float* __restrict__ bias, int* __restrict__ expert,
+                                             float* __restrict__ weight, int t, int lane, int E, int ld, int top, int renorm, int mode,
+                                             int n_groups, int keep_groups) {
     float s[NU], c[NU];
 #pragma unroll
     for (int u = 0; u < NU; ++u) {
@@ -118,15 +116,62 @@ void router_topk_kernel(const float* __restrict__ logits, const float* __restric
         const float inv = 1.0f / sum;
         if (lane < top && lane < 64) { expert[(size_t)t * top + lane] = mine_e; weight[(size_t)t * top + lane] = expf(mine_w - top_z) * inv; }
         if (top > 64 && lane == 0) for (int j = 64; j < top; ++j) weight[(size_t)t * top + j] = expf(weight[(size_t)t * top + j] - top_z) * inv;
-        return;
+        return mine_e;
     }
     const float inv = renorm ? 1.0f / (sum + 1e-20f) : 1.0f;
     if (lane < top && lane < 64) { expert[(size_t)t * top + lane] = mine_e; weight[(size_t)t * top + lane] = mine_w * inv; }
     if (renorm && top > 64 && lane == 0) for (int j = 64; j < top; ++j) weight[(size_t)t * top + j] *= inv;
+    return mine_e;
 }
 
-extern "C" int spite_router_topk(const float* logits, const float* bias, int* expert, float* weight, int T, int E, int ld, int top,
-                                 int renorm, int mode, int n_groups, int keep_groups, hipStream_t st) {
+template <int NU>
+__global__ __launch_bounds__(256)
+void router_topk_kernel(const float* __restrict__ logits, const float* __restrict__ bias, int* __restrict__ expert,
+                        float* __restrict__ weight, int T, int E, int ld, int top, int renorm, int mode,
+                        int n_groups, int keep_groups) {
+    const int t = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (t >= T) return;
+    topk_of_token<NU>(logits, bias, expert, weight, t, threadIdx.x & 63, E, ld, top, renorm, mode, n_groups, keep_groups);
+}
+
+// The choice and the row list of the grouped products (moe_plan with a fan of `top` and `shared` groups that every token
+// visits) of a step of few tokens by one workgroup: two kernels of 4.5 us each, of which next to nothing is work, become
+// one.  The entries' experts stay in LDS in between; ranks are counted as moe_plan_kernel counts them.
+#define RP_NT 512
+#define RP_MAX 512       // entries at most: each is ranked by a thread that looks at all of them
+template <int NU>
+__global__ __launch_bounds__(RP_NT)
+void router_plan_kernel(const float* __restrict__ logits, const float* __restrict__ bias, int* __restrict__ expert,
+                        float* __restrict__ weight, int T, int E, int ld, int top, int renorm, int mode, int n_groups,
+                        int keep_groups, int* __restrict__ src, float* __restrict__ scale, int* __restrict__ dst,
+                        int* __restrict__ offsets, int shared) {
+    __shared__ unsigned short e_of[RP_MAX];
+    const int lane = threadIdx.x & 63, n = T * top;
+    for (int t = threadIdx.x >> 6; t < T; t += RP_NT / 64) {
+        const int e = topk_of_token<NU>(logits, bias, expert, weight, t, lane, E, ld, top, renorm, mode, n_groups, keep_groups);
+        if (lane < top) e_of[t * top + lane] = (unsigned short)e;
+    }
+    __syncthreads();                                        // (the weights of this workgroup's waves are visible to it, too)
+    const int i = threadIdx.x;
+    if (i < n) {
+        const int me = e_of[i];
+        int rank = 0;
+        for (int j = 0; j < n; ++j) {
+            const int ej = e_of[j];
+            rank += (ej < me) || (ej == me && j < i);
+        }
+        src[rank] = i / top; scale[rank] = weight[i]; dst[rank] = i;
+    }
+    for (int j = i; j < shared * T; j += RP_NT) { src[n + j] = j % T; scale[n + j] = 1.0f; dst[n + j] = n + j; }
+    for (int g = i; g <= E + shared; g += RP_NT) {
+        int c = 0;
+        if (g <= E) for (int j = 0; j < n; ++j) c += e_of[j] < g;
+        else c = n + (g - E) * T;
+        offsets[g] = c;
+    }
+}
+
+static int topk_check(int T, int E, int ld, int top, int mode, int n_groups, int keep_groups) {
     SP_REQUIRE(mode >= 0 && mode <= 3, "router_topk: scoring %d", mode);
     SP_REQUIRE(ld >= E, "router_topk: rows of %d logits for %d experts", ld, E);
     SP_REQUIRE(n_groups >= 1 && E > 0 && E % n_groups == 0 && keep_groups >= 1 && keep_groups <= n_groups, "router_topk: %d of %d groups of %d experts",
@@ -134,14 +179,40 @@ extern "C" int spite_router_topk(const float* logits, const float* bias, int* ex
     SP_REQUIRE(top <= keep_groups * (E / n_groups), "router_topk: %d experts out of %d groups of %d", top, keep_groups, E / n_groups);
     SP_REQUIRE(T >= 0 && E > 0 && E <= 64 * TOPK_MAX_PER_LANE, "router_topk: %d experts, at most %d", E, 64 * TOPK_MAX_PER_LANE);
     SP_REQUIRE(top > 0 && top <= E, "router_topk: %d of %d experts", top, E);
+    return 0;
+}
+#define SP_BY_EXPERTS(GO) do { if (E <= 64) GO(1); else if (E <= 128) GO(2); else if (E <= 256) GO(4); else GO(TOPK_MAX_PER_LANE); } while (0)
+
+extern "C" int spite_router_topk(const float* logits, const float* bias, int* expert, float* weight, int T, int E, int ld, int top,
+                                 int renorm, int mode, int n_groups, int keep_groups, hipStream_t st) {
+    if (int rc = topk_check(T, E, ld, top, mode, n_groups, keep_groups)) return rc;
     if (T == 0) return 0;
 #define SP_RT(NU) router_topk_kernel<NU><<<(T + 3) / 4, 256, 0, st>>>(logits, bias, expert, weight, T, E, ld, top, renorm, mode, n_groups, keep_groups)
-    if (E <= 64) SP_RT(1);
-    else if (E <= 128) SP_RT(2);
-    else if (E <= 256) SP_RT(4);
-    else SP_RT(TOPK_MAX_PER_LANE);
+    SP_BY_EXPERTS(SP_RT);
 #undef SP_RT
     SP_LAUNCH_CHECK("router_topk");
+    return 0;
+}
+
+extern "C" int spite_moe_plan(int* expert, float* weight, const float* logits, int* src, float* scale, int* dst,
+                              int* offsets, int T, int E, int shared, int fan, hipStream_t st);
+
+// router_topk, then moe_plan over its T * top entries with `shared` groups of T rows behind the experts'; in one launch
+// where the entries fit a workgroup.
+extern "C" int spite_router_plan(const float* logits, const float* bias, int* expert, float* weight, int T, int E, int ld, int top,
+                                 int renorm, int mode, int n_groups, int keep_groups, int* src, float* scale, int* dst,
+                                 int* offsets, int shared, hipStream_t st) {
+    if (int rc = topk_check(T, E, ld, top, mode, n_groups, keep_groups)) return rc;
+    SP_REQUIRE(shared >= 0 && shared <= 64, "router_plan: %d shared groups", shared);
+    if (T == 0 || top > 64 || (long)T * top > RP_MAX) {
+        if (int rc = spite_router_topk(logits, bias, expert, weight, T, E, ld, top, renorm, mode, n_groups, keep_groups, st)) return rc;
+        return spite_moe_plan(expert, weight, nullptr, src, scale, dst, offsets, T * top, E, shared, top, st);
+    }
+#define SP_RP(NU) router_plan_kernel<NU><<<1, RP_NT, 0, st>>>(logits, bias, expert, weight, T, E, ld, top, renorm, mode, n_groups, \
+                                                              keep_groups, src, scale, dst, offsets, shared)
+    SP_BY_EXPERTS(SP_RP);
+#undef SP_RP
+    SP_LAUNCH_CHECK("router_plan");
     return 0;
 }
 
@@ -150,7 +221,7 @@ extern "C" int spite_router_topk(const float* logits, const float* bias, int* ex
 template <int VEC>
 __global__ __launch_bounds__(256)
 void moe_combine_kernel(const float* __restrict__ y, const float* __restrict__ weight, const float* __restrict__ extra,
-                        const float* __restrict__ gate, int ldg, float* __restrict__ out, int T, int d, int top) {
+                        const float* __restrict__ gate, int ldg, float* __restrict__ out, int T, int d, int top, int n_extra) {
     typedef float vec __attribute__((ext_vector_type(VEC)));
     const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
     const int dv = d / VEC;
@@ -166,7 +237,8 @@ void moe_combine_kernel(const float* __restrict__ y, const float* __restrict__ w
         for (int e = 0; e < VEC; ++e) acc[e] = fmaf(w, v[e], acc[e]);
     }
     if (extra) {
-        const vec x = *(const vec*)(extra + t * d + c);
+        vec x = *(const vec*)(extra + t * d + c);
+        for (int j = 1; j < n_extra; ++j) x += *(const vec*)(extra + ((size_t)j * T + t) * d + c);
         const float g = gate ? 1.0f / (1.0f + expf(-gate[t * ldg])) : 1.0f;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) acc[e] += g * x[e];
@@ -175,8 +247,8 @@ void moe_combine_kernel(const float* __restrict__ y, const float* __restrict__ w
 }
 
 extern "C" int spite_moe_combine(const float* y, const float* weight, const float* extra, const float* gate, int ldg, float* out,
-                                 int T, int d, int top, hipStream_t st) {
-    SP_REQUIRE(T >= 0 && d > 0 && top > 0, "moe_combine: bad sizes T=%d d=%d top=%d", T, d, top);
+                                 int T, int d, int top, int n_extra, hipStream_t st) {
+    SP_REQUIRE(T >= 0 && d > 0 && top > 0 && n_extra >= 1, "moe_combine: bad sizes T=%d d=%d top=%d, %d extra rows", T, d, top, n_extra);
     SP_REQUIRE(!gate || (extra && ldg >= 1), "moe_combine: a gate without the row that it gates");
     if (T == 0) return 0;
     auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
@@ -184,8 +256,8 @@ extern "C" int spite_moe_combine(const float* y, const float* weight, const floa
     const size_t n = (size_t)T * (v4 ? d / 4 : d);
     SP_REQUIRE((n + 255) / 256 < (1u << 31), "moe_combine: too many elements");
     const unsigned grid = (unsigned)((n + 255) / 256);
-    if (v4) moe_combine_kernel<4><<<grid, 256, 0, st>>>(y, weight, extra, gate, ldg, out, T, d, top);
-    else moe_combine_kernel<1><<<grid, 256, 0, st>>>(y, weight, extra, gate, ldg, out, T, d, top);
+    if (v4) moe_combine_kernel<4><<<grid, 256, 0, st>>>(y, weight, extra, gate, ldg, out, T, d, top, n_extra);
+    else moe_combine_kernel<1><<<grid, 256, 0, st>>>(y, weight, extra, gate, ldg, out, T, d, top, n_extra);
     SP_LAUNCH_CHECK("moe_combine");
     return 0;
 }

@@ -75,7 +75,8 @@ def lib():
             "spite_attn_latent_generic": [P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, P],
             "spite_attn_latent_mfma": [P, P, P, P, P, P, I, P, I, I, I, I, I, I, I, I, F, P, I, I, P],
             "spite_router_topk": [P, P, P, P, I, I, I, I, I, I, I, I, P],
-            "spite_moe_combine": [P, P, P, P, I, P, I, I, I, P],
+            "spite_router_plan": [P, P, P, P, I, I, I, I, I, I, I, I, P, P, P, P, I, P],
+            "spite_moe_combine": [P, P, P, P, I, P, I, I, I, I, P],
             "spite_gated_rows": [P, I, P, P, I, I, I, P, I, I, P],
             "spite_qkv_prepare": [P, I, I, P, P, P, F, P, P, P, P, P, P, I, F, P, I, I, I, I, I, I, I, I, I, I, I, I, F, I, I, P, I, F, P],
             "spite_attn_wide": [P, P, P, P, I, I, P, P, P, I, I, I, I, I, I, I, I, I, I, F, I, I, P, P, I, P, I, P],
@@ -285,9 +286,12 @@ def moe_plan(expert, weight, src, scale, dst, offsets, T, E, shared, logits=None
     """Row list of the grouped products from the router's choice (see the kernel).  With
     ``logits`` ([T, E] fp32) the choice is made here and written to ``expert`` and ``weight``.
     ``fan`` > 1: the T entries are ``fan`` choices in a row for each of T / fan tokens; ``src`` names
-    the token (entry // fan), ``dst`` the entry."""
-    n = 2 * T if shared else T
-    if src.numel() < n or scale.numel() < n or dst.numel() < n or offsets.numel() < E + 1 + int(bool(shared)):
+    the token (entry // fan), ``dst`` the entry.  ``shared``: so many groups behind the experts' that every
+    token visits."""
+    if T % int(fan):
+        raise KernelError(f"moe_plan: {T} entries of {fan} a token")
+    n = T + int(shared) * (T // int(fan))
+    if src.numel() < n or scale.numel() < n or dst.numel() < n or offsets.numel() < E + 1 + int(shared):
         raise KernelError("moe_plan: output arrays too small")
     if expert.numel() < T or weight.numel() < T:
         raise KernelError("moe_plan: inputs too small")
@@ -296,7 +300,7 @@ def moe_plan(expert, weight, src, scale, dst, offsets, T, E, shared, logits=None
     _check(lib().spite_moe_plan(_ptr(expert, "expert", torch.int32), _ptr(weight, "weight", torch.float32),
                                 _ptr(logits, "logits", torch.float32, True), _ptr(src, "src", torch.int32), _ptr(scale, "scale", torch.float32),
                                 _ptr(dst, "dst", torch.int32), _ptr(offsets, "offsets", torch.int32),
-                                T, E, int(bool(shared)), int(fan), _stream()), "moe_plan")
+                                T, E, int(shared), int(fan), _stream()), "moe_plan")
 
 
 def convert(src, dst):
@@ -771,6 +775,14 @@ def router_topk(logits, bias, expert, weight, top, renorm=False, scoring="sigmoi
     taken experts' logits (``softmax_taken_biased``: over the taken experts' z + bias, the bias being part of the logits); ``softmax``: scores softmax(z) over all experts, the rest as with sigmoid.  ``groups`` =
     (count, keep): only experts of the ``keep`` groups (``count`` equal groups of neighbours) whose largest choice
     value is largest can be taken.  ``n_experts``: the logits are the first so many columns of the rows."""
+    T, E, count, keep = _topk_sizes(logits, bias, expert, weight, top, scoring, groups, n_experts)
+    _check(lib().spite_router_topk(_ptr(logits, "logits", torch.float32), _ptr(bias, "bias", torch.float32, True),
+                                   _ptr(expert, "expert", torch.int32), _ptr(weight, "weight", torch.float32),
+                                   T, E, logits.shape[1], int(top), int(bool(renorm)), ROUTER_SCORING[scoring], count, keep, _stream()),
+           "router_topk")
+
+
+def _topk_sizes(logits, bias, expert, weight, top, scoring, groups, n_experts):
     T, E = logits.shape[0], int(n_experts or logits.shape[1])
     count, keep = (1, 1) if groups is None else (int(groups[0]), int(groups[1]))
     if E > logits.shape[1]:
@@ -779,25 +791,38 @@ def router_topk(logits, bias, expert, weight, top, renorm=False, scoring="sigmoi
         raise KernelError(f"router_topk: scoring {scoring!r} (known: {sorted(ROUTER_SCORING)})")
     if expert.numel() < T * top or weight.numel() < T * top or (bias is not None and bias.numel() != E):
         raise KernelError("router_topk: outputs too small or bias of the wrong size")
-    _check(lib().spite_router_topk(_ptr(logits, "logits", torch.float32), _ptr(bias, "bias", torch.float32, True),
+    return T, E, count, keep
+
+
+def router_plan(logits, bias, expert, weight, top, src, scale, dst, offsets, shared=0, renorm=False, scoring="sigmoid", groups=None,
+                n_experts=None):
+    """``router_topk``, and ``moe_plan`` over its T * top entries (``fan`` = top) with ``shared`` groups that every token
+    visits, in one launch for a step of few tokens."""
+    T, E, count, keep = _topk_sizes(logits, bias, expert, weight, top, scoring, groups, n_experts)
+    n = T * (top + int(shared))
+    if src.numel() < n or scale.numel() < n or dst.numel() < n or offsets.numel() < E + 1 + int(shared):
+        raise KernelError("router_plan: output arrays too small")
+    _check(lib().spite_router_plan(_ptr(logits, "logits", torch.float32), _ptr(bias, "bias", torch.float32, True),
                                    _ptr(expert, "expert", torch.int32), _ptr(weight, "weight", torch.float32),
-                                   T, E, logits.shape[1], int(top), int(bool(renorm)), ROUTER_SCORING[scoring], count, keep, _stream()),
-           "router_topk")
+                                   T, E, logits.shape[1], int(top), int(bool(renorm)), ROUTER_SCORING[scoring], count, keep,
+                                   _ptr(src, "src", torch.int32), _ptr(scale, "scale", torch.float32), _ptr(dst, "dst", torch.int32),
+                                   _ptr(offsets, "offsets", torch.int32), int(shared), _stream()), "router_plan")
 
 
-def moe_combine(y, weight, extra, out, T, top, gate=None):
+def moe_combine(y, weight, extra, out, T, top, gate=None, n_extra=1):
     """out[t] = sum_j weight[t*top + j] * y[t*top + j] (+ extra[t]); all fp32; ``weight`` None: every weight 1.
-    ``gate`` (fp32, [T] with any stride): the extra row is multiplied by sigmoid(gate[t])."""
+    ``gate`` (fp32, [T] with any stride): the extra row is multiplied by sigmoid(gate[t]).  ``n_extra``: the extra row
+    comes in so many parts, [n_extra * T, d], that are added."""
     if gate is not None and (gate.dim() != 1 or gate.shape[0] < T or gate.dtype != torch.float32 or not gate.is_cuda or extra is None):
         raise KernelError("moe_combine: a gate is one fp32 number a token for the extra row")
     d = out.shape[-1]
     if y.numel() < T * top * d or (weight is not None and weight.numel() < T * top) or out.numel() < T * d \
-            or (extra is not None and extra.numel() < T * d):
+            or (extra is not None and extra.numel() < n_extra * T * d):
         raise KernelError("moe_combine: arrays too small")
     _check(lib().spite_moe_combine(_ptr(y, "y", torch.float32), _ptr(weight, "weight", torch.float32, True),
                                    _ptr(extra, "extra", torch.float32, True),
                                    gate.data_ptr() if gate is not None else None, gate.stride(0) if gate is not None else 0,
-                                   _ptr(out, "out", torch.float32), T, d, int(top), _stream()), "moe_combine")
+                                   _ptr(out, "out", torch.float32), T, d, int(top), int(n_extra), _stream()), "moe_combine")
 
 
 def gated_rows(a, ids, table, col0, g):

@@ -228,6 +228,11 @@ class MoeTop1Sigmoid(FeedForward):
         return (y[:T], y[T:])
 
 
+# groups that a shared expert may make beside the routed ones: each adds a row of d numbers a token to what the combining
+# kernel reads
+SHARED_GROUPS_MAX = 4
+
+
 @register("ffn", "moe_topk_sigmoid")
 class MoeTopKSigmoid(FeedForward):
     graph_safe = True
@@ -261,6 +266,8 @@ class MoeTopKSigmoid(FeedForward):
         if self.shared_gate and self.Fs is None:
             raise ValueError("moe: a gate on a shared expert that there is not")
         self.w_router = self.bias = self.w_gate_up = self.w_down = self.ws_gate_up = self.ws_down = None
+        # how many groups of the routed experts' width the shared expert makes behind them (0: products of its own)
+        self.shared_groups = 0
 
     def params(self):
         d, F, E = self.d, self.F, self.E
@@ -285,11 +292,21 @@ class MoeTopKSigmoid(FeedForward):
         self.bias = t["correction"].contiguous() if self.score_bias else None
         dts = {t[f"e{e}.{k}"].dtype for e in range(E) for k in ("gate", "up", "down")}
         dt = torch.float32 if len(dts) > 1 else dts.pop()
-        gu = torch.stack([torch.cat([t[f"e{e}.gate"].to(dt), t[f"e{e}.up"].to(dt)], dim=0) for e in range(E)])
+        # A shared expert as wide as several routed ones is that many more groups that every token visits (its inner
+        # elements are independent of each other, and its result the sum over them): two products a layer instead of
+        # four, and more tiles in each.
+        F, m = self.F, 0
+        if self.Fs is not None and self.Fs % F == 0 and self.Fs // F <= SHARED_GROUPS_MAX and self.shared_activation == self.activation \
+                and all(t[f"shared.{x}"].dtype == dt for x in ("gate", "up", "down")):
+            m = self.Fs // F
+        self.shared_groups = m
+        part = lambda g: slice(g * F, (g + 1) * F)
+        gu = torch.stack([torch.cat([t[f"e{e}.gate"].to(dt), t[f"e{e}.up"].to(dt)], dim=0) for e in range(E)]
+                         + [torch.cat([t["shared.gate"][part(g)], t["shared.up"][part(g)]], dim=0) for g in range(m)])
         self.w_gate_up = Weight(gu, self.F % 16 == 0)
         del gu
-        self.w_down = Weight(torch.stack([t[f"e{e}.down"].to(dt) for e in range(E)]))
-        if self.Fs is not None:
+        self.w_down = Weight(torch.stack([t[f"e{e}.down"].to(dt) for e in range(E)] + [t["shared.down"][:, part(g)] for g in range(m)]))
+        if self.Fs is not None and not m:
             sdt = t["shared.gate"].dtype if t["shared.gate"].dtype == t["shared.up"].dtype else torch.float32
             self.ws_gate_up = Weight(torch.cat([t["shared.gate"].to(sdt), t["shared.up"].to(sdt)], dim=0), self.Fs % 16 == 0)
             self.ws_down = Weight(t["shared.down"])
@@ -325,29 +342,31 @@ class MoeTopKSigmoid(FeedForward):
             groups = None
             if self.scoring != "softmax_taken_biased":
                 bias = None
-        hipops.router_topk(logits, bias, expert, weight, k, renorm=self.renormalize, scoring=self.scoring, groups=groups,
-                           n_experts=E)
+        # the row list: the entries of the routed experts, then, for every group of the shared one, every token
+        # (``unused``: the entries' weights in the order of the slots; a product reads it only with ``weight_input``)
+        m = self.shared_groups
+        rows = n + m * T
+        src, dst, unused = ws.take((rows,), torch.int32), ws.take((rows,), torch.int32), ws.take((rows,), torch.float32)
+        offsets = ws.take((E + m + 1,), torch.int32)
+        hipops.router_plan(logits, bias, expert, weight, k, src, unused, dst, offsets, m, renorm=self.renormalize, scoring=self.scoring,
+                           groups=groups, n_experts=E)
         if trace is not None:                         # a testing aid: which experts each token took, [T, top_k]
             trace.setdefault("moe_experts", []).append(expert.view(T, k).clone())
-        # (``unused``: the entries' weights in the order of the slots; a product reads it only with ``weight_input``)
-        src, dst, unused = ws.take((n,), torch.int32), ws.take((n,), torch.int32), ws.take((n,), torch.float32)
-        offsets = ws.take((E + 1,), torch.int32)
-        hipops.moe_plan(expert, weight, src, unused, dst, offsets, n, E, False, fan=k)
-        live = min(n, E)
+        live = min(n, E) + m
         # slot s (entries sorted by expert) reads token src[s] and writes the entry's own row dst[s]
-        act = ws.take((n, F), x.dtype)
-        linear(x, self.w_gate_up, act, glu=self.activation, offsets=offsets, n_groups=E, a_rows=src,
-               a_scale=unused if self.weight_input else None, rows=n, max_rows=T, live_groups=live, ws=ws)
-        y = ws.take((n, d), torch.float32)
-        linear(act, self.w_down, y, offsets=offsets, n_groups=E, y_rows=dst, rows=n, max_rows=T, live_groups=live, ws=ws)
-        ys = None
-        if self.Fs is not None:
+        act = ws.take((rows, F), x.dtype)
+        linear(x, self.w_gate_up, act, glu=self.activation, offsets=offsets, n_groups=E + m, a_rows=src,
+               a_scale=unused if self.weight_input else None, rows=rows, max_rows=T, live_groups=live, ws=ws)
+        y = ws.take((rows, d), torch.float32)
+        linear(act, self.w_down, y, offsets=offsets, n_groups=E + m, y_rows=dst, rows=rows, max_rows=T, live_groups=live, ws=ws)
+        ys = y[n:] if m else None
+        if self.Fs is not None and not m:
             act_s = ws.take((T, self.Fs), x.dtype)
             linear(x, self.ws_gate_up, act_s, glu=self.shared_activation, ws=ws)
             ys = ws.take((T, d), torch.float32)
             linear(act_s, self.ws_down, ys, ws=ws)
         out = ws.take((T, d), torch.float32)
-        hipops.moe_combine(y, None if self.weight_input else weight, ys, out, T, k, gate=gate)
+        hipops.moe_combine(y, None if self.weight_input else weight, ys, out, T, k, gate=gate, n_extra=max(m, 1))
         return (out,)
 
 
