@@ -221,13 +221,16 @@ extern "C" int spite_gemm_skinny(const void* X, int ldx, const void* W, long w_g
     // takes: 16 rows of W a workgroup (variant 6) where 32 (variant 8) would leave half of the compute units without one
     // (2,048 x 2,048: 4.4 against 5.1 us, 2 groups of 2,048 x 3,072: 7.0 against 8.7) and for the experts' plain products,
     // 32 where there are enough (5,120 x 5,120: 10.6 against 12.5, 2 groups of 2 x 3,072 x 2,048 gated: 10.7 against
-    // 11.8); for the output matrix more columns of X or longer blocks.
+    // 11.8); for the output matrix more columns of X or longer blocks.  The experts' gated products run best as many small
+    // workgroups, 16 + 16 rows and four waves (variant 5: two groups of 2 x 8,192 x 5,120 50.6 us against 53.0 with
+    // variant 8, 6.6 against 6.3 TB/s; seven groups 169.6 against 173.4).
     if (variant == 0) {
         if (max_rows <= 16) {
             const long groups = !offsets ? 1 : (live_groups > 0 && live_groups < n_groups ? live_groups : n_groups);
             const bool few = (long)((N + 31) / 32) * (groups < M ? groups : M) < sp_cu_count() / 2;
-            if (offsets) variant = glu && !few ? 8 : 6;
+            if (offsets) variant = glu && !few ? 5 : 6;
             else if ((size_t)N * K >= ((size_t)1 << 28)) variant = max_rows <= 8 ? 4 : 7;
+            else if (max_rows <= 2 && (size_t)N * K >= ((size_t)1 << 27)) variant = 5;
             else variant = few ? 6 : 8;
         }
         // (the output matrix's stream outweighs the second read of its rows by two row tiles: 59 against 71 us at
@@ -247,6 +250,7 @@ extern "C" int spite_gemm_skinny(const void* X, int ldx, const void* W, long w_g
         case 2: return launch_skinny<2, 2, 2, 8>(SP_ARGS);
         case 3: return launch_skinny<2, 4, 2, 4>(SP_ARGS);
         case 4: return launch_skinny<2, 1, 4, 8>(SP_ARGS);
+        case 5: return launch_skinny<1, 1, 2, 4>(SP_ARGS);
         case 6: return launch_skinny<1, 1, 2, 8>(SP_ARGS);
         case 7: return launch_skinny<4, 1, 2, 8>(SP_ARGS);
         case 8: return launch_skinny<2, 1, 2, 8>(SP_ARGS);

@@ -8,6 +8,8 @@ library, or with a tensor that is not on the GPU, the call fails.
 from __future__ import annotations
 
 import ctypes
+import functools
+import math
 from ctypes import c_int, c_long, c_float, c_void_p, c_size_t, c_char_p
 
 import numpy as np
@@ -64,6 +66,7 @@ def lib():
             "spite_gemm_skinny": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, I, I, I, P],
             "spite_attn_decode": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
             "spite_gemm_mfma": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
+            "spite_gemm_lds": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_tiled": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_tiled_split": [P, I, P, P, I, I, I, I, I, I, P, P],
             "spite_attn_prefill": [P, P, P, P, P, P, P, P, I, P, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
@@ -112,6 +115,8 @@ def lib():
         l.spite_attn_prefill_workspace.restype = c_size_t
         l.spite_delta_chunk_workspace.argtypes = [I, I, I, I]
         l.spite_delta_chunk_workspace.restype = c_size_t
+        l.spite_gemm_lds_time.argtypes = [I, I, I, I]
+        l.spite_gemm_lds_time.restype = ctypes.c_double
         l.spite_cu_count.argtypes = []
         l.spite_cu_count.restype = c_int
         _lib = l
@@ -595,6 +600,56 @@ def gemm_tiled(a, w, y, M, N, K, *, offsets=None, n_groups=1, a_rows=None, a_sca
         M, N, K, _ptr(offsets, "offsets", torch.int32, True), n_groups, _ptr(a_rows, "a_rows", torch.int32, True),
         _ptr(a_scale, "a_scale", torch.float32, True), _ptr(y_rows, "y_rows", torch.int32, True), _act_code(glu, act),
         float(act_limit), int(shape), _stream()), "gemm_tiled")
+
+
+def gemm_lds_ok(a, w, M, N, K, glu) -> bool:
+    """Whether ``gemm_lds`` takes these operands: its loads' offsets into the rows of ``a`` and a group of ``w`` are 32-bit."""
+    return K % 64 == 0 and N % 16 == 0 and max(a.shape[0], M) * a.stride(0) * 2 < 1 << 31 and (2 if glu else 1) * N * K * 2 < 1 << 31
+
+
+# What the two tiled products take on an MI355X, in us, from products timed in a row: a tile of gemm_tiled 38 and 8.5 for
+# every 16 rows at K = 5,120; both then run a sixth slower in company than alone; adding up the runs of a sum over k costs
+# a launch and the passes over the partial sums at 4.5 TB/s.
+@functools.lru_cache(maxsize=4096)
+def lds_suits(M: int, N: int, K: int, glu: bool, runs: int) -> bool:
+    """Whether a product without groups is sooner done by ``gemm_lds`` than by ``gemm_tiled`` with its sum over k in
+    ``runs`` runs.  (Timed at 33 sizes, 128 to 2,048 rows, widths of 2,048 to 16,384: the choice is the faster one, or
+    within 4 % of it, at all of them: 1,547 x 5,120 x 5,120 78 against 99 us, 1,531 x 2,048 x 2,048 31 against 37, 300 x 16,384
+    x 5,120 gated 98 against 124; 512 x 5,120 x 8,192 stays, 70 against 115.)"""
+    cus = cu_count()
+    lds = 1.15 * lib().spite_gemm_lds_time(M, N, K, int(bool(glu))) + 3.0
+    cols, scale = -(-N // (256 if glu else 512)), 1.2 * K / 5120.0
+    if runs > 1:
+        if -(-M // 128) * -(-N // 256) < cus // 4:          # too few tiles without the cut (and below what was timed)
+            return False
+        tiled = scale * 106.0 / runs + 12.0 + (runs + 1) * M * N * 4 / 4.5e6
+    else:
+        rounds = lambda rows: -(-(-(-M // rows) * cols) // cus)
+        tiled = scale * min(106.0 * rounds(128), 89.0 * rounds(96) if not glu else math.inf)
+    return lds <= tiled
+
+
+def lds_suits_groups(M: int, n_groups: int, K: int) -> bool:
+    """The same for a product over groups whose row list holds M rows.  (Rows a group on average, us with gemm_lds / gemm_tiled:
+    397 624 / 710, 267 504 / 589, 241 864 / 928; 223 824 / 808, 182 767 / 691, 155 369 / 330; with sums over 1,024 k the tiles
+    end before their loads' depth pays: 510 77 / 72.)"""
+    return M >= 230 * n_groups and K >= 2048
+
+
+def gemm_lds(a, w, y, M, N, K, *, offsets=None, n_groups=1, a_rows=None, a_scale=None, y_rows=None, glu=False, act=None,
+             act_limit=0.0, nb=0):
+    """``gemm_tiled`` with both operands in LDS (see gemm_lds.hip), for many rows; arguments as there.  ``nb``: a plain
+    product's tile height in units of 32 rows, 0 the library's choice."""
+    rows_w = _gemm_checks(a, w, y, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, "gemm_lds")
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        raise KernelError(f"gemm_lds: bfloat16 operands only, got {a.dtype} and {w.dtype}")
+    if not gemm_lds_ok(a, w, M, N, K, glu):
+        raise KernelError(f"gemm_lds: M={M} N={N} K={K} with rows {a.stride(0)} apart: K a multiple of 64, N of 16, operands below 2 GiB")
+    _check(lib().spite_gemm_lds(
+        _ptr_rows(a, "a"), a.stride(0), _ptr(w, "w"), rows_w * K, _ptr_rows(y, "y"), dtype_code(y.dtype), y.stride(0),
+        M, N, K, _ptr(offsets, "offsets", torch.int32, True), n_groups, _ptr(a_rows, "a_rows", torch.int32, True),
+        _ptr(a_scale, "a_scale", torch.float32, True), _ptr(y_rows, "y_rows", torch.int32, True), _act_code(glu, act),
+        float(act_limit), int(nb), _stream()), "gemm_lds")
 
 
 def attn_prefill_splits(counts, H, G, max_keys) -> int:

@@ -134,9 +134,13 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
                                live_groups=live_groups, act=act, act_limit=limit)
             return
         if tiled:
-            plain = offsets is None and a_rows is None and a_scale is None and y_rows is None and not glu and tile_shape == 0 \
-                and act is None
-            runs = hipops.tiled_k_runs(M, N, K) if plain and M > 0 else 1
+            splits = offsets is None and a_rows is None and a_scale is None and y_rows is None and not glu and act is None
+            runs = hipops.tiled_k_runs(M, N, K) if splits and tile_shape == 0 and M > 0 else 1
+            if M > 0 and hipops.gemm_lds_ok(x, w, M, N, K, glu) and (
+                    hipops.lds_suits(M, N, K, bool(glu), runs) if offsets is None else hipops.lds_suits_groups(M, n_groups, K)):
+                hipops.gemm_lds(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
+                                y_rows=y_rows, glu=glu, act=act, act_limit=limit)
+                return
             part = _scratch(ws, (runs, M, N), torch.float32, x.device) if runs > 1 else None
             hipops.gemm_tiled(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
                               y_rows=y_rows, glu=glu, shape=tile_shape, part=part, act=act, act_limit=limit)
