@@ -19,8 +19,8 @@
 //    ones, whose time is the stream of their W: compute and memory are busy together.
 //  * Plain products: NB by the rounds that the tiles make on the chip: see lds_time.
 //
-// Measured on an MI355X beside gemm_tiled (us): 2,048 x 5,120 x 5,120 100 / 110, 2,048 x 5,120 x 8,192 148 / 163, 1,547 x 7,168 x
-// 5,120 101 / 114, 2,048 x 16,384 x 5,120 287 / 292, 8,192^3 848 / 890 (1.30 PFLOP/s).
+// Measured on an MI355X beside gemm_tiled (us): 2,048 x 5,120 x 5,120 91 / 101, 1,786 x 5,120 x 8,192 126 / 155, 1,547 x 7,168 x
+// 5,120 98 / 103, 1,547 x 2 x 16,384 x 5,120 gated 452 / 480, 8,192^3 848 / 890 (1.30 PFLOP/s).
 #include "common.h"
 
 typedef int i32x4 __attribute__((ext_vector_type(4)));

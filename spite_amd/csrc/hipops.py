@@ -613,9 +613,9 @@ def gemm_lds_ok(a, w, M, N, K, glu) -> bool:
 @functools.lru_cache(maxsize=4096)
 def lds_suits(M: int, N: int, K: int, glu: bool, runs: int) -> bool:
     """Whether a product without groups is sooner done by ``gemm_lds`` than by ``gemm_tiled`` with its sum over k in
-    ``runs`` runs.  (Timed at 33 sizes, 128 to 2,048 rows, widths of 2,048 to 16,384: the choice is the faster one, or
-    within 4 % of it, at all of them: 1,547 x 5,120 x 5,120 78 against 99 us, 1,531 x 2,048 x 2,048 31 against 37, 300 x 16,384
-    x 5,120 gated 98 against 124; 512 x 5,120 x 8,192 stays, 70 against 115.)"""
+    ``runs`` runs.  (Timed in turn at 31 sizes, 300 to 2,048 rows, widths of 2,048 to 16,384: the choice is the faster one, or
+    within a tenth of it, at all of them: 1,547 x 5,120 x 5,120 79 against 97 us, 1,531 x 2,048 x 2,048 31 against 36, 300 x 16,384
+    x 5,120 gated 99 against 131; 700 x 5,120 x 8,192 stays, 78 against 106.)"""
     cus = cu_count()
     lds = 1.15 * lib().spite_gemm_lds_time(M, N, K, int(bool(glu))) + 3.0
     cols, scale = -(-N // (256 if glu else 512)), 1.2 * K / 5120.0
@@ -629,11 +629,13 @@ def lds_suits(M: int, N: int, K: int, glu: bool, runs: int) -> bool:
     return lds <= tiled
 
 
-def lds_suits_groups(M: int, n_groups: int, K: int) -> bool:
-    """The same for a product over groups whose row list holds M rows.  (Rows a group on average, us with gemm_lds / gemm_tiled:
-    397 624 / 710, 267 504 / 589, 241 864 / 928; 223 824 / 808, 182 767 / 691, 155 369 / 330; with sums over 1,024 k the tiles
-    end before their loads' depth pays: 510 77 / 72.)"""
-    return M >= 230 * n_groups and K >= 2048
+def lds_suits_groups(group_rows: float, K: int) -> bool:
+    """The same for a product over groups of ``group_rows`` rows each on average (beside groups that take every row).  Fewer
+    rows make its 256 rows of W a tile ask for more operands a product than the 512 of ``gemm_tiled`` do.  (us with
+    gemm_lds / gemm_tiled at K = 5,120 gated, and at the product back: 223 rows 570 / 591 and 335 / 350, 150 rows 487 / 538 and
+    304 / 330, 128 rows 822 / 720 and 522 / 460, 97 rows 751 / 642 and 491 / 432; sums over 1,024 k end before the depth of
+    its loads pays: 383 rows 74 / 68.)"""
+    return group_rows >= 140 and K >= 2048
 
 
 def gemm_lds(a, w, y, M, N, K, *, offsets=None, n_groups=1, a_rows=None, a_scale=None, y_rows=None, glu=False, act=None,

@@ -216,10 +216,10 @@ class MoeTop1Sigmoid(FeedForward):
         # every token goes to one expert: at most min(T, E) of their groups hold rows, and the shared one
         live = min(T, E) + (groups - E)
         linear(x, self.w_gate_up, act, glu=True, offsets=offsets, n_groups=groups, a_rows=src, a_scale=scale, rows=n,
-               max_rows=T, tile_shape=shape, live_groups=live, ws=ws)
+               max_rows=T, tile_shape=shape, live_groups=live, group_rows=T / E, ws=ws)
         # slot s writes row dst[s]: rows [0,T) the routed result per token, rows [T,2T) the shared one
         linear(act, self.w_down, y, offsets=offsets, n_groups=groups, y_rows=dst, rows=n, max_rows=T,
-               tile_shape=shape_down, live_groups=live, ws=ws)
+               tile_shape=shape_down, live_groups=live, group_rows=T / E, ws=ws)
         if self.fused_shared:
             return (y[:T], y[T:])
         act_s = ws.take((T, self.Fs), x.dtype)
@@ -356,9 +356,11 @@ class MoeTopKSigmoid(FeedForward):
         # slot s (entries sorted by expert) reads token src[s] and writes the entry's own row dst[s]
         act = ws.take((rows, F), x.dtype)
         linear(x, self.w_gate_up, act, glu=self.activation, offsets=offsets, n_groups=E + m, a_rows=src,
-               a_scale=unused if self.weight_input else None, rows=rows, max_rows=T, live_groups=live, ws=ws)
+               a_scale=unused if self.weight_input else None, rows=rows, max_rows=T, live_groups=live,
+               group_rows=n / E, ws=ws)
         y = ws.take((rows, d), torch.float32)
-        linear(act, self.w_down, y, offsets=offsets, n_groups=E + m, y_rows=dst, rows=rows, max_rows=T, live_groups=live, ws=ws)
+        linear(act, self.w_down, y, offsets=offsets, n_groups=E + m, y_rows=dst, rows=rows, max_rows=T, live_groups=live,
+               group_rows=n / E, ws=ws)
         ys = y[n:] if m else None
         if self.Fs is not None and not m:
             act_s = ws.take((T, self.Fs), x.dtype)

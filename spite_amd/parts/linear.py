@@ -104,7 +104,7 @@ def grouped_tile_shape(tokens: int, groups: int, whole_groups: int = 0, col_tile
 
 
 def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale=None, y_rows=None, rows=None,
-           max_rows=None, tile_shape=0, live_groups=0, ws=None, act=None):
+           max_rows=None, tile_shape=0, live_groups=0, group_rows=None, ws=None, act=None):
     """y[r] = W . x[r] for ``rows`` rows (default: all of x; for a row list: its length).
 
     With ``glu`` the weight holds gate rows then up rows and y = act(gate) * up: ``True`` or
@@ -112,6 +112,8 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
     ``max_rows``: the most rows that one group can bring (default: ``rows``).
     ``tile_shape``: the prefill product's tile (``grouped_tile_shape``), 0 = the library's choice.
     ``live_groups``: a promise that at most this many groups hold rows (0: none).
+    ``group_rows``: the rows of a routed group on average, beside which other groups may take every row
+    (default: all groups alike).
     ``ws``: the workspace that temporaries (partial sums, widened rows) are taken from.
     ``act``: an activation on a plain product's result (``gelu``, ``gelu_tanh``, ``silu``; not beside
     ``glu``): in the epilogue of the bfloat16 weight-stream and tiled products, a pass of its own after
@@ -137,7 +139,8 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
             splits = offsets is None and a_rows is None and a_scale is None and y_rows is None and not glu and act is None
             runs = hipops.tiled_k_runs(M, N, K) if splits and tile_shape == 0 and M > 0 else 1
             if M > 0 and hipops.gemm_lds_ok(x, w, M, N, K, glu) and (
-                    hipops.lds_suits(M, N, K, bool(glu), runs) if offsets is None else hipops.lds_suits_groups(M, n_groups, K)):
+                    hipops.lds_suits(M, N, K, bool(glu), runs) if offsets is None
+                    else hipops.lds_suits_groups(M / n_groups if group_rows is None else group_rows, K)):
                 hipops.gemm_lds(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
                                 y_rows=y_rows, glu=glu, act=act, act_limit=limit)
                 return
