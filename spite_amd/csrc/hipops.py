@@ -610,14 +610,17 @@ def gemm_lds_ok(a, w, M, N, K, glu) -> bool:
 # What the two tiled products take on an MI355X, in us, from products timed in a row: a tile of gemm_tiled 38 and 8.5 for
 # every 16 rows at K = 5,120; both then run a sixth slower in company than alone; adding up the runs of a sum over k costs
 # a launch and the passes over the partial sums at 4.5 TB/s.
+def lds_us(M: int, N: int, K: int, glu: bool) -> float:
+    return 1.15 * lib().spite_gemm_lds_time(M, N, K, int(bool(glu))) + 3.0
+
+
 @functools.lru_cache(maxsize=4096)
 def lds_suits(M: int, N: int, K: int, glu: bool, runs: int) -> bool:
     """Whether a product without groups is sooner done by ``gemm_lds`` than by ``gemm_tiled`` with its sum over k in
     ``runs`` runs.  (Timed in turn at 31 sizes, 300 to 2,048 rows, widths of 2,048 to 16,384: the choice is the faster one, or
     within a tenth of it, at all of them: 1,547 x 5,120 x 5,120 79 against 97 us, 1,531 x 2,048 x 2,048 31 against 36, 300 x 16,384
     x 5,120 gated 99 against 131; 700 x 5,120 x 8,192 stays, 78 against 106.)"""
-    cus = cu_count()
-    lds = 1.15 * lib().spite_gemm_lds_time(M, N, K, int(bool(glu))) + 3.0
+    cus, lds = cu_count(), lds_us(M, N, K, glu)
     cols, scale = -(-N // (256 if glu else 512)), 1.2 * K / 5120.0
     if runs > 1:
         if -(-M // 128) * -(-N // 256) < cus // 4:          # too few tiles without the cut (and below what was timed)

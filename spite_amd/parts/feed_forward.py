@@ -42,7 +42,7 @@ import math
 import torch
 
 from .base import FeedForward, ParamSpec, register
-from .linear import SKINNY_MAX_ROWS, Weight, grouped_tile_shape, linear
+from .linear import SKINNY_MAX_ROWS, Weight, grouped_tile_shape, linear, whole_group_apart
 from ..csrc import hipops
 
 
@@ -218,6 +218,12 @@ class MoeTop1Sigmoid(FeedForward):
         linear(x, self.w_gate_up, act, glu=True, offsets=offsets, n_groups=groups, a_rows=src, a_scale=scale, rows=n,
                max_rows=T, tile_shape=shape, live_groups=live, group_rows=T / E, ws=ws)
         # slot s writes row dst[s]: rows [0,T) the routed result per token, rows [T,2T) the shared one
+        apart = whole_group_apart(T, E, d, F) if shape_down in (1, 3) and self.fused_shared and self.w_down.tiled else 0
+        if apart:
+            linear(act, self.w_down, y, offsets=offsets, n_groups=E, y_rows=dst, rows=T, max_rows=T, tile_shape=apart,
+                   group_rows=T / E, ws=ws)
+            linear(act[T:], self.w_down.group(E), y[T:], ws=ws)
+            return (y[:T], y[T:])
         linear(act, self.w_down, y, offsets=offsets, n_groups=groups, y_rows=dst, rows=n, max_rows=T,
                tile_shape=shape_down, live_groups=live, group_rows=T / E, ws=ws)
         if self.fused_shared:

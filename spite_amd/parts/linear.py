@@ -6,6 +6,7 @@
 """
 from __future__ import annotations
 
+import functools
 import math
 from typing import List
 
@@ -85,22 +86,53 @@ def grouped_tile_shape(tokens: int, groups: int, whole_groups: int = 0, col_tile
       row tiles alone are compared."""
     if groups <= 0 or tokens <= 0:
         return 1
-    mean = tokens / groups
-    sd = max(math.sqrt(tokens * (1.0 / groups) * (1.0 - 1.0 / groups)), 1e-6)
+    mean, sd = _group_size(tokens, groups)
     if groups <= 32 and mean + 4.0 * sd <= 64.0 and whole_groups * -(-tokens // 64) <= 0.25 * groups:
         return 4
-
-    def tiles(rows_per_tile):
-        extra, k = 0.0, 1
-        while k * rows_per_tile < mean + 6 * sd:
-            extra += 0.5 * math.erfc((k * rows_per_tile + 0.5 - mean) / (sd * math.sqrt(2.0)))
-            k += 1
-        return groups * (1.0 + extra) + whole_groups * -(-tokens // rows_per_tile)
     if col_tiles > 0:
-        cus = cus or hipops.cu_count()
-        rounds = lambda rows_per_tile: math.ceil(tiles(rows_per_tile) * col_tiles / cus - 1e-9)
-        return 3 if TILE_160_COST * rounds(160) < rounds(128) else 1
+        return _rounds(tokens, groups, whole_groups, col_tiles, cus or hipops.cu_count())[0]
+    tiles = lambda rows: _row_tiles(tokens, groups, whole_groups, rows)
     return 3 if 1.17 * tiles(160) < tiles(128) else 1
+
+
+def _group_size(tokens, groups):
+    """Mean and standard deviation of a group's rows."""
+    return tokens / groups, max(math.sqrt(tokens * (1.0 / groups) * (1.0 - 1.0 / groups)), 1e-6)
+
+
+def _row_tiles(tokens, groups, whole_groups, rows_per_tile, sure=False):
+    """The row tiles to expect; ``sure``: a standard deviation more (each further tile of a group comes or does not)."""
+    mean, sd = _group_size(tokens, groups)
+    extra, spread, k = 0.0, 0.0, 1
+    while k * rows_per_tile < mean + 6 * sd:
+        p = 0.5 * math.erfc((k * rows_per_tile + 0.5 - mean) / (sd * math.sqrt(2.0)))
+        extra, spread, k = extra + p, spread + p * (1.0 - p), k + 1
+    return groups * (1.0 + extra) + (math.sqrt(groups * spread) if sure else 0.0) + whole_groups * -(-tokens // rows_per_tile)
+
+
+def _rounds(tokens, groups, whole_groups, col_tiles, cus, sure=False):
+    """(tile shape, its rounds over the chip times its tile's cost)."""
+    rounds = lambda rows: math.ceil(_row_tiles(tokens, groups, whole_groups, rows, sure) * col_tiles / cus - 1e-9)
+    wide, narrow = TILE_160_COST * rounds(160), float(rounds(128))
+    return (3, wide) if wide < narrow else (1, narrow)
+
+
+@functools.lru_cache(maxsize=4096)
+def whole_group_apart(tokens: int, groups: int, N: int, K: int) -> int:
+    """Whether a plain product over ``groups`` groups that ``tokens`` rows spread over and one group that takes every row
+    is better done as two: the groups (the result is the tile shape that they then take, 0: together), and the one as a
+    product of its own with both operands in LDS.  Together the
+    tiles of the second kind fill the first one's last round; apart it may need one round fewer.  A round takes 146 us
+    at K = 5,120 and the groups no less than their weights at 5.6 TB/s (measured at 5,120 x 8,192 over 16 experts, together
+    / apart: 2,048 tokens 466 / 421 us, 1,547 426 / 360, 1,200 292 / 346).  A gated product's rounds are many and its
+    stream of weights long: there it never paid (2,048 tokens 719 / 759)."""
+    cus, round_us = hipops.cu_count(), 146.0 * K / 5120.0
+    cols = -(-N // 512)
+    together = round_us * _rounds(tokens, groups, 1, cols, cus)[1]
+    # (the groups alone need few rounds: one that they miss by a tile would cost what is to be gained)
+    shape, cost = _rounds(tokens, groups, 0, cols, cus, sure=True)
+    routed = max(round_us * cost, groups * N * K * 2 / 5.6e6)
+    return shape if routed + hipops.lds_us(tokens, N, K, False) < together else 0
 
 
 def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale=None, y_rows=None, rows=None,

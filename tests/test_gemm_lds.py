@@ -56,3 +56,24 @@ def test_refuses_what_it_cannot_do():
         ops().gemm_lds(z(4, 64), z(24, 64), z(4, 24), 4, 24, 64)           # N no multiple of 16
     with pytest.raises(ops().KernelError):
         ops().gemm_lds(z(4, 64), z(16, 64), z(4, 16), 4, 16, 64, nb=7)     # no such tile
+
+
+def test_shared_expert_apart_gives_the_same_logits(monkeypatch):
+    """The down product as two (the routed groups, the shared expert with both operands in LDS): the same sums."""
+    from spite_amd import Engine, StepEntry
+    from spite_amd.parts import feed_forward
+    cfg = dict(architectures=["Llama4ForCausalLM"], num_hidden_layers=2, hidden_size=256, num_attention_heads=4, num_key_value_heads=2,
+               head_dim=64, rms_norm_eps=1e-5, num_local_experts=4, num_experts_per_tok=1, intermediate_size=512,
+               intermediate_size_mlp=1024, interleave_moe_layer_step=1, vocab_size=512, rope_theta=1e4, torch_dtype="bfloat16")
+    tokens = torch.randint(0, 512, (300,), generator=torch.Generator().manual_seed(0)).tolist()
+    out, calls = [], []
+    for shape in (0, 1, 3):
+        monkeypatch.setattr(feed_forward, "whole_group_apart", lambda *a: shape)
+        eng = Engine(cfg, random_weights=True, seed=3, cache_tokens=512, max_requests=1)
+        seen = ops().gemm_lds
+        monkeypatch.setattr(ops(), "gemm_lds", lambda *a, **kw: (calls.append(shape), seen(*a, **kw))[1])
+        monkeypatch.setattr(ops(), "lds_suits", lambda M, N, K, glu, runs: True)
+        out.append(eng.step([StepEntry(eng.admit(), tokens, list(range(300)))]).clone())
+        monkeypatch.setattr(ops(), "gemm_lds", seen)
+    assert calls.count(1) == calls.count(0) + 2
+    assert torch.equal(out[0], out[1]) and torch.equal(out[0], out[2])

@@ -1,0 +1,23 @@
+"""The rules that choose between the prefill products, at sizes that were timed and at their edges."""
+from spite_amd.parts.linear import whole_group_apart
+
+
+def test_whole_group_apart():
+    assert whole_group_apart(2048, 16, 5120, 8192) == 3          # tiles of 128 rows alone would miss their round
+    assert whole_group_apart(1547, 16, 5120, 8192) == 1
+    for tokens in (1, 65, 600, 1024, 1200):                      # one round together, or the weights' stream is the time
+        assert whole_group_apart(tokens, 16, 5120, 8192) == 0
+    assert whole_group_apart(2048, 128, 5120, 8192) == 0
+
+
+def test_lds_suits():
+    from spite_amd.csrc.hipops import latent_splits, lds_suits, lds_suits_groups, tiled_k_runs
+    faster = {(1547, 5120, 5120): True, (1786, 5120, 8192): True, (1531, 2048, 2048): True, (1024, 7168, 5120): True,
+              (512, 5120, 8192): False, (330, 7168, 5120): False, (300, 2048, 2048): False, (100, 512, 1024): False}
+    for (M, N, K), yes in faster.items():
+        assert lds_suits(M, N, K, False, tiled_k_runs(M, N, K)) is yes, (M, N, K)
+    assert lds_suits(300, 16384, 5120, True, 1)
+    assert lds_suits_groups(223.0, 5120) and not lds_suits_groups(128.0, 5120) and not lds_suits_groups(383.0, 1024)
+    # shares of two blocks of keys, no more workgroups than compute units, shares within 4,096 keys
+    assert [latent_splits(2, k) for k in (32, 256, 1024, 4096)] == [1, 8, 16, 32]
+    assert latent_splits(16, 4096) == 16 and latent_splits(500, 4096) == 1 and latent_splits(500, 100000) == 25
