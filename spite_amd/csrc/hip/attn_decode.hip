@@ -24,20 +24,33 @@
 #include "common.h"
 #include "no_alloc.h"
 
+// What the fused form does before the attention, for rows [q | k | v] of the projection: see the kernel.
+struct ad_rope {
+    const float* inv_freq;            // [HD / 2], or null: no rotation
+    const int* slot_map;              // the token's cache row
+    float norm_eps;                   // of the weightless norm over a head; 0: none
+    int floor_scale;                  // of the queries' temperature; 0: none
+    float attn_scale;
+};
+
 // HD: width of queries and keys, VD: of values.  DIST: the scores take a bias by distance from a table.
-template <int HD, int VD, bool DIST>
+// FUSE: `q` holds the projection's rows [H + 2 G heads][HD] and the kernel does itself what rope_kvwrite does for them:
+// rotation in halves, norm over the head and temperature of its queries, and, in the workgroup that reads the request's last
+// block, the new key and value on their way into the pages.  (A decoded token then needs a kernel less, of whose 4.7 us
+// next to nothing is work; the sines come from one thread a pair, through LDS.)
+template <int HD, int VD, bool DIST, bool FUSE>
 __global__ __launch_bounds__(256)
-void attn_decode_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_pages,
-                        const bf16* __restrict__ v_pages, float* __restrict__ part, bf16* __restrict__ out,
+void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
+                        bf16* v_pages, float* __restrict__ part, bf16* __restrict__ out,
                         const int* __restrict__ positions, const int* __restrict__ seq_of_token,
                         const int* __restrict__ block_table, int max_blocks, int H, int G, int ps, int vis,
                         int span, float scale_log2e, float cap_ratio, int n_splits,
                         const float* __restrict__ slopes, float inv_scale, int Gv, const float* __restrict__ sinks,
-                        int keep, const float* __restrict__ dist_bias, int n_dist) {
+                        int keep, const float* __restrict__ dist_bias, int n_dist, ad_rope rope) {
     constexpr int NC = HD / 32;      // 32-wide chunks of the head for the score product
     constexpr int ND = VD / 16;      // 16-row tiles of the output
     constexpr int ROW = VD + 2;      // partial record: output, max, sum
-    extern __shared__ float sm[];    // [4 waves][16 heads][ROW]
+    extern __shared__ float sm[];    // [4 waves][QH heads][ROW]
     const int split = blockIdx.x, g = blockIdx.y, t = blockIdx.z;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int n = lane & 15, qd = lane >> 4;
@@ -63,9 +76,68 @@ void attn_decode_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_p
 
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
     bf16x8 qf[NC];
+    if constexpr (FUSE) {
+        const bf16* row = q + (size_t)t * (H + 2 * G) * HD;
+        float* cs = sm;                                  // [HD / 2] pairs (cosine, sine)
+        if (threadIdx.x < HD / 2) {
+            float sn = 0.f, c = 1.f;
+            if (rope.inv_freq) sincosf((float)p * rope.inv_freq[threadIdx.x], &sn, &c);
+            cs[2 * threadIdx.x] = c;
+            cs[2 * threadIdx.x + 1] = sn;
+        }
+        __syncthreads();
+        const int slot = rope.slot_map[t];
+        if (rb < re && re == nblk && slot >= 0) {        // (one workgroup of the splits)
+            const int page = slot / ps, off = slot % ps;
+            if (wave == 0) {
+                const bf16* kr = row + (size_t)(H + g) * HD;
+                bf16* kp = k_pages + ((size_t)page * G + g) * ps * HD;
+                float a = 0.f, b = 0.f;
+                if (lane < HD / 2) {
+                    const float x = (float)kr[lane], y = (float)kr[lane + HD / 2], c = cs[2 * lane], sn = cs[2 * lane + 1];
+                    a = x * c - y * sn;
+                    b = x * sn + y * c;
+                }
+                const float ss = wave_sum(a * a + b * b);
+                const float scale = rope.norm_eps > 0.f ? 1.0f / sqrtf(ss / (float)HD + rope.norm_eps) : 1.0f;
+                if (lane < HD / 2) {
+                    kp[sp_k_index(off, lane, HD, true)] = (bf16)(a * scale);
+                    kp[sp_k_index(off, lane + HD / 2, HD, true)] = (bf16)(b * scale);
+                }
+            } else if (wave == 1) {
+                const bf16* vr = row + (size_t)(H + G + g) * HD;
+                bf16* vp = v_pages + ((size_t)page * G + g) * ps * VD;
+                for (int c = lane; c < VD; c += 64) vp[sp_v_index(c, off, VD, ps, true)] = vr[c];
+            }
+        }
+        // the queries: element c * 32 + qd * 8 + e turns with the one HD / 2 further on, which this lane holds as well
+        const bf16* qr = row + (size_t)(g * QH + (n < QH ? n : 0)) * HD + qd * 8;
+        float x[NC][8], ss = 0.f;
 #pragma unroll
-    for (int c = 0; c < NC; ++c)
-        qf[c] = n < QH ? *(const bf16x8*)(q + ((size_t)t * H + g * QH + n) * HD + c * 32 + qd * 8) : zero8;
+        for (int c = 0; c < NC / 2; ++c) {
+            const bf16x8 lo = *(const bf16x8*)(qr + c * 32), hi = *(const bf16x8*)(qr + c * 32 + HD / 2);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int i = c * 32 + qd * 8 + e;
+                const float a = (float)lo[e], b = (float)hi[e], co = cs[2 * i], sn = cs[2 * i + 1];
+                x[c][e] = a * co - b * sn;
+                x[c + NC / 2][e] = a * sn + b * co;
+                ss += x[c][e] * x[c][e] + x[c + NC / 2][e] * x[c + NC / 2][e];
+            }
+        }
+        ss = rows4_sum(ss);
+        float scale = rope.norm_eps > 0.f ? 1.0f / sqrtf(ss / (float)HD + rope.norm_eps) : 1.0f;
+        if (rope.floor_scale > 0) scale *= logf((float)((p + 1) / rope.floor_scale) + 1.0f) * rope.attn_scale + 1.0f;
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+#pragma unroll
+            for (int e = 0; e < 8; ++e) qf[c][e] = n < QH ? (bf16)(x[c][e] * scale) : (bf16)0.f;
+        __syncthreads();                                 // the new key and value are where the block's loads find them
+    } else {
+#pragma unroll
+        for (int c = 0; c < NC; ++c)
+            qf[c] = n < QH ? *(const bf16x8*)(q + ((size_t)t * H + g * QH + n) * HD + c * 32 + qd * 8) : zero8;
+    }
 
     float m_run = -INFINITY, l_run = 0.f;
     // a sink (one more term exp(sinks[head]) in the softmax's denominator, with no key and no value) is the
@@ -153,27 +225,29 @@ void attn_decode_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_p
         }
     }
 
-    // the four waves' partial results meet in LDS; o[d][i] of lane (n, qd) is O[head n][d*16 + qd*4 + i]
-    float* mine = sm + ((size_t)wave * 16 + n) * ROW;
+    // the waves' partial results meet in LDS; o[d][i] of lane (n, qd) is O[head n][d*16 + qd*4 + i]
+    if (n < QH) {
+        float* mine = sm + ((size_t)wave * QH + n) * ROW;
 #pragma unroll
-    for (int d = 0; d < ND; ++d)
+        for (int d = 0; d < ND; ++d)
 #pragma unroll
-        for (int i = 0; i < 4; ++i) mine[d * 16 + qd * 4 + i] = o[d][i];
-    if (qd == 0) { mine[VD] = m_run; mine[VD + 1] = l_run; }
+            for (int i = 0; i < 4; ++i) mine[d * 16 + qd * 4 + i] = o[d][i];
+        if (qd == 0) { mine[VD] = m_run; mine[VD + 1] = l_run; }
+    }
     __syncthreads();
-    if (n_splits == 1) {                 // nothing to combine: the four waves' sums are the result
+    if (n_splits == 1) {                 // nothing to combine: the waves' sums are the result
         for (int idx = threadIdx.x; idx < QH * VD; idx += 256) {
             const int hn = idx / VD, c = idx % VD;
             float M = -INFINITY;
 #pragma unroll
-            for (int w = 0; w < 4; ++w) M = fmaxf(M, sm[((size_t)w * 16 + hn) * ROW + VD]);
+            for (int w = 0; w < 4; ++w) M = fmaxf(M, sm[((size_t)w * QH + hn) * ROW + VD]);
             float acc = 0.f, L = 0.f;
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-                const float mw = sm[((size_t)w * 16 + hn) * ROW + VD];
+                const float mw = sm[((size_t)w * QH + hn) * ROW + VD];
                 const float f = (mw == -INFINITY) ? 0.f : exp2f(mw - M);
-                acc += f * sm[((size_t)w * 16 + hn) * ROW + c];
-                L += f * sm[((size_t)w * 16 + hn) * ROW + VD + 1];
+                acc += f * sm[((size_t)w * QH + hn) * ROW + c];
+                L += f * sm[((size_t)w * QH + hn) * ROW + VD + 1];
             }
             out[((size_t)t * H + g * QH + hn) * VD + c] = (bf16)(acc * (1.0f / fmaxf(L, 1e-30f)));
         }
@@ -183,15 +257,15 @@ void attn_decode_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k_p
         const int hn = idx / ROW, c = idx % ROW;
         float M = -INFINITY;
 #pragma unroll
-        for (int w = 0; w < 4; ++w) M = fmaxf(M, sm[((size_t)w * 16 + hn) * ROW + VD]);
+        for (int w = 0; w < 4; ++w) M = fmaxf(M, sm[((size_t)w * QH + hn) * ROW + VD]);
         float acc = 0.f;
         if (c == VD) acc = M;
         else {
 #pragma unroll
             for (int w = 0; w < 4; ++w) {
-                const float mw = sm[((size_t)w * 16 + hn) * ROW + VD];
+                const float mw = sm[((size_t)w * QH + hn) * ROW + VD];
                 const float f = (mw == -INFINITY) ? 0.f : exp2f(mw - M);
-                acc += f * sm[((size_t)w * 16 + hn) * ROW + c];   // c == VD+1 sums the l's
+                acc += f * sm[((size_t)w * QH + hn) * ROW + c];   // c == VD+1 sums the l's
             }
         }
         part[(((size_t)t * H + g * QH + hn) * n_splits + split) * ROW + c] = acc;
@@ -258,11 +332,12 @@ extern "C" size_t spite_attn_decode_workspace(int T, int H, int hd, int n_splits
 // `v_dim`: width of the values (0: the keys' `hd`); the pairs (64, 32), (64, 64), (128, 64) and (128, 128) exist.
 // `keep`: with a chunk or a window the request's first so many keys are read as well.  `dist_bias` (device, fp32
 // [H][n_dist], or null): dist_bias[head][min(p - j, n_dist - 1)] is added to the scaled scores (before a cap).
-extern "C" int spite_attn_decode(const void* q, const void* k_pages, const void* v_pages, void* out, void* workspace,
-                                 const int* positions, const int* seq_of_token, const int* block_table,
-                                 int max_blocks, int T, int H, int G, int hd, int page_size, int vis, int span,
-                                 float scale, float softcap, const float* slopes, int n_splits, int value_heads,
-                                 const float* sinks, int v_dim, int keep, const float* dist_bias, int n_dist, hipStream_t st) {
+// `rope`, or null: `q` holds projection rows (see the kernel; keys and values of one width and head count).
+static int attn_decode(const void* q, const void* k_pages, const void* v_pages, void* out, void* workspace,
+                       const int* positions, const int* seq_of_token, const int* block_table,
+                       int max_blocks, int T, int H, int G, int hd, int page_size, int vis, int span,
+                       float scale, float softcap, const float* slopes, int n_splits, int value_heads,
+                       const float* sinks, int v_dim, int keep, const float* dist_bias, int n_dist, const ad_rope* rope, hipStream_t st) {
     SP_REQUIRE(softcap >= 0.f && scale > 0.f, "attn_decode: scale %g, score cap %g", scale, softcap);
     // value pages [pages][value_heads][v_dim][page]: kv head g reads value head g % value_heads (0: as many as kv heads)
     if (value_heads <= 0) value_heads = G;
@@ -281,17 +356,43 @@ extern "C" int spite_attn_decode(const void* q, const void* k_pages, const void*
     if (!sp_vis_has_span(vis)) keep = 0;
     const float sl = scale * 1.4426950408889634f, cr = softcap > 0.f ? scale / softcap : 0.f;
     dim3 grid(n_splits, G, T);
-    const size_t sh = (size_t)4 * 16 * (v_dim + 2) * sizeof(float);
-#define SP_AD(HDV, VDV) do { \
-        auto kern = dist_bias ? attn_decode_kernel<HDV, VDV, true> : attn_decode_kernel<HDV, VDV, false>; \
-        kern<<<grid, 256, sh, st>>>((const bf16*)q, (const bf16*)k_pages, (const bf16*)v_pages, (float*)workspace, (bf16*)out, positions, \
-            seq_of_token, block_table, max_blocks, H, G, page_size, vis, span, sl, cr, n_splits, slopes, 1.0f / scale, value_heads, sinks, \
-            keep, dist_bias, n_dist); } while (0)
-    if (hd == 128) { if (v_dim == 128) SP_AD(128, 128); else SP_AD(128, 64); }
+    const size_t rec = (size_t)4 * (H / G) * (v_dim + 2) * sizeof(float);
+    const size_t sh = rec > (size_t)hd * sizeof(float) ? rec : (size_t)hd * sizeof(float);
+    const ad_rope ro = rope ? *rope : ad_rope{};
+#define SP_ADK(HDV, VDV, DISTV, FUSEV) attn_decode_kernel<HDV, VDV, DISTV, FUSEV><<<grid, 256, sh, st>>>( \
+            (const bf16*)q, (bf16*)k_pages, (bf16*)v_pages, (float*)workspace, (bf16*)out, positions, seq_of_token, block_table, \
+            max_blocks, H, G, page_size, vis, span, sl, cr, n_splits, slopes, 1.0f / scale, value_heads, sinks, keep, dist_bias, n_dist, ro)
+#define SP_AD(HDV, VDV) do { if (dist_bias) SP_ADK(HDV, VDV, true, false); else SP_ADK(HDV, VDV, false, false); } while (0)
+    if (rope) { if (hd == 128) SP_ADK(128, 128, false, true); else SP_ADK(64, 64, false, true); }
+    else if (hd == 128) { if (v_dim == 128) SP_AD(128, 128); else SP_AD(128, 64); }
     else { if (v_dim == 64) SP_AD(64, 64); else SP_AD(64, 32); }
 #undef SP_AD
+#undef SP_ADK
     SP_LAUNCH_CHECK("attn_decode");
     return n_splits > 1 ? sp_attn_combine((const float*)workspace, out, T, H, v_dim, n_splits, st) : 0;
+}
+
+extern "C" int spite_attn_decode(const void* q, const void* k_pages, const void* v_pages, void* out, void* workspace,
+                                 const int* positions, const int* seq_of_token, const int* block_table,
+                                 int max_blocks, int T, int H, int G, int hd, int page_size, int vis, int span,
+                                 float scale, float softcap, const float* slopes, int n_splits, int value_heads,
+                                 const float* sinks, int v_dim, int keep, const float* dist_bias, int n_dist, hipStream_t st) {
+    return attn_decode(q, k_pages, v_pages, out, workspace, positions, seq_of_token, block_table, max_blocks, T, H, G, hd, page_size, vis,
+                       span, scale, softcap, slopes, n_splits, value_heads, sinks, v_dim, keep, dist_bias, n_dist, nullptr, st);
+}
+
+// The same over projection rows qkv [T][(H + 2 G) * hd], whose keys and values go to the pages' rows slot_map[t] on the way:
+// rotation in halves of the whole head by inv_freq (null: none), a weightless norm over each head of queries and keys
+// (norm_eps 0: none), the queries' temperature (floor_scale 0: none).  Pages in operand order.
+extern "C" int spite_attn_decode_rope(const void* qkv, void* k_pages, void* v_pages, void* out, void* workspace,
+                                      const int* positions, const int* slot_map, const int* seq_of_token, const int* block_table,
+                                      int max_blocks, int T, int H, int G, int hd, int page_size, int vis, int span, float scale,
+                                      float softcap, const float* slopes, int n_splits, const float* inv_freq, float norm_eps,
+                                      int floor_scale, float attn_scale, hipStream_t st) {
+    SP_REQUIRE(slot_map && norm_eps >= 0.f && floor_scale >= 0, "attn_decode_rope: eps %g, floor scale %d, or no cache rows", norm_eps, floor_scale);
+    const ad_rope rope{inv_freq, slot_map, norm_eps, floor_scale, attn_scale};
+    return attn_decode(qkv, k_pages, v_pages, out, workspace, positions, seq_of_token, block_table, max_blocks, T, H, G, hd, page_size, vis,
+                       span, scale, softcap, slopes, n_splits, 0, nullptr, hd, 0, nullptr, 0, &rope, st);
 }
 
 // ---- the same call for callers that cannot allocate: the partial results go to an array of

@@ -64,6 +64,7 @@ def lib():
             "spite_sample_rows": [P, I, I, I, P, P, P, P],
             "spite_filter_rows": [P, I, I, I, P, P, P, P],
             "spite_gemm_skinny": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, I, I, I, P],
+            "spite_attn_decode_rope": [P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, I, P, F, I, F, P],
             "spite_attn_decode": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
             "spite_gemm_mfma": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_lds": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
@@ -524,6 +525,43 @@ def attn_decode(q, k_pages, v_pages, out, workspace, positions, seq_of_token, bl
         block_table.shape[1], T, H, G, hd, page_size, VIS[vis], int(span or 0), float(scale), float(softcap),
         _slopes(slopes, H), int(n_splits), int(value_heads or 0), _slopes(sinks, H), Vd, int(keep), *_dist_bias(dist_bias, H),
         _stream()), "attn_decode")
+
+
+def attn_decode_splits(heads: int, longest: int) -> int:
+    """Into how many workgroups the keys of each of ``heads`` (tokens times kv heads) are dealt, none of which reads more than
+    ``longest``: about two workgroups a compute unit (more only add records to join), each with at least a block of 32 keys
+    for every one of its four waves (8 heads of 1,000 keys on an MI355X: 13.2 us with four splits, 10.2 with eight, 10.3
+    with sixteen); one, which needs no second kernel, where two of at most eight blocks would be left (256 heads of 500
+    keys: 18.6 against 21.6 us)."""
+    blocks = -(-longest // 32)
+    n = max(1, min(-(-2 * cu_count() // max(heads, 1)), -(-blocks // 4), 256))
+    return 1 if n <= 2 and blocks <= 16 else n
+
+
+def attn_decode_rope(qkv, k_pages, v_pages, out, workspace, positions, slot_map, seq_of_token, block_table, T, H, G, hd,
+                     page_size, vis, span, scale, n_splits, inv_freq=None, norm_eps=0.0, temperature=None, softcap=0.0, slopes=None):
+    """``rope_kvwrite`` and ``attn_decode`` in one for decoded tokens: ``qkv`` [T, (H+2G)*hd] are the projection's rows, whose
+    keys and values go into the pages' rows ``slot_map`` on the way.  ``inv_freq`` (or None): rotation of the whole head in
+    halves; ``norm_eps`` > 0: the weightless norm over each head; ``temperature``: (floor_scale, attn_scale) or None."""
+    if qkv.dtype != torch.bfloat16:
+        raise KernelError(f"attn_decode_rope: bfloat16 only, got {qkv.dtype}")
+    if qkv.numel() < T * (H + 2 * G) * hd or out.numel() < T * H * hd:
+        raise KernelError("attn_decode_rope: qkv or out too small")
+    _check_pages(k_pages, v_pages, G, page_size, hd, "attn_decode_rope", None, hd)
+    if block_table.dim() != 2 or positions.numel() < T or seq_of_token.numel() < T or slot_map.numel() < T:
+        raise KernelError("attn_decode_rope: metadata too small")
+    if inv_freq is not None and inv_freq.numel() < hd // 2:
+        raise KernelError(f"attn_decode_rope: {inv_freq.numel()} frequencies for heads of {hd}")
+    if workspace.numel() * workspace.element_size() < attn_decode_workspace(T, H, hd, n_splits):
+        raise KernelError("attn_decode_rope: workspace too small")
+    dt = torch.bfloat16
+    _check(lib().spite_attn_decode_rope(
+        _ptr(qkv, "qkv", dt), _ptr(k_pages, "k_pages", dt), _ptr(v_pages, "v_pages", dt), _ptr(out, "out", dt),
+        _ptr(workspace, "workspace"), _ptr(positions, "positions", torch.int32), _ptr(slot_map, "slot_map", torch.int32),
+        _ptr(seq_of_token, "seq_of_token", torch.int32), _ptr(block_table, "block_table", torch.int32),
+        block_table.shape[1], T, H, G, hd, page_size, VIS[vis], int(span or 0), float(scale), float(softcap),
+        _slopes(slopes, H), int(n_splits), _ptr(inv_freq, "inv_freq", torch.float32, True), float(norm_eps),
+        int(temperature[0]) if temperature else 0, float(temperature[1]) if temperature else 0.0, _stream()), "attn_decode_rope")
 
 
 def gemm_mfma(a, w, y, M, N, K, *, offsets=None, n_groups=1, a_rows=None, a_scale=None, y_rows=None, glu=False,

@@ -115,22 +115,30 @@ class Attention(Mixer):
     def cache_need(self):
         return CacheNeed(kv=KVNeed(self.G, self.hd, self.visibility, self.span))
 
-    def _decode(self, q, o, ctx, cache, T):
-        """The split-KV kernel over the step's first T tokens, each the only one of its request."""
+    def _decode(self, q, o, ctx, cache, T, fused=None):
+        """The split-KV kernel over the step's first T tokens, each the only one of its request.  ``fused``: ``q`` holds
+        the projection's rows, and the kernel does what this part's options (the dict) ask of them first."""
         H, G, hd = self.H, self.G, self.hd
-        # split the keys so that about two workgroups a compute unit run (measured: more splits
-        # only add partial results to combine), each with at least eight blocks of keys; the
-        # bound on the keys is the block table's width, so the launch is the same for every
-        # step of that shape
+        # the bound on the keys is the block table's width, so the launch is the same for every step of that shape
         longest = cache.block_table.shape[1] * cache.page_size
         if self.visibility != "full":
             longest = min(longest, self.span + 32)
-        blocks = -(-longest // 32)
-        n_splits = max(1, min(-(-2 * hipops.cu_count() // (T * G)), -(-blocks // 8), 256))
+        n_splits = hipops.attn_decode_splits(T * G, longest)
         scratch = ctx.ws.take((hipops.attn_decode_workspace(T, H, hd, n_splits) // 4,), torch.float32)
+        if fused is not None:
+            hipops.attn_decode_rope(q, cache.k_pages, cache.v_pages, o, scratch, ctx.positions, cache.slot_map, ctx.seq_of_token,
+                                    cache.block_table, T, H, G, hd, cache.page_size, self.visibility, self.span, self.scale, n_splits,
+                                    softcap=self.score_cap, slopes=self.slopes, **fused)
+            return
         hipops.attn_decode(q, cache.k_pages, cache.v_pages, o, scratch, ctx.positions, ctx.seq_of_token,
                            cache.block_table, T, H, G, hd, cache.page_size, self.visibility, self.span,
                            self.scale, n_splits, softcap=self.score_cap, slopes=self.slopes)
+
+    def _fusable(self, ka):
+        """Whether the decode kernel can do itself what rope_kvwrite does: the plain case (Llama 4's): the whole head turns in
+        halves, then a weightless norm."""
+        return not ka["adjacent"] and (not ka["use_rope"] or int(ka.get("rotary_dim") or self.hd) == self.hd) \
+            and not self.qk_norm_weighted and not (self.qk_norm and self.qk_norm_first) and not (self.qk_norm and self.qk_norm_eps <= 0)
 
     def _prefill(self, q, o, ctx, cache, lead, cu_seqlens):
         """The tiled kernel over the step's entries from ``lead`` on (portions of prompts)."""
@@ -159,8 +167,17 @@ class Attention(Mixer):
         if not pe.fused:
             pe.transform(qkv, ctx.positions, H, G, hd)
         ka = pe.kernel_args() if pe.fused else {"use_rope": False, "inv_freq": None, "adjacent": False}
-        q = ws.take((T, H * hd), x.dtype)
         temp = self.temperature
+        # the MFMA kernels read pages in operand order (bfloat16, sizes in multiples of 32)
+        mfma = cache.tiled and hd in (64, 128)
+        if ctx.decode_only and mfma and H // G <= 16 and cache.write and self._fusable(ka):
+            o = ws.take((T, H * hd), x.dtype)
+            self._decode(qkv, o, ctx, cache, T, fused=dict(inv_freq=ka["inv_freq"] if ka["use_rope"] else None, temperature=temp,
+                                                           norm_eps=self.qk_norm_eps if self.qk_norm else 0.0))
+            out = ws.take((T, self.d), torch.float32)
+            linear(o, self.wo, out, ws=ws)
+            return out
+        q = ws.take((T, H * hd), x.dtype)
         hipops.rope_kvwrite(qkv, q, cache.k_pages, cache.v_pages, ctx.positions, cache.slot_map, ka["inv_freq"],
                             H, G, hd, cache.page_size, use_rope=ka["use_rope"], adjacent=ka["adjacent"],
                             use_norm=self.qk_norm, norm_eps=self.qk_norm_eps, use_temp=temp is not None,
@@ -168,8 +185,6 @@ class Attention(Mixer):
                             write_kv=cache.write, kv_tiled=cache.tiled, rotary_dim=ka.get("rotary_dim"),
                             norm_weight_q=self.w_qnorm, norm_weight_k=self.w_knorm, norm_first=self.qk_norm_first)
         o = ws.take((T, H * hd), x.dtype)
-        # the MFMA kernels read pages in operand order (bfloat16, sizes in multiples of 32)
-        mfma = cache.tiled and hd in (64, 128)
         if ctx.decode_only and mfma and H // G <= 16:
             self._decode(q, o, ctx, cache, T)
         elif mfma:

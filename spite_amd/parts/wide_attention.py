@@ -246,8 +246,7 @@ class WideAttention(Mixer):
         longest = cache.block_table.shape[1] * cache.page_size
         if self.visibility != "full":
             longest = min(longest, self.span + self.keep + 32)
-        blocks = -(-longest // 32)
-        n_splits = max(1, min(-(-2 * hipops.cu_count() // (T * GK)), -(-blocks // 8), 256))
+        n_splits = hipops.attn_decode_splits(T * GK, longest)
         scratch = ctx.ws.take((hipops.attn_decode_workspace(T, HQ, self.Vd, n_splits) // 4,), torch.float32)
         hipops.attn_decode(q, cache.k_pages, cache.v_pages, o, scratch, ctx.positions, ctx.seq_of_token,
                            cache.block_table, T, HQ, GK, D, cache.page_size, self.visibility, self.span,

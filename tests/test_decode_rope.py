@@ -1,0 +1,50 @@
+"""Decode attention that rotates, norms and writes the cache itself, against the kernel that does so first: the same pages,
+outputs within the rounding of one bfloat16 query; at block and page edges, with and without each option."""
+import pytest
+import torch
+
+from test_kernels import DEV, PagedKV, ops, rnd
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("H,G,hd,ps", [(5, 1, 64, 32), (8, 2, 128, 64), (40, 8, 128, 64), (16, 1, 128, 32)])
+@pytest.mark.parametrize("rope,norm,temp", [(True, True, False), (False, False, True), (True, False, True), (False, True, False)])
+@pytest.mark.parametrize("n_splits", [1, 3])
+def test_against_the_two_kernels(H, G, hd, ps, rope, norm, temp, n_splits):
+    lens = [1, 32, 33, 64, 300, 161]
+    T = len(lens)
+    kv = PagedKV(lens, G, hd, ps, torch.bfloat16)
+    kp, vp = ops().kv_operand_order(kv.kp.to(DEV), kv.vp.to(DEV))
+    qkv = rnd(T, (H + 2 * G) * hd, dtype=torch.bfloat16, seed=4)
+    positions = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([kv.tables[s][(n - 1) // ps] * ps + (n - 1) % ps for s, n in enumerate(lens)], dtype=torch.int32, device=DEV)
+    seq, bt = torch.arange(T, dtype=torch.int32, device=DEV), kv.bt.to(DEV)
+    inv = (10000.0 ** (-torch.arange(hd // 2, dtype=torch.float64) / (hd // 2))).float().to(DEV)
+    scratch = torch.empty(ops().attn_decode_workspace(T, H, hd, n_splits) // 4, dtype=torch.float32, device=DEV)
+    q, want, got = (torch.zeros(T, H * hd, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    kp2, vp2 = kp.clone(), vp.clone()
+    ops().rope_kvwrite(qkv, q, kp, vp, positions, slots, inv, H, G, hd, ps, use_rope=rope, adjacent=False, use_norm=norm, norm_eps=1e-5,
+                       use_temp=temp, floor_scale=16, attn_scale=0.1, kv_tiled=True)
+    args = (positions, seq, bt, T, H, G, hd, ps, "full", 0, hd ** -0.5, n_splits)
+    ops().attn_decode(q, kp, vp, want, scratch, *args)
+    ops().attn_decode_rope(qkv, kp2, vp2, got, scratch, positions, slots, *args[1:], inv_freq=inv if rope else None,
+                           norm_eps=1e-5 if norm else 0.0, temperature=(16, 0.1) if temp else None)
+    assert torch.equal(vp, vp2)
+    # the sum of squares runs in another order: now and then an element rounds to the next bfloat16 (2^-8 apart at most)
+    off = (kp.float() - kp2.float()).abs()
+    assert float((off / kp.float().abs().clamp_min(1e-3)).max()) <= 2 ** -7 and float((off > 0).float().mean()) < 1e-3
+    # a query or key element that rounds the other way moves a score by 2^-8 of one of hd products; the output rounds once more
+    assert (got.float() - want.float()).abs().max() <= 1.5e-2 * max(1.0, float(want.float().abs().max()))
+
+
+def test_refuses_what_it_cannot_do():
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=DEV)
+    i32 = lambda *s: torch.zeros(*s, dtype=torch.int32, device=DEV)
+    f = torch.zeros(4096, device=DEV)
+    with pytest.raises(ops().KernelError):          # a head size that the kernel does not have
+        ops().attn_decode_rope(z(1, 6 * 32), z(1, 1, 32, 32), z(1, 1, 32, 32), z(1, 4 * 32), f, i32(1), i32(1), i32(1), i32(1, 4), 1, 4, 1, 32,
+                               32, "full", 0, 1.0, 1)
+    with pytest.raises(ops().KernelError):          # no cache row
+        ops().attn_decode_rope(z(1, 6 * 64), z(1, 1, 32, 64), z(1, 1, 64, 32), z(1, 4 * 64), f, i32(1), i32(0), i32(1), i32(1, 4), 1, 4, 1, 64,
+                               32, "full", 0, 1.0, 1)
