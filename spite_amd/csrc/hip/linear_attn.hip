@@ -50,13 +50,16 @@ extern "C" int spite_channel_decay(float* z, const float* bias, int T, int width
 // entry's tokens in order.  Thread (vc, dg) = (tid / 32, tid % 32) holds, in registers, the state's elements
 // S[d][v0 + vc] and S[d][v0 + vc + 8] for D / 32 key channels d (four consecutive ones at 4 dg, and again 128
 // further on for the widest heads; two at 2 dg for heads up to 64): 32 lanes read 512 consecutive bytes of a
-// token's q, k or decay row from LDS in one wide read without bank conflicts.  The tokens' q, k, decay and value slice go through LDS a block of tokens at a time, two buffers:
-// the next block's loads are in flight while this block is computed, and a whole block is one stretch of code:
-// only the state's FMA waits for the token before.  The sum over the key channels is a thread's own partial
-// sum, four rotations across a row of 16 lanes and one step from the lower row to the upper.  The state tile
-// goes through LDS on the way in and out, so that its rows are read and written 64 bytes at a time.
-// The walk is bound by latency, not by FMAs or bytes (about a third of a SIMD's issue slots are used): the
-// split over 32 lanes a column is there to have more waves to switch between.
+// token's q, k or decay row from LDS in one wide read without bank conflicts.  The tokens' q, k, decay and value slice go
+// through LDS a block of tokens at a time, two buffers: the next block's loads are in flight while this block is computed,
+// and nothing looks at a loaded value before that (what lies outside the head is cleared on the way into LDS).  A whole
+// block is one stretch of code: only the state's FMA waits for the token before.  The sums over the key channels are taken
+// for the tokens of a block together (la_sums).  The state tile goes through LDS on the way in and out, so that its rows
+// are read and written 64 bytes at a time.
+// Bound by the reads of q and k from LDS, which every pair of columns makes again (about 190 cycles a token at D = 128 with
+// 8 waves).  1,531 tokens, one request, V = D = 128: 127 us for 16 or 32 heads (208 and 223 with the loads waited for at
+// the head of a block, a sum a token and no read ahead), 106 for heads of 64 (181), 230 for 256 (335); decay per channel:
+// 159 (265).  Half the columns a workgroup where 128 workgroups leave CUs idle gave nothing for heads of 128.
 // The order of every sum is fixed by D alone: the bits do not depend on how a request's tokens are cut.
 #define LA_VC 16        // value columns a workgroup
 #define LA_NT 512       // threads a workgroup: 16 columns x 32 lanes
@@ -65,12 +68,38 @@ extern "C" int spite_channel_decay(float* z, const float* bias, int T, int width
 
 template <int RR> struct la_block { static constexpr int tokens = RR == 16 ? 8 : 16; };
 
-// The sum over 32 lanes (two rows of 16): the rows' sums, then the lower row's into the upper row (a row's last
-// lane to the next row, rows 1 and 3 only).  The upper 16 of the 32 lanes get it.
-__device__ __forceinline__ float row32_sum(float x) {
-    x = row16_sum(x);
-    return x + __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x142, 0xa, 0xf, false));
+// The sum over 32 lanes (two rows of 16) of each of TB values: lane l against l ^ 16, ^ 15, ^ 7, ^ 2 and ^ 1 in turn.  As
+// long as there are two values left, the lanes with the step's bit clear (4, 3, 2, 1 and 0) go on with the first half of
+// them and the others with the second half, so that a step halves the values instead of repeating itself for each: 38
+// instructions for 16 values, against 96 and a wait between most of them.  The pairs that are added do not depend on TB.
+// Lane l ends with value la_owner<TB>(l)'s sum.
+template <int CTRL> __device__ __forceinline__ float la_from(float x) {
+    return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), CTRL, 0xf, 0xf, true));
 }
+template <int CTRL, int BIT, int N> __device__ __forceinline__ void la_halve(float* x, int l) {
+    if constexpr (N > 1) {
+        const bool up = l & BIT;
+#pragma unroll
+        for (int j = 0; j < N / 2; ++j) {
+            const float keep = up ? x[j + N / 2] : x[j], give = up ? x[j] : x[j + N / 2];
+            x[j] = keep + la_from<CTRL>(give);
+        }
+    } else x[0] += la_from<CTRL>(x[0]);
+}
+template <int TB> __device__ __forceinline__ float la_sums(float* x, int l) {
+    constexpr int H = TB > 1 ? TB / 2 : 1;
+#pragma unroll
+    for (int j = 0; j < H; ++j) {                    // (the swap exchanges the first's odd rows with the second's even ones)
+        const auto w = __builtin_amdgcn_permlane16_swap(__float_as_uint(x[j]), __float_as_uint(x[TB > 1 ? j + H : j]), false, false);
+        x[j] = __uint_as_float(w[0]) + __uint_as_float(w[1]);
+    }
+    la_halve<0x140, 8, H>(x, l);                     // row_mirror
+    la_halve<0x141, 4, (H > 1 ? H / 2 : 1)>(x, l);   // row_half_mirror
+    la_halve<0x4e, 2, (H > 2 ? H / 4 : 1)>(x, l);    // quad_perm 2 3 0 1
+    la_halve<0xb1, 1, (H > 4 ? H / 8 : 1)>(x, l);    // quad_perm 1 0 3 2
+    return x[0];
+}
+template <int TB> __device__ __forceinline__ int la_owner(int l) { return TB == 16 ? l >> 1 : TB == 8 ? l >> 2 : 0; }
 
 // VEC: q, k, v (bfloat16) and the decay rows start on 16 bytes and D and V are multiples of 8: a fetch is
 // 16 bytes.  Otherwise one element.  (Plain loops and no closures: every array below stays in registers.)
@@ -96,6 +125,7 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     constexpr int PV = PR < 4 ? PR : 4;             // key channels an LDS read
+    constexpr int LOOK = TB == 1 ? 1 : RR == 16 ? 2 : 4;            // tokens whose rows are on their way from LDS
     typedef float vec __attribute__((ext_vector_type(PV)));
     using RawA = typename std::conditional<VEC, u32x4, T>::type;
     using RawB = typename std::conditional<VEC, f32x4, float>::type;
@@ -145,60 +175,65 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
                 const int ld = part == 0 ? ldq : part == 1 ? ldk : ldv;
                 const int col = part < 2 ? hq * D + d : h * V + v0 + (e0 - 2 * Dp);
                 const bool ok = j < TB && tn + j < t_hi && (part < 2 ? d < D : v0 + (e0 - 2 * Dp) < V);
-                const RawA got = *(const RawA*)(base + (size_t)(ok ? tn + j : t_lo) * ld + (ok ? col : 0));
-                na[u] = ok ? got : RawA{};
+                na[u] = *(const RawA*)(base + (size_t)(ok ? tn + j : t_lo) * ld + (ok ? col : 0));
                 ns[u] = part == 0 ? q_scale : (part == 2 && v_scale) ? v_scale[(size_t)(ok ? tn + j : t_lo) * H + h] : 1.f;
             }
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
                 const int x = tid + u * LA_NT, j = x / CB, d = (x % CB) * WB;
                 const bool ok = j < TB && tn + j < t_hi && d < D;
-                const RawB got = *(const RawB*)(decay + ((size_t)(ok ? tn + j : t_lo) * H + h) * D + (ok ? d : 0));
-                nb[u] = ok ? got : RawB{};
+                nb[u] = *(const RawB*)(decay + ((size_t)(ok ? tn + j : t_lo) * H + h) * D + (ok ? d : 0));
             }
         }
-        float accs[TB];
+        float mine = 0.f;                                           // one token's result (la_owner)
         if (it >= 0) {
             const float* cur = sm + (it & 1) * (TB * per);
             const int n_tok = t_hi - t0 < TB ? t_hi - t0 : TB;
-            // a whole block as one stretch of code: only the state's FMA waits for the token before; the reads,
-            // the sums across lanes and the stores of different tokens overlap
-// token j of the block: the state moves on, and the thread's parts of the two sums over the key channels are kept
-#define LA_TOKEN(j)                                                                         \
-            {                                                                               \
-                const float* row = cur + (j) * per;                                         \
-                const float vv = row[NQ * Dp + vc];                                         \
-                accs[j] = 0.f;                                                              \
-                _Pragma("unroll")                                                           \
-                for (int r = 0; r < PR; r += PV) {                                          \
-                    const vec q4 = *(const vec*)(row + LA_OWN(r));                          \
-                    const vec k4 = *(const vec*)(row + Dp + LA_OWN(r));                     \
-                    vec a4;                                                                 \
-                    if (CH) a4 = *(const vec*)(row + 2 * Dp + LA_OWN(r));                   \
-                    _Pragma("unroll")                                                       \
-                    for (int y = 0; y < PV; ++y) {                                          \
-                        const float a = CH ? a4[y] : hd;                                    \
-                        const float kv = k4[y] * vv;                                        \
-                        if (PRE) accs[j] = fmaf(fmaf(ub[r + y], kv, S[r + y]), q4[y], accs[j]); \
-                        S[r + y] = fmaf(a, S[r + y], kv);                                   \
-                        if (!PRE) accs[j] = fmaf(S[r + y], q4[y], accs[j]);                 \
-                    }                                                                       \
-                }                                                                           \
-            }
-            if (n_tok == TB) {
-                // no branch between the tokens of a whole block
+            float accs[TB];
+            // A whole block is one stretch of code, its tokens' rows read LOOK tokens ahead of their use (the barriers keep
+            // the compiler from moving the reads back to it): only the state's FMA waits for the token before.
+            vec q4[LOOK][PR / PV], k4[LOOK][PR / PV], a4[CH ? LOOK : 1][PR / PV];
+            float vv[LOOK];
+            auto read = [&](int j) {
+                const float* row = cur + j * per;
+                vv[j % LOOK] = row[NQ * Dp + vc];
 #pragma unroll
-                for (int j = 0; j < TB; ++j) LA_TOKEN(j)
+                for (int r = 0; r < PR; r += PV) {
+                    q4[j % LOOK][r / PV] = *(const vec*)(row + LA_OWN(r));
+                    k4[j % LOOK][r / PV] = *(const vec*)(row + Dp + LA_OWN(r));
+                    if constexpr (CH) a4[j % LOOK][r / PV] = *(const vec*)(row + 2 * Dp + LA_OWN(r));
+                }
+            };
+            auto token = [&](int j) {                               // the state moves on; the thread's part of the result
+                accs[j] = 0.f;
+#pragma unroll
+                for (int r = 0; r < PR; ++r) {
+                    float a = hd;
+                    if constexpr (CH) a = a4[j % LOOK][r / PV][r % PV];
+                    const float qr = q4[j % LOOK][r / PV][r % PV], kv = k4[j % LOOK][r / PV][r % PV] * vv[j % LOOK];
+                    if (PRE) accs[j] = fmaf(fmaf(ub[PRE ? r : 0], kv, S[r]), qr, accs[j]);
+                    S[r] = fmaf(a, S[r], kv);
+                    if (!PRE) accs[j] = fmaf(S[r], qr, accs[j]);
+                }
+            };
+            if (n_tok == TB) {
+#pragma unroll
+                for (int j = 0; j < LOOK; ++j) read(j);
+#pragma unroll
+                for (int j = 0; j < TB; ++j) {
+                    __builtin_amdgcn_sched_barrier(0x7);
+                    token(j);
+                    if (j + LOOK < TB) read(j + LOOK);
+                }
+                __builtin_amdgcn_sched_barrier(0x7);
             } else {
 #pragma unroll
                 for (int j = 0; j < TB; ++j) {
                     accs[j] = 0.f;
-                    if (j < n_tok) LA_TOKEN(j)
+                    if (j < n_tok) { read(j); token(j); }
                 }
             }
-#undef LA_TOKEN
-#pragma unroll
-            for (int j = 0; j < TB; ++j) accs[j] = row32_sum(accs[j]);
+            mine = la_sums<TB>(accs, dg);
         }
         if (more) {
             float* buf = sm + ((it + 1) & 1) * (TB * per);
@@ -208,8 +243,10 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
                 if (j < TB && tn + j < t_hi) {
                     float* dst = buf + j * per + (part < 2 ? e0 : e0 + (NQ - 2) * Dp);
                     const float m = ns[u];
+                    const bool in = ((part < 2) & (e0 % Dp < D)) | ((part >= 2) & (v0 + (e0 - 2 * Dp) < V));
+                    const RawA got = in ? na[u] : RawA{};
                     if constexpr (VEC) {
-                        const u32x4 w = na[u];
+                        const u32x4 w = got;
                         f32x4 lo, hi;
                         lo.x = __builtin_bit_cast(float, w.x << 16) * m, lo.y = __builtin_bit_cast(float, w.x & 0xffff0000u) * m;
                         lo.z = __builtin_bit_cast(float, w.y << 16) * m, lo.w = __builtin_bit_cast(float, w.y & 0xffff0000u) * m;
@@ -217,26 +254,21 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
                         hi.z = __builtin_bit_cast(float, w.w << 16) * m, hi.w = __builtin_bit_cast(float, w.w & 0xffff0000u) * m;
                         *(f32x4*)dst = lo;
                         *(f32x4*)(dst + 4) = hi;
-                    } else dst[0] = to_f32<T>(na[u]) * m;
+                    } else dst[0] = to_f32<T>(got) * m;
                 }
             }
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
                 const int x = tid + u * LA_NT, j = x / CB, d = (x % CB) * WB;
                 if (j < TB && tn + j < t_hi) {
-                    if constexpr (VEC) *(f32x4*)(buf + j * per + 2 * Dp + d) = nb[u];
-                    else buf[j * per + 2 * Dp + d] = nb[u];
+                    *(RawB*)(buf + j * per + 2 * Dp + d) = d < D ? nb[u] : RawB{};
                 }
             }
         }
         // the block's results leave after the next block's rows are in LDS: waiting for those loads does not wait for these stores
-        if (it >= 0 && dg == LA_DG - 1) {
-            const int n_tok = t_hi - t0 < TB ? t_hi - t0 : TB;
-            float* orow = out + ((size_t)t0 * H + h) * V + vcol;
-#pragma unroll
-            for (int j = 0; j < TB; ++j) {
-                if (j < n_tok && vok) orow[(size_t)j * H * V] = accs[j];
-            }
+        if (it >= 0 && dg % (LA_DG / TB) == 0) {
+            const int t = t0 + la_owner<TB>(dg);
+            if (t < t_hi && vok) out[((size_t)t * H + h) * V + vcol] = mine;
         }
         __syncthreads();
     }

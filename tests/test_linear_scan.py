@@ -1,0 +1,34 @@
+"""The linear recurrence: a request's tokens taken in blocks give the bits of the same tokens taken one by one."""
+import pytest
+import torch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["channel", "head", "bonus"])
+@pytest.mark.parametrize("H,D,V,dtype", [(2, 6, 10, torch.float32), (2, 64, 40, torch.bfloat16), (1, 128, 128, torch.bfloat16),
+                                         (1, 130, 20, torch.bfloat16), (1, 256, 72, torch.bfloat16)])
+@pytest.mark.parametrize("lens", [[1, 7, 16], [8, 9, 15], [17, 33]])
+def test_blocks_of_tokens_match_single_tokens(kind, H, D, V, dtype, lens):
+    """Blocks hold 16 tokens (8 for the widest heads): lengths below, at and above them.  Each token's sums run over the
+    same pairs of lanes whichever of the two kernels takes them, so results and states are equal, not close."""
+    from spite_amd.csrc import hipops
+    torch.manual_seed(D + V)
+    n, T = len(lens), sum(lens)
+    row = (torch.randn(T, H * (2 * D + V), device="cuda") * 0.5).to(dtype)
+    q, k, v = row[:, :H * D], row[:, H * D:2 * H * D], row[:, 2 * H * D:]
+    opt = dict(decay=torch.rand(T, H * D, device="cuda")) if kind != "head" else dict(head_decay=torch.rand(H, device="cuda"))
+    if kind == "bonus":
+        opt["bonus"] = torch.randn(H, D, device="cuda")
+    start = torch.randn(n, H, D, V, device="cuda")
+    slots = torch.arange(n, dtype=torch.int32, device="cuda")
+    first = [sum(lens[:i]) for i in range(n + 1)]
+    whole, s_whole = torch.empty(T, H * V, device="cuda"), start.clone()
+    hipops.linear_attn_scan(q, k, v, whole, s_whole, torch.tensor(first, dtype=torch.int32, device="cuda"), slots, n, H, D, V, **opt)
+    single, s_single = torch.empty(T, H * V, device="cuda"), start.clone()
+    one = torch.tensor([0, 1], dtype=torch.int32, device="cuda")
+    for i in range(n):
+        for t in range(first[i], first[i + 1]):
+            cut = dict(opt, decay=opt["decay"][t:t + 1]) if "decay" in opt else opt
+            hipops.linear_attn_scan(q[t:t + 1], k[t:t + 1], v[t:t + 1], single[t:t + 1], s_single, one, slots[i:i + 1], 1, H, D, V,
+                                    longest=1, **cut)
+    assert torch.equal(whole, single) and torch.equal(s_whole, s_single)
