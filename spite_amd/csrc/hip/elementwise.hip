@@ -51,6 +51,24 @@ extern "C" int spite_embed(const int* ids, const void* table, int dtype, float* 
 
 // (a wave's fp32 dot product, wave_dot_row, is in common.h: every kernel that forms router logits calls it)
 
+// expert[] and weight[]: the largest logit, the lowest index among equals, weight =
+// 1/(1+exp(-logit)).
+__device__ __forceinline__ int top1_of(const float* __restrict__ l, int E, float* best_out) {
+    float best = -INFINITY; int best_e = 0;
+    if ((E & 3) == 0 && (((uintptr_t)l) & 15) == 0) {           // four logits a load
+        for (int e = 0; e < E; e += 4) {
+            const f32x4 v = *(const f32x4*)(l + e);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) if (v[i] > best || (e + i == 0)) { best = v[i]; best_e = e + i; }
+        }
+    } else {
+        best = l[0];
+        for (int e = 1; e < E; ++e) { const float v = l[e]; if (v > best) { best = v; best_e = e; } }
+    }
+    if (best_out) *best_out = best;
+    return best_e;
+}
+
 // ------------------------------------------------------------------ residual add + RMSNorm
 // v = h[r] + d1[r] + d2[r]; (h[r] = v); out[i] = v * 1/sqrt(mean(v^2)+eps) * w, r = rows ? rows[i] : i.
 // One workgroup of NT threads per row; a thread keeps its elements (groups of four, strided
@@ -65,6 +83,10 @@ extern "C" int spite_embed(const int* ids, const void* table, int dtype, float* 
 // itself in the output's dtype (no norm, `w` unused): the stream as a later product's operand.
 // With `w2` and `out2` the row goes out a second time, normed with the weights w2 (two norms of
 // one stream: a layer whose mixer and feed-forward read the same rows), in `out`'s dtype.
+// With `plan` (a single row) the projection is a router's logits and the row's list for the grouped products is made here
+// too, as moe_plan makes it: one of some 4.5 us of launches that a layer of a single decoded token is made of (5,120 wide
+// over 16 experts: 11.2 us for the two kernels, 7.1 for this one).
+struct norm_plan { int* expert; float* weight; int* src; float* scale; int* dst; int* offsets; int shared; };
 #define NORM_NT 512
 #define NORM_MAX_V 8     // widths up to 4*NT*MAX_V = 16384 stay in registers
 template <typename TO, bool VEC>
@@ -75,9 +97,9 @@ void add_rmsnorm_kernel(float* __restrict__ h, const float* __restrict__ d1,
                         const int* __restrict__ rows, int d, float eps, int write_h,
                         const float* __restrict__ proj, float* __restrict__ proj_out, int P,
                         const float* __restrict__ dn, const float* __restrict__ wn, float mult, float eps_n,
-                        int plain_out, const float* __restrict__ w2, TO* __restrict__ out2) {
+                        int plain_out, const float* __restrict__ w2, TO* __restrict__ out2, norm_plan plan) {
     __shared__ float red[NORM_NT / 64];
-    extern __shared__ __attribute__((aligned(16))) float ys[];            // [d] if proj
+    extern __shared__ __attribute__((aligned(16))) float ys[];            // [d] if proj, and P logits behind it (at a multiple of 4) if plan
     const int i = blockIdx.x;
     const size_t r = rows ? (size_t)rows[i] : (size_t)i;
     float* hr = h + r * d;
@@ -189,7 +211,25 @@ void add_rmsnorm_kernel(float* __restrict__ h, const float* __restrict__ d1,
         const bool pvec = (d & 3) == 0 && (((uintptr_t)proj) & 15) == 0;
         for (int p = wave; p < P; p += NORM_NT / 64) {
             const float v = wave_dot_row(proj + (size_t)p * d, ys, d, pvec, lane);
-            if (lane == 0) proj_out[(size_t)i * P + p] = v;
+            if (lane == 0) {
+                proj_out[(size_t)i * P + p] = v;
+                if (plan.expert) ys[((d + 3) & ~3) + p] = v;
+            }
+        }
+        if (!plan.expert) return;
+        __syncthreads();
+        float best;
+        const int me = top1_of(ys + ((d + 3) & ~3), P, &best);
+        if (threadIdx.x == 0) {
+            const float wt = 1.0f / (1.0f + expf(-best));
+            plan.expert[0] = me; plan.weight[0] = wt;
+            plan.src[0] = 0; plan.scale[0] = wt; plan.dst[0] = 0;
+        }
+        for (int g = threadIdx.x; g <= P; g += NORM_NT) plan.offsets[g] = me < g;
+        if ((int)threadIdx.x < plan.shared) {
+            const int j = 1 + threadIdx.x;
+            plan.src[j] = 0; plan.scale[j] = 1.0f; plan.dst[j] = j;
+            plan.offsets[P + j] = 1 + j;
         }
     }
 }
@@ -198,20 +238,24 @@ extern "C" int spite_add_rmsnorm(float* h, const float* d1, const float* d2, con
                                  int out_dtype, float* out32, const int* rows, int n_rows, int d,
                                  float eps, int write_h, const float* proj, float* proj_out, int P,
                                  const float* dn, const float* wn, float mult, float eps_n, int plain_out,
-                                 const float* w2, void* out2, hipStream_t st) {
+                                 const float* w2, void* out2, int* expert, float* weight, int* src, float* scale, int* dst,
+                                 int* offsets, int shared, hipStream_t st) {
     SP_REQUIRE(!out2 || w2, "add_rmsnorm: a second output needs the second norm's weight");
     SP_REQUIRE(n_rows >= 0 && d > 0 && eps > 0.f, "add_rmsnorm: bad sizes rows=%d d=%d eps=%g", n_rows, d, eps);
     SP_REQUIRE(!dn || (wn && eps_n > 0.f), "add_rmsnorm: a normed increment needs its weight and eps");
     SP_REQUIRE(w || plain_out || (!out && !out32 && !proj), "add_rmsnorm: a normed output needs the norm's weight");
     SP_REQUIRE(!proj || (proj_out && P > 0), "add_rmsnorm: a projection needs its output and size");
-    const size_t sh = proj ? (size_t)d * sizeof(float) : 0;
+    SP_REQUIRE(!expert || (proj && n_rows <= 1 && P < 65535 && shared >= 0 && shared <= 64 && weight && src && scale && dst && offsets),
+               "add_rmsnorm: a plan of %d rows, %d experts, %d shared groups", n_rows, P, shared);
+    const norm_plan plan{expert, weight, src, scale, dst, offsets, shared};
+    const size_t sh = proj ? (size_t)((expert ? ((d + 3) & ~3) + P : d)) * sizeof(float) : 0;
     SP_REQUIRE(sh <= 48 * 1024, "add_rmsnorm: rows of %d do not fit the projection's LDS", d);
     if (n_rows == 0) return 0;
     auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     const bool vec = d % 4 == 0 && d <= 4 * NORM_NT * NORM_MAX_V && al(h) && al(d1) && al(d2) && al(w) && al(out32) && al(out) && al(dn) && al(wn)
         && al(w2) && al(out2);
-#define SP_NORM(TO) do { if (vec) add_rmsnorm_kernel<TO, true><<<n_rows, NORM_NT, sh, st>>>(h, d1, d2, w, (TO*)out, out32, rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2, (TO*)out2); \
-        else add_rmsnorm_kernel<TO, false><<<n_rows, NORM_NT, sh, st>>>(h, d1, d2, w, (TO*)out, out32, rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2, (TO*)out2); } while (0)
+#define SP_NORM(TO) do { if (vec) add_rmsnorm_kernel<TO, true><<<n_rows, NORM_NT, sh, st>>>(h, d1, d2, w, (TO*)out, out32, rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2, (TO*)out2, plan); \
+        else add_rmsnorm_kernel<TO, false><<<n_rows, NORM_NT, sh, st>>>(h, d1, d2, w, (TO*)out, out32, rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2, (TO*)out2, plan); } while (0)
     if (out_dtype == SP_F32) SP_NORM(float);
     else if (out_dtype == SP_BF16) SP_NORM(bf16);
     else return sp_fail("add_rmsnorm: unknown dtype %d", out_dtype);
@@ -587,24 +631,6 @@ extern "C" int spite_router_top1(const float* x, const float* wr, int* expert, f
 //   the slots behind them, `shared` groups E, E + 1, ... that every token visits: src = token, scale 1, dst[s] = s;
 //   offsets[g] = first slot of group g, g in [0, E + shared + 1).
 // With `logits` ([T, E] fp32) the kernels make the router's choice themselves and write it to
-// expert[] and weight[]: the largest logit, the lowest index among equals, weight =
-// 1/(1+exp(-logit)).
-__device__ __forceinline__ int top1_of(const float* __restrict__ l, int E, float* best_out) {
-    float best = -INFINITY; int best_e = 0;
-    if ((E & 3) == 0 && (((uintptr_t)l) & 15) == 0) {           // four logits a load
-        for (int e = 0; e < E; e += 4) {
-            const f32x4 v = *(const f32x4*)(l + e);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) if (v[i] > best || (e + i == 0)) { best = v[i]; best_e = e + i; }
-        }
-    } else {
-        best = l[0];
-        for (int e = 1; e < E; ++e) { const float v = l[e]; if (v > best) { best = v; best_e = e; } }
-    }
-    if (best_out) *best_out = best;
-    return best_e;
-}
-
 // Each thread ranks one token by counting over all tokens in shared memory: no atomics, the
 // order is the same on every run.
 __global__ void moe_plan_kernel(int* __restrict__ expert, float* __restrict__ weight,

@@ -52,7 +52,7 @@ def lib():
         P, I, L, F = c_void_p, c_int, c_long, c_float
         sigs = {
             "spite_embed": [P, P, I, P, I, I, I, F, P],
-            "spite_add_rmsnorm": [P, P, P, P, P, I, P, P, I, I, F, I, P, P, I, P, P, F, F, I, P, P, P],
+            "spite_add_rmsnorm": [P, P, P, P, P, I, P, P, I, I, F, I, P, P, I, P, P, F, F, I, P, P, P, P, P, P, P, P, I, P],
             "spite_rope_kvwrite": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, I, F, I, I, I, P, P, I, P],
             "spite_router_top1": [P, P, P, P, P, I, I, I, P],
             "spite_moe_plan": [P, P, P, P, P, P, P, I, I, I, I, P],
@@ -181,20 +181,22 @@ def embed(ids, table, h, scale=1.0):
                              _ptr(h, "h", torch.float32), T, d, table.shape[0], float(scale), _stream()), "embed")
 
 
-def add_rmsnorm_can_project(d: int) -> bool:
-    """Whether ``add_rmsnorm`` forms projections of rows of this width (the row stays in LDS)."""
-    return d * 4 <= 48 * 1024
+def add_rmsnorm_can_project(d: int, plan_experts: int = 0) -> bool:
+    """Whether ``add_rmsnorm`` forms projections of rows of this width (the row stays in LDS, and with a plan the logits
+    of ``plan_experts`` experts too)."""
+    return (-(-d // 4) * 4 + plan_experts if plan_experts else d) * 4 <= 48 * 1024
 
 
 def add_rmsnorm(h, w, eps, out=None, out32=None, d1=None, d2=None, rows=None, n_rows=None, write_h=True,
-                proj=None, proj_out=None, normed=None, plain_out=False, w2=None, out2=None):
+                proj=None, proj_out=None, normed=None, plain_out=False, w2=None, out2=None, plan=None):
     """v = h[r] + d1[r] + d2[r] (stored back if write_h); out[i] = rmsnorm(v) * w with r =
     rows[i] or i.  h, d1, d2, out32 fp32; w fp32 [d]; out fp32 or bf16.  With ``proj`` ([P, d]
     fp32) also proj_out[i] = proj . (the normed row in fp32), [n, P] fp32: the same bits as
     ``router_top1`` gives for that row.  ``normed`` = (dn, wn, mult, eps_n): a further increment
     mult * rmsnorm(dn[r]; eps_n) * wn, normed on its way in.  ``plain_out``: out[i] = v itself (no
     norm; ``w`` may be None).  ``w2`` / ``out2``: the same rows normed with a second weight (in the
-    dtype of ``out`` where there is one).  With no output at all the call only adds."""
+    dtype of ``out`` where there is one).  With no output at all the call only adds.  ``plan`` (one row, with
+    ``proj``) = (expert, weight, src, scale, dst, offsets, shared): what ``moe_plan`` leaves for these logits."""
     d = h.shape[-1]
     dn = wn = None
     mult = eps_n = 0.0
@@ -223,6 +225,16 @@ def add_rmsnorm(h, w, eps, out=None, out32=None, d1=None, d2=None, rows=None, n_
         if proj.dim() != 2 or proj.shape[1] != d or proj_out is None or proj_out.dim() != 2 \
                 or proj_out.shape[0] < n or proj_out.shape[1] != P:
             raise KernelError("add_rmsnorm: projection [P, d] with an output [rows, P]")
+    expert = weight = src = scale = dst = offsets = None
+    shared = 0
+    if plan is not None:
+        expert, weight, src, scale, dst, offsets, shared = plan
+        shared = int(shared)
+        if proj is None or n != 1 or P >= 65535 or not 0 <= shared <= 64 or not add_rmsnorm_can_project(d, P):
+            raise KernelError(f"add_rmsnorm: a plan goes with one row and its logits ({n} rows, {P} experts)")
+        if min(t.numel() for t in (src, scale, dst)) < 1 + shared or offsets.numel() < P + 1 + shared \
+                or expert.numel() < 1 or weight.numel() < 1:
+            raise KernelError("add_rmsnorm: the plan's arrays are too small")
     _check(lib().spite_add_rmsnorm(
         _ptr(h, "h", torch.float32), _ptr(d1, "d1", torch.float32, True), _ptr(d2, "d2", torch.float32, True),
         _ptr(w, "w", torch.float32, True), _ptr(out, "out", None, True),
@@ -232,7 +244,9 @@ def add_rmsnorm(h, w, eps, out=None, out32=None, d1=None, d2=None, rows=None, n_
         _ptr(proj, "proj", torch.float32, True), _ptr(proj_out, "proj_out", torch.float32, True), P,
         _ptr(dn, "normed increment", torch.float32, True), _ptr(wn, "normed increment's weight", torch.float32, True),
         float(mult), float(eps_n), int(bool(plain_out)), _ptr(w2, "w2", torch.float32, True), _ptr(out2, "out2", None, True),
-        _stream()),
+        _ptr(expert, "expert", torch.int32, True), _ptr(weight, "weight", torch.float32, True), _ptr(src, "src", torch.int32, True),
+        _ptr(scale, "scale", torch.float32, True), _ptr(dst, "dst", torch.int32, True), _ptr(offsets, "offsets", torch.int32, True),
+        shared, _stream()),
         "add_rmsnorm")
 
 

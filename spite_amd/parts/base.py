@@ -147,6 +147,11 @@ class Norm(Part):
         The norm knows what its kernel can hold."""
         return False
 
+    def can_plan(self, proj, rows: int) -> bool:
+        """Whether forward() also takes a feed-forward's ``plan_arrays`` as ``plan`` beside this ``proj`` in a step of
+        so many rows, and leaves there what the feed-forward would make of the logits."""
+        return False
+
     def forward(self, h, out, *, d1=None, d2=None, out32=None, rows=None, write_h=True) -> None:
         """h (fp32 [T,d]) += d1 + d2 (kept if write_h); out[i] (and out32[i]) = norm(h[r]), r =
         rows[i] or i."""
@@ -204,6 +209,10 @@ class FeedForward(Part):
         """An fp32 matrix [P, d] whose products with the fp32 normed input this part wants
         (router logits), or None.  A block whose norm ``projects`` then calls
         ``forward(x, None, ctx, projected=logits)`` instead of handing over x32."""
+        return None
+
+    def plan_arrays(self, rows: int, ctx):
+        """Arrays that a norm which ``can_plan`` fills from the logits, or None; ``forward`` then gets them as ``plan``."""
         return None
 
     def forward(self, x, x32, ctx, projected=None):

@@ -76,8 +76,10 @@ class PreNormBlock(Block):
         if proj is not None and self.norm2.can_project(proj):
             # the norm forms the feed-forward's small fp32 products (router logits) itself
             logits = ws.take((T, proj.shape[0]), torch.float32)
-            self.norm2.forward(h, n2, d1=delta, proj=proj, proj_out=logits)
-            state["pending"] = tuple(self.ffn.forward(n2, None, ctx, projected=logits))
+            plan = self.ffn.plan_arrays(T, ctx) if self.norm2.can_plan(proj, T) else None
+            more = {"plan": plan} if plan is not None else {}
+            self.norm2.forward(h, n2, d1=delta, proj=proj, proj_out=logits, **more)
+            state["pending"] = tuple(self.ffn.forward(n2, None, ctx, projected=logits, **more))
             return
         n2_32 = None
         if self.ffn.wants_f32_input:

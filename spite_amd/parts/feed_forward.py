@@ -168,13 +168,22 @@ class MoeTop1Sigmoid(FeedForward):
     def input_projection(self):
         return self.w_router if self.w_router is not None and self.w_router.dtype == torch.float32 else None
 
-    def forward(self, x, x32, ctx, projected=None):
+    def _arrays(self, T, ws):
+        """expert, weight, src, scale, dst, offsets of a step of T tokens, and the shared groups behind the experts'."""
+        n, groups = (2 * T, self.E + 1) if self.fused_shared else (T, self.E)
+        i32 = lambda k: ws.take((k,), torch.int32)
+        f32 = lambda k: ws.take((k,), torch.float32)
+        return i32(T), f32(T), i32(n), f32(n), i32(n), i32(groups + 1), int(self.fused_shared)
+
+    def plan_arrays(self, rows, ctx):
+        return self._arrays(rows, ctx.ws) if ctx.extras.get("trace") is None else None
+
+    def forward(self, x, x32, ctx, projected=None, plan=None):
         """``projected``: the router's logits [T, E] if the block's norm formed them; else they
-        are computed here from x32."""
+        are computed here from x32.  ``plan``: the arrays of ``plan_arrays`` if the norm has filled them too."""
         T, E, F, d = x.shape[0], self.E, self.F, self.d
         ws = ctx.ws
-        expert = ws.take((T,), torch.int32)
-        weight = ws.take((T,), torch.float32)
+        expert, weight, src, scale, dst, offsets, _ = plan if plan is not None else self._arrays(T, ws)
         trace = ctx.extras.get("trace")
         if trace is not None and trace.get("take_experts"):
             # a testing aid: the experts are given (one tensor per call, in the order of the
@@ -188,12 +197,9 @@ class MoeTop1Sigmoid(FeedForward):
             projected = torch.full_like(logits, float("-inf")).scatter_(1, take, logits.gather(1, take))
         if projected is None:
             hipops.router_top1(x32, self.w_router, expert, weight)
-        n = 2 * T if self.fused_shared else T
-        src, dst = ws.take((n,), torch.int32), ws.take((n,), torch.int32)
-        scale = ws.take((n,), torch.float32)
-        groups = E + 1 if self.fused_shared else E
-        offsets = ws.take((groups + 1,), torch.int32)
-        hipops.moe_plan(expert, weight, src, scale, dst, offsets, T, E, self.fused_shared, logits=projected)
+        n, groups = (2 * T, E + 1) if self.fused_shared else (T, E)
+        if plan is None:
+            hipops.moe_plan(expert, weight, src, scale, dst, offsets, T, E, self.fused_shared, logits=projected)
         if trace is not None:                         # a testing aid: which expert each row took
             trace.setdefault("moe_experts", []).append(expert.clone())
         act = ws.take((n, F), x.dtype)

@@ -37,14 +37,18 @@ class RMSNorm(Norm):
         return proj.dtype == torch.float32 and proj.dim() == 2 and proj.shape[1] == self.width \
             and hipops.add_rmsnorm_can_project(self.width)
 
+    def can_plan(self, proj, rows: int) -> bool:
+        # the one row's logits stay in LDS behind it
+        return rows == 1 and self.can_project(proj) and hipops.add_rmsnorm_can_project(self.width, proj.shape[0])
+
     def forward(self, h, out, *, d1=None, d2=None, out32=None, rows=None, write_h=True, proj=None, proj_out=None,
-                normed=None, second=None):
+                normed=None, second=None, plan=None):
         """``normed``: a ``NormedIncrement``'s (y, weight, mult, eps), added like d1 and d2 after its own norm.
         ``second`` = (another RMS norm of the same eps, its output): the same rows under that norm's
-        weights too, in one pass (a layer with two norms of one stream)."""
+        weights too, in one pass (a layer with two norms of one stream).  ``plan``: see ``can_plan``."""
         hipops.add_rmsnorm(h, self.weight, self.eps, out=out, out32=out32, d1=d1, d2=d2, rows=rows,
                            n_rows=(rows.numel() if rows is not None else h.shape[0]), write_h=write_h,
-                           proj=proj, proj_out=proj_out, normed=normed,
+                           proj=proj, proj_out=proj_out, normed=normed, plan=plan,
                            w2=second[0].weight if second is not None else None, out2=second[1] if second is not None else None)
 
     def takes(self, increment) -> bool:
