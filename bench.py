@@ -166,9 +166,9 @@ class KernelTimes:
     of each kind of kernel in eager steps, without a profiler."""
 
     NAMES = ("embed", "add_rmsnorm", "rope_kvwrite", "router_top1", "moe_plan", "convert", "gemm_generic",
-             "attn_generic", "gemm_skinny", "gemm_mfma", "gemm_tiled", "attn_decode", "attn_prefill",
+             "attn_generic", "gemm_skinny", "gemm_mfma", "gemm_tiled", "gemm_lds", "attn_decode", "attn_decode_rope", "attn_prefill",
              "sample_rows", "argmax_rows", "filter_rows", "latent_prepare", "attn_latent_generic", "attn_latent_mfma",
-             "router_topk", "moe_combine", "gated_rows", "add_into",
+             "router_topk", "router_plan", "moe_combine", "gated_rows", "add_into",
              "qkv_prepare", "attn_wide", "attn_finish", "token_shift", "act_rows",
              "linear_attn_scan", "channel_decay", "gated_group_norm", "scale_rows",
              "add_tanh_norm", "hash_rows", "embed_sum", "causal_conv", "shift_mix", "step_decay", "softcap_rows",

@@ -50,7 +50,7 @@ class Weight:
         if self.dtype == torch.bfloat16 and self.shape[-1] % 8:
             return [f"{name} {self.shape}: rows of {self.shape[-1]} are no multiple of 8, its products run on plain FMAs"]
         if self.dtype == torch.float32:
-            return [f"{name} {self.shape}: kept in 32-bit by the checkpoint, its products run on plain FMAs"]
+            return [f"{name} {self.shape}: kept in 32-bit by the checkpoint, and so are its products"]
         return []
 
     def group(self, g: int) -> "Weight":
