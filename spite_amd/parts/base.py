@@ -212,7 +212,8 @@ class FeedForward(Part):
         return None
 
     def plan_arrays(self, rows: int, ctx):
-        """Arrays that a norm which ``can_plan`` fills from the logits, or None; ``forward`` then gets them as ``plan``."""
+        """Arrays that a norm which ``can_plan`` fills from the logits, or None; ``forward`` then gets them as ``plan``
+        (only asked for where the ``forward`` of both takes one)."""
         return None
 
     def forward(self, x, x32, ctx, projected=None):

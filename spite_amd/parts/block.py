@@ -4,6 +4,8 @@ h += mixer(norm1(h)); h += ffn(norm2(h)) (crates/spite-models/src/llama/llama4.r
 its last increments to the next block (or the final norm) instead of adding them itself."""
 from __future__ import annotations
 
+import inspect
+
 import torch
 
 from .base import Block, NormedIncrement, NORMED_INCREMENTS, register, build as build_part, two_increments
@@ -25,10 +27,17 @@ def run_mixer(mixer, x, state, ctx, cache):
     return out
 
 
+def takes_plan(norm, ffn) -> bool:
+    """Whether both hand a plan from the one to the other (``Norm.can_plan``).  A kind of part made from one that does, with
+    a ``forward`` of its own, need not know of it, and chooses from the logits itself."""
+    return all("plan" in inspect.signature(part.forward).parameters for part in (norm, ffn))
+
+
 @register("block", "prenorm")
 class PreNormBlock(Block):
     """The feed-forward (and its norm) may be missing."""
     graph_safe = True
+    _plans = False
 
     def __init__(self, env, spec):
         self.env = env
@@ -40,6 +49,7 @@ class PreNormBlock(Block):
             self.norm2 = build_part("norm", spec.norm2, env)
             self.ffn = build_part("ffn", spec.ffn, env)
             self.children += (("norm2", self.norm2, spec.norm2), ("ffn", self.ffn, spec.ffn))
+        self._plans = self.ffn is not None and takes_plan(self.norm2, self.ffn)
         self.graph_safe = all(part.graph_safe for _, part, _ in self.children)
         self.step_arrays = tuple(sorted({a for _, part, _ in self.children for a in part.step_arrays}))
 
@@ -76,7 +86,7 @@ class PreNormBlock(Block):
         if proj is not None and self.norm2.can_project(proj):
             # the norm forms the feed-forward's small fp32 products (router logits) itself
             logits = ws.take((T, proj.shape[0]), torch.float32)
-            plan = self.ffn.plan_arrays(T, ctx) if self.norm2.can_plan(proj, T) else None
+            plan = self.ffn.plan_arrays(T, ctx) if self._plans and self.norm2.can_plan(proj, T) else None
             more = {"plan": plan} if plan is not None else {}
             self.norm2.forward(h, n2, d1=delta, proj=proj, proj_out=logits, **more)
             state["pending"] = tuple(self.ffn.forward(n2, None, ctx, projected=logits, **more))
