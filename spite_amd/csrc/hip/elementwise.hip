@@ -740,7 +740,8 @@ void moe_plan_hist_kernel(int* __restrict__ expert, float* __restrict__ weight,
 extern "C" int spite_moe_plan(int* expert, float* weight, const float* logits, int* src, float* scale, int* dst,
                               int* offsets, int T, int E, int shared, int fan, hipStream_t st) {
     SP_REQUIRE(T >= 0 && E > 0 && E < 65535, "moe_plan: bad sizes T=%d E=%d", T, E);
-    SP_REQUIRE(fan >= 1 && T % fan == 0 && (fan == 1 || !logits), "moe_plan: a fan of %d goes with given experts, T=%d a multiple of it", fan, T);
+    SP_REQUIRE(fan >= 1 && (fan == 1 || !logits), "moe_plan: a fan of %d goes with given experts", fan);
+    SP_REQUIRE(!shared || T % fan == 0, "moe_plan: shared groups of %d entries, %d a token", T, fan);
     SP_REQUIRE(shared >= 0 && shared <= 64, "moe_plan: %d shared groups", shared);
     SP_REQUIRE(T <= ((T > 256 && E <= PLAN_MAX_E) ? (1 << 22) : 32768), "moe_plan: %d entries in one step are too many", T);
     const int grid = T > 0 ? (T + 255) / 256 : 1;

@@ -308,8 +308,8 @@ def moe_plan(expert, weight, src, scale, dst, offsets, T, E, shared, logits=None
     ``fan`` > 1: the T entries are ``fan`` choices in a row for each of T / fan tokens; ``src`` names
     the token (entry // fan), ``dst`` the entry.  ``shared``: so many groups behind the experts' that every
     token visits."""
-    if T % int(fan):
-        raise KernelError(f"moe_plan: {T} entries of {fan} a token")
+    if shared and T % int(fan):
+        raise KernelError(f"moe_plan: {T} entries of {fan} a token, and shared groups of whole tokens")
     n = T + int(shared) * (T // int(fan))
     if src.numel() < n or scale.numel() < n or dst.numel() < n or offsets.numel() < E + 1 + int(shared):
         raise KernelError("moe_plan: output arrays too small")

@@ -45,3 +45,21 @@ def test_combine_adds_the_parts_of_the_extra_row(parts, d):
     hipops.moe_combine(y.to(DEV), w.to(DEV), ex.to(DEV), out, T, top, n_extra=parts)
     ref = (y.double().view(T, top, d) * w.double().view(T, top, 1)).sum(1) + ex.double().view(parts, T, d).sum(0)
     assert (out.cpu().double() - ref).abs().max() < 1e-5 * float(ref.abs().max())      # a few fp32 roundings
+
+
+@pytest.mark.parametrize("T,fan", [(7, 2), (1, 4), (601, 3)])
+def test_plan_of_entries_that_end_inside_a_token(T, fan):
+    """Without groups that every token visits, the last token may bring fewer entries than the others."""
+    from spite_amd.csrc import hipops
+    E = 5
+    expert = torch.randint(0, E, (T,), generator=torch.Generator().manual_seed(T), dtype=torch.int32)
+    weight = torch.rand(T, generator=torch.Generator().manual_seed(1))
+    src, dst, offsets = (torch.full((n,), -7, dtype=torch.int32, device=DEV) for n in (T, T, E + 1))
+    scale = torch.empty(T, device=DEV)
+    hipops.moe_plan(expert.to(DEV), weight.to(DEV), src, scale, dst, offsets, T, E, False, fan=fan)
+    order = torch.argsort(expert, stable=True)
+    assert torch.equal(dst.cpu().long(), order) and torch.equal(src.cpu().long(), order // fan) and torch.equal(scale.cpu(), weight[order])
+    assert offsets.cpu().tolist() == [int((expert < e).sum()) for e in range(E + 1)]
+    with pytest.raises(hipops.KernelError):                # (a group of whole tokens has no row list then)
+        hipops.moe_plan(expert.to(DEV), weight.to(DEV), torch.cat([src] * 2), torch.cat([scale] * 2), torch.cat([dst] * 2),
+                        torch.cat([offsets] * 2), T, E, True, fan=fan)
