@@ -135,10 +135,14 @@ void router_topk_kernel(const float* __restrict__ logits, const float* __restric
 }
 
 // The choice and the row list of the grouped products (moe_plan with a fan of `top` and `shared` groups that every token
-// visits) of a step of few tokens by one workgroup: two kernels of 4.5 us each, of which next to nothing is work, become
-// one.  The entries' experts stay in LDS in between; ranks are counted as moe_plan_kernel counts them.
+// visits) of a step of a few tokens by one workgroup, a wave a token: two kernels become one.  Both are a chain of
+// latencies: the logits' load, then six steps of shuffles for every expert that is taken.  Measured on an
+// MI355X, one launch against two, us: 1 token, 1 of 16 experts 3.1 / 4.0, 4 of 64 5.1 / 6.0; 8 tokens, 2 of 16 4.5 / 5.7, 8 of
+// 128 11.0 / 11.7, 8 of 512 17.7 / 18.4.  No second token a wave: its choice would wait for the first one's, which
+// router_topk's further workgroups do not (16 tokens, 8 of 64 17.8 / 12.9; 64 tokens, 8 of 128 72 / 16; 512 tokens, 1 of 16
+// 95 / 9.7).  The entries' experts stay in LDS in between; ranks are counted as moe_plan_kernel counts them.
 #define RP_NT 512
-#define RP_MAX 512       // entries at most: each is ranked by a thread that looks at all of them
+#define RP_MAX (RP_NT / 64 * 64)       // entries: a token a wave, up to 64 experts each; a thread ranks one
 template <int NU>
 __global__ __launch_bounds__(RP_NT)
 void router_plan_kernel(const float* __restrict__ logits, const float* __restrict__ bias, int* __restrict__ expert,
@@ -147,7 +151,8 @@ void router_plan_kernel(const float* __restrict__ logits, const float* __restric
                         int* __restrict__ offsets, int shared) {
     __shared__ unsigned short e_of[RP_MAX];
     const int lane = threadIdx.x & 63, n = T * top;
-    for (int t = threadIdx.x >> 6; t < T; t += RP_NT / 64) {
+    const int t = threadIdx.x >> 6;
+    if (t < T) {
         const int e = topk_of_token<NU>(logits, bias, expert, weight, t, lane, E, ld, top, renorm, mode, n_groups, keep_groups);
         if (lane < top) e_of[t * top + lane] = (unsigned short)e;
     }
@@ -197,14 +202,17 @@ extern "C" int spite_router_topk(const float* logits, const float* bias, int* ex
 extern "C" int spite_moe_plan(int* expert, float* weight, const float* logits, int* src, float* scale, int* dst,
                               int* offsets, int T, int E, int shared, int fan, hipStream_t st);
 
+// Whether router_plan makes choice and row list in one launch.
+extern "C" int spite_router_plan_is_one_launch(int T, int top) { return T > 0 && T <= RP_NT / 64 && top <= 64; }
+
 // router_topk, then moe_plan over its T * top entries with `shared` groups of T rows behind the experts'; in one launch
-// where the entries fit a workgroup.
+// for a few tokens.
 extern "C" int spite_router_plan(const float* logits, const float* bias, int* expert, float* weight, int T, int E, int ld, int top,
                                  int renorm, int mode, int n_groups, int keep_groups, int* src, float* scale, int* dst,
                                  int* offsets, int shared, hipStream_t st) {
     if (int rc = topk_check(T, E, ld, top, mode, n_groups, keep_groups)) return rc;
     SP_REQUIRE(shared >= 0 && shared <= 64, "router_plan: %d shared groups", shared);
-    if (T == 0 || top > 64 || (long)T * top > RP_MAX) {
+    if (!spite_router_plan_is_one_launch(T, top)) {
         if (int rc = spite_router_topk(logits, bias, expert, weight, T, E, ld, top, renorm, mode, n_groups, keep_groups, st)) return rc;
         return spite_moe_plan(expert, weight, nullptr, src, scale, dst, offsets, T * top, E, shared, top, st);
     }

@@ -116,6 +116,8 @@ def lib():
         l.spite_attn_prefill_workspace.restype = c_size_t
         l.spite_delta_chunk_workspace.argtypes = [I, I, I, I]
         l.spite_delta_chunk_workspace.restype = c_size_t
+        l.spite_router_plan_is_one_launch.argtypes = [I, I]
+        l.spite_router_plan_is_one_launch.restype = c_int
         l.spite_gemm_lds_time.argtypes = [I, I, I, I]
         l.spite_gemm_lds_time.restype = ctypes.c_double
         l.spite_cu_count.argtypes = []
@@ -909,7 +911,7 @@ def _topk_sizes(logits, bias, expert, weight, top, scoring, groups, n_experts):
 def router_plan(logits, bias, expert, weight, top, src, scale, dst, offsets, shared=0, renorm=False, scoring="sigmoid", groups=None,
                 n_experts=None):
     """``router_topk``, and ``moe_plan`` over its T * top entries (``fan`` = top) with ``shared`` groups that every token
-    visits, in one launch for a step of few tokens."""
+    visits, in one launch for a step of few tokens (the kernel's comment has both sides' times)."""
     T, E, count, keep = _topk_sizes(logits, bias, expert, weight, top, scoring, groups, n_experts)
     n = T * (top + int(shared))
     if src.numel() < n or scale.numel() < n or dst.numel() < n or offsets.numel() < E + 1 + int(shared):

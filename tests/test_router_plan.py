@@ -63,3 +63,8 @@ def test_plan_of_entries_that_end_inside_a_token(T, fan):
     with pytest.raises(hipops.KernelError):                # (a group of whole tokens has no row list then)
         hipops.moe_plan(expert.to(DEV), weight.to(DEV), torch.cat([src] * 2), torch.cat([scale] * 2), torch.cat([dst] * 2),
                         torch.cat([offsets] * 2), T, E, True, fan=fan)
+
+
+@pytest.mark.parametrize("T,E,top,shared", [(8, 512, 64, 1), (8, 4, 1, 2), (9, 16, 4, 1), (10, 64, 50, 0)])
+def test_on_both_sides_of_a_token_a_wave(T, E, top, shared):
+    test_router_plan(T, E, top, shared, "sigmoid", None)
