@@ -29,3 +29,13 @@ def test_router_plan_is_one_launch_for_a_token_a_wave():
     one = lib().spite_router_plan_is_one_launch
     assert all(one(T, top) for T in (1, 5, 8) for top in (1, 8, 64))
     assert not any(one(T, top) for T in (0, 9, 64, 512) for top in (1, 8)) and not one(4, 65)
+
+
+def test_latent_splits_beyond_a_window_and_for_many_items():
+    """Sizes at which both sides were timed: long contexts for few items, and more items than half the compute units."""
+    from spite_amd.csrc.hipops import latent_splits
+    at = lambda n, *row: [latent_splits(n, k, *row) for k in (4096, 8192, 16384, 32768)]
+    assert at(1) == [32, 64, 128, 256] and at(2) == [32, 64, 128, 128] and at(4) == [32, 64, 64, 64] and at(8) == [32] * 4
+    assert latent_splits(1, 131072) == 256 and latent_splits(6, 16384) == 42
+    for n in (100, 150, 200, 255):                       # narrow rows: several workgroups a unit
+        assert latent_splits(n, 2048, 192, 128) == -(-256 // n) and latent_splits(n, 2048) == 256 // n
