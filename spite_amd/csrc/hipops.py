@@ -545,13 +545,26 @@ def attn_decode(q, k_pages, v_pages, out, workspace, positions, seq_of_token, bl
 
 def attn_decode_splits(heads: int, longest: int) -> int:
     """Into how many workgroups the keys of each of ``heads`` (tokens times kv heads) are dealt, none of which reads more than
-    ``longest``: about two workgroups a compute unit (more only add records to join), each with at least a block of 32 keys
-    for every one of its four waves (8 heads of 1,000 keys on an MI355X: 13.2 us with four splits, 10.2 with eight, 10.3
-    with sixteen); one, which needs no second kernel, where two of at most eight blocks would be left (256 heads of 500
-    keys: 18.6 against 21.6 us)."""
-    blocks = -(-longest // 32)
-    n = max(1, min(-(-2 * cu_count() // max(heads, 1)), -(-blocks // 4), 256))
-    return 1 if n <= 2 and blocks <= 16 else n
+    ``longest``: about two workgroups a compute unit at most (more only add records to join).  (us on an MI355X, one layer's
+    attention.)  One split needs no second kernel: up to 12 blocks of 32 keys for few heads (8 heads, 12 blocks: 7.6 us with one, 9.1 with two).  Beyond, shares of
+    five blocks and more for few heads, of which a wave each takes one or two (8 heads of 1,000 keys: 11.2 with four splits,
+    8.2 with eight, 8.6 with sixteen), beyond 64 splits of eight (4 heads, 256 blocks: 11.0 with 61, 14.3 with 122); in powers of two
+    and multiples of eight, as the joining kernel has eight records' loads in flight (16 heads, 64 blocks: 9.6 with sixteen,
+    11.7 with twelve, 14.1 with six).  From 64 heads on a few blocks fill the chip as they are: shares of eight blocks (64
+    heads, 12 blocks: 11.7 with three, 14.1 with six); two splits of up to 32 blocks are worth less than their second kernel
+    (256 heads of 500 keys: 14.8 with one, 19.0 with two).  (``longest`` is the width of a table, which the contexts fill by
+    half at least: timed at 1, 1.5 and 1.95 times the keys.)"""
+    blocks, room = -(-longest // 32), max(1, -(-2 * cu_count() // max(heads, 1)))
+    if room <= 2 and blocks <= 32:
+        return 1
+    if heads >= 64 and blocks < 32:
+        return min(room, -(-blocks // 8))
+    if blocks <= 12:
+        return 1
+    n = min(room, max(blocks // 5, 8), 256)
+    if n < 128:
+        n = 1 << (n.bit_length() - 1)
+    return n if n <= 64 else max(64, min(n, blocks // 8) // 8 * 8)
 
 
 def attn_decode_rope(qkv, k_pages, v_pages, out, workspace, positions, slot_map, seq_of_token, block_table, T, H, G, hd,

@@ -39,3 +39,17 @@ def test_latent_splits_beyond_a_window_and_for_many_items():
     assert latent_splits(1, 131072) == 256 and latent_splits(6, 16384) == 42
     for n in (100, 150, 200, 255):                       # narrow rows: several workgroups a unit
         assert latent_splits(n, 2048, 192, 128) == -(-256 // n) and latent_splits(n, 2048) == 256 // n
+
+
+def test_decode_attention_splits():
+    """Where the rule's lines lie, at sizes that were timed with every count of splits."""
+    from spite_amd.csrc.hipops import attn_decode_splits
+    at = lambda heads, *blocks: [attn_decode_splits(heads, 32 * b) for b in blocks]
+    assert at(8, 1, 12, 13, 32, 64, 128, 256, 500, 1000, 4000) == [1, 1, 8, 8, 8, 16, 32, 64, 64, 64]
+    assert at(2, 320, 500, 1024, 2000) == [64, 64, 128, 248]            # shares of eight blocks, not of four
+    assert at(64, 8, 12, 31, 32, 1000) == [1, 2, 4, 8, 8] and at(128, 16, 31, 500) == [2, 4, 4]
+    assert at(256, 9, 32, 33) == [1, 1, 2] and at(512, 500) == [1] and at(5000, 5000) == [1]
+    for heads in (1, 3, 40, 100, 300):
+        for blocks in range(1, 2100, 7):
+            n = attn_decode_splits(heads, 32 * blocks)
+            assert 1 <= n <= 256 and n <= -(-512 // heads) and (n < 8 or n % 8 == 0)
