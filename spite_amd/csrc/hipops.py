@@ -567,6 +567,14 @@ def attn_decode_splits(heads: int, longest: int) -> int:
     return n if n <= 64 else max(64, min(n, blocks // 8) // 8 * 8)
 
 
+def attn_decode_rope_suits(heads: int) -> bool:
+    """Whether rotation and cache write are better done inside the decode attention of ``heads`` (tokens times kv heads): up to
+    two workgroups a compute unit, where they cost a launch less, about 2 us.  Beyond, every further workgroup that a unit
+    takes up waits for its sines and its query's norm before it asks for keys (4,096 workgroups of 256 keys: 115 us against 108
+    in two kernels; 1,536 of 4,096: 313 against 305)."""
+    return heads <= 2 * cu_count()
+
+
 def attn_decode_rope(qkv, k_pages, v_pages, out, workspace, positions, slot_map, seq_of_token, block_table, T, H, G, hd,
                      page_size, vis, span, scale, n_splits, inv_freq=None, norm_eps=0.0, temperature=None, softcap=0.0, slopes=None):
     """``rope_kvwrite`` and ``attn_decode`` in one for decoded tokens: ``qkv`` [T, (H+2G)*hd] are the projection's rows, whose

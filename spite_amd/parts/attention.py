@@ -170,7 +170,7 @@ class Attention(Mixer):
         temp = self.temperature
         # the MFMA kernels read pages in operand order (bfloat16, sizes in multiples of 32)
         mfma = cache.tiled and hd in (64, 128)
-        if ctx.decode_only and mfma and H // G <= 16 and cache.write and self._fusable(ka):
+        if ctx.decode_only and mfma and H // G <= 16 and cache.write and self._fusable(ka) and hipops.attn_decode_rope_suits(T * G):
             o = ws.take((T, H * hd), x.dtype)
             self._decode(qkv, o, ctx, cache, T, fused=dict(inv_freq=ka["inv_freq"] if ka["use_rope"] else None, temperature=temp,
                                                            norm_eps=self.qk_norm_eps if self.qk_norm else 0.0))
