@@ -707,13 +707,17 @@ def lds_suits(M: int, N: int, K: int, glu: bool, runs: int) -> bool:
     return lds <= tiled
 
 
-def lds_suits_groups(group_rows: float, K: int) -> bool:
-    """The same for a product over groups of ``group_rows`` rows each on average (beside groups that take every row).  Fewer
-    rows make its 256 rows of W a tile ask for more operands a product than the 512 of ``gemm_tiled`` do.  (us with
-    gemm_lds / gemm_tiled at K = 5,120 gated, and at the product back: 223 rows 570 / 591 and 335 / 350, 150 rows 487 / 538 and
-    304 / 330, 128 rows 822 / 720 and 522 / 460, 97 rows 751 / 642 and 491 / 432; sums over 1,024 k end before the depth of
-    its loads pays: 383 rows 74 / 68.)"""
-    return group_rows >= 140 and K >= 2048
+def lds_suits_groups(group_rows: float, K: int, tiles: int = 0, lds_tiles: int = 0) -> bool:
+    """The same for a product over groups of ``group_rows`` rows each on average (beside groups that take every row), which
+    are to be ``tiles`` tiles of ``gemm_tiled`` and ``lds_tiles`` of ``gemm_lds``: where the first ones leave three of eight
+    compute units and more without a tile and the others, half as wide, still fit one round.  With more tiles the 256
+    rows of W a tile ask for more operands a product than the 512 of ``gemm_tiled`` do.  (Timed at 520 products of 2 to 128
+    groups of 60 to 4,000 rows; us with gemm_lds / gemm_tiled.  One round: 384 rows x 2 x 2,048 x 7,168, 140 / 192; 308 x 2 x
+    2,048 x 4,096 75 / 96; the 48 that the line takes in at any rows a group are 15 % faster on average, one of them 2 % slower.
+    More: 32 groups of 128 rows 822 / 720; 8 of 165 346 / 252; 16 of 415 586 / 539; 4 of 1,152, unevenly, 152 / 104.  Sums
+    over 2,048 k and fewer end before the depth of its loads pays: 59 / 53 in one round.)"""
+    cus = cu_count()
+    return group_rows >= 140 and K >= 2560 and tiles <= 5 * cus // 8 and lds_tiles <= cus
 
 
 def gemm_lds(a, w, y, M, N, K, *, offsets=None, n_groups=1, a_rows=None, a_scale=None, y_rows=None, glu=False, act=None,

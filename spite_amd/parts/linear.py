@@ -135,6 +135,15 @@ def whole_group_apart(tokens: int, groups: int, N: int, K: int) -> int:
     return shape if routed + hipops.lds_us(tokens, N, K, False) < together else 0
 
 
+def _group_tiles(M, n_groups, most, group_rows, N, glu):
+    """The tiles of ``gemm_tiled`` and of ``gemm_lds`` to expect of a product over groups (arguments as ``linear``'s)."""
+    mean = M / n_groups if group_rows is None else group_rows
+    # the groups that take every row: what the rows of the call leave over the routed ones'
+    whole = min(max(round((M - n_groups * mean) / (most - mean)), 0), n_groups - 1) if most > mean else 0
+    tiles = lambda rows, cols: ((n_groups - whole) * math.ceil(mean / rows) + whole * -(-most // rows)) * -(-N // cols)
+    return tiles(128, 256 if glu else 512), tiles(256, 128 if glu else 256)
+
+
 def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale=None, y_rows=None, rows=None,
            max_rows=None, tile_shape=0, live_groups=0, group_rows=None, ws=None, act=None):
     """y[r] = W . x[r] for ``rows`` rows (default: all of x; for a row list: its length).
@@ -172,7 +181,8 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
             runs = hipops.tiled_k_runs(M, N, K) if splits and tile_shape == 0 and M > 0 else 1
             if M > 0 and hipops.gemm_lds_ok(x, w, M, N, K, glu) and (
                     hipops.lds_suits(M, N, K, bool(glu), runs) if offsets is None
-                    else hipops.lds_suits_groups(M / n_groups if group_rows is None else group_rows, K)):
+                    else hipops.lds_suits_groups(M / n_groups if group_rows is None else group_rows, K,
+                                                 *_group_tiles(M, n_groups, most, group_rows, N, bool(glu)))):
                 hipops.gemm_lds(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
                                 y_rows=y_rows, glu=glu, act=act, act_limit=limit)
                 return

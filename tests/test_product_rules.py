@@ -53,3 +53,17 @@ def test_decode_attention_splits():
         for blocks in range(1, 2100, 7):
             n = attn_decode_splits(heads, 32 * blocks)
             assert 1 <= n <= 256 and n <= -(-512 // heads) and (n < 8 or n % 8 == 0)
+
+
+def test_groups_of_many_tiles_stay_with_the_tiled_product():
+    """The line between the two products over groups, at sizes that were timed on both sides of it."""
+    from spite_amd.csrc.hipops import lds_suits_groups
+    from spite_amd.parts.linear import _group_tiles
+    def suits(T, E, top, whole, N, K, glu):
+        return lds_suits_groups(T * top / E, K, *_group_tiles(T * (top + whole), E + whole, T, T * top / E, N, glu))
+    assert _group_tiles(2 * 2048, 17, 2048, 128.0, 8192, True) == (32 * 32, 24 * 64)       # 16 experts and a shared one
+    assert _group_tiles(700, 7, 700, None, 512, False) == (7, 14)
+    assert suits(692, 8, 4, 0, 1024, 4096, True) and suits(533, 4, 2, 0, 2048, 5120, False)
+    for slower in ((1416, 8, 1, 1, 5120, 8192, False), (4608, 4, 1, 1, 2048, 3072, False), (694, 4, 2, 1, 3072, 2048, True),
+                   (3199, 8, 1, 1, 5120, 8192, False), (1786, 16, 2, 2, 4096, 5120, True), (6992, 128, 4, 1, 1024, 2048, True)):
+        assert not suits(*slower), slower
