@@ -100,19 +100,19 @@ def _group_size(tokens, groups):
     return tokens / groups, max(math.sqrt(tokens * (1.0 / groups) * (1.0 - 1.0 / groups)), 1e-6)
 
 
-def _row_tiles(tokens, groups, whole_groups, rows_per_tile, sure=False):
-    """The row tiles to expect; ``sure``: a standard deviation more (each further tile of a group comes or does not)."""
+def _row_tiles(tokens, groups, whole_groups, rows_per_tile, deviations=0.0):
+    """The row tiles to expect, and so many standard deviations more (each further tile of a group comes or does not)."""
     mean, sd = _group_size(tokens, groups)
     extra, spread, k = 0.0, 0.0, 1
     while k * rows_per_tile < mean + 6 * sd:
         p = 0.5 * math.erfc((k * rows_per_tile + 0.5 - mean) / (sd * math.sqrt(2.0)))
         extra, spread, k = extra + p, spread + p * (1.0 - p), k + 1
-    return groups * (1.0 + extra) + (math.sqrt(groups * spread) if sure else 0.0) + whole_groups * -(-tokens // rows_per_tile)
+    return groups * (1.0 + extra) + deviations * math.sqrt(groups * spread) + whole_groups * -(-tokens // rows_per_tile)
 
 
-def _rounds(tokens, groups, whole_groups, col_tiles, cus, sure=False):
-    """(tile shape, its rounds over the chip times its tile's cost)."""
-    rounds = lambda rows: math.ceil(_row_tiles(tokens, groups, whole_groups, rows, sure) * col_tiles / cus - 1e-9)
+def _rounds(tokens, groups, whole_groups, col_tiles, cus, deviations=0.0, full=1.0):
+    """(tile shape, its rounds over the chip times its tile's cost); ``full``: how much of a round may be counted on."""
+    rounds = lambda rows: math.ceil(_row_tiles(tokens, groups, whole_groups, rows, deviations) * col_tiles / (full * cus) - 1e-9)
     wide, narrow = TILE_160_COST * rounds(160), float(rounds(128))
     return (3, wide) if wide < narrow else (1, narrow)
 
@@ -121,18 +121,21 @@ def _rounds(tokens, groups, whole_groups, col_tiles, cus, sure=False):
 def whole_group_apart(tokens: int, groups: int, N: int, K: int) -> int:
     """Whether a plain product over ``groups`` groups that ``tokens`` rows spread over and one group that takes every row
     is better done as two: the groups (the result is the tile shape that they then take, 0: together), and the one as a
-    product of its own with both operands in LDS.  Together the
-    tiles of the second kind fill the first one's last round; apart it may need one round fewer.  A round takes 146 us
-    at K = 5,120 and the groups no less than their weights at 5.6 TB/s (measured at 5,120 x 8,192 over 16 experts, together
-    / apart: 2,048 tokens 466 / 421 us, 1,547 426 / 360, 1,200 292 / 346).  A gated product's rounds are many and its
-    stream of weights long: there it never paid (2,048 tokens 719 / 759)."""
-    cus, round_us = hipops.cu_count(), 146.0 * K / 5120.0
-    cols = -(-N // 512)
-    together = round_us * _rounds(tokens, groups, 1, cols, cus)[1]
-    # (the groups alone need few rounds: one that they miss by a tile would cost what is to be gained)
-    shape, cost = _rounds(tokens, groups, 0, cols, cus, sure=True)
+    product of its own.  Together the tiles of the second kind fill the first one's last round; apart it may need one round
+    fewer.  A round takes 146 us at K = 5,120 and the groups no less than their weights at 5.6 TB/s.  Routers do not
+    spread their rows quite evenly, and a round that the groups miss by a tile costs more than is to be gained: with a standard
+    deviation of tiles more they have to fit 85 % of their rounds, and the two to be 6 % faster than all tiles together with a
+    deviation fewer.
+    (Measured at 300 sizes, 2 to 64 experts, 200 to 6,000 tokens: of the 29 that this takes in none is slower apart, on
+    average they are 10 % faster; with neither margin 15 of 58 were slower, by up to 42 %.  5,120 x 8,192 over 16 experts,
+    together / apart: 1,454 tokens 433 / 346 us, 1,547 425 / 362, 2,048 448 / 432; over 8: 1,806 398 / 345; 3,072 x 8,192 over 16:
+    3,107 431 / 360.)  A gated product's rounds are many and its stream of weights long: there it never paid (2,048 tokens
+    719 / 759)."""
+    cus, round_us, cols = hipops.cu_count(), 146.0 * K / 5120.0, -(-N // 512)
+    together = round_us * _rounds(tokens, groups, 1, cols, cus, deviations=-1.0)[1]
+    shape, cost = _rounds(tokens, groups, 0, cols, cus, deviations=1.0, full=0.85)
     routed = max(round_us * cost, groups * N * K * 2 / 5.6e6)
-    return shape if routed + hipops.lds_us(tokens, N, K, False) < together else 0
+    return shape if routed + hipops.lds_us(tokens, N, K, False) < 0.94 * together else 0
 
 
 def _group_tiles(M, n_groups, most, group_rows, N, glu):

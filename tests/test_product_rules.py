@@ -67,3 +67,13 @@ def test_groups_of_many_tiles_stay_with_the_tiled_product():
     for slower in ((1416, 8, 1, 1, 5120, 8192, False), (4608, 4, 1, 1, 2048, 3072, False), (694, 4, 2, 1, 3072, 2048, True),
                    (3199, 8, 1, 1, 5120, 8192, False), (1786, 16, 2, 2, 4096, 5120, True), (6992, 128, 4, 1, 1024, 2048, True)):
         assert not suits(*slower), slower
+
+
+def test_whole_group_stays_where_apart_was_slower():
+    """Rounds that the groups alone would miss by a tile, and sizes at which the two take the same time."""
+    for tokens, groups, N, K in ((2889, 8, 5120, 4096), (2510, 16, 5120, 4096), (2520, 16, 5120, 8192), (5548, 16, 5120, 4096),
+                                 (4291, 16, 5120, 8192), (3252, 2, 5120, 4096), (5255, 8, 2560, 1024), (4096, 32, 5120, 4096),
+                                 (2500, 8, 5120, 8192), (6000, 8, 2560, 1024)):
+        assert whole_group_apart(tokens, groups, N, K) == 0, (tokens, groups, N, K)
+    for tokens, groups, N, K in ((1454, 16, 5120, 8192), (1806, 8, 5120, 8192), (3107, 16, 3072, 8192), (2553, 8, 4096, 14336)):
+        assert whole_group_apart(tokens, groups, N, K) == 1, (tokens, groups, N, K)
