@@ -240,9 +240,12 @@ class MoeTop1Sigmoid(FeedForward):
         return (y[:T], y[T:])
 
 
-# groups that a shared expert may make beside the routed ones: each adds a row of d numbers a token to what the combining
-# kernel reads
-SHARED_GROUPS_MAX = 4
+# Groups that a shared expert may make beside the routed ones.  Each adds a row of d numbers a token to what the product
+# back writes and the combining kernel reads, where one product of its own adds up over k: in long prompts that outweighs
+# the launches from three groups on.  (A layer's experts against the same with products of their own, on an MI355X, 1 to 6,000
+# tokens: one group 0.78 to 1.02 of the time at five sizes, two 0.71 to 1.03 at three; three 4,096 x 1,024 over 64 experts
+# 1.04 and four 5,120 x 2,048 over 32 1.03 to 1.06 from 2,300 tokens on.)
+SHARED_GROUPS_MAX = 2
 
 
 @register("ffn", "moe_topk_sigmoid")
