@@ -309,9 +309,11 @@ class MoeTopKSigmoid(FeedForward):
         dt = torch.float32 if len(dts) > 1 else dts.pop()
         # A shared expert as wide as several routed ones is that many more groups that every token visits (its inner
         # elements are independent of each other, and its result the sum over them): two products a layer instead of
-        # four, and more tiles in each.
+        # four, and more tiles in each.  Not where its whole width has what the width of one lacks: rows in operand order
+        # (multiples of 64, 16 beside each other), or such as the matrix units read at all (8; in 32-bit 4).
         F, m = self.F, 0
         if self.Fs is not None and self.Fs % F == 0 and self.Fs // F <= SHARED_GROUPS_MAX and self.shared_activation == self.activation \
+                and all((self.Fs % q == 0) == (F % q == 0) for q in (4, 8, 16, 64)) \
                 and all(t[f"shared.{x}"].dtype == dt for x in ("gate", "up", "down")):
             m = self.Fs // F
         self.shared_groups = m

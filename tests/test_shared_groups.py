@@ -22,3 +22,10 @@ def groups_of(F, Fs, dtype=torch.bfloat16):
 def test_up_to_two_groups(F, Fs, m):
     """From three on the rows that the product back writes for each cost long prompts more than the launches they save."""
     assert groups_of(F, Fs) == m
+
+
+@pytest.mark.parametrize("F,Fs,m", [(20, 40, 0), (24, 48, 0), (32, 64, 0), (96, 192, 0), (40, 80, 0), (48, 96, 2), (12, 24, 0), (10, 20, 0), (16, 32, 2), (10, 10, 1)])
+def test_no_groups_that_lose_the_matrix_units_or_the_operand_order(F, Fs, m):
+    """The whole width is a multiple of 8, 16 or 64 where the groups' width is not: their products would run on plain FMAs,
+    or read rows where tiles were."""
+    assert groups_of(F, Fs) == m
