@@ -195,6 +195,53 @@ static int launch_skinny(const void* X, int ldx, const void* W, long wgs, void* 
     return 0;
 }
 
+// Which variant a product takes.  `n_groups` 0: no groups.
+//
+// Measured on an MI355X, launches in a row over weights that the caches do not hold.  Up to 16 rows the time is the
+// stream of W, so what counts is workgroups enough to keep it busy, and no more of the fixed part of each than that
+// takes: 16 rows of W a workgroup (variant 6) where 32 (variant 8) would leave half of the compute units without one
+// (2,048 x 2,048: 4.4 against 5.1 us, 2 groups of 2,048 x 3,072: 7.0 against 8.7) and for the experts' plain products,
+// 32 where there are enough (5,120 x 5,120: 10.6 against 12.5, 2 groups of 2 x 3,072 x 2,048 gated: 10.7 against
+// 11.8); for the output matrix more columns of X or longer blocks.  The experts' gated products run best as many small
+// workgroups, 16 + 16 rows and four waves (variant 5: two groups of 2 x 8,192 x 5,120 50.6 us against 53.0 with
+// variant 8, 6.6 against 6.3 TB/s; seven groups 169.6 against 173.4), and so do one or two rows times a table of
+// 2^27 elements and up, if those are four a compute unit (variant 5 / 8: 16,384 x 8,192 41.7 / 44.4, 26,496 x 5,120
+// 42.8 / 46.2, 65,536 x 2,048 40.9 / 42.2; fewer: 14,736 x 10,432 50.2 / 46.9).
+static int skinny_variant(int M, int N, int K, int n_groups, int live_groups, bool glu, int max_rows) {
+    const long cus = sp_cu_count();
+    const size_t nk = (size_t)N * K;
+    if (max_rows <= 16) {
+        const long groups = !n_groups ? 1 : (live_groups > 0 && live_groups < n_groups ? live_groups : n_groups);
+        const bool few = (long)((N + 31) / 32) * (groups < M ? groups : M) < cus / 2;
+        if (n_groups) return glu && !few ? 5 : 6;
+        if (nk >= ((size_t)1 << 28)) return max_rows <= 8 ? 4 : 7;
+        if (max_rows <= 2 && nk >= ((size_t)1 << 27) && N / 16 >= 4 * cus) return 5;
+        return few ? 6 : 8;
+    }
+    if (max_rows <= 32) {
+        // The output matrix's stream outweighs the second read of its rows by two row tiles: 64 rows of W a workgroup
+        // (variant 10) instead of 32 (variant 2).  Between 2^27 and 2^28 elements that holds for more than 24 rows and
+        // workgroups that leave less than a seventh of the last round of compute units without one (10 / 2: 32,768 x 5,120
+        // 60 / 67 us at 32 rows, 57 / 56 at 17; 32,768 x 7,168 80 / 89; 32,768 x 4,096, the worst, 53 / 52; with 1.25 and
+        // 2.5 rounds 20,480 x 7,168 70 / 65, 40,960 x 4,096 70 / 65).
+        const long wide = (N + 63) / 64, filled = (wide + cus - 1) / cus * cus;
+        if (!n_groups && (nk >= ((size_t)1 << 28) || (!glu && max_rows > 24 && nk >= ((size_t)1 << 27) && 7 * wide >= 6 * filled))) return 10;
+        return 2;
+    }
+    // (groups of experts at 33 to 64 tokens hold a few rows each, only the shared one all:
+    // 32 columns a workgroup and a second row tile for that group beat 64 columns for all)
+    if (n_groups) return glu ? 2 : 10;
+    // (a plain product's time grows with the tokens, whose rows every workgroup reads from
+    // L2 beside its rows of W: from about 50 tokens on, 64 rows of W a workgroup with two row
+    // tiles of 32 columns beat 32 rows of W with all 64 columns; where 64 rows of W would leave
+    // the chip half empty, 32 with two row tiles: 3,072 x 2,048 8.4 against 11.1 us)
+    if ((N + 63) / 64 * 2 < cus / 2) return 2;
+    return max_rows > 48 ? 10 : 9;
+}
+extern "C" int spite_gemm_skinny_variant(int M, int N, int K, int n_groups, int live_groups, int glu, int max_rows) {
+    return skinny_variant(M, N, K, n_groups, live_groups, glu != 0, max_rows);
+}
+
 // `max_rows`: the most rows any group brings (M itself for a plain product); picks how many
 // token columns a workgroup carries.  `live_groups`: the caller's promise that no more groups than
 // this hold rows (0: no promise); the grid is cut to the row tiles that can exist.
@@ -216,36 +263,7 @@ extern "C" int spite_gemm_skinny(const void* X, int ldx, const void* W, long w_g
     SP_REQUIRE(!w_tiled || (K % 32 == 0 && N % 16 == 0), "gemm_skinny: operand order needs K=%d a multiple of 32 and N=%d of 16", K, N);
     if (M == 0) return 0;
 #define SP_ARGS X, ldx, W, w_group_stride, Y, y_dtype, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, w_tiled, live_groups, st
-    // Measured on an MI355X, launches in a row over weights that the caches do not hold.  Up to 16 rows the time is the
-    // stream of W, so what counts is workgroups enough to keep it busy, and no more of the fixed part of each than that
-    // takes: 16 rows of W a workgroup (variant 6) where 32 (variant 8) would leave half of the compute units without one
-    // (2,048 x 2,048: 4.4 against 5.1 us, 2 groups of 2,048 x 3,072: 7.0 against 8.7) and for the experts' plain products,
-    // 32 where there are enough (5,120 x 5,120: 10.6 against 12.5, 2 groups of 2 x 3,072 x 2,048 gated: 10.7 against
-    // 11.8); for the output matrix more columns of X or longer blocks.  The experts' gated products run best as many small
-    // workgroups, 16 + 16 rows and four waves (variant 5: two groups of 2 x 8,192 x 5,120 50.6 us against 53.0 with
-    // variant 8, 6.6 against 6.3 TB/s; seven groups 169.6 against 173.4).
-    if (variant == 0) {
-        if (max_rows <= 16) {
-            const long groups = !offsets ? 1 : (live_groups > 0 && live_groups < n_groups ? live_groups : n_groups);
-            const bool few = (long)((N + 31) / 32) * (groups < M ? groups : M) < sp_cu_count() / 2;
-            if (offsets) variant = glu && !few ? 5 : 6;
-            else if ((size_t)N * K >= ((size_t)1 << 28)) variant = max_rows <= 8 ? 4 : 7;
-            else if (max_rows <= 2 && (size_t)N * K >= ((size_t)1 << 27)) variant = 5;
-            else variant = few ? 6 : 8;
-        }
-        // (the output matrix's stream outweighs the second read of its rows by two row tiles: 59 against 71 us at
-        // 32 rows of 32,768 x 5,120)
-        else if (max_rows <= 32) variant = !offsets && (size_t)N * K >= ((size_t)1 << 27) ? 10 : 2;
-        // (groups of experts at 33 to 64 tokens hold a few rows each, only the shared one all:
-        // 32 columns a workgroup and a second row tile for that group beat 64 columns for all)
-        else if (offsets) variant = glu ? 2 : 10;
-        // (a plain product's time grows with the tokens, whose rows every workgroup reads from
-        // L2 beside its rows of W: from about 50 tokens on, 64 rows of W a workgroup with two row
-        // tiles of 32 columns beat 32 rows of W with all 64 columns; where 64 rows of W would leave
-        // the chip half empty, 32 with two row tiles: 3,072 x 2,048 8.4 against 11.1 us)
-        else if ((N + 63) / 64 * 2 < sp_cu_count() / 2) variant = 2;
-        else variant = max_rows > 48 ? 10 : 9;
-    }
+    if (variant == 0) variant = skinny_variant(M, N, K, offsets ? n_groups : 0, live_groups, glu != 0, max_rows);
     switch (variant) {
         case 2: return launch_skinny<2, 2, 2, 8>(SP_ARGS);
         case 3: return launch_skinny<2, 4, 2, 4>(SP_ARGS);

@@ -118,6 +118,8 @@ def lib():
         l.spite_delta_chunk_workspace.restype = c_size_t
         l.spite_router_plan_is_one_launch.argtypes = [I, I]
         l.spite_router_plan_is_one_launch.restype = c_int
+        l.spite_gemm_skinny_variant.argtypes = [I] * 7
+        l.spite_gemm_skinny_variant.restype = c_int
         l.spite_gemm_lds_time.argtypes = [I, I, I, I]
         l.spite_gemm_lds_time.restype = ctypes.c_double
         l.spite_cu_count.argtypes = []

@@ -77,3 +77,18 @@ def test_whole_group_stays_where_apart_was_slower():
         assert whole_group_apart(tokens, groups, N, K) == 0, (tokens, groups, N, K)
     for tokens, groups, N, K in ((1454, 16, 5120, 8192), (1806, 8, 5120, 8192), (3107, 16, 3072, 8192), (2553, 8, 4096, 14336)):
         assert whole_group_apart(tokens, groups, N, K) == 1, (tokens, groups, N, K)
+
+
+def test_variants_of_the_weight_stream():
+    """Tables between 2^27 and 2^28 elements, on either side of the lines that were timed."""
+    from spite_amd.csrc.hipops import lib
+    plain = lambda rows, N, K, glu=0: lib().spite_gemm_skinny_variant(rows, N, K, 0, 0, glu, rows)
+    assert [plain(r, 32768, 5120) for r in (1, 2, 3, 16, 17, 24, 25, 32)] == [5, 5, 8, 8, 2, 2, 10, 10]
+    assert [plain(1, N, K) for N, K in ((16384, 8192), (14736, 10432), (15168, 9536), (16384, 5120), (65536, 4096))] == [5, 8, 8, 8, 4]
+    assert [plain(32, N, K) for N, K in ((36864, 5120), (40960, 4096), (24576, 6144), (18432, 14336), (30720, 8192), (28672, 5120))] == [2, 2, 2, 2, 10, 10]
+    assert plain(25, 18688, 13760, 1) == 2 and plain(25, 202048, 5120, 0) == 10 and plain(20, 202048, 5120) == 10
+    # as it was: few rows, experts' groups, 33 to 64 rows
+    assert [plain(1, N, K) for N, K in ((2048, 2048), (5120, 5120), (202048, 5120))] == [6, 8, 4] and plain(16, 202048, 5120) == 7
+    group = lambda rows, N, K, glu, live: lib().spite_gemm_skinny_variant(rows * 2, N, K, 17, live, glu, rows)
+    assert group(8, 8192, 5120, 1, 9) == 5 and group(8, 5120, 8192, 0, 9) == 6 and group(40, 8192, 5120, 1, 17) == 2 and group(40, 5120, 8192, 0, 17) == 10
+    assert plain(40, 5120, 5120) == 9 and plain(60, 5120, 5120) == 10 and plain(60, 3072, 2048) == 2
