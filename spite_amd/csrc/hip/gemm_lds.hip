@@ -232,16 +232,17 @@ void gemm_lds_kernel(gl_args a) {
 }
 
 // Which NB suits a plain product, and what it takes then, in us: a round of tiles over the compute units takes (4.3 + 1.95 NB)
-// ns a k (measured at NB = 4, 5, 6, 8 and K = 5,120: 62, 71, 81 and 102 us).
+// ns a k (measured at NB = 4, 5, 6, 8 and K = 5,120: 62, 71, 81 and 102 us), and every round but the first 10 us for its
+// tiles' start and end, which short sums over k do not hide (448 k, 18 rounds: 401 us).
 static double lds_time(int M, int N, int K, bool glu, int* nb_out) {
     const long cus = sp_cu_count(), cols = (N + (glu ? 127 : 255)) / (glu ? 128 : 256);
-    double least = -1.0;
+    double least = -1.0, further = 0.0;
     for (int nb : {8, 6, 5, 4}) {
-        const long tiles = (M + 32 * nb - 1) / (32 * nb) * cols;
-        const double t = (double)((tiles + cus - 1) / cus) * K * (4.3e-3 + 1.95e-3 * nb);
-        if (least < 0.0 || t < least) { *nb_out = nb; least = t; }
+        const long tiles = (M + 32 * nb - 1) / (32 * nb) * cols, rounds = (tiles + cus - 1) / cus;
+        const double t = (double)rounds * K * (4.3e-3 + 1.95e-3 * nb);
+        if (least < 0.0 || t < least) { *nb_out = nb; least = t; further = 10.4 * (double)(rounds - 1); }
     }
-    return least;
+    return least + further;
 }
 extern "C" double spite_gemm_lds_time(int M, int N, int K, int glu) { int nb; return lds_time(M, N, K, glu != 0, &nb); }
 

@@ -685,8 +685,8 @@ def gemm_lds_ok(a, w, M, N, K, glu) -> bool:
 
 
 # What the two tiled products take on an MI355X, in us, from products timed in a row: a tile of gemm_tiled 38 and 8.5 for
-# every 16 rows at K = 5,120; both then run a sixth slower in company than alone; adding up the runs of a sum over k costs
-# a launch and the passes over the partial sums at 4.5 TB/s.
+# every 16 rows at K = 5,120, and every round but the first 6 more; both then run a sixth slower in company than alone;
+# adding up the runs of a sum over k costs a launch and the passes over the partial sums at 4.5 TB/s.
 def lds_us(M: int, N: int, K: int, glu: bool) -> float:
     return 1.15 * lib().spite_gemm_lds_time(M, N, K, int(bool(glu))) + 3.0
 
@@ -694,9 +694,10 @@ def lds_us(M: int, N: int, K: int, glu: bool) -> float:
 @functools.lru_cache(maxsize=4096)
 def lds_suits(M: int, N: int, K: int, glu: bool, runs: int) -> bool:
     """Whether a product without groups is sooner done by ``gemm_lds`` than by ``gemm_tiled`` with its sum over k in
-    ``runs`` runs.  (Timed in turn at 31 sizes, 300 to 2,048 rows, widths of 2,048 to 16,384: the choice is the faster one, or
-    within a tenth of it, at all of them: 1,547 x 5,120 x 5,120 79 against 97 us, 1,531 x 2,048 x 2,048 31 against 36, 300 x 16,384
-    x 5,120 gated 99 against 131; 700 x 5,120 x 8,192 stays, 78 against 106.)"""
+    ``runs`` runs.  (Timed in turn at 224 sizes, 65 to 8,192 rows, widths of 512 to 32,768, sums over 64 to 16,384: none of the
+    95 that the line takes in is more than 2 % slower, on average they are 27 % faster: 1,547 x 5,120 x 5,120 79 against 97 us,
+    1,531 x 2,048 x 2,048 31 against 36, 300 x 16,384 x 5,120 gated 99 against 131; 700 x 5,120 x 8,192 stays, 78 against 106, and
+    7,902 x 18,304 x 448 gated, 367 against 401.)"""
     cus, lds = cu_count(), lds_us(M, N, K, glu)
     cols, scale = -(-N // (256 if glu else 512)), 1.2 * K / 5120.0
     if runs > 1:
@@ -704,8 +705,10 @@ def lds_suits(M: int, N: int, K: int, glu: bool, runs: int) -> bool:
             return False
         tiled = scale * 106.0 / runs + 12.0 + (runs + 1) * M * N * 4 / 4.5e6
     else:
-        rounds = lambda rows: -(-(-(-M // rows) * cols) // cus)
-        tiled = scale * min(106.0 * rounds(128), 89.0 * rounds(96) if not glu else math.inf)
+        def rounds(rows, tile_us):
+            n = -(-(-(-M // rows) * cols) // cus)
+            return scale * tile_us * n + 6.0 * (n - 1)
+        tiled = min(rounds(128, 106.0), rounds(96, 89.0) if not glu else math.inf)
     return lds <= tiled
 
 

@@ -92,3 +92,12 @@ def test_variants_of_the_weight_stream():
     group = lambda rows, N, K, glu, live: lib().spite_gemm_skinny_variant(rows * 2, N, K, 17, live, glu, rows)
     assert group(8, 8192, 5120, 1, 9) == 5 and group(8, 5120, 8192, 0, 9) == 6 and group(40, 8192, 5120, 1, 17) == 2 and group(40, 5120, 8192, 0, 17) == 10
     assert plain(40, 5120, 5120) == 9 and plain(60, 5120, 5120) == 10 and plain(60, 3072, 2048) == 2
+
+
+def test_short_sums_of_many_rounds_stay_with_the_tiled_product():
+    """Products that both were timed at and that were 3 to 10 % slower with both operands in LDS."""
+    from spite_amd.csrc.hipops import lds_suits, tiled_k_runs
+    for M, N, K, glu in ((7902, 18304, 448, True), (3601, 8320, 896, False), (7489, 22032, 448, False), (6362, 23024, 128, True),
+                         (6907, 28704, 320, True), (7136, 20448, 256, False), (1822, 28224, 2048, True), (2933, 4256, 1536, True),
+                         (5743, 10352, 768, False), (1871, 28704, 768, False)):
+        assert not lds_suits(M, N, K, glu, 1 if glu else tiled_k_runs(M, N, K)), (M, N, K, glu)
