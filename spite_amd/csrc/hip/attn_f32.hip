@@ -1,10 +1,11 @@
 // fp32 attention over row-major pages (head sizes in multiples of 16 up to 128, pages in multiples of 4 keys): the true
 // 32-bit path at the sizes that models have; attn_generic.hip keeps the others.
 //
-// A workgroup of eight waves per (token, query head).  Keys are walked in tiles of 32 that start at multiples of 32
-// positions, tile t by wave t % 8, each wave with its own running maximum, sum and output; the eight meet in LDS at the
-// end, in their order.  So the order of every sum depends on the query's position alone, as in the plain kernel: a token
-// gives the same bits whether it comes in a whole prompt, a portion or alone.
+// A workgroup of W waves per (token, query head): eight, or fewer where a window or a chunk never shows a query that many
+// tiles.  Keys are walked in tiles of 32 that start at multiples of 32 positions, the tiles dealt to the waves in turn, each
+// wave with its own running maximum, sum and output; they meet in LDS at the end, in their order.  So the order of every
+// sum depends on the layer and the query's position alone, as in the plain kernel: a token gives the same bits whether it
+// comes in a whole prompt, a portion or alone.
 //
 // Bound by latency (decode: a chain of loads, table entry - keys - values, over few workgroups) or by the loads' path
 // (prompts).  Hence tiles of 32 over eight waves, so that 256 keys are one such chain; 16-byte loads over whole lines,
@@ -12,18 +13,17 @@
 // partial sums of its four keys until the end instead of summing across lanes in every tile.
 #include "common.h"
 
-#define AF_WAVES 8
 #define AF_KEYS 32
 
-template <int NI>     // the head size in units of 16, at most
-__global__ __launch_bounds__(64 * AF_WAVES)
+template <int NI, int W>     // NI: the head size in units of 16, at most
+__global__ __launch_bounds__(64 * W)
 void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pages, const float* __restrict__ v_pages,
                      float* __restrict__ out, const int* __restrict__ positions, const int* __restrict__ seq_of_token,
                      const int* __restrict__ block_table, int max_blocks, int H, int G, int hd, int ps, int vis, int span,
                      float scale, float softcap, const float* __restrict__ slopes) {
-    __shared__ __align__(16) float p_sh[AF_WAVES][AF_KEYS];
-    __shared__ float o_sh[AF_WAVES][NI * 16];
-    __shared__ float ml_sh[AF_WAVES][2];
+    __shared__ __align__(16) float p_sh[W][AF_KEYS];
+    __shared__ float o_sh[W][NI * 16];
+    __shared__ float ml_sh[W][2];
     const int t = blockIdx.x, h = blockIdx.y, lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int g = h / (H / G), ni = hd >> 4;
@@ -45,7 +45,7 @@ void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pa
     for (int i = 0; i < NI * 2; ++i) o[i] = 0.f;
     float m = -INFINITY, l = 0.f;
 
-    for (int j0 = (lo & ~(AF_KEYS - 1)) + wave * AF_KEYS; j0 <= p; j0 += AF_KEYS * AF_WAVES) {
+    for (int j0 = (lo & ~(AF_KEYS - 1)) + wave * AF_KEYS; j0 <= p; j0 += AF_KEYS * W) {
         // the table entries of this tile's keys and values, then every row of keys, before anything waits for them
         int page[2];
         bool seen[2];
@@ -129,10 +129,10 @@ void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pa
     if (c >= hd) return;
     float mm = ml_sh[0][0];
 #pragma unroll
-    for (int w = 1; w < AF_WAVES; ++w) mm = fmaxf(mm, ml_sh[w][0]);
+    for (int w = 1; w < W; ++w) mm = fmaxf(mm, ml_sh[w][0]);
     float ll = 0.f, a = 0.f;
 #pragma unroll
-    for (int w = 0; w < AF_WAVES; ++w) {
+    for (int w = 0; w < W; ++w) {
         const float f = ml_sh[w][0] == -INFINITY ? 0.f : expf(ml_sh[w][0] - mm);   // a wave without tiles
         ll += ml_sh[w][1] * f;
         a += o_sh[w][c] * f;
@@ -145,10 +145,20 @@ int sp_attn_f32(const float* q, const float* k_pages, const float* v_pages, floa
                 const int* seq_of_token, const int* block_table, int max_blocks, int T, int H, int G, int hd, int page_size,
                 int vis, int span, float scale, float softcap, const float* slopes, hipStream_t st) {
     if (hd % 16 || hd > 128 || page_size % 4 || ((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages) % 16) return 1;
+    // Waves for no more tiles than a query sees, lanes for no more of the head than there is: 3,000 tokens of a prompt, 4 heads
+    // of 16 behind a window of 64 keys, 25 us (46 with eight waves and heads padded to 64, 60 for the plain kernel); 1,000 tokens,
+    // 16 heads of 128, 170 (332, 751).  A few keys are the plain kernel's, a wave a row: a window of one, 1,000 tokens, 16 heads
+    // of 128, 47 against 82 us; of eight, 4 heads of 16, 3,000 tokens, 17 against 27; of 33 35 against 16.
+    if (sp_vis_has_span(vis) && span <= 8) return 1;
     dim3 grid(T, H);
-#define AF_GO(NI) attn_f32_kernel<NI><<<grid, 64 * AF_WAVES, 0, st>>>(q, k_pages, v_pages, out, positions, seq_of_token, block_table, \
+    const long tiles = sp_vis_has_span(vis) ? ((long)span + 30) / 32 + 1 : 8;      // that a query sees at most
+#define AF_GO(NI, W) attn_f32_kernel<NI, W><<<grid, 64 * W, 0, st>>>(q, k_pages, v_pages, out, positions, seq_of_token, block_table, \
         max_blocks, H, G, hd, page_size, vis, span, scale, softcap, slopes)
-    if (hd <= 64) AF_GO(4); else AF_GO(8);
+#define AF_HEAD(W) do { if (hd <= 16) AF_GO(1, W); else if (hd <= 32) AF_GO(2, W); else if (hd <= 64) AF_GO(4, W); else AF_GO(8, W); } while (0)
+    if (tiles <= 2) AF_HEAD(2);
+    else if (tiles <= 4) AF_HEAD(4);
+    else AF_HEAD(8);
+#undef AF_HEAD
 #undef AF_GO
     SP_LAUNCH_CHECK("attn_f32");
     return 0;
