@@ -246,10 +246,11 @@ static double lds_time(int M, int N, int K, bool glu, int* nb_out) {
 }
 extern "C" double spite_gemm_lds_time(int M, int N, int K, int glu) { int nb; return lds_time(M, N, K, glu != 0, &nb); }
 
-// Arguments as spite_gemm_tiled's; `nb`: the plain product's tile height in units of 32 rows (4, 5, 6 or 8), 0 the library's choice.
+// Arguments as spite_gemm_tiled's; `nb`: the plain product's tile height in units of 32 rows (4, 5, 6 or 8), 0 the library's choice;
+// `x_rows`: how many rows X has, which a row list's entries stay below (0 without one: M).
 extern "C" int spite_gemm_lds(const void* X, int ldx, const void* W, long w_group_stride, void* Y, int y_dtype, int ldy, int M,
                               int N, int K, const int* offsets, int n_groups, const int* a_rows, const float* a_scale,
-                              const int* y_rows, int glu, float act_limit, int nb, hipStream_t st) {
+                              const int* y_rows, int glu, float act_limit, int nb, int x_rows, hipStream_t st) {
     SP_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldy >= N, "gemm_lds: bad sizes M=%d N=%d K=%d", M, N, K);
     SP_REQUIRE(K % 64 == 0 && N % 16 == 0, "gemm_lds: operand order needs K=%d a multiple of 64 and N=%d of 16", K, N);
     SP_REQUIRE(ldx % 8 == 0, "gemm_lds: the row stride %d must be a multiple of 8", ldx);
@@ -261,9 +262,10 @@ extern "C" int spite_gemm_lds(const void* X, int ldx, const void* W, long w_grou
     glu &= 15;
     SP_REQUIRE(!(glu && unary) && unary <= SP_UNARY_TANH, "gemm_lds: activation code %d", glu | (unary << 4));
     SP_REQUIRE(glu <= SP_ACT_LAST && (glu != SP_ACT_CLAMPED || act_limit > 0.f), "gemm_lds: activation code %d with bound %g", glu, act_limit);
-    // the loads' offsets are 32-bit: rows of X (a row list names rows below M) and a group's W
-    SP_REQUIRE((size_t)M * ldx * 2 < ((size_t)1 << 31) && (size_t)(glu ? 2 : 1) * N * K * 2 < ((size_t)1 << 31),
-               "gemm_lds: operands of 2 GiB and more (M=%d N=%d K=%d)", M, N, K);
+    SP_REQUIRE(!a_rows || x_rows > 0, "gemm_lds: a row list over %d rows of X", x_rows);
+    // the loads' offsets are 32-bit: rows of X and a group's W
+    SP_REQUIRE((size_t)(a_rows ? x_rows : M) * ldx * 2 < ((size_t)1 << 31) && (size_t)(glu ? 2 : 1) * N * K * 2 < ((size_t)1 << 31),
+               "gemm_lds: operands of 2 GiB and more (M=%d, %d rows of X, N=%d K=%d)", M, x_rows, N, K);
     if (M == 0) return 0;
     gl_args a{(const bf16*)X, ldx, (const bf16*)W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows,
               0, 0, 0, glu ? glu : -unary, act_limit};

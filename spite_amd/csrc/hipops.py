@@ -67,7 +67,7 @@ def lib():
             "spite_attn_decode_rope": [P, P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, I, P, F, I, F, P],
             "spite_attn_decode": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
             "spite_gemm_mfma": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
-            "spite_gemm_lds": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
+            "spite_gemm_lds": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, I, P],
             "spite_gemm_tiled": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_tiled_split": [P, I, P, P, I, I, I, I, I, I, P, P],
             "spite_attn_prefill": [P, P, P, P, P, P, P, P, I, P, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
@@ -738,7 +738,7 @@ def gemm_lds(a, w, y, M, N, K, *, offsets=None, n_groups=1, a_rows=None, a_scale
         _ptr_rows(a, "a"), a.stride(0), _ptr(w, "w"), rows_w * K, _ptr_rows(y, "y"), dtype_code(y.dtype), y.stride(0),
         M, N, K, _ptr(offsets, "offsets", torch.int32, True), n_groups, _ptr(a_rows, "a_rows", torch.int32, True),
         _ptr(a_scale, "a_scale", torch.float32, True), _ptr(y_rows, "y_rows", torch.int32, True), _act_code(glu, act),
-        float(act_limit), int(nb), _stream()), "gemm_lds")
+        float(act_limit), int(nb), a.shape[0], _stream()), "gemm_lds")
 
 
 def attn_prefill_splits(counts, H, G, max_keys) -> int:
