@@ -48,3 +48,37 @@ def test_refuses_what_it_cannot_do():
     with pytest.raises(ops().KernelError):          # no cache row
         ops().attn_decode_rope(z(1, 6 * 64), z(1, 1, 32, 64), z(1, 1, 64, 32), z(1, 4 * 64), f, i32(1), i32(0), i32(1), i32(1, 4), 1, 4, 1, 64,
                                32, "full", 0, 1.0, 1)
+
+
+@pytest.mark.parametrize("vis,span", [("full", 0), ("chunk", 64), ("window", 45), ("window", 1)])
+@pytest.mark.parametrize("softcap,sloped", [(0.0, False), (4.0, False), (0.0, True), (3.0, True)])
+@pytest.mark.parametrize("n_splits", [1, 2, 13])
+@pytest.mark.parametrize("hd", [64, 128])
+def test_what_a_query_sees_caps_slopes_and_rows_without_a_place(vis, span, softcap, sloped, n_splits, hd):
+    """Queries that open a chunk or a block, windows whose first key lies inside a block, more splits than blocks (the one
+    that holds the last block writes the row), and a token without a cache row, which leaves the pages alone."""
+    lens, H, G, ps = [1, 32, 33, 65, 64, 300, 129, 97], 6, 2, 32
+    T = len(lens)
+    kv = PagedKV(lens, G, hd, ps, torch.bfloat16)
+    kp, vp = ops().kv_operand_order(kv.kp.to(DEV), kv.vp.to(DEV))
+    before = kp.clone(), vp.clone()
+    qkv = rnd(T, (H + 2 * G) * hd, dtype=torch.bfloat16, seed=9)
+    positions = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([kv.tables[s][(n - 1) // ps] * ps + (n - 1) % ps for s, n in enumerate(lens)], dtype=torch.int32, device=DEV)
+    slots[5] = -1
+    seq, bt = torch.arange(T, dtype=torch.int32, device=DEV), kv.bt.to(DEV)
+    inv = (10000.0 ** (-torch.arange(hd // 2, dtype=torch.float64) / (hd // 2))).float().to(DEV)
+    slopes = (0.02 * (1 + torch.arange(H))).float().to(DEV) if sloped else None
+    scratch = torch.empty(ops().attn_decode_workspace(T, H, hd, n_splits) // 4, dtype=torch.float32, device=DEV)
+    q, want, got = (torch.zeros(T, H * hd, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    kp2, vp2 = kp.clone(), vp.clone()
+    ops().rope_kvwrite(qkv, q, kp, vp, positions, slots, inv, H, G, hd, ps, use_rope=True, adjacent=False, use_norm=False, norm_eps=0.0,
+                       use_temp=False, floor_scale=0, attn_scale=0.0, kv_tiled=True)
+    args = (positions, seq, bt, T, H, G, hd, ps, vis, span, hd ** -0.5, n_splits)
+    ops().attn_decode(q, kp, vp, want, scratch, *args, softcap=softcap, slopes=slopes)
+    ops().attn_decode_rope(qkv, kp2, vp2, got, scratch, positions, slots, *args[1:], inv_freq=inv, softcap=softcap, slopes=slopes)
+    assert torch.equal(kp, kp2) and torch.equal(vp, vp2)         # (without a norm: no sum whose order could differ)
+    page = kv.tables[5][299 // ps]
+    assert torch.equal(kp2[page], before[0][page]) and torch.equal(vp2[page], before[1][page])
+    assert not torch.equal(kp2, before[0])
+    assert torch.equal(got, want)
