@@ -51,8 +51,7 @@ extern "C" int spite_embed(const int* ids, const void* table, int dtype, float* 
 
 // (a wave's fp32 dot product, wave_dot_row, is in common.h: every kernel that forms router logits calls it)
 
-// expert[] and weight[]: the largest logit, the lowest index among equals, weight =
-// 1/(1+exp(-logit)).
+// The index of the largest logit, the lowest among equals, and (if asked for) the logit.
 __device__ __forceinline__ int top1_of(const float* __restrict__ l, int E, float* best_out) {
     float best = -INFINITY; int best_e = 0;
     if ((E & 3) == 0 && (((uintptr_t)l) & 15) == 0) {           // four logits a load
@@ -631,6 +630,9 @@ extern "C" int spite_router_top1(const float* x, const float* wr, int* expert, f
 //   the slots behind them, `shared` groups E, E + 1, ... that every token visits: src = token, scale 1, dst[s] = s;
 //   offsets[g] = first slot of group g, g in [0, E + shared + 1).
 // With `logits` ([T, E] fp32) the kernels make the router's choice themselves and write it to
+// expert[] and weight[]: the largest logit, the lowest index among equals, weight =
+// 1/(1+exp(-logit)).
+//
 // Each thread ranks one token by counting over all tokens in shared memory: no atomics, the
 // order is the same on every run.
 __global__ void moe_plan_kernel(int* __restrict__ expert, float* __restrict__ weight,

@@ -11,8 +11,8 @@
 //    rows of W (GLU: 16 of each half) and gives one run of k to each of its eight waves, so that a product with
 //    2,048 output rows has 1,024 waves in flight; the runs' sums meet in LDS.
 //  gemm_f32_tile: many rows, bound by the MFMAs (256 FLOP a clock and compute unit).  64 rows of X times 64 rows of W a
-//    workgroup: X through double-buffered LDS, read by all four waves; a wave's 16 rows of W straight into registers, a
-//    step ahead.  The smaller tile than a large product would want is for the sizes at hand: 301 tokens times 2,048
+//    workgroup: X through double-buffered LDS, a step ahead, read by all four waves; a wave's 16 rows of W straight into
+//    registers, two steps ahead.  The smaller tile than a large product would want is for the sizes at hand: 301 tokens times 2,048
 //    columns are 160 workgroups.
 //
 // SP_F32_ROWS_MAX: up to 64 rows the first one reads each byte of W once, beyond it would read W again for every
@@ -127,8 +127,8 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
 #define F32_LD (F32_TK + 4)       // LDS row: 16 bytes more than a step, so that 16 rows' reads spread over the banks
 
 // The loop over k for a tile whose first LIVE groups of 16 rows hold rows (an expert's last tile is seldom full).  Loads
-// are unconditional, a step ahead of their use, and scaled only when they go to LDS, so that nothing waits for them
-// before the step's MFMAs; a chain of four MFMAs is spread over the accumulators.
+// are unconditional, X's a step ahead of its use and W's two (three sets of registers in turn), and X is scaled only when it
+// goes to LDS, so that nothing waits for them before the step's MFMAs; a chain of four MFMAs is spread over the accumulators.
 template <int NB, int LIVE>
 __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp, const float* const* xp, const float* sc, int K,
                                               int seg, int lr, int lk, int r, int q, f32x4 (&tot)[4][NB]) {

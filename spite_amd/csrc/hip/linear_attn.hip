@@ -102,7 +102,8 @@ template <int TB> __device__ __forceinline__ float la_sums(float* x, int l) {
 template <int TB> __device__ __forceinline__ int la_owner(int l) { return TB == 16 ? l >> 1 : TB == 8 ? l >> 2 : 0; }
 
 // VEC: q, k, v (bfloat16) and the decay rows start on 16 bytes and D and V are multiples of 8: a fetch is
-// 16 bytes.  Otherwise one element.  (Plain loops and no closures: every array below stays in registers.)
+// 16 bytes.  Otherwise one element.  (Every loop over the arrays below is unrolled and both lambdas are inlined, so that
+// the arrays stay in registers.)
 #define LA_OWN(r) (PR >= 4 ? ((r) / 4) * 128 + dg * 4 + ((r) % 4) : dg * PR + (r))    // the thread's r-th key channel
 // TB: tokens a block: 16 (8 for the widest heads), or 1 for steps of single tokens, whose workgroups then hold
 // little LDS and few registers, so that many are resident and their round trips to memory overlap.

@@ -1,4 +1,4 @@
-"""The 32-bit product and attention on the matrix units and over whole runs, at the edges of their tiles."""
+"""The 32-bit product on the matrix units and the 32-bit attention over tiles of keys, at the edges of their tiles."""
 import math
 
 import pytest
