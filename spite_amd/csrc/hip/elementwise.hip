@@ -82,13 +82,13 @@ __device__ __forceinline__ int top1_of(const float* __restrict__ l, int E, float
 // itself in the output's dtype (no norm, `w` unused): the stream as a later product's operand.
 // With `w2` and `out2` the row goes out a second time, normed with the weights w2 (two norms of
 // one stream: a layer whose mixer and feed-forward read the same rows), in `out`'s dtype.
-// With `plan` (a single row) the projection is a router's logits and the row's list for the grouped products is made here
+// PLAN (a single row): the projection is a router's logits and the row's list for the grouped products is made here
 // too, as moe_plan makes it: one of some 4.5 us of launches that a layer of a single decoded token is made of (5,120 wide
 // over 16 experts: 11.2 us for the two kernels, 7.1 for this one).
 struct norm_plan { int* expert; float* weight; int* src; float* scale; int* dst; int* offsets; int shared; };
 #define NORM_NT 512
 #define NORM_MAX_V 8     // widths up to 4*NT*MAX_V = 16384 stay in registers
-template <typename TO, bool VEC>
+template <typename TO, bool VEC, bool PLAN>
 __global__ __launch_bounds__(NORM_NT)
 void add_rmsnorm_kernel(float* __restrict__ h, const float* __restrict__ d1,
                         const float* __restrict__ d2, const float* __restrict__ w,
@@ -212,10 +212,10 @@ void add_rmsnorm_kernel(float* __restrict__ h, const float* __restrict__ d1,
             const float v = wave_dot_row(proj + (size_t)p * d, ys, d, pvec, lane);
             if (lane == 0) {
                 proj_out[(size_t)i * P + p] = v;
-                if (plan.expert) ys[((d + 3) & ~3) + p] = v;
+                if (PLAN) ys[((d + 3) & ~3) + p] = v;
             }
         }
-        if (!plan.expert) return;
+        if (!PLAN) return;
         __syncthreads();
         float best;
         const int me = top1_of(ys + ((d + 3) & ~3), P, &best);
@@ -253,11 +253,14 @@ extern "C" int spite_add_rmsnorm(float* h, const float* d1, const float* d2, con
     auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     const bool vec = d % 4 == 0 && d <= 4 * NORM_NT * NORM_MAX_V && al(h) && al(d1) && al(d2) && al(w) && al(out32) && al(out) && al(dn) && al(wn)
         && al(w2) && al(out2);
-#define SP_NORM(TO) do { if (vec) add_rmsnorm_kernel<TO, true><<<n_rows, NORM_NT, sh, st>>>(h, d1, d2, w, (TO*)out, out32, rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2, (TO*)out2, plan); \
-        else add_rmsnorm_kernel<TO, false><<<n_rows, NORM_NT, sh, st>>>(h, d1, d2, w, (TO*)out, out32, rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2, (TO*)out2, plan); } while (0)
-    if (out_dtype == SP_F32) SP_NORM(float);
-    else if (out_dtype == SP_BF16) SP_NORM(bf16);
+#define SP_NORM(TO, VEC, PLAN) add_rmsnorm_kernel<TO, VEC, PLAN><<<n_rows, NORM_NT, sh, st>>>(h, d1, d2, w, (TO*)out, out32, rows, d, eps, \
+        write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2, (TO*)out2, plan)
+#define SP_NORM_TO(TO) do { if (expert) { if (vec) SP_NORM(TO, true, true); else SP_NORM(TO, false, true); } \
+        else { if (vec) SP_NORM(TO, true, false); else SP_NORM(TO, false, false); } } while (0)
+    if (out_dtype == SP_F32) SP_NORM_TO(float);
+    else if (out_dtype == SP_BF16) SP_NORM_TO(bf16);
     else return sp_fail("add_rmsnorm: unknown dtype %d", out_dtype);
+#undef SP_NORM_TO
 #undef SP_NORM
     SP_LAUNCH_CHECK("add_rmsnorm");
     return 0;
