@@ -1,0 +1,343 @@
+// Products over groups of rows (experts) for many rows: Y[M,N] = X[M,K] . W[g][N,K]^T, bf16 in, fp32 accumulation on MFMA
+// 16x16x32, W in MFMA operand order (see gemm_tiled.hip), plain or gated with silu.
+//
+// A step's groups differ: a router gives each expert a few rows or a few hundred, a shared expert takes every one.  A tile
+// of one height for all multiplies padding for the small groups and reads W again for the large ones; here every group
+// takes as few tiles as `cap` rows (128 or 160) allow, all of the height, in units of 16 rows, that then covers it.
+//
+// A workgroup of NW waves (eight or four) owns 64 * NW rows of W (GLU: 32 * NW gate rows and the matching up rows) and one tile
+// of 16 * NB rows of X; a wave owns 64 rows of W and every row of X: 4 x NB accumulator tiles.
+//  * W never touches LDS: S rotating sets of operand registers (six up to 96 rows, four above), each asked for again as soon as
+//    its products are issued, S - 1 half steps of 32 k ahead.  A group of one tile reads its W once: non-temporal loads.
+//  * X goes straight to LDS (buffer loads with the lds bit), four buffers of 64 k, asked for three steps ahead: no register
+//    waits for it, and waiting for it (loads are counted in order) waits for no younger W.  The 16-byte pieces of a row are
+//    exchanged by XOR with half its number, so that an operand read spreads over all banks.  One barrier per 64 k.
+//  * Rows past the group and steps past K (K is cut into rounds of S / 2 steps of 64) are loads beyond the buffer's end, which
+//    give zeros: no branch in the loop, and products of zeros cost the matrix units less power, which is what bounds the
+//    clock here.
+//  * Workgroups go to the eight XCDs in turn; XCD x takes the x-th eighth of the tiles, the row tile running fastest, so that
+//    those which run at a time share what they read.
+// The sum over k runs in the order of gemm_tiled and gemm_lds: the same bits.
+//
+// Measured on an MI355X against gemm_tiled's best tile (us; 16 experts of which a token takes `top`, beside them one or two
+// groups of every token): 2,048 tokens x 2 x 8,192 x 5,120 gated 639 / 722, 1,547 553 / 656, 330 453 / 476; 1,786, top 2,
+// 2 x 4,096 x 5,120 548 / 653; 1,531, top 4, 2 x 1,024 x 2,048 80 / 109; 1,200 x 2,048 x 3,072 57 / 70; over 220 sizes of 4 to 128
+// groups and 65 to 6,000 tokens 0.86 of the time on average.  At 2,048 tokens what bounds it is the power limit (the clock falls
+// to 1.6 GHz with the matrix units half busy), at 330 the stream of W (6.5 TB/s).
+#include <math.h>
+#include "common.h"
+
+struct gg_args {
+    const bf16* X; int ldx; const bf16* W; long w_group_stride; void* Y; int ldy, M, N, K;
+    const int* offsets; int n_groups; const int* a_rows; const float* a_scale; const int* y_rows;
+    int m_tiles, n_tiles, cap;
+};
+#define GG_PAST ((int)0x80000000)      // an offset beyond every buffer's end: loads give zeros
+
+// 16 bytes a lane from the buffer at voff + soff to LDS at lds + lane * 16 (written out: the compiler would wait for every such
+// load before any read of LDS; the waits are the kernel's own)
+__device__ __forceinline__ void gg_load_lds(__amdgpu_buffer_rsrc_t buf, int voff, int soff, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :: "v"(voff), "s"(buf), "s"(soff), "s"(lds) : "memory", "m0");
+}
+// A buffer of 2 GiB from p on (the operands' offsets are checked on the host), p the same in every lane.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t gg_buffer(const void* p) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    const uint64_t u = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)u, 0, 0x7fffffff, 0x00020000);
+}
+
+// One tile: rows row0 .. of the group g whose rows end at row_end, columns of the result from n0 on.
+template <int NW, int NB, int S, bool GLU, typename TY, bool NTW>
+__device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, int g, int row0, int row_end, int n0) {
+    constexpr int XB = 16 * NB * 128;                            // bytes of a step of X
+    constexpr int XI = (2 * NB + NW - 1) / NW;                   // load instructions a wave: a step of X (eight rows each)
+    constexpr int TG = GLU ? 2 : 4;                              // bands that name distinct columns
+    static_assert(S % 2 == 0, "whole steps a round");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4, N = p.N, nu = p.K / 64, kt = 2 * nu;
+    const __amdgpu_buffer_rsrc_t xbuf = gg_buffer(p.X), wbuf = gg_buffer(p.W + (size_t)g * p.w_group_stride);
+    int xoff[XI], xblk[XI];
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        xblk[i] = i * NW + wave < 2 * NB ? i * NW + wave : 2 * NB - 1;       // blocks past the tile's last: that one again
+        const int row = xblk[i] * 8 + (lane >> 3), s = row0 + row;
+        const int at = s < row_end ? s : row_end - 1;
+        xoff[i] = (p.a_rows ? p.a_rows[at] : at) * p.ldx * 2 + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
+        if (s >= row_end) xoff[i] = GG_PAST;
+    }
+    int wband[4];
+#pragma unroll
+    for (int a = 0; a < 4; ++a) {
+        int band = n0 / 16 + wave * TG + a % TG;
+        band = band < N / 16 ? band : N / 16 - 1;                // bands past N read the last one again
+        if (GLU && a >= TG) band += N / 16;
+        wband[a] = band * kt * 1024;
+    }
+    const int wlane = lane * 16;
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+    auto load_x = [&](int u) {
+        const int k0 = (u < nu ? u : 0) * 128, past = u < nu ? 0 : GG_PAST;
+#pragma unroll
+        for (int i = 0; i < XI; ++i) gg_load_lds(xbuf, xoff[i] | past, k0, lds0 + (u & 3) * XB + xblk[i] * 1024);
+    };
+    auto load_w = [&](bf16x8 (&ws)[4], int t) {
+        const int at = (t < kt ? t : 0) * 1024, past = t < kt ? 0 : GG_PAST;
+#pragma unroll
+        for (int a = 0; a < 4; ++a)          // (2: non-temporal)
+            ws[a] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, wlane | past, wband[a] + at, NTW ? 2 : 0));
+    };
+    f32x4 acc[4][NB];          // [W band a][slot tile b]
+#pragma unroll
+    for (int a = 0; a < 4; ++a)
+#pragma unroll
+        for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int swz = (r >> 1) & 7, xl0 = r * 128 + ((q ^ swz) * 16), xl1 = r * 128 + (((4 + q) ^ swz) * 16);
+    auto mul = [&](bf16x8 (&ws)[4], int buf, int kk) {
+        const unsigned char* xs = lds + buf * XB + (kk ? xl1 : xl0);
+        constexpr int NX = NB == 9 ? 3 : 4;                      // slot tiles read from LDS at a time
+#pragma unroll
+        for (int b0 = 0; b0 < NB; b0 += NX) {
+            bf16x8 xf[NX];
+#pragma unroll
+            for (int b = 0; b < NX; ++b)
+                if (b0 + b < NB) xf[b] = *(const bf16x8*)(xs + (b0 + b) * 2048);
+#pragma unroll
+            for (int a = 0; a < 4; ++a)
+#pragma unroll
+                for (int b = 0; b < NX; ++b)
+                    if (b0 + b < NB)
+                        acc[a][b0 + b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ws[a], xf[b], acc[a][b0 + b], 0, 0, 0);
+        }
+    };
+    // Step u: half steps 2u and 2u + 1 with the X of buffer u % 4, while X of step u + 3 goes to the buffer that step u - 1 has
+    // left (every wave has passed the barrier behind it).  Before the barrier each wave waits until its own loads of X for
+    // step u + 1 are there: younger than those are two steps of X and the W asked for since, three steps of eight loads or,
+    // with fewer sets, at least the sets of the start and one step.
+    constexpr int PENDING = 2 * XI + (8 + 4 * S < 24 ? 8 + 4 * S : 24);
+#define GG_MEET(pending) do { \
+        asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(pending) : "memory"); \
+        __builtin_amdgcn_s_barrier(); \
+        __builtin_amdgcn_sched_barrier(0); } while (0)
+    bf16x8 w[S][4];
+    load_x(0);
+    load_x(1);
+    load_x(2);
+#pragma unroll
+    for (int s = 0; s < S; ++s) load_w(w[s], s);
+    GG_MEET(2 * XI + 4 * S);
+    auto step = [&](bf16x8 (&wa)[4], bf16x8 (&wb)[4], int u) {
+        load_x(u + 3);
+        __builtin_amdgcn_sched_barrier(0);
+        mul(wa, u & 3, 0);
+        load_w(wa, 2 * u + S);
+        __builtin_amdgcn_sched_barrier(0);
+        mul(wb, u & 3, 1);
+        load_w(wb, 2 * u + S + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        GG_MEET(PENDING);
+    };
+    for (int u = 0; u < nu; u += S / 2) {
+#pragma unroll
+        for (int j = 0; j < S / 2; ++j) step(w[2 * j], w[2 * j + 1], u + j);
+    }
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");  // no load into LDS outlives the workgroup
+#undef GG_MEET
+
+    // acc[a][b][i] of lane (r, q): column n0 + (wave * TG + a) * 16 + q * 4 + i, slot row0 + b * 16 + r; four columns a store
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const int s = row0 + b * 16 + r;
+        if (s >= row_end) continue;
+        const float sc = p.a_scale ? p.a_scale[s] : 1.0f;
+        TY* yrow = (TY*)p.Y + (p.y_rows ? (size_t)p.y_rows[s] : (size_t)s) * p.ldy;
+#pragma unroll
+        for (int a = 0; a < TG; ++a) {
+            const int n = n0 + (wave * TG + a) * 16 + q * 4;
+            if (n >= N) continue;
+            float v[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                v[i] = acc[a][b][i] * sc;
+                if constexpr (GLU) v[i] = sp_gated(v[i], acc[a + 2][b][i] * sc, SP_ACT_SILU, 0.f, true);
+            }
+            if constexpr (sizeof(TY) == 2) {
+                bf16x4 o;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[i] = (bf16)v[i];
+                *(bf16x4*)(yrow + n) = o;
+            } else {
+                *(f32x4*)(yrow + n) = f32x4{v[0], v[1], v[2], v[3]};
+            }
+        }
+    }
+}
+
+// The tiles of a group of `rows` rows, and their height in units of 16 rows (2, 4 and every one from 5 to 10).
+__device__ __host__ __forceinline__ int gg_group_tiles(int rows, int cap, int& nb) {
+    const int tiles = (rows + cap - 1) / cap, each = tiles ? (rows + tiles - 1) / tiles : 0;
+    nb = (each + 15) / 16;
+    nb = nb <= 2 ? 2 : nb <= 4 ? 4 : nb;
+    return tiles;
+}
+
+template <int NW, bool GLU, typename TY>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_groups_kernel(gg_args p) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const int units = p.m_tiles * p.n_tiles, per_xcd = (units + 7) / 8;
+    const int unit = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if ((int)(blockIdx.x / 8) >= per_xcd || unit >= units) return;
+    // the group of the row tile, 64 groups at a time: a prefix sum over the lanes (one after another the loads of the offsets
+    // cost half a microsecond a group); what it finds is kept in scalar registers
+    const int mt = unit % p.m_tiles, lane = threadIdx.x & 63;
+    int g = -1, row0 = 0, row_end = 0, nb = 8, tiles = 0, base = 0;
+    for (int c = 0; c < p.n_groups; c += 64) {
+        int b = 0, e = 0, h = 0;
+        if (c + lane < p.n_groups) { b = p.offsets[c + lane]; e = p.offsets[c + lane + 1]; }
+        const int nt = gg_group_tiles(e - b, p.cap, h);
+        int incl = nt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
+        const int total = __builtin_amdgcn_readlane(incl, 63);
+        if (mt < base + total) {
+            const bool mine = mt >= base + incl - nt && mt < base + incl;
+            const int src = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(mine)) - 1);
+            g = c + src;
+            nb = __builtin_amdgcn_readlane(h, src);
+            tiles = __builtin_amdgcn_readlane(nt, src);
+            row_end = __builtin_amdgcn_readlane(e, src);
+            row0 = __builtin_amdgcn_readlane(b, src) + (mt - base - __builtin_amdgcn_readlane(incl - nt, src)) * 16 * nb;
+            break;
+        }
+        base += total;
+    }
+    // (no such tile; or, with heights rounded up, the group's rows end before its last tile)
+    if (g < 0 || row0 >= row_end) return;
+    const int n0 = unit / p.m_tiles * (GLU ? 32 * NW : 64 * NW);
+#define GG_TILE(NB, S, NT) gg_tile<NW, NB, S, GLU, TY, NT>(p, lds, g, row0, row_end, n0)
+#define GG_TILES(NT) switch (nb) { \
+        case 2: GG_TILE(2, 6, NT); break; \
+        case 4: GG_TILE(4, 6, NT); break; \
+        case 5: GG_TILE(5, 6, NT); break; \
+        case 6: GG_TILE(6, 6, NT); break; \
+        case 7: GG_TILE(7, 4, NT); break; \
+        case 8: GG_TILE(8, 4, NT); break; \
+        case 9: GG_TILE(9, 4, NT); break; \
+        default: GG_TILE(10, 4, NT); }
+    if (tiles == 1) GG_TILES(true) else GG_TILES(false)
+#undef GG_TILES
+#undef GG_TILE
+}
+
+template <int NW, bool GLU, typename TY>
+static int gg_launch(gg_args p, hipStream_t st) {
+    const int cols = (GLU ? 32 : 64) * NW;
+    p.n_tiles = (p.N + cols - 1) / cols;
+    // row tiles: a group of r rows has ceil(r / cap): at most r / cap + 1
+    p.m_tiles = p.M / p.cap + (p.n_groups < p.M ? p.n_groups : p.M);
+    SP_REQUIRE((long)p.m_tiles * p.n_tiles < (1L << 30), "gemm_groups: too many tiles");
+    const int grid = (p.m_tiles * p.n_tiles + 7) / 8 * 8;
+    static bool allowed = false;
+    if (!allowed) {
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_groups_kernel<NW, GLU, TY>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 160 * 128);
+        SP_REQUIRE(e == hipSuccess, "gemm_groups: 80 KB of LDS refused: %s", hipGetErrorString(e));
+        allowed = true;
+    }
+    gemm_groups_kernel<NW, GLU, TY><<<grid, NW * 64, (size_t)4 * p.cap * 128, st>>>(p);
+    SP_LAUNCH_CHECK("gemm_groups");
+    return 0;
+}
+
+// Arguments as spite_gemm_lds's (`x_rows`: how many rows X has); `waves` 4 or 8, `cap` 128 or 160.  Gated with silu
+// (`glu` SP_ACT_SILU) or plain (0); rows of Y that 16-byte stores can take.
+extern "C" int spite_gemm_groups(const void* X, int ldx, const void* W, long w_group_stride, void* Y, int y_dtype, int ldy, int M,
+                                 int N, int K, const int* offsets, int n_groups, const int* a_rows, const float* a_scale,
+                                 const int* y_rows, int glu, int waves, int cap, int x_rows, hipStream_t st) {
+    SP_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldy >= N, "gemm_groups: bad sizes M=%d N=%d K=%d", M, N, K);
+    SP_REQUIRE(offsets && n_groups > 0, "gemm_groups: no groups");
+    SP_REQUIRE(K % 64 == 0 && N % 16 == 0, "gemm_groups: operand order needs K=%d a multiple of 64 and N=%d of 16", K, N);
+    SP_REQUIRE(ldx % 8 == 0 && ((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0, "gemm_groups: operands must be 16-byte aligned");
+    SP_REQUIRE(ldy % 4 == 0 && ((uintptr_t)Y & 15) == 0, "gemm_groups: rows of Y must be 16-byte aligned");
+    SP_REQUIRE(y_dtype == SP_BF16 || y_dtype == SP_F32, "gemm_groups: output dtype %d", y_dtype);
+    SP_REQUIRE(glu == 0 || glu == SP_ACT_SILU, "gemm_groups: activation code %d", glu);
+    SP_REQUIRE((waves == 4 || waves == 8) && (cap == 128 || cap == 160), "gemm_groups: %d waves, tiles of %d rows", waves, cap);
+    SP_REQUIRE(x_rows > 0 && (a_rows || x_rows >= M), "gemm_groups: %d rows of X", x_rows);
+    // the loads' offsets are 32-bit: rows of X and a group's W
+    SP_REQUIRE((size_t)x_rows * ldx * 2 < ((size_t)1 << 31) && (size_t)(glu ? 2 : 1) * N * K * 2 < ((size_t)1 << 31),
+               "gemm_groups: operands of 2 GiB and more (%d rows of X, N=%d K=%d)", x_rows, N, K);
+    if (M == 0) return 0;
+    const gg_args p{(const bf16*)X, ldx, (const bf16*)W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, 0, 0, cap};
+    if (waves == 8) {
+        if (glu) return y_dtype == SP_BF16 ? gg_launch<8, true, bf16>(p, st) : gg_launch<8, true, float>(p, st);
+        return y_dtype == SP_BF16 ? gg_launch<8, false, bf16>(p, st) : gg_launch<8, false, float>(p, st);
+    }
+    if (glu) return y_dtype == SP_BF16 ? gg_launch<4, true, bf16>(p, st) : gg_launch<4, true, float>(p, st);
+    return y_dtype == SP_BF16 ? gg_launch<4, false, bf16>(p, st) : gg_launch<4, false, float>(p, st);
+}
+
+// Which waves and cap suit a product whose `routed` groups hold `mean` rows each on average (sizes taken as normal about it),
+// beside `whole` groups that take all `tokens` rows: waves * 256 + cap, or 0: gemm_tiled.
+//
+// The estimate: the tiles to expect and their mean height nb; a tile takes (a + b nb) us at K = 5,120, eight waves alone on a
+// compute unit, four in pairs (one alone a third of that); rounds of tiles over the slots, a last one that is not full counts
+// for most of one with eight waves and for a third with four; beside it the stream of the weights; then the two together,
+// between their maximum and their sum.  Fitted to 220 sizes (4 to 128 groups, 65 to 6,000 tokens, N and K of 512 to 8,192, plain
+// and gated) timed with each choice and with gemm_tiled: the choice is 14 % faster than gemm_tiled's best tile by its own
+// rules on average; nine are 2 % and more slower, most of them sizes where a tile more or less starts a round (4 x 220 rows x 6,912 x
+// 4,672: 127 against 100 until a deviation of tiles more was counted).
+// Where the tiles of eight waves are one for every second compute unit and up to one for each, and the time is the stream of
+// W, four waves, with a tile for some units and two for others, stream no faster; plain products stay with gemm_tiled
+// there (69 rows, 16 groups and one of all x 5,120 x 8,192: 246 with eight and 266 with four against 210), gated ones
+// take eight (300 rows x 2 x 3,072 x 2,048: 72 and 75 against 85).
+extern "C" int spite_gemm_groups_choice(int tokens, int routed, double mean, int whole, int N, int K, int glu) {
+    if (tokens <= 0 || routed <= 0 || mean <= 0.0) return 0;
+    static const double Z[11] = {-1.6, -1.0, -0.67, -0.43, -0.2, 0.0, 0.2, 0.43, 0.67, 1.0, 1.6};
+    const double cus = sp_cu_count(), share = mean / tokens < 1.0 ? mean / tokens : 1.0;
+    const double sd = sqrt(tokens * share * (1.0 - share));
+    const double live = routed * mean < routed ? routed * mean : routed;
+    const double stream = (live + whole) * (double)N * K * (glu ? 4 : 2) * 1e-6;       // MB
+    int best = 0;
+    double least = 0.0;
+    bool pairs = true;
+    for (int waves : {8, 4}) {
+        if (waves == 4 && !pairs) continue;
+        for (int cap : {160, 128}) {
+            double n = 0.0, sum = 0.0, squares = 0.0;
+            int most = 2, nb;
+            for (double z : Z) {
+                const int rows = (int)(mean + z * sd + 0.5);
+                if (rows <= 0) continue;
+                const int t = gg_group_tiles(rows, cap, nb);
+                n += t; sum += (double)t * nb; squares += (double)t * t;
+                most = nb > most ? nb : most;
+            }
+            // (a standard deviation of tiles more: a round that the tiles miss by one costs more than is to be gained)
+            const double spread = sqrt(fmax(routed * (squares / 11.0 - n / 11.0 * (n / 11.0)), 0.0));
+            n *= routed / 11.0; sum *= routed / 11.0;
+            if (whole) {
+                const int t = gg_group_tiles(tokens, cap, nb);
+                n += (double)whole * t; sum += (double)whole * t * nb;
+                most = nb > most ? nb : most;
+            }
+            if (n <= 0.0) return 0;
+            const double cols = (N + (glu ? 32 : 64) * waves - 1) / ((glu ? 32 : 64) * waves), tiles = (n + spread) * cols, nbm = sum / n;
+            double us;
+            if (waves == 8) {
+                const double r = tiles / cus, c = K / 5120.0 * (71.0 + 6.5 * nbm), alone = K / 5120.0 * (71.0 + 6.5 * most);
+                if (cap == 160 && r > 0.5 && r <= 0.95 && K / 5120.0 * (68.7 + 7.76 * nbm) * r < 0.7 * stream / 6.5) {
+                    if (!glu) return 0;
+                    pairs = false;
+                }
+                const double work = r <= 1.0 ? alone : c * (r + 0.8 * (ceil(r) - r));
+                us = 7.9 + pow(pow(work, 2.4) + pow(stream / 6.45, 2.4), 1.0 / 2.4);
+            } else {
+                const double r = tiles / (2.0 * cus), c = K / 5120.0 * (37.0 + 11.0 * nbm), alone = 0.31 * K / 5120.0 * (37.0 + 11.0 * most);
+                const double work = r <= 0.5 ? alone : r <= 1.0 ? (c > alone ? c : alone) : c * (r + 0.33 * (ceil(r) - r));
+                us = 8.2 + pow(pow(work, 1.6) + pow(stream / 6.8, 1.6), 1.0 / 1.6);
+            }
+            if (best == 0 || us <= least) { best = waves * 256 + cap; least = us; }
+        }
+    }
+    return best;
+}

@@ -68,6 +68,7 @@ def lib():
             "spite_attn_decode": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
             "spite_gemm_mfma": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_lds": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, I, P],
+            "spite_gemm_groups": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, I, I, I, P],
             "spite_gemm_tiled": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_tiled_split": [P, I, P, P, I, I, I, I, I, I, P, P],
             "spite_attn_prefill": [P, P, P, P, P, P, P, P, I, P, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
@@ -120,6 +121,8 @@ def lib():
         l.spite_router_plan_is_one_launch.restype = c_int
         l.spite_gemm_skinny_variant.argtypes = [I] * 7
         l.spite_gemm_skinny_variant.restype = c_int
+        l.spite_gemm_groups_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I]
+        l.spite_gemm_groups_choice.restype = c_int
         l.spite_gemm_lds_time.argtypes = [I, I, I, I]
         l.spite_gemm_lds_time.restype = ctypes.c_double
         l.spite_cu_count.argtypes = []
@@ -739,6 +742,33 @@ def gemm_lds(a, w, y, M, N, K, *, offsets=None, n_groups=1, a_rows=None, a_scale
         M, N, K, _ptr(offsets, "offsets", torch.int32, True), n_groups, _ptr(a_rows, "a_rows", torch.int32, True),
         _ptr(a_scale, "a_scale", torch.float32, True), _ptr(y_rows, "y_rows", torch.int32, True), _act_code(glu, act),
         float(act_limit), int(nb), a.shape[0], _stream()), "gemm_lds")
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_groups_choice(tokens: int, routed: int, mean: float, whole: int, N: int, K: int, glu: bool):
+    """(waves, cap) for ``gemm_groups``, or None where ``gemm_tiled`` is the faster one: ``routed`` groups of ``mean`` rows each on
+    average beside ``whole`` groups that take all ``tokens`` rows (the rule, and what it was timed against, in gemm_groups.hip)."""
+    code = lib().spite_gemm_groups_choice(tokens, routed, mean, whole, N, K, int(bool(glu)))
+    return divmod(code, 256) if code else None
+
+
+def gemm_groups_ok(a, y, M, N, K, glu) -> bool:
+    """Whether ``gemm_groups`` takes these operands: 32-bit offsets into the rows of ``a`` and a group of W, rows of ``y`` that
+    16-byte stores can take, silu or no gate."""
+    return glu in (0, 1) and gemm_lds_ok(a, None, M, N, K, glu) and y.stride(0) % 4 == 0 and y.data_ptr() % 16 == 0
+
+
+def gemm_groups(a, w, y, M, N, K, *, offsets, n_groups, a_rows=None, a_scale=None, y_rows=None, glu=False, waves=8, cap=128):
+    """Tiled bf16 product over groups, each in tiles of the height that suits it (see gemm_groups.hip); arguments as gemm_generic,
+    ``glu`` with silu.  ``waves`` (4 or 8) and ``cap`` (128 or 160): see ``gemm_groups_choice``."""
+    rows_w = _gemm_checks(a, w, y, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, "gemm_groups")
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        raise KernelError(f"gemm_groups: bfloat16 operands only, got {a.dtype} and {w.dtype}")
+    _check(lib().spite_gemm_groups(
+        _ptr_rows(a, "a"), a.stride(0), _ptr(w, "w"), rows_w * K, _ptr_rows(y, "y"), dtype_code(y.dtype), y.stride(0),
+        M, N, K, _ptr(offsets, "offsets", torch.int32), n_groups, _ptr(a_rows, "a_rows", torch.int32, True),
+        _ptr(a_scale, "a_scale", torch.float32, True), _ptr(y_rows, "y_rows", torch.int32, True), int(bool(glu)),
+        int(waves), int(cap), a.shape[0], _stream()), "gemm_groups")
 
 
 def attn_prefill_splits(counts, H, G, max_keys) -> int:

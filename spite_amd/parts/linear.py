@@ -138,11 +138,16 @@ def whole_group_apart(tokens: int, groups: int, N: int, K: int) -> int:
     return shape if routed + hipops.lds_us(tokens, N, K, False) < 0.94 * together else 0
 
 
+def _routed_and_whole(M, n_groups, most, group_rows):
+    """A routed group's rows on average and how many groups take every row: what the rows of the call leave over the routed
+    ones' (arguments as ``linear``'s)."""
+    mean = M / n_groups if group_rows is None else group_rows
+    return mean, min(max(round((M - n_groups * mean) / (most - mean)), 0), n_groups - 1) if most > mean else 0
+
+
 def _group_tiles(M, n_groups, most, group_rows, N, glu):
     """The tiles of ``gemm_tiled`` and of ``gemm_lds`` to expect of a product over groups (arguments as ``linear``'s)."""
-    mean = M / n_groups if group_rows is None else group_rows
-    # the groups that take every row: what the rows of the call leave over the routed ones'
-    whole = min(max(round((M - n_groups * mean) / (most - mean)), 0), n_groups - 1) if most > mean else 0
+    mean, whole = _routed_and_whole(M, n_groups, most, group_rows)
     tiles = lambda rows, cols: ((n_groups - whole) * math.ceil(mean / rows) + whole * -(-most // rows)) * -(-N // cols)
     return tiles(128, 256 if glu else 512), tiles(256, 128 if glu else 256)
 
@@ -182,6 +187,13 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
         if tiled:
             splits = offsets is None and a_rows is None and a_scale is None and y_rows is None and not glu and act is None
             runs = hipops.tiled_k_runs(M, N, K) if splits and tile_shape == 0 and M > 0 else 1
+            if offsets is not None and M > 0 and act is None and hipops.gemm_groups_ok(x, y, M, N, K, glu):
+                mean, whole = _routed_and_whole(M, n_groups, most, group_rows)
+                choice = hipops.gemm_groups_choice(most, n_groups - whole, float(mean), whole, N, K, bool(glu))
+                if choice is not None:
+                    hipops.gemm_groups(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
+                                       y_rows=y_rows, glu=bool(glu), waves=choice[0], cap=choice[1])
+                    return
             if M > 0 and hipops.gemm_lds_ok(x, w, M, N, K, glu) and (
                     hipops.lds_suits(M, N, K, bool(glu), runs) if offsets is None
                     else hipops.lds_suits_groups(M / n_groups if group_rows is None else group_rows, K,

@@ -1,0 +1,60 @@
+"""The product over groups in tiles of several heights: every height and both ends of it, one step of K and a last round that K
+does not fill, against float64 and, bit for bit, against the tiled product (both add k in the same order)."""
+import pytest
+import torch
+
+from test_kernels import DEV, ops, rnd, run_gemm
+
+HEIGHTS = [0, 1, 32, 33, 64, 65, 80, 81, 96, 97, 112, 113, 128, 129, 144, 145, 160, 161, 0, 257, 321]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,groups", [(70, 48, 64, 5), (400, 272, 128, 3), (900, 528, 192, 4), (90, 16, 320, 70), (300, 144, 448, 130)])
+@pytest.mark.parametrize("glu,out_dtype", [(False, torch.float32), (False, torch.bfloat16), (True, torch.bfloat16), (True, torch.float32)])
+@pytest.mark.parametrize("waves,cap", [(4, 128), (4, 160), (8, 128), (8, 160)])
+def test_groups_with_row_lists(M, N, K, groups, glu, out_dtype, waves, cap):
+    def fn(a, w, y, M, N, K, **kw):
+        ops().gemm_groups(a, ops().operand_order(w), y, M, N, K, waves=waves, cap=cap, **kw)
+    run_gemm(fn, torch.bfloat16, out_dtype, M, N, K, glu, True, groups)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("waves,cap", [(4, 128), (4, 160), (8, 128), (8, 160)])
+@pytest.mark.parametrize("K", [64, 192, 320])
+def test_groups_of_every_height_equal_the_tiled_product(glu, waves, cap, K):
+    """What the local memory held before must not show: a product whose rows are not numbers runs first."""
+    M, N, G = sum(HEIGHTS), 272, len(HEIGHTS)
+    a, w = rnd(M, K, dtype=torch.bfloat16), ops().operand_order(rnd(G, 2 * N if glu else N, K, dtype=torch.bfloat16, seed=1))
+    offsets = torch.tensor([sum(HEIGHTS[:g]) for g in range(G + 1)], dtype=torch.int32, device=DEV)
+    y, z = torch.zeros(M, N, device=DEV), torch.ones(M, N, device=DEV)
+    ops().gemm_tiled(a, w, y, M, N, K, offsets=offsets, n_groups=G, glu=glu, shape=1)
+    ops().gemm_groups(torch.full_like(a, float("nan")), w, z, M, N, K, offsets=offsets, n_groups=G, glu=glu, waves=waves, cap=cap)
+    ops().gemm_groups(a, w, z, M, N, K, offsets=offsets, n_groups=G, glu=glu, waves=waves, cap=cap)
+    assert torch.equal(y, z)
+
+
+@pytest.mark.gpu
+def test_refuses_what_it_cannot_do():
+    z = lambda *s: torch.zeros(*s, dtype=torch.bfloat16, device=DEV)
+    o = torch.tensor([0, 4], dtype=torch.int32, device=DEV)
+    call = lambda a, w, y, K=64, **kw: ops().gemm_groups(a, w, y, 4, y.shape[1], K, offsets=o, n_groups=1, **kw)
+    for a, w, y, kw in ((z(4, 96), z(1, 16, 96), z(4, 16), dict(K=96)), (z(4, 64), z(1, 24, 64), z(4, 24), {}),
+                        (z(4, 64), z(1, 16, 64), z(4, 18)[:, :16], {}), (z(4, 64), z(1, 16, 64), z(4, 16), dict(waves=6)),
+                        (z(4, 64), z(1, 16, 64), z(4, 16), dict(cap=96))):
+        with pytest.raises(ops().KernelError):
+            call(a, w, y, **kw)
+    assert not ops().gemm_groups_ok(z(4, 64), z(4, 16), 4, 16, 64, ops().gate_code("relu")[0])
+    assert not ops().gemm_groups_ok(z(4, 64), z(4, 18)[:, :16], 4, 16, 64, 0) and ops().gemm_groups_ok(z(4, 64), z(4, 16), 4, 16, 64, 1)
+
+
+def test_choice_of_waves_and_height():
+    """Sizes that were timed: long prompts and short ones, narrow experts, and streams of W that the tiled product keeps."""
+    from spite_amd.csrc.hipops import gemm_groups_choice
+    at = lambda T, E, top, whole, N, K, glu: gemm_groups_choice(T, E, T * top / E, whole, N, K, glu)
+    assert at(2048, 16, 1, 1, 8192, 5120, True) == (8, 160) and at(1547, 16, 1, 1, 8192, 5120, True) == (8, 128)
+    assert at(330, 16, 1, 1, 8192, 5120, True)[0] == 4 and at(1531, 16, 4, 2, 1024, 2048, True) == (4, 128)
+    assert at(1200, 16, 1, 1, 2048, 3072, False)[0] == 4
+    for T in (69, 228, 425):
+        assert at(T, 16, 1, 1, 5120, 8192, False) is None
+    assert at(300, 4, 1, 0, 1216, 4416, False) == (4, 128) and gemm_groups_choice(0, 16, 0.0, 0, 64, 64, False) is None
