@@ -10,16 +10,14 @@
 //  gemm_f32_rows: few rows.  Bound by the stream of W (one row of X makes 0.5 FLOP a byte).  A workgroup takes 16
 //    rows of W (GLU: 16 of each half) and gives one run of k to each of its eight waves, so that a product with
 //    2,048 output rows has 1,024 waves in flight; the runs' sums meet in LDS.
-//  gemm_f32_tile: many rows, bound by the MFMAs (256 FLOP a clock and compute unit).  64 rows of X times 64 rows of W a
-//    workgroup: X through double-buffered LDS, a step ahead, read by all four waves; a wave's 16 rows of W straight into
-//    registers, two steps ahead.  The smaller tile than a large product would want is for the sizes at hand: 301 tokens times 2,048
-//    columns are 160 workgroups.
+//  gemm_f32_tile: many rows, bound by the MFMAs (256 FLOP a clock and compute unit).  TM (64 or 32) rows of X times 64 rows of
+//    W a workgroup: X through double-buffered LDS, a step ahead, read by all four waves; a wave's 16 rows of W straight into
+//    registers, two steps ahead.  One workgroup a compute unit reaches 45 % of the units' rate, since nothing fills its waits;
+//    several 70 %.
 //
-// SP_F32_ROWS_MAX: up to 64 rows the first one reads each byte of W once, beyond it would read W again for every
-// further 64 rows.
+// Which one, and its tile: see f32_variant.
 #include "common.h"
 
-#define SP_F32_ROWS_MAX 64
 
 // sum of one step of 16 k: the lane's four k of each operand
 __device__ __forceinline__ void f32_step(f32x4& acc, f32x4 w, f32x4 x) {
@@ -122,18 +120,17 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
     f32_store(Y, y_rows ? (size_t)y_rows[s] : (size_t)s, ldy, n0 + q * 4, N, t[0], vec_y);
 }
 
-#define F32_TM 64                 // rows of X a workgroup
 #define F32_TK 64                 // k a step through LDS
 #define F32_LD (F32_TK + 4)       // LDS row: 16 bytes more than a step, so that 16 rows' reads spread over the banks
 
 // The loop over k for a tile whose first LIVE groups of 16 rows hold rows (an expert's last tile is seldom full).  Loads
 // are unconditional, X's a step ahead of its use and W's two (three sets of registers in turn), and X is scaled only when it
 // goes to LDS, so that nothing waits for them before the step's MFMAs; a chain of four MFMAs is spread over the accumulators.
-template <int NB, int LIVE>
+template <int TM, int NB, int LIVE>
 __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp, const float* const* xp, const float* sc, int K,
-                                              int seg, int lr, int lk, int r, int q, f32x4 (&tot)[4][NB]) {
+                                              int seg, int lr, int lk, int r, int q, f32x4 (&tot)[TM / 16][NB]) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    constexpr int U = F32_TK / 16, XL = F32_TM * F32_TK / 1024;      // steps of 16 k, 16-byte pieces of X a thread
+    constexpr int U = F32_TK / 16, XL = TM * F32_TK / 1024;      // steps of 16 k, 16-byte pieces of X a thread
     f32x4 acc[LIVE][NB], w0[U][NB], w1[U][NB], w2[U][NB], xv[XL];
 #pragma unroll
     for (int m = 0; m < LIVE; ++m)
@@ -149,7 +146,7 @@ __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp,
     _Pragma("unroll") for (int i = 0; i < XL; ++i) xv[i] = *(const f32x4*)(xp[i] + kx); } while (0)
 #define F32_PUT(buf, k0) do { \
     _Pragma("unroll") for (int i = 0; i < XL; ++i) \
-        *(f32x4*)(xs + (buf) * (F32_TM * F32_LD) + (lr + i * (F32_TM / XL)) * F32_LD + lk) = (k0) + lk < K ? xv[i] * sc[i] : zero; } while (0)
+        *(f32x4*)(xs + (buf) * (TM * F32_LD) + (lr + i * (TM / XL)) * F32_LD + lk) = (k0) + lk < K ? xv[i] * sc[i] : zero; } while (0)
     // Step k0 multiplies the set wa with the rows in buffer `buf`; the rows of the next step and W of the step after the
     // next are asked for first, in this order: waiting for the rows leaves W on its way.
 #define F32_STEP(wa, wc) do { \
@@ -161,7 +158,7 @@ __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp,
     F32_X(k0 + F32_TK); \
     F32_W(wc, k0 + 2 * F32_TK); \
     __builtin_amdgcn_sched_barrier(0); \
-    const float* xb = xs + buf * (F32_TM * F32_LD); \
+    const float* xb = xs + buf * (TM * F32_LD); \
     _Pragma("unroll") for (int u = 0; u < U; ++u) { \
         if (k0 + u * 16 + 16 > K) { \
             const bool in = k0 + u * 16 + q * 4 < K; \
@@ -197,19 +194,21 @@ __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp,
 #undef F32_PUT
 }
 
-template <int GLU>
+template <int TM, int GLU>
 __global__ __launch_bounds__(256)
 void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, long w_group_stride,
                           float* __restrict__ Y, int ldy, int M, int N, int K, const int* __restrict__ offsets, int n_groups,
                           const int* __restrict__ a_rows, const float* __restrict__ a_scale, const int* __restrict__ y_rows,
                           int act, float act_limit, int vec_y) {
     constexpr int NB = GLU ? 2 : 1;
-    __shared__ __align__(16) float xs[2 * F32_TM * F32_LD];
+    __shared__ __align__(16) float xs[2 * TM * F32_LD];
     int g = 0, row0 = 0, row_end = M;
     if (offsets) {
-        if (!sp_find_tile(offsets, n_groups, F32_TM, blockIdx.y, g, row0, row_end)) return;
+        // the last groups' tiles start first: a group that every row visits comes last and has the full ones, an expert's
+        // hold a few rows and fill the end (17 groups, 301 rows over 16 and all of them, 2 x 3,072 x 2,048 gated: 264 / 287 us; 16 x 20 rows 208 / 252)
+        if (!sp_find_tile(offsets, n_groups, TM, gridDim.y - 1 - blockIdx.y, g, row0, row_end)) return;
     } else {
-        row0 = blockIdx.y * F32_TM;
+        row0 = blockIdx.y * TM;
     }
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;
@@ -220,28 +219,33 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
     wp[0] = Wg + (size_t)wn * K;
     if (GLU) wp[NB - 1] = Wg + (size_t)(N + wn) * K;
     // the loader: a thread brings 4 k of every XL-th part of the rows
-    constexpr int XL = F32_TM * F32_TK / 1024, PIECES = F32_TK / 4;
+    constexpr int XL = TM * F32_TK / 1024, PIECES = F32_TK / 4;
     const int lk = (threadIdx.x % PIECES) * 4, lr = threadIdx.x / PIECES;
     const float* xp[XL];
     float sc[XL];
 #pragma unroll
     for (int i = 0; i < XL; ++i) {
-        const int s = row0 + lr + i * (F32_TM / XL), ss = s < row_end ? s : row0;
+        const int s = row0 + lr + i * (TM / XL), ss = s < row_end ? s : row0;
         xp[i] = A + (size_t)(a_rows ? a_rows[ss] : ss) * lda;
         sc[i] = a_scale ? a_scale[ss] : 1.0f;
     }
-    f32x4 tot[4][NB];
+    f32x4 tot[TM / 16][NB];
 #pragma unroll
-    for (int m = 0; m < 4; ++m)
+    for (int m = 0; m < TM / 16; ++m)
 #pragma unroll
         for (int b = 0; b < NB; ++b) tot[m][b] = {0.f, 0.f, 0.f, 0.f};
     const int rows = row_end - row0, seg = f32_seg(K);
-    if (rows > 48) f32_tile_loop<NB, 4>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
-    else if (rows > 32) f32_tile_loop<NB, 3>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
-    else if (rows > 16) f32_tile_loop<NB, 2>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
-    else f32_tile_loop<NB, 1>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+    bool done = false;
+    if constexpr (TM == 64) {
+        if (rows > 48) f32_tile_loop<TM, NB, 4>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+        else if (rows > 32) f32_tile_loop<TM, NB, 3>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+        done = rows > 32;
+    }
+    if (done) {}
+    else if (rows > 16) f32_tile_loop<TM, NB, 2>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+    else f32_tile_loop<TM, NB, 1>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
 #pragma unroll
-    for (int m = 0; m < 4; ++m) {
+    for (int m = 0; m < TM / 16; ++m) {
         const int s = row0 + m * 16 + r;
         if (s >= row_end) continue;
         f32x4 t = tot[m][0];
@@ -252,20 +256,46 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
     }
 }
 
+// Rows of X a workgroup takes: of gemm_f32_rows (16, 32 or 64), or minus those of gemm_f32_tile (32 or 64).  `n_groups` 0: no groups.
+//
+// Measured on an MI355X (us), products in a row over weights that the caches do not hold; "gate/up" 2 x 3,072 x 2,048 gated and
+// "down" 2,048 x 3,072 over 16 experts and a shared one, `t` tokens:
+//  * groups of up to eight rows on average: the stream of every group's W, 16 rows a workgroup, whatever the call's rows are
+//    (t = 16: gate/up 124, with 32 rows a workgroup 190; t = 32 169, with 64 rows 331, tiles of 32 211; t = 64 184 / tiles 207;
+//    the shared group's W comes from L2 for its further rows).
+//  * no groups: the stream up to 64 rows, unless W is tall enough for two workgroups of tiles a compute unit (32,768 x 2,048: 9 rows
+//    54 with the stream, 48 with tiles of 32; 16: 64 / 49; 64: 198 / 98; 8 51 / 52; 3,072 x 2,048 stays, 64 rows 26 / 35).
+//  * tiles of 32 rows where those of 64 would be fewer than four a compute unit (3,072 x 2,048, 100 rows: 35 / 53, 301: 54 / 60;
+//    2,048 x 2,048, 200: 35 / 52; down, t = 200: 109 / 133; gate/up, t = 150: 214 / 237, but t = 200, over the line: 264 / 247;
+//    32,768 x 2,048, 100 rows, over the line: 188 / 168).
+static int f32_variant(int M, int N, int n_groups) {
+    const long cus = sp_cu_count(), cols = (N + 63) / 64;
+    if (n_groups && M <= 8L * n_groups && M / 16L + n_groups <= 65535) return 16;      // (the grid's limit)
+    if (M <= 64 && (n_groups || M <= 8 || cols * ((M + 31) / 32) < 2 * cus)) return M > 32 ? 64 : M > 16 ? 32 : 16;
+    const long tiles = (n_groups ? M / 64 + (n_groups < M ? n_groups : M) : (M + 63) / 64) * cols;
+    return tiles < 4 * cus ? -32 : -64;
+}
+extern "C" int spite_gemm_f32_variant(int M, int N, int n_groups) { return f32_variant(M, N, n_groups); }
+
 // The product if its rows can be read 16 bytes at a time (returns 0, or an error), else 1: the plain kernel's.
 int sp_gemm_f32(const float* A, int lda, const float* W, long w_group_stride, float* Y, int ldy, int M, int N, int K,
                 const int* offsets, int n_groups, const int* a_rows, const float* a_scale, const int* y_rows, int glu,
                 float act_limit, hipStream_t st) {
     if (K % 4 || lda % 4 || w_group_stride % 4 || ((uintptr_t)A | (uintptr_t)W) % 16) return 1;
     const int vec_y = ldy % 4 == 0 && (uintptr_t)Y % 16 == 0;
-    const int tile = M > SP_F32_ROWS_MAX ? F32_TM : M > 32 ? 64 : M > 16 ? 32 : 16;
+    const int variant = f32_variant(M, N, offsets ? n_groups : 0), tile = variant > 0 ? variant : -variant;
     const int m_tiles = offsets ? M / tile + (n_groups < M ? n_groups : M) : (M + tile - 1) / tile;
     SP_REQUIRE(m_tiles <= 65535, "gemm: too many row tiles (%d)", m_tiles);
 #define SP_F32_ARGS A, lda, W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, act_limit, vec_y
-    if (M > SP_F32_ROWS_MAX) {
+    if (variant < 0) {
         dim3 grid((N + 63) / 64, m_tiles);
-        if (glu) gemm_f32_tile_kernel<1><<<grid, 256, 0, st>>>(SP_F32_ARGS);
-        else gemm_f32_tile_kernel<0><<<grid, 256, 0, st>>>(SP_F32_ARGS);
+        if (tile == 32) {
+            if (glu) gemm_f32_tile_kernel<32, 1><<<grid, 256, 0, st>>>(SP_F32_ARGS);
+            else gemm_f32_tile_kernel<32, 0><<<grid, 256, 0, st>>>(SP_F32_ARGS);
+        } else {
+            if (glu) gemm_f32_tile_kernel<64, 1><<<grid, 256, 0, st>>>(SP_F32_ARGS);
+            else gemm_f32_tile_kernel<64, 0><<<grid, 256, 0, st>>>(SP_F32_ARGS);
+        }
         SP_LAUNCH_CHECK("gemm_f32_tile");
         return 0;
     }

@@ -123,6 +123,8 @@ def lib():
         l.spite_gemm_skinny_variant.restype = c_int
         l.spite_gemm_groups_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I]
         l.spite_gemm_groups_choice.restype = c_int
+        l.spite_gemm_f32_variant.argtypes = [I, I, I]
+        l.spite_gemm_f32_variant.restype = c_int
         l.spite_gemm_lds_time.argtypes = [I, I, I, I]
         l.spite_gemm_lds_time.restype = ctypes.c_double
         l.spite_cu_count.argtypes = []

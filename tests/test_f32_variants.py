@@ -1,0 +1,34 @@
+"""Which of the 32-bit products a call takes, and the same bits from each of them."""
+import pytest
+import torch
+
+from test_kernels import DEV, ops, rnd, run_gemm
+
+
+def test_lines_lie_where_both_sides_were_timed():
+    from spite_amd.csrc.hipops import lib
+    at = lib().spite_gemm_f32_variant
+    assert [at(2 * t, 3072, 17) for t in (1, 16, 32, 64, 68, 150, 200)] == [16, 16, 16, 16, 16, -32, -64]
+    assert [at(m, 32768, 0) for m in (1, 8, 9, 64, 65, 100)] == [16, 16, -32, -32, -64, -64]
+    assert [at(m, 3072, 0) for m in (16, 17, 64, 65, 301)] == [16, 32, 64, -32, -32]
+    assert at(400000, 64, 50000) == -64 and at(64, 64, 2) == 64
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,groups", [(200, 40), (70, 5), (300, 5), (40, 3)])
+@pytest.mark.parametrize("N,K,glu", [(80, 292, False), (80, 292, True), (16400, 36, False)])
+def test_groups(M, groups, N, K, glu):
+    run_gemm(ops().gemm_generic, torch.float32, torch.float32, M, N, K, glu, True, groups)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("rows", [1, 8, 9, 16, 17, 32, 33, 48, 49, 64, 65, 100])
+def test_a_row_of_a_tall_matrix_has_the_same_bits_in_every_variant(rows):
+    N, K = 16400 * 2, 132
+    a, w = rnd(130, K), rnd(N, K, seed=1)
+    whole, part = torch.empty(130, N, device=DEV), torch.empty(rows, N, device=DEV)
+    ops().gemm_generic(a, w, whole, 130, N, K)
+    ops().gemm_generic(a[:rows].contiguous(), w, part, rows, N, K)
+    narrow = torch.empty(rows, 48, device=DEV)
+    ops().gemm_generic(a[:rows].contiguous(), w[:48].contiguous(), narrow, rows, 48, K)
+    assert torch.equal(part, whole[:rows]) and torch.equal(narrow, whole[:rows, :48])
