@@ -143,6 +143,9 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
 // ... and the lanes' sums meet in a butterfly.  Every kernel that forms router logits calls
 // this, so a logit has the same bits wherever it is computed; its order of summation depends
 // on the width alone.
+__device__ __forceinline__ float dot4_add(float acc, const f32x4& w, const f32x4& x) {
+    return acc + (w[0] * x[0] + w[1] * x[1] + w[2] * x[2] + w[3] * x[3]);
+}
 __device__ __forceinline__ float wave_dot_row(const float* __restrict__ w, const float* xs, int d, bool vec, int lane) {
     float acc = 0.f;
     if (vec) {
@@ -151,7 +154,7 @@ __device__ __forceinline__ float wave_dot_row(const float* __restrict__ w, const
         for (int c = lane; c < nv; c += 64) {          // independent 16-byte loads, ten in flight
             const f32x4 ww = ((const f32x4*)w)[c];
             const f32x4 xx = ((const f32x4*)xs)[c];
-            acc += ww[0] * xx[0] + ww[1] * xx[1] + ww[2] * xx[2] + ww[3] * xx[3];
+            acc = dot4_add(acc, ww, xx);
         }
     } else {
         for (int c = lane; c < d; c += 64) acc += w[c] * xs[c];

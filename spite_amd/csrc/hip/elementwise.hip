@@ -84,153 +84,226 @@ __device__ __forceinline__ int top1_of(const float* __restrict__ l, int E, float
 // one stream: a layer whose mixer and feed-forward read the same rows), in `out`'s dtype.
 // PLAN (a single row): the projection is a router's logits and the row's list for the grouped products is made here
 // too, as moe_plan makes it: one of some 4.5 us of launches that a layer of a single decoded token is made of (5,120 wide
-// over 16 experts: 11.2 us for the two kernels, 7.1 for this one).
+// over 16 experts: 11.2 us for the two kernels, 6.8 for this one).
 struct norm_plan { int* expert; float* weight; int* src; float* scale; int* dst; int* offsets; int shared; };
 #define NORM_NT 512
-#define NORM_MAX_V 8     // widths up to 4*NT*MAX_V = 16384 stay in registers
-template <typename TO, bool VEC, bool PLAN>
+#define NORM_R 2         // rows a workgroup of many rows with a projection
+#define NORM_MAX_V 8     // rows of up to 4*NT*MAX_V = 16384 that 16-byte loads can take stay in registers
+struct norm_args {
+    float* h; const float *d1, *d2, *w; float* out32; const int* rows; int n_rows, d; float eps; int write_h;
+    const float* proj; float* proj_out; int P; const float *dn, *wn; float mult, eps_n; int plain_out; const float* w2; norm_plan plan;
+};
+
+// The row's list from its P logits (in LDS): what moe_plan makes of a single row.
+__device__ __forceinline__ void norm_make_plan(const norm_plan& plan, const float* logits, int P) {
+    float best;
+    const int me = top1_of(logits, P, &best);
+    if (threadIdx.x == 0) {
+        const float wt = 1.0f / (1.0f + expf(-best));
+        plan.expert[0] = me; plan.weight[0] = wt;
+        plan.src[0] = 0; plan.scale[0] = wt; plan.dst[0] = 0;
+    }
+    for (int g = threadIdx.x; g <= P; g += NORM_NT) plan.offsets[g] = me < g;
+    if ((int)threadIdx.x < plan.shared) {
+        const int j = 1 + threadIdx.x;
+        plan.src[j] = 0; plan.scale[j] = 1.0f; plan.dst[j] = j;
+        plan.offsets[P + j] = 1 + j;
+    }
+}
+
+// Rows that 16-byte loads can take: V groups of four a thread.
+//  Few rows (a decoded batch): one workgroup a row, most of the chip idle, and what counts is how many times it waits for
+//  memory.  Every load that depends on nothing is asked for at once, without a condition (groups past the row read its last one
+//  again): the stream, its increments and all weights.  On an MI355X, launches in a row, against loads group by group as they
+//  are needed (us): one row of 5,120 3.3 / 4.0, of 2,048 2.3 / 2.9, with 16 rows of proj 6.1 / 7.0 and 4.2 / 5.6; 2,048 rows of 5,120
+//  29 / 33 (6.5 TB/s), of 2,048 14 / 17.  Two rows of proj a wave in flight where the row is short (2,048: 4.2, one 5.0; 5,120: 8.1
+//  / 6.1).
+//  Many rows with a projection: R rows a workgroup, since each workgroup reads all of `proj` from L2 (16 x 5,120: 320 KB beside
+//  60 KB of the row; 2,048 rows 41 / 43, four rows a workgroup, for which LDS has less room, 59; 330 rows 10.1 / 11.3).
+template <typename TO, int V, int R, bool PLAN>
 __global__ __launch_bounds__(NORM_NT)
-void add_rmsnorm_kernel(float* __restrict__ h, const float* __restrict__ d1,
-                        const float* __restrict__ d2, const float* __restrict__ w,
-                        TO* __restrict__ out, float* __restrict__ out32,
-                        const int* __restrict__ rows, int d, float eps, int write_h,
-                        const float* __restrict__ proj, float* __restrict__ proj_out, int P,
-                        const float* __restrict__ dn, const float* __restrict__ wn, float mult, float eps_n,
-                        int plain_out, const float* __restrict__ w2, TO* __restrict__ out2, norm_plan plan) {
+void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ out2) {
     __shared__ float red[NORM_NT / 64];
-    extern __shared__ __attribute__((aligned(16))) float ys[];            // [d] if proj, and P logits behind it (at a multiple of 4) if plan
-    const int i = blockIdx.x;
-    const size_t r = rows ? (size_t)rows[i] : (size_t)i;
-    float* hr = h + r * d;
-    const float* a = d1 ? d1 + r * d : nullptr;
-    const float* b = d2 ? d2 + r * d : nullptr;
-    const float* nr = dn ? dn + r * d : nullptr;
+    extern __shared__ __attribute__((aligned(16))) float ys[];            // [R][d] if proj, and P logits behind it if PLAN
+    const int d = p.d, nv = d >> 2, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    int at[V];                                                            // the thread's groups
+#pragma unroll
+    for (int u = 0; u < V; ++u) at[u] = tid + u * NORM_NT < nv ? tid + u * NORM_NT : nv - 1;
+    f32x4 ww[V], ww2[V];
+    const bool outputs = out || p.out32 || p.proj || out2, normed = outputs && !p.plain_out;
+    const int first = blockIdx.x * R, rows = R == 1 ? 1 : (p.n_rows - first < R ? p.n_rows - first : R);
+    for (int rr = 0; rr < rows; ++rr) {
+        const int i = first + rr;
+        const size_t r = p.rows ? (size_t)p.rows[i] : (size_t)i;
+        float* hr = p.h + r * d;
+        f32x4 v[V], x1[V], x2[V], xn[V], wn[V];
+        if (p.dn)
+#pragma unroll
+            for (int u = 0; u < V; ++u) xn[u] = ((const f32x4*)(p.dn + r * d))[at[u]];
+#pragma unroll
+        for (int u = 0; u < V; ++u) v[u] = ((const f32x4*)hr)[at[u]];
+        if (p.d1)
+#pragma unroll
+            for (int u = 0; u < V; ++u) x1[u] = ((const f32x4*)(p.d1 + r * d))[at[u]];
+        if (p.d2)
+#pragma unroll
+            for (int u = 0; u < V; ++u) x2[u] = ((const f32x4*)(p.d2 + r * d))[at[u]];
+        if (p.dn)
+#pragma unroll
+            for (int u = 0; u < V; ++u) wn[u] = ((const f32x4*)p.wn)[at[u]];
+        if (rr == 0 && normed) {
+#pragma unroll
+            for (int u = 0; u < V; ++u) ww[u] = ((const f32x4*)p.w)[at[u]];
+            if (out2)
+#pragma unroll
+                for (int u = 0; u < V; ++u) ww2[u] = ((const f32x4*)p.w2)[at[u]];
+        }
+        float sn = 0.f, ss = 0.f;
+        if (p.dn) {
+            float sq = 0.f;
+#pragma unroll
+            for (int u = 0; u < V; ++u) {
+                const float t = xn[u][0] * xn[u][0] + xn[u][1] * xn[u][1] + xn[u][2] * xn[u][2] + xn[u][3] * xn[u][3];
+                if (tid + u * NORM_NT < nv) sq += t;
+            }
+            sn = p.mult / sqrtf(block_sum<NORM_NT>(sq, red) / (float)d + p.eps_n);
+        }
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            if (p.d1) v[u] += x1[u];
+            if (p.d2) v[u] += x2[u];
+            if (p.dn)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) v[u][e] += xn[u][e] * sn * wn[u][e];
+            const float t = v[u][0] * v[u][0] + v[u][1] * v[u][1] + v[u][2] * v[u][2] + v[u][3] * v[u][3];
+            if (tid + u * NORM_NT < nv) {
+                ss += t;
+                if (p.write_h) ((f32x4*)hr)[tid + u * NORM_NT] = v[u];
+            }
+        }
+        if (!outputs) continue;                            // the additions were all that was asked for
+        const float scale = p.plain_out ? 1.f : 1.0f / sqrtf(block_sum<NORM_NT>(ss, red) / (float)d + p.eps);
+#pragma unroll
+        for (int u = 0; u < V; ++u) {
+            const int c = tid + u * NORM_NT;
+            if (c >= nv) continue;
+            f32x4 y = v[u];
+            if (!p.plain_out)
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y[e] = v[u][e] * scale * ww[u][e];
+            if (p.out32) ((f32x4*)(p.out32 + (size_t)i * d))[c] = y;
+            if (p.proj) ((f32x4*)(ys + rr * d))[c] = y;
+            auto put = [&](TO* dst, const f32x4& yy) {
+                if constexpr (sizeof(TO) == 2) {             // four bf16 in one 8-byte store
+                    bf16x4 o4;
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) o4[e] = (bf16)yy[e];
+                    *(bf16x4*)((bf16*)dst + (size_t)i * d + 4 * c) = o4;
+                } else {
+                    ((f32x4*)((float*)dst + (size_t)i * d))[c] = yy;
+                }
+            };
+            if (out) put(out, y);
+            if (out2) {                                      // the same row under a second norm's weights
+                f32x4 y2;
+#pragma unroll
+                for (int e = 0; e < 4; ++e) y2[e] = v[u][e] * scale * ww2[u][e];
+                put(out2, y2);
+            }
+        }
+    }
+    if (!p.proj) return;
+    __syncthreads();
+    float* logits = ys + ((d + 3) & ~3);
+    constexpr int NE = R == 1 && V == 1 ? 2 : 1, NWV = NORM_NT / 64;      // rows of proj a wave has in flight
+    for (int e = wave; e < p.P; e += NE * NWV) {
+        float acc[NE][R];
+#pragma unroll
+        for (int j = 0; j < NE; ++j)
+#pragma unroll
+            for (int rr = 0; rr < R; ++rr) acc[j][rr] = 0.f;
+        const f32x4* pr[NE];
+#pragma unroll
+        for (int j = 0; j < NE; ++j) pr[j] = (const f32x4*)(p.proj + (size_t)(e + j * NWV < p.P ? e + j * NWV : e) * d);
+#pragma unroll 10
+        for (int c = lane; c < nv; c += 64) {
+#pragma unroll
+            for (int j = 0; j < NE; ++j) {
+                const f32x4 w4 = pr[j][c];
+#pragma unroll
+                for (int rr = 0; rr < R; ++rr) acc[j][rr] = dot4_add(acc[j][rr], w4, ((const f32x4*)(ys + rr * d))[c]);
+            }
+        }
+#pragma unroll
+        for (int j = 0; j < NE; ++j)
+#pragma unroll
+        for (int rr = 0; rr < R; ++rr) {
+            const float t = wave_sum(acc[j][rr]);
+            if (lane == 0 && rr < rows && e + j * NWV < p.P) {
+                p.proj_out[(size_t)(first + rr) * p.P + e + j * NWV] = t;
+                if (PLAN) logits[e + j * NWV] = t;
+            }
+        }
+    }
+    if (!PLAN) return;
+    __syncthreads();
+    norm_make_plan(p.plan, logits, p.P);
+}
+
+// Any row, an element a thread at a time.
+template <typename TO, bool PLAN>
+__global__ __launch_bounds__(NORM_NT)
+void add_rmsnorm_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ out2) {
+    __shared__ float red[NORM_NT / 64];
+    extern __shared__ __attribute__((aligned(16))) float ys[];            // as above
+    const int i = blockIdx.x, d = p.d, write_h = p.write_h, plain_out = p.plain_out, P = p.P;
+    const float eps = p.eps, mult = p.mult, eps_n = p.eps_n, *w = p.w, *w2 = p.w2, *wn = p.wn, *proj = p.proj;
+    const size_t r = p.rows ? (size_t)p.rows[i] : (size_t)i;
+    float *hr = p.h + r * d, *out32 = p.out32;
+    const float* a = p.d1 ? p.d1 + r * d : nullptr;
+    const float* b = p.d2 ? p.d2 + r * d : nullptr;
+    const float* nr = p.dn ? p.dn + r * d : nullptr;
     float ss = 0.f;
-    if (VEC) {
-        // d is a multiple of 4 and at most 4*NT*MAX_V
-        f32x4 v[NORM_MAX_V];
-        const int nv = d >> 2;
-        float sn = 0.f;
-        if (nr) {
-            float sq = 0.f;
-#pragma unroll
-            for (int u = 0; u < NORM_MAX_V; ++u) {
-                const int c = threadIdx.x + u * NORM_NT;
-                if (c < nv) {
-                    const f32x4 x = ((const f32x4*)nr)[c];
-                    v[u] = x;
-                    sq += x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
-                }
-            }
-            sn = mult / sqrtf(block_sum<NORM_NT>(sq, red) / (float)d + eps_n);
-        }
-#pragma unroll
-        for (int u = 0; u < NORM_MAX_V; ++u) {
-            const int c = threadIdx.x + u * NORM_NT;
-            if (c < nv) {
-                f32x4 x = ((const f32x4*)hr)[c];
-                if (a) x += ((const f32x4*)a)[c];
-                if (b) x += ((const f32x4*)b)[c];
-                if (nr) {
-                    const f32x4 ww = ((const f32x4*)wn)[c];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) x[e] += v[u][e] * sn * ww[e];
-                }
-                if (write_h) ((f32x4*)hr)[c] = x;
-                v[u] = x;
-                ss += x[0] * x[0] + x[1] * x[1] + x[2] * x[2] + x[3] * x[3];
-            }
-        }
-        if (!out && !out32 && !proj && !out2) return;      // the additions were all that was asked for
-        const float ms = block_sum<NORM_NT>(ss, red) / (float)d;
-        const float scale = 1.0f / sqrtf(ms + eps);
-#pragma unroll
-        for (int u = 0; u < NORM_MAX_V; ++u) {
-            const int c = threadIdx.x + u * NORM_NT;
-            if (c < nv) {
-                f32x4 y = v[u];
-                if (!plain_out) {
-                    const f32x4 ww = ((const f32x4*)w)[c];
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y[e] = v[u][e] * scale * ww[e];
-                }
-                if (out32) ((f32x4*)(out32 + (size_t)i * d))[c] = y;
-                if (proj) ((f32x4*)ys)[c] = y;
-                auto put = [&](TO* dst, const f32x4& yy) {
-                    if constexpr (sizeof(TO) == 2) {             // four bf16 in one 8-byte store (d % 4 == 0 here)
-                        bf16x4 o4;
-#pragma unroll
-                        for (int e = 0; e < 4; ++e) o4[e] = (bf16)yy[e];
-                        *(bf16x4*)((bf16*)dst + (size_t)i * d + 4 * c) = o4;
-                    } else {
-                        ((f32x4*)((float*)dst + (size_t)i * d))[c] = yy;
-                    }
-                };
-                if (out) put(out, y);
-                if (out2) {                                      // the same row under a second norm's weights
-                    const f32x4 ww = ((const f32x4*)w2)[c];
-                    f32x4 y2;
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) y2[e] = v[u][e] * scale * ww[e];
-                    put(out2, y2);
-                }
-            }
-        }
-    } else {
-        float sn = 0.f;
-        if (nr) {
-            float sq = 0.f;
-            for (int c = threadIdx.x; c < d; c += NORM_NT) sq += nr[c] * nr[c];
-            sn = mult / sqrtf(block_sum<NORM_NT>(sq, red) / (float)d + eps_n);
-        }
-        for (int c = threadIdx.x; c < d; c += NORM_NT) {
-            float x = hr[c];
-            if (a) x += a[c];
-            if (b) x += b[c];
-            if (nr) x += nr[c] * sn * wn[c];
-            if (write_h) hr[c] = x;
-            ss += x * x;
-        }
-        if (!out && !out32 && !proj && !out2) return;
-        const float ms = block_sum<NORM_NT>(ss, red) / (float)d;
-        const float scale = 1.0f / sqrtf(ms + eps);
-        for (int c = threadIdx.x; c < d; c += NORM_NT) {
-            float x = hr[c];
-            if (!write_h) { if (a) x += a[c]; if (b) x += b[c]; if (nr) x += nr[c] * sn * wn[c]; }
-            const float y = plain_out ? x : x * scale * w[c];
-            if (out) out[(size_t)i * d + c] = from_f32<TO>(y);
-            if (out2) out2[(size_t)i * d + c] = from_f32<TO>(x * scale * w2[c]);
-            if (out32) out32[(size_t)i * d + c] = y;
-            if (proj) ys[c] = y;
+    float sn = 0.f;
+    if (nr) {
+        float sq = 0.f;
+        for (int c = threadIdx.x; c < d; c += NORM_NT) sq += nr[c] * nr[c];
+        sn = mult / sqrtf(block_sum<NORM_NT>(sq, red) / (float)d + eps_n);
+    }
+    for (int c = threadIdx.x; c < d; c += NORM_NT) {
+        float x = hr[c];
+        if (a) x += a[c];
+        if (b) x += b[c];
+        if (nr) x += nr[c] * sn * wn[c];
+        if (write_h) hr[c] = x;
+        ss += x * x;
+    }
+    if (!out && !out32 && !proj && !out2) return;
+    const float ms = block_sum<NORM_NT>(ss, red) / (float)d;
+    const float scale = 1.0f / sqrtf(ms + eps);
+    for (int c = threadIdx.x; c < d; c += NORM_NT) {
+        float x = hr[c];
+        if (!write_h) { if (a) x += a[c]; if (b) x += b[c]; if (nr) x += nr[c] * sn * wn[c]; }
+        const float y = plain_out ? x : x * scale * w[c];
+        if (out) out[(size_t)i * d + c] = from_f32<TO>(y);
+        if (out2) out2[(size_t)i * d + c] = from_f32<TO>(x * scale * w2[c]);
+        if (out32) out32[(size_t)i * d + c] = y;
+        if (proj) ys[c] = y;
+    }
+    if (!proj) return;
+    __syncthreads();
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const bool pvec = (d & 3) == 0 && (((uintptr_t)proj) & 15) == 0;
+    for (int e = wave; e < P; e += NORM_NT / 64) {
+        const float v = wave_dot_row(proj + (size_t)e * d, ys, d, pvec, lane);
+        if (lane == 0) {
+            p.proj_out[(size_t)i * P + e] = v;
+            if (PLAN) ys[((d + 3) & ~3) + e] = v;
         }
     }
-    if (proj) {
-        __syncthreads();
-        const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-        const bool pvec = (d & 3) == 0 && (((uintptr_t)proj) & 15) == 0;
-        for (int p = wave; p < P; p += NORM_NT / 64) {
-            const float v = wave_dot_row(proj + (size_t)p * d, ys, d, pvec, lane);
-            if (lane == 0) {
-                proj_out[(size_t)i * P + p] = v;
-                if (PLAN) ys[((d + 3) & ~3) + p] = v;
-            }
-        }
-        if (!PLAN) return;
-        __syncthreads();
-        float best;
-        const int me = top1_of(ys + ((d + 3) & ~3), P, &best);
-        if (threadIdx.x == 0) {
-            const float wt = 1.0f / (1.0f + expf(-best));
-            plan.expert[0] = me; plan.weight[0] = wt;
-            plan.src[0] = 0; plan.scale[0] = wt; plan.dst[0] = 0;
-        }
-        for (int g = threadIdx.x; g <= P; g += NORM_NT) plan.offsets[g] = me < g;
-        if ((int)threadIdx.x < plan.shared) {
-            const int j = 1 + threadIdx.x;
-            plan.src[j] = 0; plan.scale[j] = 1.0f; plan.dst[j] = j;
-            plan.offsets[P + j] = 1 + j;
-        }
-    }
+    if (!PLAN) return;
+    __syncthreads();
+    norm_make_plan(p.plan, ys + ((d + 3) & ~3), P);
 }
 
 extern "C" int spite_add_rmsnorm(float* h, const float* d1, const float* d2, const float* w, void* out,
@@ -246,21 +319,41 @@ extern "C" int spite_add_rmsnorm(float* h, const float* d1, const float* d2, con
     SP_REQUIRE(!proj || (proj_out && P > 0), "add_rmsnorm: a projection needs its output and size");
     SP_REQUIRE(!expert || (proj && n_rows <= 1 && P < 65535 && shared >= 0 && shared <= 64 && weight && src && scale && dst && offsets),
                "add_rmsnorm: a plan of %d rows, %d experts, %d shared groups", n_rows, P, shared);
-    const norm_plan plan{expert, weight, src, scale, dst, offsets, shared};
-    const size_t sh = proj ? (size_t)((expert ? ((d + 3) & ~3) + P : d)) * sizeof(float) : 0;
+    const norm_args p{h, d1, d2, w, out32, rows, n_rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2,
+                      norm_plan{expert, weight, src, scale, dst, offsets, shared}};
+    size_t sh = proj ? (size_t)((expert ? ((d + 3) & ~3) + P : d)) * sizeof(float) : 0;
     SP_REQUIRE(sh <= 48 * 1024, "add_rmsnorm: rows of %d do not fit the projection's LDS", d);
+    SP_REQUIRE(out_dtype == SP_F32 || out_dtype == SP_BF16, "add_rmsnorm: unknown dtype %d", out_dtype);
     if (n_rows == 0) return 0;
-    auto al = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
+    auto al = [](const void* q) { return ((uintptr_t)q & 15) == 0; };
     const bool vec = d % 4 == 0 && d <= 4 * NORM_NT * NORM_MAX_V && al(h) && al(d1) && al(d2) && al(w) && al(out32) && al(out) && al(dn) && al(wn)
         && al(w2) && al(out2);
-#define SP_NORM(TO, VEC, PLAN) add_rmsnorm_kernel<TO, VEC, PLAN><<<n_rows, NORM_NT, sh, st>>>(h, d1, d2, w, (TO*)out, out32, rows, d, eps, \
-        write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2, (TO*)out2, plan)
-#define SP_NORM_TO(TO) do { if (expert) { if (vec) SP_NORM(TO, true, true); else SP_NORM(TO, false, true); } \
-        else { if (vec) SP_NORM(TO, true, false); else SP_NORM(TO, false, false); } } while (0)
-    if (out_dtype == SP_F32) SP_NORM_TO(float);
-    else if (out_dtype == SP_BF16) SP_NORM_TO(bf16);
-    else return sp_fail("add_rmsnorm: unknown dtype %d", out_dtype);
-#undef SP_NORM_TO
+#define SP_NORM(KERNEL, GRID) do { if (out_dtype == SP_BF16) { typedef bf16 TO; KERNEL<<<GRID, NORM_NT, sh, st>>>(p, (TO*)out, (TO*)out2); } \
+                                   else { typedef float TO; KERNEL<<<GRID, NORM_NT, sh, st>>>(p, (TO*)out, (TO*)out2); } } while (0)
+#define SP_COMMA ,
+    if (!vec || (proj && !al(proj))) {
+        if (expert) SP_NORM(add_rmsnorm_kernel<TO SP_COMMA true>, n_rows);
+        else SP_NORM(add_rmsnorm_kernel<TO SP_COMMA false>, n_rows);
+        SP_LAUNCH_CHECK("add_rmsnorm");
+        return 0;
+    }
+    const int v = (d / 4 + NORM_NT - 1) / NORM_NT;
+    const bool many = proj && n_rows > (v == 1 ? 2 : 1) * sp_cu_count() && v <= 3;
+    if (many) sh = (size_t)NORM_R * d * sizeof(float);
+#define SP_NORM_V(V) do { \
+        if (!proj) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA false>, n_rows); \
+        else if (expert) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA true>, n_rows); \
+        else if (many) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA (V <= 3 ? V : 1) SP_COMMA NORM_R SP_COMMA false>, (n_rows + NORM_R - 1) / NORM_R); \
+        else SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA false>, n_rows); } while (0)
+    switch (v) {
+        case 1: SP_NORM_V(1); break;
+        case 2: SP_NORM_V(2); break;
+        case 3: SP_NORM_V(3); break;
+        case 4: SP_NORM_V(4); break;
+        default: SP_NORM_V(8);
+    }
+#undef SP_NORM_V
+#undef SP_COMMA
 #undef SP_NORM
     SP_LAUNCH_CHECK("add_rmsnorm");
     return 0;
