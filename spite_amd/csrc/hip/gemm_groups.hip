@@ -49,13 +49,13 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t gg_buffer(const void* p) {
 
 // One tile: rows row0 .. of the group g whose rows end at row_end, columns of the result from n0 on.
 template <int NW, int NB, int S, bool GLU, typename TY, bool NTW>
-__device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, int g, int row0, int row_end, int n0) {
+__device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, int g, int row0, int row_end, int n0, int u_first, int nu, TY* Y) {
     constexpr int XB = 16 * NB * 128;                            // bytes of a step of X
     constexpr int XI = (2 * NB + NW - 1) / NW;                   // load instructions a wave: a step of X (eight rows each)
     constexpr int TG = GLU ? 2 : 4;                              // bands that name distinct columns
     static_assert(S % 2 == 0, "whole steps a round");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int r = lane & 15, q = lane >> 4, N = p.N, nu = p.K / 64, kt = 2 * nu;
+    const int r = lane & 15, q = lane >> 4, N = p.N, kt = 2 * nu;
     const __amdgpu_buffer_rsrc_t xbuf = gg_buffer(p.X), wbuf = gg_buffer(p.W + (size_t)g * p.w_group_stride);
     int xoff[XI], xblk[XI];
 #pragma unroll
@@ -72,14 +72,14 @@ __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, in
         int band = n0 / 16 + wave * TG + a % TG;
         band = band < N / 16 ? band : N / 16 - 1;                // bands past N read the last one again
         if (GLU && a >= TG) band += N / 16;
-        wband[a] = band * kt * 1024;
+        wband[a] = (band * (p.K / 32) + 2 * u_first) * 1024;
     }
     const int wlane = lane * 16;
     const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
     auto load_x = [&](int u) {
-        const int k0 = (u < nu ? u : 0) * 128, past = u < nu ? 0 : GG_PAST;
+        const int k0 = (u_first + (u < nu ? u : 0)) * 128, past = u < nu ? 0 : GG_PAST;
 #pragma unroll
-        for (int i = 0; i < XI; ++i) gg_load_lds(xbuf, xoff[i] | past, k0, lds0 + (u & 3) * XB + xblk[i] * 1024);
+        for (int i = 0; i < XI; ++i) gg_load_lds(xbuf, xoff[i] | past, __builtin_amdgcn_readfirstlane(k0), lds0 + (u & 3) * XB + xblk[i] * 1024);
     };
     auto load_w = [&](bf16x8 (&ws)[4], int t) {
         const int at = (t < kt ? t : 0) * 1024, past = t < kt ? 0 : GG_PAST;
@@ -150,7 +150,7 @@ __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, in
         const int s = row0 + b * 16 + r;
         if (s >= row_end) continue;
         const float sc = p.a_scale ? p.a_scale[s] : 1.0f;
-        TY* yrow = (TY*)p.Y + (p.y_rows ? (size_t)p.y_rows[s] : (size_t)s) * p.ldy;
+        TY* yrow = Y + (p.y_rows ? (size_t)p.y_rows[s] : (size_t)s) * p.ldy;
 #pragma unroll
         for (int a = 0; a < TG; ++a) {
             const int n = n0 + (wave * TG + a) * 16 + q * 4;
@@ -215,7 +215,7 @@ void gemm_groups_kernel(gg_args p) {
     // (no such tile; or, with heights rounded up, the group's rows end before its last tile)
     if (g < 0 || row0 >= row_end) return;
     const int n0 = unit / p.m_tiles * (GLU ? 32 * NW : 64 * NW);
-#define GG_TILE(NB, S, NT) gg_tile<NW, NB, S, GLU, TY, NT>(p, lds, g, row0, row_end, n0)
+#define GG_TILE(NB, S, NT) gg_tile<NW, NB, S, GLU, TY, NT>(p, lds, g, row0, row_end, n0, 0, p.K / 64, (TY*)p.Y)
 #define GG_TILES(NT) switch (nb) { \
         case 2: GG_TILE(2, 6, NT); break; \
         case 4: GG_TILE(4, 6, NT); break; \
@@ -247,6 +247,111 @@ static int gg_launch(gg_args p, hipStream_t st) {
     gemm_groups_kernel<NW, GLU, TY><<<grid, NW * 64, (size_t)4 * p.cap * 128, st>>>(p);
     SP_LAUNCH_CHECK("gemm_groups");
     return 0;
+}
+
+// Plain products of some tens to some hundreds of rows, by the same tiles: four waves and 256 rows of W a workgroup, tiles of
+// 16 * NB rows, the sum over k cut into `runs` runs, each a workgroup of its own that writes its partial sums to Y + run * M * N
+// (one run: the result).  The chip takes one workgroup a compute unit at a time: what bounds these sizes is the stream of W
+// and, since a workgroup's waits are filled by no other, the number of its steps; so as many runs as make up to one
+// workgroup a unit, and no more (rounds of them cost twice: 330 x 7,168 x 5,120 in 3 runs of 7 x 16 rows 39 us, in 6 54).
+//
+// Measured on an MI355X against the best of gemm_tiled (its runs of 128 x 512), gemm_lds and, up to 64 rows, gemm_skinny, launches in
+// a row over weights that the caches do not hold, with the sum of the runs (us): 64 x 32,768 x 5,120 62 / 119, 64 x 5,120 x 8,192
+// 26 / 34, 80 x 7,168 x 5,120 26 / 34, 330 39 / 55, 500 x 5,120 x 5,120 39 / 55, 500 x 2,048 x 2,048 23 / 30, 1,531 x 576 x 5,120 27 / 37.
+template <int NB, int S, typename TY>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
+void gemm_runs_kernel(gg_args p, int runs) {
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    const int units = p.m_tiles * p.n_tiles * runs, per_xcd = (units + 7) / 8;
+    const int unit = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if ((int)(blockIdx.x / 8) >= per_xcd || unit >= units) return;
+    const int tile = unit / p.m_tiles, ks = tile % runs, all = p.K / 64;
+    // (quotients: in scalar registers again)
+    const int mt = __builtin_amdgcn_readfirstlane(unit % p.m_tiles), n0 = __builtin_amdgcn_readfirstlane(tile / runs) * 256;
+    const int each = __builtin_amdgcn_readfirstlane((all + runs - 1) / runs), first = __builtin_amdgcn_readfirstlane(ks) * each;
+    gg_tile<4, NB, S, false, TY, true>(p, lds, 0, mt * 16 * NB, p.M, n0, first, all - first < each ? all - first : each,
+                                       (TY*)p.Y + (size_t)ks * p.M * p.N);
+}
+
+template <int NB, int S, typename TY>
+static int gr_launch(gg_args p, int runs, hipStream_t st) {
+    constexpr int SH = 4 * NB * 16 * 128;
+    p.n_tiles = (p.N + 255) / 256;
+    p.m_tiles = (p.M + 16 * NB - 1) / (16 * NB);
+    static bool allowed = false;
+    if (!allowed) {
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_runs_kernel<NB, S, TY>, hipFuncAttributeMaxDynamicSharedMemorySize, SH);
+        SP_REQUIRE(e == hipSuccess, "gemm_runs: %d bytes of LDS refused: %s", SH, hipGetErrorString(e));
+        allowed = true;
+    }
+    SP_REQUIRE((long)p.m_tiles * p.n_tiles * runs < (1L << 30), "gemm_runs: too many tiles");
+    gemm_runs_kernel<NB, S, TY><<<(p.m_tiles * p.n_tiles * runs + 7) / 8 * 8, 256, SH, st>>>(p, runs);
+    SP_LAUNCH_CHECK("gemm_runs");
+    return 0;
+}
+template <typename TY>
+static int gr_launch_nb(const gg_args& p, int runs, int nb, hipStream_t st) {
+    switch (nb) {
+        case 2: return gr_launch<2, 6, TY>(p, runs, st);
+        case 4: return gr_launch<4, 6, TY>(p, runs, st);
+        case 5: return gr_launch<5, 6, TY>(p, runs, st);
+        case 6: return gr_launch<6, 6, TY>(p, runs, st);
+        case 7: return gr_launch<7, 4, TY>(p, runs, st);
+        case 8: return gr_launch<8, 4, TY>(p, runs, st);
+        case 9: return gr_launch<9, 4, TY>(p, runs, st);
+        case 10: return gr_launch<10, 4, TY>(p, runs, st);
+        default: return sp_fail("gemm_runs: tiles of %d rows", 16 * nb);
+    }
+}
+
+int sp_add_runs(const float* part, int runs, void* Y, int y_dtype, int ldy, int M, int N, hipStream_t st);       // gemm_tiled.hip
+
+// Y[M,N] = X[M,K] . W[N,K]^T, W in operand order.  `nb`: a tile's rows in units of 16 (2, 4 .. 10); `part`: [runs][M][N] floats where there
+// is more than one run (aligned to 16 bytes, as rows of Y are where there is one).
+extern "C" int spite_gemm_runs(const void* X, int ldx, const void* W, void* Y, int y_dtype, int ldy, int M, int N, int K, int runs, int nb,
+                               float* part, hipStream_t st) {
+    SP_REQUIRE(M > 0 && N > 0 && K > 0 && ldx >= K && ldy >= N, "gemm_runs: bad sizes M=%d N=%d K=%d", M, N, K);
+    SP_REQUIRE(K % 64 == 0 && N % 16 == 0, "gemm_runs: operand order needs K=%d a multiple of 64 and N=%d of 16", K, N);
+    SP_REQUIRE(ldx % 8 == 0 && ((uintptr_t)X & 15) == 0 && ((uintptr_t)W & 15) == 0, "gemm_runs: operands must be 16-byte aligned");
+    SP_REQUIRE(y_dtype == SP_BF16 || y_dtype == SP_F32, "gemm_runs: output dtype %d", y_dtype);
+    const int all = K / 64;
+    SP_REQUIRE(runs >= 1 && runs <= 64 && (all + runs - 1) / runs * (runs - 1) < all, "gemm_runs: %d runs over %d steps leave a run empty", runs, all);
+    SP_REQUIRE(runs == 1 ? ldy % 4 == 0 && ((uintptr_t)Y & 15) == 0 : part && ((uintptr_t)part & 15) == 0, "gemm_runs: rows of the result must be 16-byte aligned");
+    // the loads' offsets are 32-bit
+    SP_REQUIRE((size_t)M * ldx * 2 < ((size_t)1 << 31) && (size_t)N * K * 2 < ((size_t)1 << 31), "gemm_runs: operands of 2 GiB and more (M=%d N=%d K=%d)", M, N, K);
+    gg_args p{(const bf16*)X, ldx, (const bf16*)W, 0, Y, ldy, M, N, K, nullptr, 1, nullptr, nullptr, nullptr, 0, 0, 0};
+    if (runs == 1) return y_dtype == SP_BF16 ? gr_launch_nb<bf16>(p, 1, nb, st) : gr_launch_nb<float>(p, 1, nb, st);
+    p.Y = part;
+    p.ldy = N;
+    const int rc = gr_launch_nb<float>(p, runs, nb, st);
+    return rc ? rc : sp_add_runs(part, runs, Y, y_dtype, ldy, M, N, st);
+}
+
+// The runs and tile (runs * 16 + nb) that suit a plain product, and what it takes then, in us; 0 if the tiles alone are more than one a
+// compute unit.  A step of 64 k takes 0.457 + 0.038 nb us, or what the stream of W needs for 32 KB a workgroup (8.3 TB/s: row
+// tiles share it); more than one run a launch, and the passes over the partial sums at 6.8 TB/s.  Fitted to 296 sizes (20 to 3,000
+// rows, N and K of 128 to 20,000), each with several choices; the choice is within 1 % of the best of them on average.
+extern "C" int spite_gemm_runs_choice(int M, int N, int K, double* us) {
+    const long cus = sp_cu_count(), cols = (N + 255) / 256;
+    const int steps = K / 64;
+    int best = 0;
+    *us = 0.0;
+    for (int rt = (M + 159) / 160; rt <= (M + 63) / 64 && rt * cols <= cus; ++rt) {
+        int nb = ((M + rt - 1) / rt + 15) / 16;
+        nb = nb <= 2 ? 2 : nb <= 4 ? 4 : nb;
+        if ((M + 16 * nb - 1) / (16 * nb) != rt) continue;
+        long most = cus / (rt * cols) < 16 ? cus / (rt * cols) : 16;
+        if (most > steps / 2) most = steps / 2;
+        while (most > 1 && (steps + most - 1) / most * (most - 1) >= steps) --most;      // no run may be empty
+        for (long runs : {most, 1L}) {
+            if (runs < 1) continue;
+            const double step = fmax(0.457 + 0.038 * nb, 0.0328 * (double)(cols * runs) / 8.27);
+            const double t = 9.2 + (double)((steps + runs - 1) / runs) * step
+                           + (runs > 1 ? 1.7 + (2.0 * runs + 1.0) * M * N * 4e-6 / 6.76 : 0.0);
+            if (best == 0 || t < *us) { best = (int)runs * 16 + nb; *us = t; }
+        }
+    }
+    return best;
 }
 
 // Arguments as spite_gemm_lds's (`x_rows`: how many rows X has); `waves` 4 or 8, `cap` 128 or 160.  Gated with silu

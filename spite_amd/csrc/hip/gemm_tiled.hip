@@ -383,6 +383,30 @@ void add_runs_kernel(const float* __restrict__ part, int runs, size_t stride, TY
     }
 }
 
+// Adds up the `runs` partial sums [run][M][N] of a product whose sum over k was cut (N % 4 == 0).
+int sp_add_runs(const float* part, int runs, void* Y, int y_dtype, int ldy, int M, int N, hipStream_t st) {
+    const size_t stride = (size_t)M * N;
+    const size_t blocks = (stride / 4 + 255) / 256;
+    const int grid = (int)(blocks < 8192 ? blocks : 8192);
+    const int vec = ldy % 4 == 0 && ((uintptr_t)Y & 15) == 0;
+#define SP_ADD(R) do { \
+        if (y_dtype == SP_BF16) add_runs_kernel<bf16, R><<<grid, 256, 0, st>>>(part, runs, stride, (bf16*)Y, ldy, M, N, vec); \
+        else add_runs_kernel<float, R><<<grid, 256, 0, st>>>(part, runs, stride, (float*)Y, ldy, M, N, vec); \
+        } while (0)
+    switch (runs) {
+        case 2: SP_ADD(2); break;
+        case 3: SP_ADD(3); break;
+        case 4: SP_ADD(4); break;
+        case 5: SP_ADD(5); break;
+        case 6: SP_ADD(6); break;
+        case 7: SP_ADD(7); break;
+        default: SP_ADD(8);
+    }
+#undef SP_ADD
+    SP_LAUNCH_CHECK("add_runs");
+    return 0;
+}
+
 // A plain product (no groups, no row lists, no GLU) over few tiles, the sum over k cut into
 // `k_splits` runs so that the chip is filled: `workspace` holds k_splits * M * N floats.
 extern "C" int spite_gemm_tiled_split(const void* X, int ldx, const void* W, void* Y, int y_dtype, int ldy, int M, int N,
@@ -400,25 +424,7 @@ extern "C" int spite_gemm_tiled_split(const void* X, int ldx, const void* W, voi
     int rc = launch_tiled_kernel<8, 1, 8, false, float, true>(X, ldx, W, 0, workspace, N, M, N, K, nullptr, 1, nullptr, nullptr, nullptr,
                                                         k_splits, stride, st);
     if (rc) return rc;
-    const size_t blocks = (stride / 4 + 255) / 256;
-    const int grid = (int)(blocks < 8192 ? blocks : 8192);
-    const int vec = ldy % 4 == 0 && ((uintptr_t)Y & 15) == 0;
-#define SP_ADD(R) do { \
-        if (y_dtype == SP_BF16) add_runs_kernel<bf16, R><<<grid, 256, 0, st>>>((const float*)workspace, k_splits, stride, (bf16*)Y, ldy, M, N, vec); \
-        else add_runs_kernel<float, R><<<grid, 256, 0, st>>>((const float*)workspace, k_splits, stride, (float*)Y, ldy, M, N, vec); \
-        } while (0)
-    switch (k_splits) {
-        case 2: SP_ADD(2); break;
-        case 3: SP_ADD(3); break;
-        case 4: SP_ADD(4); break;
-        case 5: SP_ADD(5); break;
-        case 6: SP_ADD(6); break;
-        case 7: SP_ADD(7); break;
-        default: SP_ADD(8);
-    }
-#undef SP_ADD
-    SP_LAUNCH_CHECK("add_runs");
-    return 0;
+    return sp_add_runs((const float*)workspace, k_splits, Y, y_dtype, ldy, M, N, st);
 }
 
 // W in operand order (see above), every group N (2N with GLU) rows of K.

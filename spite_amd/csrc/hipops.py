@@ -69,6 +69,8 @@ def lib():
             "spite_gemm_mfma": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_lds": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, I, P],
             "spite_gemm_groups": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, I, I, I, P],
+            "spite_gemm_runs": [P, I, P, P, I, I, I, I, I, I, I, P, P],
+            "spite_gemm_runs_choice": [I, I, I, P],
             "spite_gemm_tiled": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_tiled_split": [P, I, P, P, I, I, I, I, I, I, P, P],
             "spite_attn_prefill": [P, P, P, P, P, P, P, P, I, P, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
@@ -703,18 +705,50 @@ def lds_suits(M: int, N: int, K: int, glu: bool, runs: int) -> bool:
     95 that the line takes in is more than 2 % slower, on average they are 27 % faster: 1,547 x 5,120 x 5,120 79 against 97 us,
     1,531 x 2,048 x 2,048 31 against 36, 300 x 16,384 x 5,120 gated 99 against 131; 700 x 5,120 x 8,192 stays, 78 against 106, and
     7,902 x 18,304 x 448 gated, 367 against 401.)"""
-    cus, lds = cu_count(), lds_us(M, N, K, glu)
-    cols, scale = -(-N // (256 if glu else 512)), 1.2 * K / 5120.0
+    if runs > 1 and -(-M // 128) * -(-N // 256) < cu_count() // 4:      # too few tiles without the cut (and below what was timed)
+        return False
+    return lds_us(M, N, K, glu) <= tiled_us(M, N, K, glu, runs)
+
+
+def tiled_us(M: int, N: int, K: int, glu: bool, runs: int) -> float:
+    """What ``gemm_tiled`` takes for a product without groups, its sum over k in ``runs`` runs (see above)."""
+    cus, cols, scale = cu_count(), -(-N // (256 if glu else 512)), 1.2 * K / 5120.0
     if runs > 1:
-        if -(-M // 128) * -(-N // 256) < cus // 4:          # too few tiles without the cut (and below what was timed)
-            return False
-        tiled = scale * 106.0 / runs + 12.0 + (runs + 1) * M * N * 4 / 4.5e6
-    else:
-        def rounds(rows, tile_us):
-            n = -(-(-(-M // rows) * cols) // cus)
-            return scale * tile_us * n + 6.0 * (n - 1)
-        tiled = min(rounds(128, 106.0), rounds(96, 89.0) if not glu else math.inf)
-    return lds <= tiled
+        return scale * 106.0 / runs + 12.0 + (runs + 1) * M * N * 4 / 4.5e6
+
+    def rounds(rows, tile_us):
+        n = -(-(-(-M // rows) * cols) // cus)
+        return scale * tile_us * n + 6.0 * (n - 1)
+    return min(rounds(128, 106.0), rounds(96, 89.0) if not glu else math.inf)
+
+
+@functools.lru_cache(maxsize=4096)
+def gemm_runs_choice(M: int, N: int, K: int):
+    """(runs, nb) for ``gemm_runs``, or None where another product is the faster one.  Up to 32 rows the stream of W of
+    ``gemm_skinny`` is; up to 64 it is for matrices of fewer than 26 M elements (64 rows: 3,072 x 2,048 12.7 against 17.6 us, 5,120 x
+    5,120 24.4 against 23.3, 32,768 x 5,120 119 against 62).  Beyond, by what each is estimated to take: up to 800 rows the estimate
+    of the others is the lower side of what was timed (149 sizes, 25 % faster on average, 2 of them up to 3 % slower); above, where
+    two rounds of small tiles stand against one of large ones, it has to be a tenth to gain."""
+    if M <= 32 or (M <= 64 and N * K < 26_000_000):
+        return None
+    us = ctypes.c_double()
+    code = lib().spite_gemm_runs_choice(M, N, K, ctypes.addressof(us))
+    if not code or (M > 64 and us.value >= (1.1 if M <= 800 else 0.9)
+                    * min(lds_us(M, N, K, False), tiled_us(M, N, K, False, tiled_k_runs(M, N, K)))):
+        return None
+    return divmod(code, 16)
+
+
+def gemm_runs(a, w, y, M, N, K, *, runs, nb, part=None):
+    """Plain bf16 product of some tens to hundreds of rows, its sum over k in ``runs`` runs (``part``: fp32 [runs, M, N] where there is
+    more than one) and tiles of 16 * ``nb`` rows (see gemm_groups.hip and ``gemm_runs_choice``)."""
+    _gemm_checks(a, w, y, M, N, K, None, 1, None, None, None, False, "gemm_runs")
+    if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
+        raise KernelError(f"gemm_runs: bfloat16 operands only, got {a.dtype} and {w.dtype}")
+    if runs > 1 and (part is None or part.numel() < runs * M * N):
+        raise KernelError(f"gemm_runs: partial sums {None if part is None else tuple(part.shape)} for {runs} runs of M={M} N={N}")
+    _check(lib().spite_gemm_runs(_ptr_rows(a, "a"), a.stride(0), _ptr(w, "w"), _ptr_rows(y, "y"), dtype_code(y.dtype), y.stride(0), M, N, K,
+                                 int(runs), int(nb), _ptr(part, "part", torch.float32, True), _stream()), "gemm_runs")
 
 
 def lds_suits_groups(group_rows: float, K: int, tiles: int = 0, lds_tiles: int = 0) -> bool:

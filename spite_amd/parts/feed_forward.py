@@ -211,9 +211,9 @@ class MoeTop1Sigmoid(FeedForward):
             # at 64 tokens over 16 experts: 658 against 683 us for the two products of a layer)
             linear(x, self.w_gate_up, act, glu=True, offsets=offsets, n_groups=E, a_rows=src, a_scale=scale, rows=T,
                    max_rows=16, ws=ws)
-            linear(x, self.w_gate_up.group(E), act[T:], glu=True, a_rows=src[T:], a_scale=scale[T:], rows=T, ws=ws)
+            linear(x, self.w_gate_up.group(E), act[T:], glu=True, ws=ws)
             linear(act, self.w_down, y, offsets=offsets, n_groups=E, y_rows=dst, rows=T, max_rows=16, ws=ws)
-            linear(act[T:], self.w_down.group(E), y, y_rows=dst[T:], rows=T, ws=ws)
+            linear(act[T:], self.w_down.group(E), y[T:], ws=ws)
             return (y[:T], y[T:])
         # the tile of either product, by the rounds that its tiles make on the chip (gate and up
         # rows share a tile of 512 W rows: 256 columns of the result; the down product's tile has 512)

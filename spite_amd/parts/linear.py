@@ -177,6 +177,14 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
     most = max_rows if max_rows is not None else M
     if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and K % 8 == 0 and x.stride(0) % 8 == 0 \
             and x.data_ptr() % 16 == 0:
+        if tiled and M > 32 and tile_shape == 0 and offsets is None and a_rows is None and a_scale is None and y_rows is None and act is None \
+                and not glu and hipops.gemm_groups_ok(x, y, M, N, K, glu):
+            choice = hipops.gemm_runs_choice(M, N, K)
+            if choice is not None:
+                runs, nb = choice
+                part = _scratch(ws, (runs, M, N), torch.float32, x.device) if runs > 1 else None
+                hipops.gemm_runs(x, w, y, M, N, K, runs=runs, nb=nb, part=part)
+                return
         # few rows: the time is the weights' stream (a very tall matrix, the output table, is
         # streamed faster by the tiled kernel from 33 rows on)
         if most <= SKINNY_MAX_ROWS and not (tiled and most > 32 and offsets is None and N >= 65536):
