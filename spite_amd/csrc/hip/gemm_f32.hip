@@ -38,13 +38,16 @@ __device__ __forceinline__ void f32_store(float* __restrict__ Y, size_t row, int
         for (int r = 0; r < 4; ++r) if (n + r < N) y[r] = v[r];
 }
 
-template <int MT, int GLU>
+// HALVES (GLU, N a multiple of 8): a workgroup takes eight rows of each half, in one MFMA operand: twice as many workgroups, where
+// those of sixteen would be up to three a compute unit and some units have one more than others (2 x 3,072 x 2,048, two groups of a
+// row 27.3 -> 23.9 us, three 36.1 -> 31.5; five, 3.75 a unit, 46.2 with either).
+template <int MT, int GLU, bool HALVES = false>
 __global__ __launch_bounds__(512)
 void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, long w_group_stride,
                           float* __restrict__ Y, int ldy, int M, int N, int K, const int* __restrict__ offsets, int n_groups,
                           const int* __restrict__ a_rows, const float* __restrict__ a_scale, const int* __restrict__ y_rows,
                           int act, float act_limit, int vec_y) {
-    constexpr int NB = GLU ? 2 : 1;
+    constexpr int NB = GLU && !HALVES ? 2 : 1;
     __shared__ f32x4 red[8][MT * NB][64];
     int g = 0, row0 = 0, row_end = M;
     if (offsets) {
@@ -54,12 +57,12 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
     }
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4;
-    const int n0 = blockIdx.x * 16;
+    const int n0 = blockIdx.x * (HALVES ? 8 : 16);
     const float* Wg = W + (size_t)g * w_group_stride;
     const int wn = n0 + r < N ? n0 + r : N - 1;
     const float* wp[NB];
-    wp[0] = Wg + (size_t)wn * K;
-    if (GLU) wp[NB - 1] = Wg + (size_t)(N + wn) * K;
+    wp[0] = Wg + (size_t)(HALVES ? n0 + (r & 7) + (r < 8 ? 0 : N) : wn) * K;
+    if (NB == 2) wp[NB - 1] = Wg + (size_t)(N + wn) * K;
     const float* xp[MT];
     float sc[MT];
     bool live[MT];
@@ -113,8 +116,14 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
 #pragma unroll
         for (int i = 0; i < 8; ++i) t[b] += red[i][m * NB + b][lane];
     }
-    if (s >= row_end) return;
-    if (GLU)
+    if (HALVES)                                        // rows 8 to 15, the up half's: 32 lanes further on
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const float up = __shfl_down(t[0][e], 32, 64);
+            t[0][e] = sp_gated(t[0][e], up, act, act_limit, false);
+        }
+    if (s >= row_end || (HALVES && q >= 2)) return;
+    if (GLU && !HALVES)
 #pragma unroll
         for (int e = 0; e < 4; ++e) t[0][e] = sp_gated(t[0][e], t[NB - 1][e], act, act_limit, false);
     f32_store(Y, y_rows ? (size_t)y_rows[s] : (size_t)s, ldy, n0 + q * 4, N, t[0], vec_y);
@@ -302,7 +311,9 @@ int sp_gemm_f32(const float* A, int lda, const float* W, long w_group_stride, fl
     dim3 grid((N + 15) / 16, m_tiles);
 #define SP_F32_ROWS(MT) do { if (glu) gemm_f32_rows_kernel<MT, 1><<<grid, 512, 0, st>>>(SP_F32_ARGS); \
                              else gemm_f32_rows_kernel<MT, 0><<<grid, 512, 0, st>>>(SP_F32_ARGS); } while (0)
-    if (tile == 16) SP_F32_ROWS(1);
+    if (tile == 16 && glu && N % 8 == 0 && (long)((N + 15) / 16) * (offsets ? (n_groups < M ? n_groups : M) : 1) <= 3L * sp_cu_count())
+        gemm_f32_rows_kernel<1, 1, true><<<dim3(N / 8, m_tiles), 512, 0, st>>>(SP_F32_ARGS);
+    else if (tile == 16) SP_F32_ROWS(1);
     else if (tile == 32) SP_F32_ROWS(2);
     else SP_F32_ROWS(4);
 #undef SP_F32_ROWS

@@ -32,3 +32,16 @@ def test_a_row_of_a_tall_matrix_has_the_same_bits_in_every_variant(rows):
     narrow = torch.empty(rows, 48, device=DEV)
     ops().gemm_generic(a[:rows].contiguous(), w[:48].contiguous(), narrow, rows, 48, K)
     assert torch.equal(part, whole[:rows]) and torch.equal(narrow, whole[:rows, :48])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 8, 36), (5, 24, 516), (16, 2056, 260), (3, 20, 64)])
+@pytest.mark.parametrize("groups", [0, 4])
+def test_gated_rows_with_both_halves_in_one_operand(M, N, K, groups):
+    """Eight columns a workgroup (N a multiple of 8) and sixteen, the last ones part of their tile."""
+    run_gemm(ops().gemm_generic, torch.float32, torch.float32, M, N, K, True, groups > 0, max(groups, 1))
+    a, w = rnd(M, K), rnd(2 * N, K, seed=1)
+    y, many = torch.empty(M, N, device=DEV), torch.empty(M + 100, N, device=DEV)
+    ops().gemm_generic(a, w, y, M, N, K, glu=True)
+    ops().gemm_generic(torch.cat([a, rnd(100, K, seed=3)]), w, many, M + 100, N, K, glu=True)
+    assert torch.equal(y, many[:M])
