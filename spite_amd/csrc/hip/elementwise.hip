@@ -130,7 +130,7 @@ void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ 
 #pragma unroll
     for (int u = 0; u < V; ++u) at[u] = tid + u * NORM_NT < nv ? tid + u * NORM_NT : nv - 1;
     f32x4 ww[V], ww2[V];
-    const bool outputs = out || p.out32 || p.proj || out2, normed = outputs && !p.plain_out;
+    const bool outputs = out || p.out32 || p.proj || out2, normed = outputs && (!p.plain_out || out2);   // (out2 is normed beside a plain row too)
     const int first = blockIdx.x * R, rows = R == 1 ? 1 : (p.n_rows - first < R ? p.n_rows - first : R);
     for (int rr = 0; rr < rows; ++rr) {
         const int i = first + rr;
@@ -152,8 +152,9 @@ void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ 
 #pragma unroll
             for (int u = 0; u < V; ++u) wn[u] = ((const f32x4*)p.wn)[at[u]];
         if (rr == 0 && normed) {
+            if (!p.plain_out)
 #pragma unroll
-            for (int u = 0; u < V; ++u) ww[u] = ((const f32x4*)p.w)[at[u]];
+                for (int u = 0; u < V; ++u) ww[u] = ((const f32x4*)p.w)[at[u]];
             if (out2)
 #pragma unroll
                 for (int u = 0; u < V; ++u) ww2[u] = ((const f32x4*)p.w2)[at[u]];
@@ -182,7 +183,7 @@ void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ 
             }
         }
         if (!outputs) continue;                            // the additions were all that was asked for
-        const float scale = p.plain_out ? 1.f : 1.0f / sqrtf(block_sum<NORM_NT>(ss, red) / (float)d + p.eps);
+        const float scale = !normed ? 1.f : 1.0f / sqrtf(block_sum<NORM_NT>(ss, red) / (float)d + p.eps);
 #pragma unroll
         for (int u = 0; u < V; ++u) {
             const int c = tid + u * NORM_NT;

@@ -50,3 +50,14 @@ def test_rows_by_a_list_and_without_outputs(d, rows):
     assert ((out.double() - want).abs() <= 2e-6 * want.abs().max()).all()
     ops().add_rmsnorm(hh, None, 1e-5, d1=d1)
     assert torch.equal(hh, h + d1)
+
+
+@pytest.mark.parametrize("d", [2048, 5120, 5121])
+def test_a_second_norm_beside_a_plain_row(d):
+    h, d1, w2 = rnd(3, d), rnd(3, d, seed=1), rnd(d, seed=2)
+    plain, out2 = torch.empty(3, d, device=DEV), torch.empty(3, d, device=DEV)
+    ops().add_rmsnorm(h, None, 1e-5, out=plain, d1=d1, plain_out=True, w2=w2, out2=out2, write_h=False)
+    assert torch.equal(plain, h + d1)
+    v = (h + d1).double()
+    want = v / (v.pow(2).mean(1, keepdim=True) + 1e-5).sqrt() * w2.double()
+    assert ((out2.double() - want).abs() <= 2e-6 * want.abs().max()).all()      # fp32 sums of d terms in a tree
