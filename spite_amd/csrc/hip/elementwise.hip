@@ -471,51 +471,126 @@ void rope_kvwrite_kernel(const T* __restrict__ qkv, T* __restrict__ q_out,
     }
 }
 
+// Values of 32 tokens and one kv head into their pages, which hold a column's keys side by side: written by a token at a time
+// they are stores of two bytes, 16 lanes of as many lines each.  Here the rows go through LDS, and wherever eight tokens fill
+// eight places in a row, the first a multiple of eight, a column's are one 16-byte store; the others go one by one.  A token
+// belongs to such a piece or not by the slots alone: pieces that begin in another block's tokens are that block's.
+// Measured on an MI355X, the whole rotation and cache write, 40 heads and 8 kv heads of 128, tokens of one prompt, against a token at a
+// time (us): 2,048 15.6 / 24.9 (59 MB: 3.8 TB/s), 700 7.9 / 12.9, 330 6.1 / 9.3; 330 tokens of as many requests 7.2 / 8.9.
+#define ROPE_VT 32
+#define ROPE_VROWS (ROPE_VT + 7)
+__device__ __forceinline__ void rope_value_block(const bf16* __restrict__ qkv, bf16* __restrict__ v_pages, const int* __restrict__ slot_map,
+                                                 int T, int H, int G, int hd, int ps, int kv_tiled, int t0, int g, bf16* rows) {
+    __shared__ int piece[ROPE_VT], single[ROPE_VT], count[2];        // tokens of the block: a piece's first; on their own
+    __shared__ int page_of[ROPE_VT], off_of[ROPE_VT];
+    const int tid = threadIdx.x, ld = hd + 2, per_row = hd >> 2;
+    const size_t row_w = (size_t)(H + 2 * G) * hd;
+    const bf16* src = qkv + (size_t)(H + G + g) * hd;
+    if (tid < 64) {
+        const int t = t0 + tid;
+        const int slot = tid < ROPE_VT && t < T ? slot_map[t] : -1;
+        const int i = t - (slot & 7);                                // where its piece would begin
+        bool whole = slot >= 0 && i >= 0 && i + 7 < T;
+        if (whole)
+#pragma unroll
+            for (int m = 0; m < 8; ++m) whole = whole && slot_map[i + m] == (slot & ~7) + m;
+        const unsigned long long heads = __ballot(whole && i == t), alone = __ballot(slot >= 0 && !whole);
+        const unsigned long long below = (1ull << tid) - 1;
+        if (whole && i == t) piece[__popcll(heads & below)] = tid;
+        if (slot >= 0 && !whole) single[__popcll(alone & below)] = tid;
+        if (tid == 0) { count[0] = __popcll(heads); count[1] = __popcll(alone); }
+        if (slot >= 0) { page_of[tid] = slot / ps; off_of[tid] = slot % ps; }
+    }
+    for (int x = tid; x < ROPE_VROWS * per_row; x += 256) {
+        const int j = x / per_row, c = (x - j * per_row) * 4;
+        if (t0 + j >= T) break;
+        const uint2 v = *(const uint2*)(src + (size_t)(t0 + j) * row_w + c);
+        unsigned* at = (unsigned*)(rows + j * ld + c);               // (rows of hd + 2: columns' reads spread over the banks)
+        at[0] = v.x;
+        at[1] = v.y;
+    }
+    __syncthreads();
+    const int np = count[0], n1 = count[1], bits = __ffs(hd) - 1;    // (hd: a power of two)
+    auto place = [&](int j, int c) { return ((size_t)page_of[j] * G + g) * (size_t)hd * ps + sp_v_index(c, off_of[j], hd, ps, kv_tiled); };
+    for (int x = tid; x < np * hd; x += 256) {                       // neighbouring lanes: a column's pieces
+        const int c = x / np, j = piece[x - c * np];
+        bf16x8 v;
+#pragma unroll
+        for (int m = 0; m < 8; ++m) v[m] = rows[(j + m) * ld + c];
+        *(bf16x8*)(v_pages + place(j, c)) = v;
+    }
+#pragma unroll 4
+    for (int x = tid; x < n1 * hd; x += 256) {
+        const int j = single[x >> bits], c = x & (hd - 1);
+        v_pages[place(j, c)] = rows[j * ld + c];
+    }
+}
+
 // The same for bfloat16 rows whose head size gives every head a power-of-two group of lanes with
 // four pairs each (hd = 32, 64, 128, 256, 512): a lane reads and writes eight bytes at a time
 // instead of two, and a wave handles 64 / (hd/8) heads at once.  Every value is computed by the
 // same operations in the same order as in the kernel above; only the sum of squares of the
-// qk-norm meets in a different order.
+// qk-norm meets in a different order.  A token's sines and cosines are formed once a workgroup and shared through LDS, and the
+// next heads' loads are asked for before this one's are worked on.
+// `v_blocks` > 0: the first workgroups (of y = 0) write the values, 32 tokens of a kv head each, and n_heads counts queries and
+// keys; tokens go to the eight XCDs in eighths, so that keys that share a line of the pages meet in one L2.
 __global__ __launch_bounds__(256)
 void rope_kvwrite_vec_kernel(const bf16* __restrict__ qkv, bf16* __restrict__ q_out,
                              bf16* __restrict__ k_pages, bf16* __restrict__ v_pages,
                              const int* __restrict__ positions, const int* __restrict__ slot_map,
-                             const float* __restrict__ inv_freq, int H, int G, int hd, int ps,
+                             const float* __restrict__ inv_freq, int T, int H, int G, int hd, int ps,
                              int use_rope, int adjacent, int use_norm, float norm_eps,
-                             int use_temp, int floor_scale, float attn_scale, int n_heads, int hpw, int kv_tiled) {
-    const int t = blockIdx.x;
+                             int use_temp, int floor_scale, float attn_scale, int n_heads, int hpw, int kv_tiled, int v_blocks) {
+    extern __shared__ __attribute__((aligned(16))) unsigned char lds[];
+    int t = blockIdx.x;
+    if (v_blocks) {
+        if (t < v_blocks) {
+            if (blockIdx.y == 0) rope_value_block(qkv, v_pages, slot_map, T, H, G, hd, ps, kv_tiled, t / G * ROPE_VT, t % G, (bf16*)lds);
+            return;
+        }
+        t = (t - v_blocks) % 8 * ((T + 7) / 8) + (t - v_blocks) / 8;
+        if (t >= T) return;
+    }
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int half = hd >> 1;
     const int lph = half >> 2;                   // lanes a head: four pairs each
     const int sub = lane / lph, l = lane % lph;  // which head of the wave's group, which four pairs
     const int hpi = 64 / lph;                    // heads a wave takes at once
     const int row_w = (H + 2 * G) * hd;
+    // the four pairs' elements: half-split (4l+u, half+4l+u) or adjacent (8l+2u, 8l+2u+1)
+    const int c0 = adjacent ? 8 * l : 4 * l, c1 = adjacent ? 8 * l + 4 : half + 4 * l;
+    auto head = [&](int it) { return (blockIdx.y * 4 * hpw + it * 4 + wave) * hpi + sub; };
+    auto source = [&](int it) { const int hh = head(it); return qkv + (size_t)t * row_w + (size_t)(hh < n_heads ? hh : 0) * hd; };
+    bf16x4 lo_next = *(const bf16x4*)(source(0) + c0), hi_next = *(const bf16x4*)(source(0) + c1);
     const int pos = positions[t];
     const int slot = slot_map ? slot_map[t] : -1;
     float sn[4], cs[4];
     if (use_rope) {
+        float *sines = (float*)lds, *cosines = sines + half;
+        for (int i = threadIdx.x; i < half; i += 256) sincosf((float)pos * inv_freq[i], &sines[i], &cosines[i]);
+        __syncthreads();
 #pragma unroll
-        for (int u = 0; u < 4; ++u) sincosf((float)pos * inv_freq[4 * l + u], &sn[u], &cs[u]);
+        for (int u = 0; u < 4; ++u) { sn[u] = sines[4 * l + u]; cs[u] = cosines[4 * l + u]; }
     }
     float temp = 1.f;
     if (use_temp) temp = logf((float)((pos + 1) / floor_scale) + 1.0f) * attn_scale + 1.0f;
 
     for (int it = 0; it < hpw; ++it) {
-        const int hh = (blockIdx.y * 4 * hpw + it * 4 + wave) * hpi + sub;
+        const int hh = head(it);
         const bool have = hh < n_heads;          // lanes past the last head idle, but join the shuffles
-        const bf16* src = qkv + (size_t)t * row_w + (size_t)(have ? hh : 0) * hd;
         const bool is_q = hh < H;
         const bool is_v = hh >= H + G;
         const int g = is_v ? hh - H - G : hh - H;
         const size_t page = slot >= 0 ? slot / ps : 0;
         const int off = slot >= 0 ? slot % ps : 0;
-        // the four pairs' elements: half-split (4l+u, half+4l+u) or adjacent (8l+2u, 8l+2u+1)
-        bf16x4 lo4 = *(const bf16x4*)(src + (adjacent ? 8 * l : 4 * l));
-        bf16x4 hi4 = *(const bf16x4*)(src + (adjacent ? 8 * l + 4 : half + 4 * l));
+        const bf16x4 lo4 = lo_next, hi4 = hi_next;
+        if (it + 1 < hpw) {
+            lo_next = *(const bf16x4*)(source(it + 1) + c0);
+            hi_next = *(const bf16x4*)(source(it + 1) + c1);
+        }
         if (have && is_v) {
             if (slot >= 0) {
                 bf16* slab = v_pages + (page * G + g) * (size_t)hd * ps;
-                const int c0 = adjacent ? 8 * l : 4 * l, c1 = adjacent ? 8 * l + 4 : half + 4 * l;
 #pragma unroll
                 for (int u = 0; u < 4; ++u) {
                     slab[sp_v_index(c0 + u, off, hd, ps, kv_tiled)] = lo4[u];
@@ -561,7 +636,6 @@ void rope_kvwrite_vec_kernel(const bf16* __restrict__ qkv, bf16* __restrict__ q_
                 o_lo[u] = ya; o_hi[u] = yb;
             }
         }
-        const int c0 = adjacent ? 8 * l : 4 * l, c1 = adjacent ? 8 * l + 4 : half + 4 * l;
         if (is_q) {
             bf16* dst = q_out + ((size_t)t * H + hh) * hd;
             *(bf16x4*)(dst + c0) = o_lo;
@@ -604,10 +678,16 @@ extern "C" int spite_rope_kvwrite(const void* qkv, void* q_out, void* k_pages, v
     if (plain && dtype == SP_BF16 && hd % 8 == 0 && lph >= 1 && lph <= 64 && (lph & (lph - 1)) == 0 && al8(qkv) && al8(q_out)
         && al8(k_pages) && (page_size % 4 == 0 || !write_kv)) {
         const int hpi = 64 / lph;
-        dim3 grid(T, (n_heads + 4 * hpw * hpi - 1) / (4 * hpw * hpi));
-        rope_kvwrite_vec_kernel<<<grid, 256, 0, st>>>((const bf16*)qkv, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages,
-            positions, slot_map, inv_freq, H, G, hd, page_size, use_rope, adjacent, use_norm, norm_eps, use_temp,
-            floor_scale, attn_scale, n_heads, hpw, kv_tiled);
+        // (values by blocks: with 16 heads, 4 of them kv, of 128, 256 tokens of one prompt 4.8 / 6.3 us and of as many requests 5.7 / 6.3, but
+        // 200 of as many requests 5.6 / 4.6; larger heads, 8 and 2 of 256: 330 tokens 5.9 and 8.6 against 7.4, 700 6.3 and 9.5 against 10 and 9.5)
+        const bool values = write_kv && T >= 256 && T >= 2 * hd && page_size % 8 == 0 && ((uintptr_t)v_pages & 15) == 0;
+        const int heads = values ? H + G : n_heads, v_blocks = values ? (T + ROPE_VT - 1) / ROPE_VT * G : 0;
+        const int even = (heads + 4 * hpi - 1) / (4 * hpi), each = even < hpw ? even : hpw;
+        const size_t sh = values ? (size_t)ROPE_VROWS * (hd + 2) * sizeof(bf16) : (size_t)hd * sizeof(float);
+        dim3 grid(values ? v_blocks + (T + 7) / 8 * 8 : T, (heads + 4 * each * hpi - 1) / (4 * each * hpi));
+        rope_kvwrite_vec_kernel<<<grid, 256, sh, st>>>((const bf16*)qkv, (bf16*)q_out, (bf16*)k_pages, (bf16*)v_pages,
+            positions, slot_map, inv_freq, T, H, G, hd, page_size, use_rope, adjacent, use_norm, norm_eps, use_temp,
+            floor_scale, attn_scale, heads, each, kv_tiled, v_blocks);
         SP_LAUNCH_CHECK("rope_kvwrite");
         return 0;
     }
