@@ -23,7 +23,7 @@
 // groups of every token): 2,048 tokens x 2 x 8,192 x 5,120 gated 639 / 722, 1,547 553 / 656, 330 453 / 476; 1,786, top 2,
 // 2 x 4,096 x 5,120 548 / 653; 1,531, top 4, 2 x 1,024 x 2,048 80 / 109; 1,200 x 2,048 x 3,072 57 / 70; over 220 sizes of 4 to 128
 // groups and 65 to 6,000 tokens 0.86 of the time on average.  At 2,048 tokens what bounds it is the power limit (the clock falls
-// to 1.6 GHz with the matrix units half busy), at 330 the stream of W (6.5 TB/s).
+// to 1.6 GHz with the matrix units half busy), at 330 the stream of W (6.3 TB/s).
 #include <math.h>
 #include "common.h"
 
