@@ -95,8 +95,7 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
                 float a = 0.f, b = 0.f;
                 if (lane < HD / 2) {
                     const float x = (float)kr[lane], y = (float)kr[lane + HD / 2], c = cs[2 * lane], sn = cs[2 * lane + 1];
-                    a = x * c - y * sn;
-                    b = x * sn + y * c;
+                    sp_rotate(x, y, c, sn, a, b);
                 }
                 const float ss = wave_sum(a * a + b * b);
                 const float scale = rope.norm_eps > 0.f ? 1.0f / sqrtf(ss / (float)HD + rope.norm_eps) : 1.0f;
@@ -120,8 +119,7 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
             for (int e = 0; e < 8; ++e) {
                 const int i = c * 32 + qd * 8 + e;
                 const float a = (float)lo[e], b = (float)hi[e], co = cs[2 * i], sn = cs[2 * i + 1];
-                x[c][e] = a * co - b * sn;
-                x[c + NC / 2][e] = a * sn + b * co;
+                sp_rotate(a, b, co, sn, x[c][e], x[c + NC / 2][e]);
                 ss += x[c][e] * x[c][e] + x[c + NC / 2][e] * x[c + NC / 2][e];
             }
         }

@@ -138,6 +138,15 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     return t;
 }
 
+// ------------------------------------------------------------------ rotation of a pair
+// (a cos - b sin, b cos + a sin) with one rounded product and one fused multiply-add each, written out: left to the
+// compiler, which product is fused depends on the code around it, and a key would round one way when a prompt writes it and
+// another when a decoded token does.
+__device__ __forceinline__ void sp_rotate(float a, float b, float cs, float sn, float& ra, float& rb) {
+    ra = fmaf(a, cs, -(b * sn));
+    rb = fmaf(b, cs, a * sn);
+}
+
 // ------------------------------------------------------------------ a wave's fp32 dot product
 // sum_c w[c] * xs[c] over a row xs in LDS, by one wave: lane l takes the 16-byte groups l, l+64,
 // ... and the lanes' sums meet in a butterfly.  Every kernel that forms router logits calls

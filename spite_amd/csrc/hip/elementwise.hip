@@ -400,6 +400,11 @@ void rope_kvwrite_kernel(const T* __restrict__ qkv, T* __restrict__ q_out,
         sn[u] = 0.f; cs[u] = 1.f;                    // pairs that do not rotate
         if (use_rope && i < rhalf) sincosf((float)pos * inv_freq[i], &sn[u], &cs[u]);
     }
+    // (here the second element's fused product is the sine's, in sp_rotate the cosine's: a last bit of 32 apart)
+    auto rotate = [&](float& a, float& b, int u) {
+        const float ra = fmaf(a, cs[u], -(b * sn[u])), rb = fmaf(a, sn[u], b * cs[u]);
+        a = ra; b = rb;
+    };
     float temp = 1.f;
     if (use_temp) temp = logf((float)((pos + 1) / floor_scale) + 1.0f) * attn_scale + 1.0f;
 
@@ -436,9 +441,7 @@ void rope_kvwrite_kernel(const T* __restrict__ qkv, T* __restrict__ q_out,
             if (i < half) {
                 float a = to_f32<T>(src[first_of(i)]), b = to_f32<T>(src[second_of(i)]);
                 if (use_rope && !norm_first) {
-                    const float ra = a * cs[u] - b * sn[u];
-                    const float rb = a * sn[u] + b * cs[u];
-                    a = ra; b = rb;
+                    rotate(a, b, u);
                 }
                 x0[u] = a; x1[u] = b;
                 ss += a * a + b * b;
@@ -458,9 +461,7 @@ void rope_kvwrite_kernel(const T* __restrict__ qkv, T* __restrict__ q_out,
                 float a = x0[u] * scale, b = x1[u] * scale;
                 if (use_norm && wn) { a *= wn[i0]; b *= wn[i1]; }
                 if (use_rope && norm_first) {
-                    const float ra = a * cs[u] - b * sn[u];
-                    const float rb = a * sn[u] + b * cs[u];
-                    a = ra; b = rb;
+                    rotate(a, b, u);
                 }
                 if (!use_norm || wn || norm_first) { a *= last; b *= last; }
                 else { a = x0[u] * (scale * last); b = x1[u] * (scale * last); }   // the plain case's one product
@@ -528,9 +529,9 @@ __device__ __forceinline__ void rope_value_block(const bf16* __restrict__ qkv, b
 
 // The same for bfloat16 rows whose head size gives every head a power-of-two group of lanes with
 // four pairs each (hd = 32, 64, 128, 256, 512): a lane reads and writes eight bytes at a time
-// instead of two, and a wave handles 64 / (hd/8) heads at once.  Every value is computed by the
-// same operations in the same order as in the kernel above; only the sum of squares of the
-// qk-norm meets in a different order.  A token's sines and cosines are formed once a workgroup and shared through LDS, and the
+// instead of two, and a wave handles 64 / (hd/8) heads at once.  A pair rotates as in the fused
+// decode attention (sp_rotate), bit for bit: a prompt's and a decoded token's keys round alike.
+// The sum of squares of the qk-norm meets in another order than in the kernel above.  A token's sines and cosines are formed once a workgroup and shared through LDS, and the
 // next heads' loads are asked for before this one's are worked on.
 // `v_blocks` > 0: the first workgroups (of y = 0) write the values, 32 tokens of a kv head each, and n_heads counts queries and
 // keys; tokens go to the eight XCDs in eighths, so that keys that share a line of the pages meet in one L2.
@@ -610,10 +611,8 @@ void rope_kvwrite_vec_kernel(const bf16* __restrict__ qkv, bf16* __restrict__ q_
                 a = (float)lo4[u]; b = (float)hi4[u];
             }
             if (use_rope) {
-                const int su = adjacent ? u : u;
-                // adjacent pairing: pair index 4l+u as well
-                const float ra = a * cs[su] - b * sn[su];
-                const float rb = a * sn[su] + b * cs[su];
+                float ra, rb;            // (adjacent pairing: pair index 4l+u as well)
+                sp_rotate(a, b, cs[u], sn[u], ra, rb);
                 a = ra; b = rb;
             }
             x0[u] = a; x1[u] = b;
