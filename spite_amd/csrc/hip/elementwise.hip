@@ -118,10 +118,11 @@ __device__ __forceinline__ void norm_make_plan(const norm_plan& plan, const floa
 //  are needed (us): one row of 5,120 3.3 / 4.0, of 2,048 2.3 / 2.9, with 16 rows of proj 6.1 / 7.0 and 4.2 / 5.6; 2,048 rows of 5,120
 //  29 / 33 (6.5 TB/s), of 2,048 14 / 17.  Two rows of proj a wave in flight where the row is short (2,048: 4.2, one 5.0; 5,120: 8.1
 //  / 6.1).
-//  Many rows with a projection: R rows a workgroup, since each workgroup reads all of `proj` from L2 (16 x 5,120: 320 KB beside
-//  60 KB of the row; 2,048 rows 41 / 43, four rows a workgroup, for which LDS has less room, 59; 330 rows 10.1 / 11.3).
-template <typename TO, int V, int R, bool PLAN>
-__global__ __launch_bounds__(NORM_NT)
+//  AHEAD false: each group's loads as they are needed, in half of the registers, so that two workgroups share a compute unit:
+//  wide rows in greater numbers.  With a projection, R rows a workgroup, since each workgroup reads all of `proj` from L2.
+//  Where either pays: see norm_variant.
+template <typename TO, int V, int R, bool PLAN, bool AHEAD>
+__global__ __launch_bounds__(NORM_NT, AHEAD ? 1 : 4)
 void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ out2) {
     __shared__ float red[NORM_NT / 64];
     extern __shared__ __attribute__((aligned(16))) float ys[];            // [R][d] if proj, and P logits behind it if PLAN
@@ -137,33 +138,38 @@ void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ 
         const size_t r = p.rows ? (size_t)p.rows[i] : (size_t)i;
         float* hr = p.h + r * d;
         f32x4 v[V], x1[V], x2[V], xn[V], wn[V];
+        auto past = [&](int u) { return !AHEAD && tid + u * NORM_NT >= nv; };     // (loads as they are needed are skipped past the row)
         if (p.dn)
 #pragma unroll
-            for (int u = 0; u < V; ++u) xn[u] = ((const f32x4*)(p.dn + r * d))[at[u]];
+            for (int u = 0; u < V; ++u)
+                if (!past(u)) xn[u] = ((const f32x4*)(p.dn + r * d))[at[u]];
+        if (AHEAD) {
 #pragma unroll
-        for (int u = 0; u < V; ++u) v[u] = ((const f32x4*)hr)[at[u]];
-        if (p.d1)
+            for (int u = 0; u < V; ++u) v[u] = ((const f32x4*)hr)[at[u]];
+            if (p.d1)
 #pragma unroll
-            for (int u = 0; u < V; ++u) x1[u] = ((const f32x4*)(p.d1 + r * d))[at[u]];
-        if (p.d2)
+                for (int u = 0; u < V; ++u) x1[u] = ((const f32x4*)(p.d1 + r * d))[at[u]];
+            if (p.d2)
 #pragma unroll
-            for (int u = 0; u < V; ++u) x2[u] = ((const f32x4*)(p.d2 + r * d))[at[u]];
-        if (p.dn)
+                for (int u = 0; u < V; ++u) x2[u] = ((const f32x4*)(p.d2 + r * d))[at[u]];
+            if (p.dn)
 #pragma unroll
-            for (int u = 0; u < V; ++u) wn[u] = ((const f32x4*)p.wn)[at[u]];
-        if (rr == 0 && normed) {
-            if (!p.plain_out)
+                for (int u = 0; u < V; ++u) wn[u] = ((const f32x4*)p.wn)[at[u]];
+            if (rr == 0 && normed) {
+                if (!p.plain_out)
 #pragma unroll
-                for (int u = 0; u < V; ++u) ww[u] = ((const f32x4*)p.w)[at[u]];
-            if (out2)
+                    for (int u = 0; u < V; ++u) ww[u] = ((const f32x4*)p.w)[at[u]];
+                if (out2)
 #pragma unroll
-                for (int u = 0; u < V; ++u) ww2[u] = ((const f32x4*)p.w2)[at[u]];
+                    for (int u = 0; u < V; ++u) ww2[u] = ((const f32x4*)p.w2)[at[u]];
+            }
         }
         float sn = 0.f, ss = 0.f;
         if (p.dn) {
             float sq = 0.f;
 #pragma unroll
             for (int u = 0; u < V; ++u) {
+                if (past(u)) continue;
                 const float t = xn[u][0] * xn[u][0] + xn[u][1] * xn[u][1] + xn[u][2] * xn[u][2] + xn[u][3] * xn[u][3];
                 if (tid + u * NORM_NT < nv) sq += t;
             }
@@ -171,11 +177,15 @@ void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ 
         }
 #pragma unroll
         for (int u = 0; u < V; ++u) {
-            if (p.d1) v[u] += x1[u];
-            if (p.d2) v[u] += x2[u];
-            if (p.dn)
+            if (past(u)) continue;
+            if (!AHEAD) v[u] = ((const f32x4*)hr)[at[u]];
+            if (p.d1) v[u] += AHEAD ? x1[u] : ((const f32x4*)(p.d1 + r * d))[at[u]];
+            if (p.d2) v[u] += AHEAD ? x2[u] : ((const f32x4*)(p.d2 + r * d))[at[u]];
+            if (p.dn) {
+                const f32x4 w4 = AHEAD ? wn[u] : ((const f32x4*)p.wn)[at[u]];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) v[u][e] += xn[u][e] * sn * wn[u][e];
+                for (int e = 0; e < 4; ++e) v[u][e] += xn[u][e] * sn * w4[e];
+            }
             const float t = v[u][0] * v[u][0] + v[u][1] * v[u][1] + v[u][2] * v[u][2] + v[u][3] * v[u][3];
             if (tid + u * NORM_NT < nv) {
                 ss += t;
@@ -189,9 +199,11 @@ void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ 
             const int c = tid + u * NORM_NT;
             if (c >= nv) continue;
             f32x4 y = v[u];
-            if (!p.plain_out)
+            if (!p.plain_out) {
+                const f32x4 w4 = AHEAD ? ww[u] : ((const f32x4*)p.w)[c];
 #pragma unroll
-                for (int e = 0; e < 4; ++e) y[e] = v[u][e] * scale * ww[u][e];
+                for (int e = 0; e < 4; ++e) y[e] = v[u][e] * scale * w4[e];
+            }
             if (p.out32) ((f32x4*)(p.out32 + (size_t)i * d))[c] = y;
             if (p.proj) ((f32x4*)(ys + rr * d))[c] = y;
             auto put = [&](TO* dst, const f32x4& yy) {
@@ -206,9 +218,10 @@ void add_rmsnorm_vec_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ 
             };
             if (out) put(out, y);
             if (out2) {                                      // the same row under a second norm's weights
+                const f32x4 w4 = AHEAD ? ww2[u] : ((const f32x4*)p.w2)[c];
                 f32x4 y2;
 #pragma unroll
-                for (int e = 0; e < 4; ++e) y2[e] = v[u][e] * scale * ww2[u][e];
+                for (int e = 0; e < 4; ++e) y2[e] = v[u][e] * scale * w4[e];
                 put(out2, y2);
             }
         }
@@ -307,6 +320,29 @@ void add_rmsnorm_kernel(norm_args p, TO* __restrict__ out, TO* __restrict__ out2
     norm_make_plan(p.plan, ys + ((d + 3) & ~3), P);
 }
 
+// Rows a workgroup takes, and 256 where it asks for every load ahead, for rows that 16-byte loads can take with P rows of a
+// projection (0: none).
+//
+// Measured on an MI355X, launches in a row (us):
+//  * rows of more than 8,192, with increments: up to a row a compute unit ahead (64 x 12,288 6.4, as needed 7.1), beyond as needed
+//    (300 x 12,288 12.6, ahead 14.2; 2,048 76.7 / 78.9; with 128 rows of a projection 475 / 644; 520 x 16,384 stays, 4 % behind).
+//  * up to 2,048 wide one row a workgroup, whatever P is (2,048 x 2,048 with 128 rows of a projection one 84, two 107).
+//  * up to 4,096 two where rows are more than two a compute unit (2,048 x 2,560 with 16 24.4 / one 27.0, with 128 67 / 95; 330
+//    with 16 8.2 / 7.2); for fewer only where P is 64 to 128 and the row neither short nor long (330 with 128: of 2,560 20.8 / 25.0,
+//    of 2,304 31.3 / 27.9, of 3,840 13 % behind).
+//  * up to 6,144 two from 5,120 on (4,608 lost at every size: 2,048 with 16 55.7 / 49.5) and from 32 or 64 rows of a projection
+//    (5,120: 330 with 16 10.8 / 11.2 but 600 21.5 / 18.3, 2,048 47.6 / 47.0; with 64 330 20.3 / 25.6; with 128 2,048 137 / 186); a
+//    little over two rows a compute unit, which two rows a workgroup start a second round with, seldom (600 x 6,144 with 128 101 / 93).
+static int norm_variant(int n_rows, int d, int P) {
+    const int v = (d / 4 + NORM_NT - 1) / NORM_NT, cus = sp_cu_count();
+    bool two = false;
+    if (P > 0 && v == 2) two = n_rows > 2 * cus ? P >= 16 : n_rows > cus && d >= 2560 && d <= 3072 && P >= 64 && P <= 128;
+    if (P > 0 && v == 3 && n_rows > cus && d >= 5120)
+        two = n_rows > 2 * cus && n_rows <= 3 * cus ? P >= 128 && d <= 5376 : P >= (d <= 5632 ? 32 : 64);
+    return (two ? NORM_R : 1) + (v <= 4 || n_rows <= cus ? 256 : 0);
+}
+extern "C" int spite_add_rmsnorm_variant(int n_rows, int d, int P) { return norm_variant(n_rows, d, P); }
+
 extern "C" int spite_add_rmsnorm(float* h, const float* d1, const float* d2, const float* w, void* out,
                                  int out_dtype, float* out32, const int* rows, int n_rows, int d,
                                  float eps, int write_h, const float* proj, float* proj_out, int P,
@@ -339,13 +375,15 @@ extern "C" int spite_add_rmsnorm(float* h, const float* d1, const float* d2, con
         return 0;
     }
     const int v = (d / 4 + NORM_NT - 1) / NORM_NT;
-    const bool many = proj && n_rows > (v == 1 ? 2 : 1) * sp_cu_count() && v <= 3;
-    if (many) sh = (size_t)NORM_R * d * sizeof(float);
+    const int variant = norm_variant(n_rows, d, proj ? P : 0);
+    const bool ahead = variant >= 256, two = variant % 256 == NORM_R;
+    if (two) sh = (size_t)NORM_R * d * sizeof(float);
 #define SP_NORM_V(V) do { \
-        if (!proj) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA false>, n_rows); \
-        else if (expert) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA true>, n_rows); \
-        else if (many) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA (V <= 3 ? V : 1) SP_COMMA NORM_R SP_COMMA false>, (n_rows + NORM_R - 1) / NORM_R); \
-        else SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA false>, n_rows); } while (0)
+        if (!ahead) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA false SP_COMMA (V <= 4)>, n_rows); \
+        else if (expert) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA true SP_COMMA true>, n_rows); \
+        else if (two) SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA (V <= 3 ? V : 2) SP_COMMA (V == 2 || V == 3 ? NORM_R : 1) SP_COMMA false SP_COMMA true>, \
+                              (n_rows + NORM_R - 1) / NORM_R); \
+        else SP_NORM(add_rmsnorm_vec_kernel<TO SP_COMMA V SP_COMMA 1 SP_COMMA false SP_COMMA true>, n_rows); } while (0)
     switch (v) {
         case 1: SP_NORM_V(1); break;
         case 2: SP_NORM_V(2); break;

@@ -51,6 +51,7 @@ def lib():
         l.spite_hip_last_error.restype = c_char_p
         P, I, L, F = c_void_p, c_int, c_long, c_float
         sigs = {
+            "spite_add_rmsnorm_variant": [I, I, I],
             "spite_embed": [P, P, I, P, I, I, I, F, P],
             "spite_add_rmsnorm": [P, P, P, P, P, I, P, P, I, I, F, I, P, P, I, P, P, F, F, I, P, P, P, P, P, P, P, P, I, P],
             "spite_rope_kvwrite": [P, P, P, P, I, P, P, P, I, I, I, I, I, I, I, I, F, I, I, F, I, I, I, P, P, I, P],
