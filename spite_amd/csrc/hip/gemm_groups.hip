@@ -185,21 +185,29 @@ template <int NW, bool GLU, typename TY>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_groups_kernel(gg_args p) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
-    const int units = p.m_tiles * p.n_tiles, per_xcd = (units + 7) / 8;
-    const int unit = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if ((int)(blockIdx.x / 8) >= per_xcd || unit >= units) return;
-    // the group of the row tile, 64 groups at a time: a prefix sum over the lanes (one after another the loads of the offsets
-    // cost half a microsecond a group); what it finds is kept in scalar registers
-    const int mt = unit % p.m_tiles, lane = threadIdx.x & 63;
-    int g = -1, row0 = 0, row_end = 0, nb = 8, tiles = 0, base = 0;
-    for (int c = 0; c < p.n_groups; c += 64) {
-        int b = 0, e = 0, h = 0;
+    // The groups' tiles, 64 groups at a time: a prefix sum over the lanes (one after another the loads of the offsets cost half a
+    // microsecond a group); what it finds is kept in scalar registers.  The launch is as large as the rows allow, up to a tile a group more than there are.
+    // Those that there are are dealt evenly to the XCDs and go to their first workgroups: with empty ones among them an XCD got
+    // more than its eighth, and two tiles met on one compute unit while others had none (126 rows of 4 of 4 experts and of one more x 2 x
+    // 5,120 x 16,384 gated, 200 tiles of four waves, 506 -> 292 us; 1,483 of 8 of 32 x 768 x 16,384, eight waves, 846 -> 483; over 559 sizes 0.96).
+    const int lane = threadIdx.x & 63;
+    int b = 0, e = 0, h = 0, nt = 0, incl = 0, all = 0;
+    auto scan = [&](int c) {
+        b = e = 0;
         if (c + lane < p.n_groups) { b = p.offsets[c + lane]; e = p.offsets[c + lane + 1]; }
-        const int nt = gg_group_tiles(e - b, p.cap, h);
-        int incl = nt;
+        nt = incl = gg_group_tiles(e - b, p.cap, h);
 #pragma unroll
         for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
-        const int total = __builtin_amdgcn_readlane(incl, 63);
+        return __builtin_amdgcn_readlane(incl, 63);
+    };
+    for (int c = 0; c < p.n_groups; c += 64) all += scan(c);
+    const int units = all * p.n_tiles, per_xcd = (units + 7) / 8;
+    const int unit = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+    if ((int)(blockIdx.x / 8) >= per_xcd || unit >= units) return;
+    const int mt = __builtin_amdgcn_readfirstlane(unit % all);
+    int g = -1, row0 = 0, row_end = 0, nb = 8, tiles = 0, base = 0;
+    for (int c = 0; c < p.n_groups; c += 64) {
+        const int total = p.n_groups <= 64 ? all : scan(c);
         if (mt < base + total) {
             const bool mine = mt >= base + incl - nt && mt < base + incl;
             const int src = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(mine)) - 1);
@@ -212,9 +220,8 @@ void gemm_groups_kernel(gg_args p) {
         }
         base += total;
     }
-    // (no such tile; or, with heights rounded up, the group's rows end before its last tile)
-    if (g < 0 || row0 >= row_end) return;
-    const int n0 = unit / p.m_tiles * (GLU ? 32 * NW : 64 * NW);
+    if (g < 0) return;
+    const int n0 = __builtin_amdgcn_readfirstlane(unit / all) * (GLU ? 32 * NW : 64 * NW);
 #define GG_TILE(NB, S, NT) gg_tile<NW, NB, S, GLU, TY, NT>(p, lds, g, row0, row_end, n0, 0, p.K / 64, (TY*)p.Y)
 #define GG_TILES(NT) switch (nb) { \
         case 2: GG_TILE(2, 6, NT); break; \

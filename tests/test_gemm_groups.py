@@ -58,3 +58,20 @@ def test_choice_of_waves_and_height():
     for T in (69, 228, 425):
         assert at(T, 16, 1, 1, 5120, 8192, False) is None
     assert at(300, 4, 1, 0, 1216, 4416, False) == (4, 128) and gemm_groups_choice(0, 16, 0.0, 0, 64, 64, False) is None
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("waves,cap", [(4, 128), (8, 160)])
+@pytest.mark.parametrize("G,rows", [(1, [300]), (9, [0] * 8 + [5]), (64, [0, 0, 161] + [0] * 60 + [40]), (65, [1] * 65), (200, [0] * 70 + [3] + [0] * 128 + [170]),
+                                    (129, [0] * 129)])
+def test_groups_of_which_few_hold_rows(waves, cap, G, rows):
+    """The launch is sized by the rows and the number of groups; what holds rows is found among them, and nothing else is written."""
+    M, N, K = sum(rows), 272, 128
+    a, w = rnd(max(M, 1), K, dtype=torch.bfloat16), ops().operand_order(rnd(G, N, K, dtype=torch.bfloat16, seed=1))
+    offsets = torch.tensor([sum(rows[:g]) for g in range(G + 1)], dtype=torch.int32, device=DEV)
+    M = M + 200                                                  # room for more rows than the offsets name
+    a = torch.cat([a, rnd(200, K, dtype=torch.bfloat16, seed=2)])
+    y, z = torch.full((M, N), 7.0, device=DEV), torch.full((M, N), 7.0, device=DEV)
+    ops().gemm_tiled(a, w, y, M, N, K, offsets=offsets, n_groups=G, shape=1)
+    ops().gemm_groups(a, w, z, M, N, K, offsets=offsets, n_groups=G, waves=waves, cap=cap)
+    assert torch.equal(y, z) and (z[sum(rows):] == 7.0).all()
