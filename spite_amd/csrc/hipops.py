@@ -728,14 +728,16 @@ def gemm_runs_choice(M: int, N: int, K: int):
     """(runs, nb) for ``gemm_runs``, or None where another product is the faster one.  Up to 32 rows the stream of W of
     ``gemm_skinny`` is; up to 64 it is for matrices of fewer than 26 M elements (64 rows: 3,072 x 2,048 12.7 against 17.6 us, 5,120 x
     5,120 24.4 against 23.3, 32,768 x 5,120 119 against 62).  Beyond, by what each is estimated to take: up to 800 rows the estimate
-    of the others is the lower side of what was timed (149 sizes, 25 % faster on average, 2 of them up to 3 % slower); above, where
-    two rounds of small tiles stand against one of large ones, it has to be a tenth to gain."""
+    of the others is the lower side of what was timed; above, small tiles in one run lose to the large ones of ``gemm_lds`` (1,547 x
+    5,120 x 8,192 125 against 101, 1,922 x 3,072 x 14,336 210 against 166), and more runs have an eighth to gain.  (Timed at 757 sizes that
+    it takes in: 29 % faster on average, one of them 4 % slower.)"""
     if M <= 32 or (M <= 64 and N * K < 26_000_000):
         return None
     us = ctypes.c_double()
     code = lib().spite_gemm_runs_choice(M, N, K, ctypes.addressof(us))
-    if not code or (M > 64 and us.value >= (1.1 if M <= 800 else 0.9)
-                    * min(lds_us(M, N, K, False), tiled_us(M, N, K, False, tiled_k_runs(M, N, K)))):
+    if not code or (M > 800 and code < 32):
+        return None
+    if M > 64 and us.value >= (1.1 if M <= 800 else 0.87) * min(lds_us(M, N, K, False), tiled_us(M, N, K, False, tiled_k_runs(M, N, K))):
         return None
     return divmod(code, 16)
 
