@@ -388,68 +388,101 @@ extern "C" int spite_gemm_groups(const void* X, int ldx, const void* W, long w_g
     return y_dtype == SP_BF16 ? gg_launch<4, false, bf16>(p, st) : gg_launch<4, false, float>(p, st);
 }
 
-// Which waves and cap suit a product whose `routed` groups hold `mean` rows each on average (sizes taken as normal about it),
-// beside `whole` groups that take all `tokens` rows: waves * 256 + cap, or 0: gemm_tiled.
+// What a product over groups takes, in us: `routed` groups that hold `mean` rows each on average (sizes taken as normal about it)
+// beside `whole` groups that take all `tokens` rows.
 //
-// The estimate: the tiles to expect and their mean height nb; a tile takes (a + b nb) us at K = 5,120, eight waves alone on a
-// compute unit, four in pairs (one alone a third of that); rounds of tiles over the slots, a last one that is not full counts
-// for most of one with eight waves and for a third with four; beside it the stream of the weights; then the two together,
-// between their maximum and their sum.  Fitted to 220 sizes (4 to 128 groups, 65 to 6,000 tokens, N and K of 512 to 8,192, plain
-// and gated) timed with each choice and with gemm_tiled: the choice is 14 % faster than gemm_tiled's best tile by its own
-// rules on average; nine are 2 % and more slower, most of them sizes where a tile more or less starts a round (4 x 220 rows x 6,912 x
-// 4,672: 127 against 100 until a deviation of tiles more was counted).
-// Where the tiles of eight waves are one for every second compute unit and up to one for each, and the time is the stream of
-// W, four waves, with a tile for some units and two for others, stream no faster; plain products stay with gemm_tiled
-// there (69 rows, 16 groups and one of all x 5,120 x 8,192: 246 with eight and 266 with four against 210), gated ones
-// take eight (300 rows x 2 x 3,072 x 2,048: 72 and 75 against 85).
-extern "C" int spite_gemm_groups_choice(int tokens, int routed, double mean, int whole, int N, int K, int glu) {
-    if (tokens <= 0 || routed <= 0 || mean <= 0.0) return 0;
-    static const double Z[11] = {-1.6, -1.0, -0.67, -0.43, -0.2, 0.0, 0.2, 0.43, 0.67, 1.0, 1.6};
-    const double cus = sp_cu_count(), share = mean / tokens < 1.0 ? mean / tokens : 1.0;
-    const double sd = sqrt(tokens * share * (1.0 - share));
-    const double live = routed * mean < routed ? routed * mean : routed;
-    const double stream = (live + whole) * (double)N * K * (glu ? 4 : 2) * 1e-6;       // MB
-    int best = 0;
-    double least = 0.0;
-    bool pairs = true;
-    for (int waves : {8, 4}) {
-        if (waves == 4 && !pairs) continue;
-        for (int cap : {160, 128}) {
-            double n = 0.0, sum = 0.0, squares = 0.0;
-            int most = 2, nb;
-            for (double z : Z) {
-                const int rows = (int)(mean + z * sd + 0.5);
-                if (rows <= 0) continue;
-                const int t = gg_group_tiles(rows, cap, nb);
-                n += t; sum += (double)t * nb; squares += (double)t * t;
-                most = nb > most ? nb : most;
-            }
-            // (a standard deviation of tiles more: a round that the tiles miss by one costs more than is to be gained)
-            const double spread = sqrt(fmax(routed * (squares / 11.0 - n / 11.0 * (n / 11.0)), 0.0));
-            n *= routed / 11.0; sum *= routed / 11.0;
-            if (whole) {
-                const int t = gg_group_tiles(tokens, cap, nb);
-                n += (double)whole * t; sum += (double)whole * t * nb;
-                most = nb > most ? nb : most;
-            }
-            if (n <= 0.0) return 0;
-            const double cols = (N + (glu ? 32 : 64) * waves - 1) / ((glu ? 32 : 64) * waves), tiles = (n + spread) * cols, nbm = sum / n;
-            double us;
-            if (waves == 8) {
-                const double r = tiles / cus, c = K / 5120.0 * (71.0 + 6.5 * nbm), alone = K / 5120.0 * (71.0 + 6.5 * most);
-                if (cap == 160 && r > 0.5 && r <= 0.95 && K / 5120.0 * (68.7 + 7.76 * nbm) * r < 0.7 * stream / 6.5) {
-                    if (!glu) return 0;
-                    pairs = false;
-                }
-                const double work = r <= 1.0 ? alone : c * (r + 0.8 * (ceil(r) - r));
-                us = 7.9 + pow(pow(work, 2.4) + pow(stream / 6.45, 2.4), 1.0 / 2.4);
-            } else {
-                const double r = tiles / (2.0 * cus), c = K / 5120.0 * (37.0 + 11.0 * nbm), alone = 0.31 * K / 5120.0 * (37.0 + 11.0 * most);
-                const double work = r <= 0.5 ? alone : r <= 1.0 ? (c > alone ? c : alone) : c * (r + 0.33 * (ceil(r) - r));
-                us = 8.2 + pow(pow(work, 1.6) + pow(stream / 6.8, 1.6), 1.0 / 1.6);
-            }
-            if (best == 0 || us <= least) { best = waves * 256 + cap; least = us; }
-        }
+// The tiles to expect go to eight XCDs and, in turn, to the four shader engines of each; gemm_tiled and gemm_lds have a
+// launch's empty tiles among the others, so that an engine may get more than its share of real ones.  A tile takes `tile` us and, for
+// every 5,120 of K, `w` and `x` for each 16 rows (gemm_lds: 32) of its height; where none waits for another `alone` of that; rounds of
+// them, of which a last one that is not full counts for `part` and what fills it.  Beside it the stream of the weights of the
+// groups that hold rows; the two together between their maximum and their sum.  A gated product takes `gated` of it, one whose bands of
+// W lie multiples of 64 KB apart `aligned` (they meet in the same memory channels), and the result is written at `out` TB/s.
+// Fitted to 3,600 products (4 to 128 groups of 1 to 8 a token, 65 to 6,000 tokens, N of 512 to 8,192, K of 512 to 16,384, gated in
+// bfloat16 and plain in fp32), each timed with every kernel: 7 to 9 % off (gemm_lds 11), much of it alike for all of one size.
+struct gg_fit { int rows, cols; double start, tile, w, x, tbs, power, part, alone, gated, out, aligned; };
+static const gg_fit GG_FITS[8] = {       // gemm_groups with four waves and tiles of up to 128 and 160 rows, and eight; gemm_tiled's three; gemm_lds
+    {128, 256, 7.15, 2.46, 73.6, 6.2, 9, 1.3, 0.32, 0.444, 0.957, 4.77, 1.03},
+    {160, 256, 6.86, 3.15, 86.8, 6.28, 8.58, 1.49, 0.334, 0.45, 0.962, 4.54, 1.02},
+    {128, 512, 3.56, 7.1, 99, 2.34, 9, 1.56, 0.784, 0.892, 0.971, 6.32, 1.06},
+    {160, 512, 4.23, 7.44, 105, 2.87, 9, 1.71, 0.764, 0.846, 0.98, 5.19, 1.05},
+    {128, 512, 6.34, 6.22, 74.1, 6.16, 9, 1.67, 0.654, 0.821, 1.01, 5.73, 0.992},
+    {160, 512, 11.1, 5.39, 80.7, 6.63, 7.06, 2.33, 0.659, 0.792, 1.02, 5.3, 1},
+    {64, 512, 1.25, 6.7, 72.8, 6.27, 8.59, 1.65, 0.896, 0.922, 1.02, 2, 0.987},
+    {256, 256, 2.24, 12.1, 12.9, 12.9, 7.19, 1.47, 0.75, 0.827, 0.979, 6.65, 1.01}
+};
+static int gg_fit_tiles(int kind, int rows, int& nb) {
+    if (kind < 4) return gg_group_tiles(rows, GG_FITS[kind].rows, nb);
+    const int height = GG_FITS[kind].rows, tiles = (rows + height - 1) / height;
+    nb = height / 16;
+    if (kind == 7) {                     // as gemm_lds takes them
+        const int each = tiles ? (rows + tiles - 1) / tiles : 0;
+        nb = each > 192 ? 8 : each > 160 ? 6 : each > 128 ? 5 : each > 96 ? 4 : 3;
     }
-    return best;
+    return tiles;
+}
+static double gg_estimate(int kind, int tokens, int routed, double mean, int whole, int N, int K, int glu) {
+    static const double Z[11] = {-1.6, -1.0, -0.67, -0.43, -0.2, 0.0, 0.2, 0.43, 0.67, 1.0, 1.6};
+    const gg_fit& f = GG_FITS[kind];
+    const double share = mean / tokens < 1.0 ? mean / tokens : 1.0, sd = sqrt(tokens * share * (1.0 - share));
+    double n = 0.0, sum = 0.0;
+    int most = 2, nb;
+    for (double z : Z) {
+        const int rows = (int)(mean + z * sd + 0.5);
+        if (rows <= 0) continue;
+        const int t = gg_fit_tiles(kind, rows, nb);
+        n += t; sum += (double)t * nb;
+        most = nb > most ? nb : most;
+    }
+    n *= routed / 11.0; sum *= routed / 11.0;
+    if (whole) {
+        const int t = gg_fit_tiles(kind, tokens, nb);
+        n += (double)whole * t; sum += (double)whole * t * nb;
+        most = nb > most ? nb : most;
+    }
+    if (n <= 0.0) return 0.0;
+    const long cols = (N + f.cols / (glu ? 2 : 1) - 1) / (f.cols / (glu ? 2 : 1));
+    const double rows = (double)routed * mean + (double)whole * tokens, cus = sp_cu_count();
+    double u;                            // rounds of tiles
+    if (kind < 4) {
+        u = ceil(n * cols / 8.0) / (cus / 8.0 * (kind < 2 ? 2.0 : 1.0));
+    } else {
+        const long real = n > 1.0 ? (long)(n + 0.5) : 1, groups = routed + whole;
+        long launched = (long)(rows / f.rows) + (groups < (long)rows ? groups : (long)rows), most_tiles = 0;
+        if (launched < real) launched = real;
+        const long units = launched * cols, per = (units + 7) / 8;
+        for (long first = 0; first < units; first += per)
+            for (long engine = 0; engine < 4; ++engine) {
+                long c = 0;
+                for (long unit = first + engine; unit < first + per && unit < units; unit += 4) c += unit % launched < real;
+                most_tiles = c > most_tiles ? c : most_tiles;
+            }
+        u = most_tiles / (cus / 32.0);
+    }
+    const double tile = f.tile + K / 5120.0 * (f.w + f.x * sum / n), tallest = f.tile + K / 5120.0 * (f.w + f.x * most);
+    double work = f.alone * tallest;
+    if (kind < 2 && u > 0.5) work = u <= 1.0 ? fmax(tile, work) : tile * (u + f.part * (ceil(u - 1e-9) - u));
+    if (kind >= 2 && u > 1.0) work = tile * (u + f.part * (ceil(u - 1e-9) - u));
+    const double live = routed * (1.0 - pow(1.0 - share, tokens));
+    const double stream = (live + whole) * N * K * (glu ? 4e-6 : 2e-6) / f.tbs;
+    const double us = f.start + pow(pow(work, f.power) + pow(stream, f.power), 1.0 / f.power);
+    return us * (glu ? f.gated : 1.0) * (K % 2048 == 0 ? f.aligned : 1.0) + rows * N * (glu ? 2e-6 : 4e-6) / f.out;
+}
+
+// Which waves and cap suit it: waves * 256 + cap, or 0 where the other product, gemm_lds (`lds`) or gemm_tiled with its tile `shape`, is
+// estimated within 2 % of the best of them.  us[0]: what the taken one is estimated to take.  Over those products the choice is 18 %
+// faster than the others on average; at 93 it is 2 % and more slower, at 43 of them by 5 % and more (a quarter of those where one
+// group took a quarter of the rows, which the estimate cannot know).  16 experts and a shared one: 1,547 tokens x 2 x 8,192 x 5,120
+// gated tiles of eight waves (553 us, gemm_tiled 656), 1,512 x 3,072 x 2,048 stays (gemm_groups 71, gemm_tiled 61).
+extern "C" int spite_gemm_groups_choice(int tokens, int routed, double mean, int whole, int N, int K, int glu, int shape, int lds, double* us) {
+    *us = 0.0;
+    if (tokens <= 0 || routed <= 0 || mean <= 0.0) return 0;
+    const double other = gg_estimate(lds ? 7 : shape == 3 ? 5 : shape == 4 || shape == 5 ? 6 : 4, tokens, routed, mean, whole, N, K, glu);
+    int best = 0;
+    for (int kind = 0; kind < 4; ++kind) {
+        const double t = gg_estimate(kind, tokens, routed, mean, whole, N, K, glu);
+        if (best == 0 || t < *us) { best = (kind < 2 ? 4 : 8) * 256 + GG_FITS[kind].rows; *us = t; }
+    }
+    if (*us < 0.98 * other) return best;
+    *us = other;
+    return 0;
 }

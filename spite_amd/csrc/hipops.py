@@ -124,7 +124,7 @@ def lib():
         l.spite_router_plan_is_one_launch.restype = c_int
         l.spite_gemm_skinny_variant.argtypes = [I] * 7
         l.spite_gemm_skinny_variant.restype = c_int
-        l.spite_gemm_groups_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I]
+        l.spite_gemm_groups_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I, I, I, P]
         l.spite_gemm_groups_choice.restype = c_int
         l.spite_gemm_f32_variant.argtypes = [I, I, I]
         l.spite_gemm_f32_variant.restype = c_int
@@ -784,11 +784,18 @@ def gemm_lds(a, w, y, M, N, K, *, offsets=None, n_groups=1, a_rows=None, a_scale
 
 
 @functools.lru_cache(maxsize=4096)
-def gemm_groups_choice(tokens: int, routed: int, mean: float, whole: int, N: int, K: int, glu: bool):
-    """(waves, cap) for ``gemm_groups``, or None where ``gemm_tiled`` is the faster one: ``routed`` groups of ``mean`` rows each on
-    average beside ``whole`` groups that take all ``tokens`` rows (the rule, and what it was timed against, in gemm_groups.hip)."""
-    code = lib().spite_gemm_groups_choice(tokens, routed, mean, whole, N, K, int(bool(glu)))
-    return divmod(code, 256) if code else None
+def gemm_groups_estimate(tokens: int, routed: int, mean: float, whole: int, N: int, K: int, glu: bool, shape: int = 0, lds: bool = False):
+    """((waves, cap) for ``gemm_groups``, or None where the other product is the faster one; what the taken one is estimated to
+    take, in us): ``routed`` groups of ``mean`` rows each on average beside ``whole`` groups that take all ``tokens`` rows.  The other
+    product is ``gemm_lds`` (``lds``) or ``gemm_tiled`` with tile ``shape`` (the rule, and what it was timed against, in gemm_groups.hip)."""
+    us = ctypes.c_double()
+    code = lib().spite_gemm_groups_choice(tokens, routed, mean, whole, N, K, int(bool(glu)), int(shape), int(bool(lds)), ctypes.addressof(us))
+    return (divmod(code, 256) if code else None), us.value
+
+
+def gemm_groups_choice(tokens: int, routed: int, mean: float, whole: int, N: int, K: int, glu: bool, shape: int = 0, lds: bool = False):
+    """The choice of ``gemm_groups_estimate``."""
+    return gemm_groups_estimate(tokens, routed, mean, whole, N, K, glu, shape, lds)[0]
 
 
 def gemm_groups_ok(a, y, M, N, K, glu) -> bool:

@@ -195,17 +195,18 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
         if tiled:
             splits = offsets is None and a_rows is None and a_scale is None and y_rows is None and not glu and act is None
             runs = hipops.tiled_k_runs(M, N, K) if splits and tile_shape == 0 and M > 0 else 1
+            lds = M > 0 and hipops.gemm_lds_ok(x, w, M, N, K, glu) and (
+                hipops.lds_suits(M, N, K, bool(glu), runs) if offsets is None
+                else hipops.lds_suits_groups(M / n_groups if group_rows is None else group_rows, K,
+                                             *_group_tiles(M, n_groups, most, group_rows, N, bool(glu))))
             if offsets is not None and M > 0 and act is None and hipops.gemm_groups_ok(x, y, M, N, K, glu):
                 mean, whole = _routed_and_whole(M, n_groups, most, group_rows)
-                choice = hipops.gemm_groups_choice(most, n_groups - whole, float(mean), whole, N, K, bool(glu))
+                choice = hipops.gemm_groups_choice(most, n_groups - whole, float(mean), whole, N, K, bool(glu), tile_shape, lds)
                 if choice is not None:
                     hipops.gemm_groups(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
                                        y_rows=y_rows, glu=bool(glu), waves=choice[0], cap=choice[1])
                     return
-            if M > 0 and hipops.gemm_lds_ok(x, w, M, N, K, glu) and (
-                    hipops.lds_suits(M, N, K, bool(glu), runs) if offsets is None
-                    else hipops.lds_suits_groups(M / n_groups if group_rows is None else group_rows, K,
-                                                 *_group_tiles(M, n_groups, most, group_rows, N, bool(glu)))):
+            if lds:
                 hipops.gemm_lds(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
                                 y_rows=y_rows, glu=glu, act=act, act_limit=limit)
                 return
