@@ -122,15 +122,17 @@ def whole_group_apart(tokens: int, groups: int, N: int, K: int) -> int:
     """Whether a plain product over ``groups`` groups that ``tokens`` rows spread over and one group that takes every row
     is better done as two: the groups (the result is the tile shape that they then take, 0: together), and the one as a
     product of its own.  Together the tiles of the second kind fill the first one's last round; apart it may need one round
-    fewer.  A round takes 146 us at K = 5,120 and the groups no less than their weights at 5.6 TB/s.  Routers do not
-    spread their rows quite evenly, and a round that the groups miss by a tile costs more than is to be gained: with a standard
-    deviation of tiles more they have to fit 85 % of their rounds, and the two to be 6 % faster than all tiles together with a
-    deviation fewer.
-    (Measured at 300 sizes, 2 to 64 experts, 200 to 6,000 tokens: of the 29 that this takes in none is slower apart, on
-    average they are 10 % faster; with neither margin 15 of 58 were slower, by up to 42 %.  5,120 x 8,192 over 16 experts,
-    together / apart: 1,454 tokens 433 / 346 us, 1,547 425 / 362, 2,048 448 / 432; over 8: 1,806 398 / 345; 3,072 x 8,192 over 16:
-    3,107 431 / 360.)  A gated product's rounds are many and its stream of weights long: there it never paid (2,048 tokens
-    719 / 759)."""
+    fewer, and each has the kernel that suits it.  The price is ``gemm_tiled``'s: a round takes 146 us at K = 5,120 and the groups no
+    less than their weights at 5.6 TB/s; the tiles of several heights that the products may take instead (``gemm_groups``) move both sides
+    by less than the margins.  Routers do not spread their rows quite evenly, and a round that the groups miss by a tile costs more
+    than is to be gained: with a standard deviation of tiles more they have to fit 85 % of their rounds, and the two to be 6 % faster
+    than all tiles together with a deviation fewer.
+    (Measured with whichever kernel each product then takes, at 420 sizes, 4 to 32 experts, 130 to 6,000 tokens: of the 30 that this takes
+    in 7 are 2 % and more slower apart, most of them by 7, on average they are 4 % faster; never apart loses 46 of the 420 to what
+    they took with gemm_tiled alone, this 30, and the estimates of those kernels, tried in its place, 36 to 49.  5,120 x 8,192 over 16
+    experts, together / apart: 1,547 tokens 428 / 360 us, 1,685 408 / 371, 2,048 462 / 433; over 8: 1,629 367 / 322, 1,743 360 / 339; 3,072
+    x 8,192 over 16: 3,192 401 / 378, over 32: 1,865 406 / 379.)  A gated product's rounds are many and its stream of weights long: there
+    it never paid (2,048 tokens 719 / 759)."""
     cus, round_us, cols = hipops.cu_count(), 146.0 * K / 5120.0, -(-N // 512)
     together = round_us * _rounds(tokens, groups, 1, cols, cus, deviations=-1.0)[1]
     shape, cost = _rounds(tokens, groups, 0, cols, cus, deviations=1.0, full=0.85)

@@ -10,6 +10,13 @@ def test_whole_group_apart():
     assert whole_group_apart(2048, 128, 5120, 8192) == 0
 
 
+def test_whole_group_apart_where_it_was_timed_beside_tiles_of_several_heights():
+    for tokens, groups, N, K in ((1522, 8, 5120, 8192), (1629, 8, 5120, 8192), (1743, 8, 5120, 8192), (1685, 16, 5120, 8192), (1865, 32, 3072, 8192)):
+        assert whole_group_apart(tokens, groups, N, K) == 1, (tokens, groups, N, K)
+    for tokens, groups, N, K in ((850, 4, 2048, 3072), (2048, 8, 2048, 8192), (1200, 4, 3072, 8192), (1000, 8, 5120, 8192), (2600, 16, 5120, 8192)):
+        assert whole_group_apart(tokens, groups, N, K) == 0, (tokens, groups, N, K)
+
+
 def test_lds_suits():
     from spite_amd.csrc.hipops import latent_splits, lds_suits, lds_suits_groups, tiled_k_runs
     faster = {(1547, 5120, 5120): True, (1786, 5120, 8192): True, (1531, 2048, 2048): True, (1024, 7168, 5120): True,
