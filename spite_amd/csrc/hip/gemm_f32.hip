@@ -39,8 +39,8 @@ __device__ __forceinline__ void f32_store(float* __restrict__ Y, size_t row, int
 }
 
 // HALVES (GLU, N a multiple of 8): a workgroup takes eight rows of each half, in one MFMA operand: twice as many workgroups, where
-// those of sixteen would be up to three a compute unit and some units have one more than others (2 x 3,072 x 2,048, two groups of a
-// row 27.3 -> 23.9 us, three 36.1 -> 31.5; five, 3.75 a unit, 46.2 with either).
+// those of sixteen are few or some compute units have one more than others (2 x 3,072 x 2,048, two groups of a row 27.3 -> 23.9 us, three 36.1 ->
+// 31.5; five, 3.75 a unit, 46.2 with either).
 template <int MT, int GLU, bool HALVES = false>
 __global__ __launch_bounds__(512)
 void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, long w_group_stride,
@@ -265,26 +265,41 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
     }
 }
 
-// Rows of X a workgroup takes: of gemm_f32_rows (16, 32 or 64), or minus those of gemm_f32_tile (32 or 64).  `n_groups` 0: no groups.
+// Rows of X a workgroup takes: of gemm_f32_rows (16, 32 or 64; 8: 16 rows, eight columns), or minus those of gemm_f32_tile (32 or
+// 64).  `n_groups` 0: no groups.
 //
-// Measured on an MI355X (us), products in a row over weights that the caches do not hold; "gate/up" 2 x 3,072 x 2,048 gated and
-// "down" 2,048 x 3,072 over 16 experts and a shared one, `t` tokens:
-//  * groups of up to eight rows on average: the stream of every group's W, 16 rows a workgroup, whatever the call's rows are
-//    (t = 16: gate/up 124, with 32 rows a workgroup 190; t = 32 169, with 64 rows 331, tiles of 32 211; t = 64 184 / tiles 207;
-//    the shared group's W comes from L2 for its further rows).
+// Both kernels take a time that follows from the most workgroups that a compute unit gets, c: for 2,048 of K, on an MI355X (us), the
+// stream of 16 rows 7 c (gated 11.5 c), tiles of 32 rows 14 + 19.5 c (14 + 47 c), of 64 17 + 36 c (19 + 82 c); the stream gives each
+// of its eight waves a run of 64 k and more, so that shorter sums than 512 leave some idle.  The lines lie where 14,900 products (1
+// to 1,500 tokens, up to 128 groups of 1 to 8 a token, K of 128 to 8,192) were timed with every variant:
+//  * groups of up to eight rows on average: the stream of every group's W, 16 rows a workgroup (16 groups and one of all t rows, 2 x
+//    3,072 x 2,048 gated: t = 16 124, with 32 rows a workgroup 190; t = 64 184 / tiles 207), but tiles of 32 rows where sums are
+//    short and tiles enough (K <= 512 and more than one a compute unit; plain K <= 1,024 and more than two: 129 groups x 2,048 x 768,
+//    535 rows, 151 / stream 233).  A group that holds most of the rows has its W read once every 16 of them, which the rule does not
+//    know (128 groups of one row a token and one of all, 2,048 x 2,048, t = 318: gated 2 x 2,048, t = 451, 881 / 887, but plain 449 /
+//    380).
 //  * no groups: the stream up to 64 rows, unless W is tall enough for two workgroups of tiles a compute unit (32,768 x 2,048: 9 rows
 //    54 with the stream, 48 with tiles of 32; 16: 64 / 49; 64: 198 / 98; 8 51 / 52; 3,072 x 2,048 stays, 64 rows 26 / 35).
-//  * tiles of 32 rows where those of 64 would be fewer than four a compute unit (3,072 x 2,048, 100 rows: 35 / 53, 301: 54 / 60;
-//    2,048 x 2,048, 200: 35 / 52; down, t = 200: 109 / 133; gate/up, t = 150: 214 / 237, but t = 200, over the line: 264 / 247;
-//    32,768 x 2,048, 100 rows, over the line: 188 / 168).
-static int f32_variant(int M, int N, int n_groups) {
-    const long cus = sp_cu_count(), cols = (N + 63) / 64;
-    if (n_groups && M <= 8L * n_groups && M / 16L + n_groups <= 65535) return 16;      // (the grid's limit)
-    if (M <= 64 && (n_groups || M <= 8 || cols * ((M + 31) / 32) < 2 * cus)) return M > 32 ? 64 : M > 16 ? 32 : 16;
-    const long tiles = (n_groups ? M / 64 + (n_groups < M ? n_groups : M) : (M + 63) / 64) * cols;
-    return tiles < 4 * cus ? -32 : -64;
+//  * more rows: tiles of 32 up to three of them a compute unit, gated two, with groups two and a quarter (3,072 x 2,048, 100 rows: 35
+//    / 53, 301: 54 / 60; 16,384 x 3,072, 186 rows, over the line, 215 / 191; gated 16,384 x 4,096, 78 rows, 346 / 255; gated, 8
+//    groups and one of all x 512 x 2,048, t = 212, 105 / 172), and where groups hold up to 20 rows, plain ones 160 (17 groups, 2 x
+//    3,072 x 2,048, t = 150 214 / 237, t = 200, over the line, 264 / 247); none past 128 a compute unit, more than was timed.
+//  * eight columns: up to a workgroup of sixteen a compute unit, up to three for K of 2,048 and more (3,072 x 2,048, two groups of a
+//    row 23.9 / 27.3; 5 rows x 6,144 x 768, over the line, 16.9 / 15.3).
+static int f32_variant(int M, int N, int K, int n_groups, int glu) {
+    const long cus = sp_cu_count(), cols = (N + 63) / 64, live = n_groups ? (n_groups < M ? n_groups : M) : 1, streams = (N + 15) / 16 * live;
+    const bool halves = glu && N % 8 == 0 && (streams <= cus || (streams <= 3 * cus && K >= 2048));
+    const bool few = n_groups && M > 16 && M <= 8L * n_groups;
+    const bool short_sum = (K <= 512 && live * cols > cus) || (!glu && K <= 1024 && live * cols > 2 * cus);
+    if (few && !short_sum && M / 16L + n_groups <= 65535) return halves ? 8 : 16;      // (the grid's limit)
+    if (!few && M <= 64 && (n_groups || M <= 8 || cols * ((M + 31) / 32) < 2 * cus)) return M > 32 ? 64 : M > 16 ? 32 : halves ? 8 : 16;
+    const double tiles = (n_groups ? M / 32.0 + 0.5 * live : (M + 31) / 32) * cols / cus;         // of 32 rows, a compute unit
+    if (tiles <= (!glu ? 3.0 : n_groups ? 2.25 : 2.0) || (!n_groups && M <= 64)) return -32;
+    return tiles <= 128.0 && (M <= 20L * n_groups || (!glu && M <= 160L * n_groups)) ? -32 : -64;
 }
-extern "C" int spite_gemm_f32_variant(int M, int N, int n_groups) { return f32_variant(M, N, n_groups); }
+extern "C" int spite_gemm_f32_choice(int M, int N, int K, int n_groups, int glu) { return f32_variant(M, N, K, n_groups, glu); }
+// Gated, K = 2,048: the rows alone.
+extern "C" int spite_gemm_f32_variant(int M, int N, int n_groups) { const int v = f32_variant(M, N, 2048, n_groups, 1); return v == 8 ? 16 : v; }
 
 // The product if its rows can be read 16 bytes at a time (returns 0, or an error), else 1: the plain kernel's.
 int sp_gemm_f32(const float* A, int lda, const float* W, long w_group_stride, float* Y, int ldy, int M, int N, int K,
@@ -292,7 +307,7 @@ int sp_gemm_f32(const float* A, int lda, const float* W, long w_group_stride, fl
                 float act_limit, hipStream_t st) {
     if (K % 4 || lda % 4 || w_group_stride % 4 || ((uintptr_t)A | (uintptr_t)W) % 16) return 1;
     const int vec_y = ldy % 4 == 0 && (uintptr_t)Y % 16 == 0;
-    const int variant = f32_variant(M, N, offsets ? n_groups : 0), tile = variant > 0 ? variant : -variant;
+    const int variant = f32_variant(M, N, K, offsets ? n_groups : 0, glu), tile = variant == 8 ? 16 : variant > 0 ? variant : -variant;
     const int m_tiles = offsets ? M / tile + (n_groups < M ? n_groups : M) : (M + tile - 1) / tile;
     SP_REQUIRE(m_tiles <= 65535, "gemm: too many row tiles (%d)", m_tiles);
 #define SP_F32_ARGS A, lda, W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, act_limit, vec_y
@@ -311,7 +326,7 @@ int sp_gemm_f32(const float* A, int lda, const float* W, long w_group_stride, fl
     dim3 grid((N + 15) / 16, m_tiles);
 #define SP_F32_ROWS(MT) do { if (glu) gemm_f32_rows_kernel<MT, 1><<<grid, 512, 0, st>>>(SP_F32_ARGS); \
                              else gemm_f32_rows_kernel<MT, 0><<<grid, 512, 0, st>>>(SP_F32_ARGS); } while (0)
-    if (tile == 16 && glu && N % 8 == 0 && (long)((N + 15) / 16) * (offsets ? (n_groups < M ? n_groups : M) : 1) <= 3L * sp_cu_count())
+    if (variant == 8)
         gemm_f32_rows_kernel<1, 1, true><<<dim3(N / 8, m_tiles), 512, 0, st>>>(SP_F32_ARGS);
     else if (tile == 16) SP_F32_ROWS(1);
     else if (tile == 32) SP_F32_ROWS(2);

@@ -128,6 +128,8 @@ def lib():
         l.spite_gemm_groups_choice.restype = c_int
         l.spite_gemm_f32_variant.argtypes = [I, I, I]
         l.spite_gemm_f32_variant.restype = c_int
+        l.spite_gemm_f32_choice.argtypes = [I] * 5
+        l.spite_gemm_f32_choice.restype = c_int
         l.spite_gemm_lds_time.argtypes = [I, I, I, I]
         l.spite_gemm_lds_time.restype = ctypes.c_double
         l.spite_cu_count.argtypes = []

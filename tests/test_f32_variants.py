@@ -13,6 +13,15 @@ def test_lines_lie_where_both_sides_were_timed():
     assert [at(m, 3072, 0) for m in (16, 17, 64, 65, 301)] == [16, 32, 64, -32, -32]
     assert at(400000, 64, 50000) == -64 and at(64, 64, 2) == 64
 
+    at = lib().spite_gemm_f32_choice             # 8: a workgroup takes eight columns of each half
+    assert [at(2 * t, 2048, k, 129, 0) for t in (107, 267) for k in (768, 1024, 1536)] == [-32, -32, 16] * 2
+    assert [at(120, 1024, k, 33, 1) for k in (512, 768)] == [-32, 16] and at(20, 256, 512, 4, 1) == 8
+    assert [at(m, 16384, 2048, 0, 1) for m in (64, 65, 166)] == [-32, -64, -64]
+    assert [at(m, 16384, 2048, 0, 0) for m in (65, 96, 97, 186)] == [-32, -32, -64, -64]
+    assert [at(m, 6144, 2048, 0, 1) for m in (158, 161)] == [-32, -64]
+    assert [at(1908, 512, 2048, 9, g) for g in (0, 1)] == [-32, -32] and at(3000, 1536, 2048, 65, 1) == -64
+    assert [at(1, 6144, k, 0, 1) for k in (512, 2047, 2048)] == [16, 16, 8] and at(1, 4096, 128, 0, 1) == 8 and at(1, 4100, 2048, 0, 1) == 16
+
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,groups", [(200, 40), (70, 5), (300, 5), (40, 3)])
