@@ -356,7 +356,8 @@ extern "C" int spite_add_rmsnorm(float* h, const float* d1, const float* d2, con
     SP_REQUIRE(!proj || (proj_out && P > 0), "add_rmsnorm: a projection needs its output and size");
     SP_REQUIRE(!expert || (proj && n_rows <= 1 && P < 65535 && shared >= 0 && shared <= 64 && weight && src && scale && dst && offsets),
                "add_rmsnorm: a plan of %d rows, %d experts, %d shared groups", n_rows, P, shared);
-    const norm_args p{h, d1, d2, w, out32, rows, n_rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain_out, w2,
+    const int plain = plain_out || !w;                       // (the second output alone: the kernels read no w that is not there)
+    const norm_args p{h, d1, d2, w, out32, rows, n_rows, d, eps, write_h, proj, proj_out, P, dn, wn, mult, eps_n, plain, w2,
                       norm_plan{expert, weight, src, scale, dst, offsets, shared}};
     size_t sh = proj ? (size_t)((expert ? ((d + 3) & ~3) + P : d)) * sizeof(float) : 0;
     SP_REQUIRE(sh <= 48 * 1024, "add_rmsnorm: rows of %d do not fit the projection's LDS", d);

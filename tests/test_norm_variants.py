@@ -55,3 +55,13 @@ def test_a_row_alone_and_among_many(d, rows, P, dtype):
     if P:
         ref = (want * w.double()) @ proj.double().T
         assert ((got[4].double() - ref).abs() <= 4e-6 * d ** 0.5 * ref.abs().max()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,rows", [(2048, 3), (2046, 3), (12288, 300)])
+def test_the_second_output_alone_needs_no_first_weight(d, rows):
+    h, w, w2 = rnd(rows, d), rnd(d, seed=1) + 2.0, rnd(d, seed=2) + 2.0
+    got, both, out = (torch.empty(rows, d, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    ops().add_rmsnorm(h, None, 1e-5, w2=w2, out2=got)
+    ops().add_rmsnorm(h, w, 1e-5, out=out, w2=w2, out2=both)
+    assert torch.equal(got, both)
