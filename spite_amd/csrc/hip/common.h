@@ -148,13 +148,17 @@ __device__ __forceinline__ void sp_rotate(float a, float b, float cs, float sn, 
 }
 
 // ------------------------------------------------------------------ a wave's fp32 dot product
-// sum_c w[c] * xs[c] over a row xs in LDS, by one wave: lane l takes the 16-byte groups l, l+64,
-// ... and the lanes' sums meet in a butterfly.  Every kernel that forms router logits calls
-// this, so a logit has the same bits wherever it is computed; its order of summation depends
-// on the width alone.
+// Four terms of a router logit, one rounded product and three fused multiply-adds, and their addition to the lane's sum, written
+// out: the compiler might join products and sums one way in one kernel and another way in the next.
 __device__ __forceinline__ float dot4_add(float acc, const f32x4& w, const f32x4& x) {
-    return acc + (w[0] * x[0] + w[1] * x[1] + w[2] * x[2] + w[3] * x[3]);
+#pragma clang fp contract(off)
+    return acc + fmaf(w[3], x[3], fmaf(w[2], x[2], fmaf(w[0], x[0], w[1] * x[1])));
 }
+// sum_c w[c] * xs[c] over a row xs in LDS, by one wave: lane l takes the 16-byte groups l, l+64,
+// ... and the lanes' sums meet in a butterfly.  A kernel that forms router logits calls this, or, where
+// it takes several rows at once (add_rmsnorm's 16-byte rows, router_top1's four tokens), goes through the same groups
+// in the same order with dot4_add and ends in the same butterfly: a logit has the same bits wherever it is
+// computed; its order of summation depends on the width alone.
 __device__ __forceinline__ float wave_dot_row(const float* __restrict__ w, const float* xs, int d, bool vec, int lane) {
     float acc = 0.f;
     if (vec) {

@@ -49,8 +49,6 @@ extern "C" int spite_embed(const int* ids, const void* table, int dtype, float* 
     return 0;
 }
 
-// (a wave's fp32 dot product, wave_dot_row, is in common.h: every kernel that forms router logits calls it)
-
 // The index of the largest logit, the lowest among equals, and (if asked for) the logit.
 __device__ __forceinline__ int top1_of(const float* __restrict__ l, int E, float* best_out) {
     float best = -INFINITY; int best_e = 0;
@@ -787,7 +785,7 @@ void router_top1_kernel(const float* __restrict__ x, const float* __restrict__ w
 #pragma unroll
                 for (int u = 0; u < TB; ++u) {
                     const f32x4 xx = ((const f32x4*)(xs + (size_t)u * d))[c];
-                    acc[u] += ww[0] * xx[0] + ww[1] * xx[1] + ww[2] * xx[2] + ww[3] * xx[3];
+                    acc[u] = dot4_add(acc[u], ww, xx);
                 }
             }
         } else {

@@ -65,3 +65,19 @@ def test_the_second_output_alone_needs_no_first_weight(d, rows):
     ops().add_rmsnorm(h, None, 1e-5, w2=w2, out2=got)
     ops().add_rmsnorm(h, w, 1e-5, out=out, w2=w2, out2=both)
     assert torch.equal(got, both)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("d,P", [(516, 17), (2048, 17), (2048, 130), (5120, 64), (5120, 130), (8192, 16), (9216, 5)])
+@pytest.mark.parametrize("rows", [1, 255, 256, 331])
+def test_logits_are_the_routers(d, P, rows):
+    """Two rows of the projection a wave, two rows a workgroup, four tokens a workgroup of the router (from 256 on), and one."""
+    h, w, proj = rnd(rows, d), rnd(d, seed=1) + 2.0, rnd(P, d, seed=2)
+    out32, logits, again = torch.empty(rows, d, device=DEV), torch.empty(rows, P, device=DEV), torch.empty(rows, P, device=DEV)
+    ops().add_rmsnorm(h, w, 1e-5, out32=out32, proj=proj, proj_out=logits)
+    expert, weight = torch.empty(rows, dtype=torch.int32, device=DEV), torch.empty(rows, device=DEV)
+    ops().router_top1(out32, proj, expert, weight, again)
+    assert torch.equal(logits, again)
+    exact, size = out32.double() @ proj.double().T, out32.double().abs() @ proj.double().abs().T
+    # a lane adds d/256 fours of four roundings each, then six steps of the butterfly
+    assert ((logits.double() - exact).abs() <= (d / 256 + 11) * 2.0 ** -24 * size).all()
