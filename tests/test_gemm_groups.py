@@ -96,3 +96,20 @@ def test_choice_against_the_product_that_would_run_otherwise():
         assert at(*in_lds, lds=True) is None, in_lds
     assert at(2048, 16, 1, 1, 8192, 5120, True) == (8, 160) and at(1531, 16, 4, 2, 1024, 2048, True) == (4, 128)
     assert at(126, 4, 4, 1, 5120, 16384, True) == (4, 128) and at(1483, 32, 8, 1, 768, 16384, False) == (8, 128)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("waves,cap", [(4, 128), (4, 160), (8, 128), (8, 160)])
+def test_row_lists_scales_and_scattered_rows_equal_the_tiled_product(glu, out_dtype, waves, cap):
+    M, N, K, G = sum(HEIGHTS), 272, 192, len(HEIGHTS)
+    g = torch.Generator().manual_seed(3)
+    a, w = rnd(M + 3, K, dtype=torch.bfloat16), ops().operand_order(rnd(G, 2 * N if glu else N, K, dtype=torch.bfloat16, seed=1))
+    kw = dict(offsets=torch.tensor([sum(HEIGHTS[:g]) for g in range(G + 1)], dtype=torch.int32, device=DEV), n_groups=G, glu=glu,
+              a_rows=torch.randint(0, M + 3, (M,), generator=g).to(torch.int32).to(DEV), a_scale=(torch.rand(M, generator=g) + 0.5).to(DEV),
+              y_rows=torch.randperm(M + 2, generator=g)[:M].to(torch.int32).to(DEV))
+    y, z = torch.zeros(M + 2, N, dtype=out_dtype, device=DEV), torch.zeros(M + 2, N, dtype=out_dtype, device=DEV)
+    ops().gemm_tiled(a, w, y, M, N, K, shape=1, **kw)
+    ops().gemm_groups(a, w, z, M, N, K, waves=waves, cap=cap, **kw)
+    assert torch.equal(y, z)

@@ -84,3 +84,28 @@ def test_many_rows_take_runs_where_that_was_faster():
         assert at(M, N, K) is None, (M, N, K)
     for M, N, K, runs in ((900, 1024, 5120, 5), (1531, 576, 5120, 5), (1200, 2048, 4096, 4), (800, 5120, 5120, 2)):
         assert at(M, N, K)[0] == runs, (M, N, K, at(M, N, K))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(65, 64, 768), (40, 32768, 832), (40, 5184, 5120), (100, 272, 1472)])
+@pytest.mark.parametrize("out_dtype", [torch.bfloat16, torch.float32])
+def test_linear_takes_the_runs(M, N, K, out_dtype, monkeypatch):
+    """One run and several, with the partial sums from a workspace and without one, against float64."""
+    from spite_amd.parts import linear as parts
+    seen, inner = [], ops().gemm_runs
+    monkeypatch.setattr(parts.hipops, "gemm_runs", lambda *a, **kw: (seen.append((kw["runs"], kw["part"])), inner(*a, **kw)))
+
+    class Taken(list):
+        def take(self, shape, dtype):
+            self.append(torch.full(shape, float("nan"), dtype=dtype, device=DEV))
+            return self[-1]
+    x, w = rnd(M, K, dtype=torch.bfloat16), rnd(N, K, dtype=torch.bfloat16, seed=1)
+    y, z, ws = torch.empty(M, N, dtype=out_dtype, device=DEV), torch.empty(M, N, dtype=out_dtype, device=DEV), Taken()
+    parts.linear(x, parts.Weight(w), y, ws=ws)
+    parts.linear(x, parts.Weight(w), z)
+    runs = ops().gemm_runs_choice(M, N, K)[0]
+    assert [r for r, _ in seen] == [runs] * 2 and (runs == 1) == (N == 32768) and [tuple(t.shape) for t in ws] == [(runs, M, N)] * (runs > 1)
+    assert torch.equal(y, z) and (runs == 1 or seen[0][1] is ws[0])
+    exact, size = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
+    last = 2.0 ** -8 if out_dtype == torch.bfloat16 else 0.0
+    assert ((y.double() - exact).abs() <= size * K * 2.0 ** -24 + exact.abs() * last).all()
