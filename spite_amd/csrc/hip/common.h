@@ -138,6 +138,15 @@ __device__ __forceinline__ float block_sum(float v, float* red) {
     return t;
 }
 
+// ------------------------------------------------------------------ loads straight to LDS
+// 16 bytes a lane from the buffer (a resource descriptor) at voff + soff to LDS at lds + lane * 16 (written out: the compiler would
+// wait for every such load before any read of LDS; the waits are the kernel's own).
+template <typename BUF>
+__device__ __forceinline__ void sp_load_lds(BUF buf, int voff, int soff, unsigned lds) {
+    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
+                 :: "v"(voff), "s"(buf), "s"(soff), "s"(lds) : "memory", "m0");
+}
+
 // ------------------------------------------------------------------ rotation of a pair
 // (a cos - b sin, b cos + a sin) with one rounded product and one fused multiply-add each, written out: left to the
 // compiler, which product is fused depends on the code around it, and a key would round one way when a prompt writes it and

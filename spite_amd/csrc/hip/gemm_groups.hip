@@ -20,10 +20,10 @@
 // The sum over k runs in the order of gemm_tiled and gemm_lds: the same bits.
 //
 // Measured on an MI355X against gemm_tiled's best tile (us; 16 experts of which a token takes `top`, beside them one or two
-// groups of every token): 2,048 tokens x 2 x 8,192 x 5,120 gated 639 / 722, 1,547 553 / 656, 330 453 / 476; 1,786, top 2,
-// 2 x 4,096 x 5,120 548 / 653; 1,531, top 4, 2 x 1,024 x 2,048 80 / 109; 1,200 x 2,048 x 3,072 57 / 70; over 220 sizes of 4 to 128
-// groups and 65 to 6,000 tokens 0.86 of the time on average.  At 2,048 tokens what bounds it is the power limit (the clock falls
-// to 1.6 GHz with the matrix units half busy), at 330 the stream of W (6.3 TB/s).
+// groups of every token): 2,048 tokens x 2 x 8,192 x 5,120 gated 640 / 718, 1,547 579 / 630, 330 444 / 481; 1,786, top 2,
+// 2 x 4,096 x 5,120 550 / 590; 1,531, top 4, 2 x 1,024 x 2,048 79 / 108; 1,200 x 2,048 x 3,072 59 / 74; but 1,512 x 3,072 x 2,048, which
+// stays with gemm_tiled, 67 / 60.  At 2,048 tokens what bounds it is the power limit (the clock falls to 1.6 GHz with the matrix units
+// half busy), at 330 the stream of W (6.4 TB/s).
 #include <math.h>
 #include "common.h"
 
@@ -34,12 +34,6 @@ struct gg_args {
 };
 #define GG_PAST ((int)0x80000000)      // an offset beyond every buffer's end: loads give zeros
 
-// 16 bytes a lane from the buffer at voff + soff to LDS at lds + lane * 16 (written out: the compiler would wait for every such
-// load before any read of LDS; the waits are the kernel's own)
-__device__ __forceinline__ void gg_load_lds(__amdgpu_buffer_rsrc_t buf, int voff, int soff, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :: "v"(voff), "s"(buf), "s"(soff), "s"(lds) : "memory", "m0");
-}
 // A buffer of 2 GiB from p on (the operands' offsets are checked on the host), p the same in every lane.
 __device__ __forceinline__ __amdgpu_buffer_rsrc_t gg_buffer(const void* p) {
     const uint64_t a = (uint64_t)(uintptr_t)p;
@@ -79,7 +73,7 @@ __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, in
     auto load_x = [&](int u) {
         const int k0 = (u_first + (u < nu ? u : 0)) * 128, past = u < nu ? 0 : GG_PAST;
 #pragma unroll
-        for (int i = 0; i < XI; ++i) gg_load_lds(xbuf, xoff[i] | past, __builtin_amdgcn_readfirstlane(k0), lds0 + (u & 3) * XB + xblk[i] * 1024);
+        for (int i = 0; i < XI; ++i) sp_load_lds(xbuf, xoff[i] | past, __builtin_amdgcn_readfirstlane(k0), lds0 + (u & 3) * XB + xblk[i] * 1024);
     };
     auto load_w = [&](bf16x8 (&ws)[4], int t) {
         const int at = (t < kt ? t : 0) * 1024, past = t < kt ? 0 : GG_PAST;
@@ -265,6 +259,7 @@ static int gg_launch(gg_args p, hipStream_t st) {
 // Measured on an MI355X against the best of gemm_tiled (its runs of 128 x 512), gemm_lds and, up to 64 rows, gemm_skinny, launches in
 // a row over weights that the caches do not hold, with the sum of the runs (us): 64 x 32,768 x 5,120 62 / 119, 64 x 5,120 x 8,192
 // 26 / 34, 80 x 7,168 x 5,120 26 / 34, 330 39 / 55, 500 x 5,120 x 5,120 39 / 55, 500 x 2,048 x 2,048 23 / 30, 1,531 x 576 x 5,120 27 / 37.
+// (W's loads are non-temporal however many row tiles read it; cached ones were not timed there.)
 template <int NB, int S, typename TY>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 void gemm_runs_kernel(gg_args p, int runs) {
@@ -472,7 +467,7 @@ static double gg_estimate(int kind, int tokens, int routed, double mean, int who
 // estimated within 2 % of the best of them.  us[0]: what the taken one is estimated to take.  Over those products the choice is 18 %
 // faster than the others on average; at 93 it is 2 % and more slower, at 43 of them by 5 % and more (a quarter of those where one
 // group took a quarter of the rows, which the estimate cannot know).  16 experts and a shared one: 1,547 tokens x 2 x 8,192 x 5,120
-// gated tiles of eight waves (553 us, gemm_tiled 656), 1,512 x 3,072 x 2,048 stays (gemm_groups 71, gemm_tiled 61).
+// gated tiles of eight waves (579 us, gemm_tiled 630), 1,512 x 3,072 x 2,048 stays (gemm_groups 67, gemm_tiled 60).
 extern "C" int spite_gemm_groups_choice(int tokens, int routed, double mean, int whole, int N, int K, int glu, int shape, int lds, double* us) {
     *us = 0.0;
     if (tokens <= 0 || routed <= 0 || mean <= 0.0) return 0;

@@ -38,12 +38,6 @@ __device__ __forceinline__ i32x4 gl_buffer(const void* p) {
     r[3] = 0x00020000;
     return r;
 }
-// 16 bytes a lane from the buffer at voff + soff to LDS at lds + lane * 16.  (Written out so that the compiler, which does not
-// know which buffer of LDS a later read touches, does not wait for every load before it; the waits are the kernel's own.)
-__device__ __forceinline__ void gl_load(i32x4 buf, int voff, int soff, unsigned lds) {
-    asm volatile("s_mov_b32 m0, %3\n\ts_nop 0\n\tbuffer_load_dwordx4 %0, %1, %2 offen lds"
-                 :: "v"(voff), "s"(buf), "s"(soff), "s"(lds) : "memory", "m0");
-}
 
 struct gl_args {
     const bf16* X; int ldx; const bf16* W; long w_group_stride; void* Y; int ldy, M, N, K;
@@ -86,12 +80,12 @@ __device__ __forceinline__ void gl_tile(const gl_args& a, unsigned char* lds, co
     auto load_x = [&](int v, int xb) {
         const int k = (v < nu ? v : nu - 1) * 128;
 #pragma unroll
-        for (int i = 0; i < XI; ++i) gl_load(xbuf, xoff[i], k, lds0 + xb * XB + xblk[i] * 1024);
+        for (int i = 0; i < XI; ++i) sp_load_lds(xbuf, xoff[i], k, lds0 + xb * XB + xblk[i] * 1024);
     };
     auto load_w = [&](int t) {
         const int k = (t < kt ? t : kt - 1) * 1024;
 #pragma unroll
-        for (int i = 0; i < WI; ++i) gl_load(wbuf, wvoff, wbase[i] + k, lds0 + 3 * XB + (t & 3) * GL_WB + (wave * WI + i) * 1024);
+        for (int i = 0; i < WI; ++i) sp_load_lds(wbuf, wvoff, wbase[i] + k, lds0 + 3 * XB + (t & 3) * GL_WB + (wave * WI + i) * 1024);
     };
     f32x4 acc[4][NB];
 #pragma unroll

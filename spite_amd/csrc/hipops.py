@@ -760,7 +760,9 @@ def lds_suits_groups(group_rows: float, K: int, tiles: int = 0, lds_tiles: int =
     """The same for a product over groups of ``group_rows`` rows each on average (beside groups that take every row), which
     are to be ``tiles`` tiles of ``gemm_tiled`` and ``lds_tiles`` of ``gemm_lds``: where the first ones leave three of eight
     compute units and more without a tile and the others, half as wide, still fit one round.  With more tiles the 256
-    rows of W a tile ask for more operands a product than the 512 of ``gemm_tiled`` do.  (Timed at 520 products of 2 to 128
+    rows of W a tile ask for more operands a product than the 512 of ``gemm_tiled`` do.  Of the products that this takes in,
+    plain ones and those gated with silu are weighed once more, against the tiles of several heights (``gemm_groups_choice``); other
+    gates, an activation and rows that 16-byte stores cannot take stay.  (Timed against ``gemm_tiled`` at 520 products of 2 to 128
     groups of 60 to 4,000 rows; us with gemm_lds / gemm_tiled.  One round: 384 rows x 2 x 2,048 x 7,168, 140 / 192; 308 x 2 x
     2,048 x 4,096 75 / 96; the 48 that the line takes in at any rows a group are 15 % faster on average, one of them 2 % slower.
     More: 32 groups of 128 rows 822 / 720; 8 of 165 346 / 252; 16 of 415 586 / 539; 4 of 1,152, unevenly, 152 / 104.  Sums

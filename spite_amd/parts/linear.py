@@ -67,9 +67,11 @@ TILE_160_COST = 1.16
 
 
 def grouped_tile_shape(tokens: int, groups: int, whole_groups: int = 0, col_tiles: int = 0, cus: int = 0) -> int:
-    """Which tile of the prefill product suits ``tokens`` rows that spread evenly over ``groups``
+    """Which tile of ``gemm_tiled`` suits ``tokens`` rows that spread evenly over ``groups``
     groups (experts that a router picks), beside ``whole_groups`` groups that take every row.
-    A group costs whole row tiles, each of which streams the group's weights once.
+    A group costs whole row tiles, each of which streams the group's weights once.  (The product
+    then takes that tile only where ``linear`` estimates no other kernel to be the faster one:
+    ``hipops.gemm_groups_choice`` weighs the tiles of several heights against it.)
 
     * Few rows a group and few groups (a short prompt over a few experts): the time is the stream
       of the weights from memory and there are too few workgroups to keep it busy; the 64-row
