@@ -274,10 +274,10 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
 // to 1,500 tokens, up to 128 groups of 1 to 8 a token, K of 128 to 8,192) were timed with every variant:
 //  * groups of up to eight rows on average: the stream of every group's W, 16 rows a workgroup (16 groups and one of all t rows, 2 x
 //    3,072 x 2,048 gated: t = 16 124, with 32 rows a workgroup 190; t = 64 184 / tiles 207), but tiles of 32 rows where sums are
-//    short and tiles enough (K <= 512 and more than one a compute unit; plain K <= 1,024 and more than two: 129 groups x 2,048 x 768,
-//    535 rows, 151 / stream 233).  A group that holds most of the rows has its W read once every 16 of them, which the rule does not
-//    know (128 groups of one row a token and one of all, 2,048 x 2,048, t = 318: gated 2 x 2,048, t = 451, 881 / 887, but plain 449 /
-//    380).
+//    short and tiles enough (K <= 512 and more than one a compute unit; plain K < 2,048 and more than two: 129 groups x 2,048 x 768,
+//    535 rows, 151 / stream 233; 128 x 4,096 x 1,536, 885 rows, 567 / 794; at K = 2,048 either is as fast).  A group that holds most of
+//    the rows has its W read once every 16 of them, which the rule does not know (128 groups of one row a token and one of all, 2,048 x
+//    2,048: gated t = 451 881 / 887, but plain t = 318 449 / 380).
 //  * no groups: the stream up to 64 rows, unless W is tall enough for two workgroups of tiles a compute unit (32,768 x 2,048: 9 rows
 //    54 with the stream, 48 with tiles of 32; 16: 64 / 49; 64: 198 / 98; 8 51 / 52; 3,072 x 2,048 stays, 64 rows 26 / 35).
 //  * more rows: tiles of 32 up to three of them a compute unit, gated two, with groups two and a quarter (3,072 x 2,048, 100 rows: 35
@@ -290,7 +290,7 @@ static int f32_variant(int M, int N, int K, int n_groups, int glu) {
     const long cus = sp_cu_count(), cols = (N + 63) / 64, live = n_groups ? (n_groups < M ? n_groups : M) : 1, streams = (N + 15) / 16 * live;
     const bool halves = glu && N % 8 == 0 && (streams <= cus || (streams <= 3 * cus && K >= 2048));
     const bool few = n_groups && M > 16 && M <= 8L * n_groups;
-    const bool short_sum = (K <= 512 && live * cols > cus) || (!glu && K <= 1024 && live * cols > 2 * cus);
+    const bool short_sum = (K <= 512 && live * cols > cus) || (!glu && K < 2048 && live * cols > 2 * cus);
     if (few && !short_sum && M / 16L + n_groups <= 65535) return halves ? 8 : 16;      // (the grid's limit)
     if (!few && M <= 64 && (n_groups || M <= 8 || cols * ((M + 31) / 32) < 2 * cus)) return M > 32 ? 64 : M > 16 ? 32 : halves ? 8 : 16;
     const double tiles = (n_groups ? M / 32.0 + 0.5 * live : (M + 31) / 32) * cols / cus;         // of 32 rows, a compute unit

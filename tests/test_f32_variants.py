@@ -14,7 +14,7 @@ def test_lines_lie_where_both_sides_were_timed():
     assert at(400000, 64, 50000) == -64 and at(64, 64, 2) == 64
 
     at = lib().spite_gemm_f32_choice             # 8: a workgroup takes eight columns of each half
-    assert [at(2 * t, 2048, k, 129, 0) for t in (107, 267) for k in (768, 1024, 1536)] == [-32, -32, 16] * 2
+    assert [at(2 * t, 2048, k, 129, 0) for t in (107, 267) for k in (768, 1024, 1536, 2048)] == [-32, -32, -32, 16] * 2
     assert [at(120, 1024, k, 33, 1) for k in (512, 768)] == [-32, 16] and at(20, 256, 512, 4, 1) == 8
     assert [at(m, 16384, 2048, 0, 1) for m in (64, 65, 166)] == [-32, -64, -64]
     assert [at(m, 16384, 2048, 0, 0) for m in (65, 96, 97, 186)] == [-32, -32, -64, -64]
