@@ -24,6 +24,8 @@
 #include "common.h"
 #include "no_alloc.h"
 
+typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+
 // What the fused form does before the attention, for rows [q | k | v] of the projection: see the kernel.
 struct ad_rope {
     const float* inv_freq;            // [HD / 2], or null: no rotation
@@ -50,14 +52,15 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
     constexpr int NC = HD / 32;      // 32-wide chunks of the head for the score product
     constexpr int ND = VD / 16;      // 16-row tiles of the output
     constexpr int ROW = VD + 2;      // partial record: output, max, sum
-    extern __shared__ float sm[];    // [4 waves][QH heads][ROW]
+    extern __shared__ __align__(16) float sm[];    // [4 waves][QH heads][ROW]
     const int split = blockIdx.x, g = blockIdx.y, t = blockIdx.z;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int n = lane & 15, qd = lane >> 4;
     const int QH = H / G;
-    const int p = positions[t];
+    int p = positions[t], seq = seq_of_token[t];
+    asm volatile("" : "+s"(p), "+s"(seq));               // (both asked for at once)
     const int lo = sp_first_visible(p, vis, span);
-    const int* bt = block_table + (size_t)seq_of_token[t] * max_blocks;
+    const int* bt = block_table + (size_t)seq * max_blocks;
     // a bias slope * (key - query position) on the scaled score of head n, as an addend of the raw score
     const float slope = (slopes && n < QH) ? slopes[g * QH + n] * inv_scale : 0.f;
 
@@ -75,51 +78,101 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
     const int re = (rb + per < nblk) ? rb + per : nblk;
 
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
+    // Block i of the split, its page and first key, and its keys and values on their way.
+    int key0 = 0, page = 0;
+    bf16x8 kf[2][NC];
+    u32x4 vf[ND];                    // (pairs of values: they are masked as such)
+#pragma unroll
+    for (int c = 0; c < 2 * NC; ++c) kf[c & 1][c >> 1] = zero8;
+#pragma unroll
+    for (int d = 0; d < ND; ++d) vf[d] = u32x4{0, 0, 0, 0};
+    auto find_block = [&](int i) {
+        key0 = (i < b_kept ? i : b_first + (i - b_kept)) * 32;
+        page = bt[key0 / ps];
+    };
+    auto load_block = [&]() {
+        const size_t pg = (size_t)(page < 0 ? 0 : page) * G + g;
+        const int blk = key0 % ps >> 5;                              // the block of 32 keys inside the page
+        const bf16* kbase = k_pages + pg * ps * HD + (size_t)blk * 2 * NC * 512 + lane * 8;
+        // (value heads may be fewer than key heads: key head g reads value head g % Gv)
+        const bf16* vbase = v_pages + ((size_t)(page < 0 ? 0 : page) * Gv + g % Gv) * VD * ps + (size_t)blk * ND * 512 + lane * 8;
+#pragma unroll
+        for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+                kf[tt][c] = __builtin_nontemporal_load((const bf16x8*)(kbase + (tt * NC + c) * 512));
+#pragma unroll
+        for (int d = 0; d < ND; ++d) vf[d] = __builtin_nontemporal_load((const u32x4*)(vbase + d * 512));
+    };
+    int i = rb + wave;
     bf16x8 qf[NC];
+    // the fused form's own key and value, for the wave that reads their block
+    bf16* own = (bf16*)(sm + HD);                        // [HD] rotated key, [VD] value, behind the sines
+    int own_slot = -1;
     if constexpr (FUSE) {
+        // Everything that is read is asked for before the sines and the barrier, the first block of keys and values too
+        // (the token's own key in it is a stale one, replaced in registers below): one trip to memory where there were four in a row.
+        // With the join's loads taken together, a layer's attention in us before and now (40 heads over 8): 8 tokens of 4,096 keys
+        // 29.7 / 27.8, 16 of 1,211 22.9 / 20.2, 32 of 300 13.8 / 12.7, 64 of 1,000 51.2 / 48.7, one of 14,000 19.8 / 18.4; one of 1,000
+        // and fewer 9.2 / 9.3, most of it the sines and the query's norm.
         const bf16* row = q + (size_t)t * (H + 2 * G) * HD;
+        const bf16* qr = row + (size_t)(g * QH + (n < QH ? n : 0)) * HD + qd * 8;
+        bf16x8 qlo[NC / 2], qhi[NC / 2];
+#pragma unroll
+        for (int c = 0; c < NC / 2; ++c) { qlo[c] = *(const bf16x8*)(qr + c * 32); qhi[c] = *(const bf16x8*)(qr + c * 32 + HD / 2); }
+        const bool mine = rb < re && re == nblk;         // (one workgroup of the splits has the last block)
+        const int slot = rope.slot_map[t];
+        const bf16* kr = row + (size_t)(H + g) * HD + (HD == 64 ? lane & 31 : lane);
+        const bf16* vr = row + (size_t)(H + G + g) * HD + lane;
+        bf16 kx = kr[0], ky = kr[HD / 2], v0 = vr[0], v1 = vr[VD - 64];
         float* cs = sm;                                  // [HD / 2] pairs (cosine, sine)
+        float freq = rope.inv_freq ? rope.inv_freq[threadIdx.x & (HD / 2 - 1)] : 0.f;
+        if (i < re) find_block(i);
+        // these are there before the long loads go out: a wait for them would be one for those too
+#pragma unroll
+        for (int c = 0; c < NC / 2; ++c) asm volatile("" : "+v"(qlo[c]), "+v"(qhi[c]));
+        asm volatile("" : "+v"(kx), "+v"(ky), "+v"(v0), "+v"(v1), "+v"(freq), "+s"(page));
+        if (i < re) load_block();
         if (threadIdx.x < HD / 2) {
             float sn = 0.f, c = 1.f;
-            if (rope.inv_freq) sincosf((float)p * rope.inv_freq[threadIdx.x], &sn, &c);
+            if (rope.inv_freq) sincosf((float)p * freq, &sn, &c);
             cs[2 * threadIdx.x] = c;
             cs[2 * threadIdx.x + 1] = sn;
         }
         __syncthreads();
-        const int slot = rope.slot_map[t];
-        if (rb < re && re == nblk && slot >= 0) {        // (one workgroup of the splits)
-            const int page = slot / ps, off = slot % ps;
+        if (mine && slot >= 0) {
+            own_slot = slot;
+            const int at = slot / ps, off = slot % ps;
             if (wave == 0) {
-                const bf16* kr = row + (size_t)(H + g) * HD;
-                bf16* kp = k_pages + ((size_t)page * G + g) * ps * HD;
+                bf16* kp = k_pages + ((size_t)at * G + g) * ps * HD;
                 float a = 0.f, b = 0.f;
-                if (lane < HD / 2) {
-                    const float x = (float)kr[lane], y = (float)kr[lane + HD / 2], c = cs[2 * lane], sn = cs[2 * lane + 1];
-                    sp_rotate(x, y, c, sn, a, b);
-                }
+                if (lane < HD / 2) sp_rotate((float)kx, (float)ky, cs[2 * lane], cs[2 * lane + 1], a, b);
                 const float ss = wave_sum(a * a + b * b);
                 const float scale = rope.norm_eps > 0.f ? 1.0f / sqrtf(ss / (float)HD + rope.norm_eps) : 1.0f;
                 if (lane < HD / 2) {
+                    own[lane] = (bf16)(a * scale);
+                    own[lane + HD / 2] = (bf16)(b * scale);
                     kp[sp_k_index(off, lane, HD, true)] = (bf16)(a * scale);
                     kp[sp_k_index(off, lane + HD / 2, HD, true)] = (bf16)(b * scale);
                 }
             } else if (wave == 1) {
-                const bf16* vr = row + (size_t)(H + G + g) * HD;
-                bf16* vp = v_pages + ((size_t)page * G + g) * ps * VD;
-                for (int c = lane; c < VD; c += 64) vp[sp_v_index(c, off, VD, ps, true)] = vr[c];
+                bf16* vp = v_pages + ((size_t)at * G + g) * ps * VD;
+                own[HD + lane] = v0;
+                vp[sp_v_index(lane, off, VD, ps, true)] = v0;
+                if (VD > 64) {
+                    own[HD + lane + 64] = v1;
+                    vp[sp_v_index(lane + 64, off, VD, ps, true)] = v1;
+                }
             }
         }
         // the queries: element c * 32 + qd * 8 + e turns with the one HD / 2 further on, which this lane holds as well
-        const bf16* qr = row + (size_t)(g * QH + (n < QH ? n : 0)) * HD + qd * 8;
         float x[NC][8], ss = 0.f;
 #pragma unroll
         for (int c = 0; c < NC / 2; ++c) {
-            const bf16x8 lo = *(const bf16x8*)(qr + c * 32), hi = *(const bf16x8*)(qr + c * 32 + HD / 2);
 #pragma unroll
             for (int e = 0; e < 8; ++e) {
-                const int i = c * 32 + qd * 8 + e;
-                const float a = (float)lo[e], b = (float)hi[e], co = cs[2 * i], sn = cs[2 * i + 1];
-                sp_rotate(a, b, co, sn, x[c][e], x[c + NC / 2][e]);
+                const f32x4 two = *(const f32x4*)(cs + 2 * (c * 32 + qd * 8 + (e & 6)));
+                sp_rotate((float)qlo[c][e], (float)qhi[c][e], two[2 * (e & 1)], two[2 * (e & 1) + 1], x[c][e], x[c + NC / 2][e]);
                 ss += x[c][e] * x[c][e] + x[c + NC / 2][e] * x[c + NC / 2][e];
             }
         }
@@ -130,11 +183,12 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
         for (int c = 0; c < NC; ++c)
 #pragma unroll
             for (int e = 0; e < 8; ++e) qf[c][e] = n < QH ? (bf16)(x[c][e] * scale) : (bf16)0.f;
-        __syncthreads();                                 // the new key and value are where the block's loads find them
+        __syncthreads();                                 // the own key and value are in LDS
     } else {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
             qf[c] = n < QH ? *(const bf16x8*)(q + ((size_t)t * H + g * QH + n) * HD + c * 32 + qd * 8) : zero8;
+        if (i < re) { find_block(i); load_block(); }
     }
 
     float m_run = -INFINITY, l_run = 0.f;
@@ -145,33 +199,42 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
 #pragma unroll
     for (int d = 0; d < ND; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    for (int i = rb + wave; i < re; i += 4) {
-        const int key0 = (i < b_kept ? i : b_first + (i - b_kept)) * 32;
-        const int page = bt[key0 / ps];
-        const int off0 = key0 % ps;
-        const size_t pg = (size_t)(page < 0 ? 0 : page) * G + g;
-        const int blk = off0 >> 5;                                   // the block of 32 keys inside the page
-        const bf16* kbase = k_pages + pg * ps * HD + (size_t)blk * 2 * NC * 512 + lane * 8;
-        // (value heads may be fewer than key heads: key head g reads value head g % Gv)
-        const bf16* vbase = v_pages + ((size_t)(page < 0 ? 0 : page) * Gv + g % Gv) * VD * ps + (size_t)blk * ND * 512 + lane * 8;
-        bf16x8 kf[2][NC];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-            for (int c = 0; c < NC; ++c)
-                kf[tt][c] = __builtin_nontemporal_load((const bf16x8*)(kbase + (tt * NC + c) * 512));
-        bf16x8 vf[ND];
-#pragma unroll
-        for (int d = 0; d < ND; ++d) vf[d] = __builtin_nontemporal_load((const bf16x8*)(vbase + d * 512));
-        if (key0 + 31 > p) {
-            // the block that holds the query's own key: the rows behind it still hold what the
+    if (i < re) for (;;) {
+        if (FUSE ? key0 + 31 >= p : key0 + 31 > p) {
+            // The block that holds the query's own key: the rows behind it still hold what the
             // page's last owner left, and a probability of zero times a value that is not finite
-            // is not zero; those values are taken as zero (this lane's keys are key0 + qd*8 + e)
+            // is not zero; those values are taken as zero (this lane's keys are key0 + qd*8 + e).
+            // Masks of two values each: few instructions, as every one of this kernel is fetched for a single use.
+            const int behind = p - (key0 + qd * 8);                  // elements e > behind are past the query
+            u32x4 keep2, own2 = {0, 0, 0, 0};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const bool dead = key0 + qd * 8 + e > p;
+            for (int j = 0; j < 4; ++j) keep2[j] = (2 * j <= behind ? 0xffffu : 0u) | (2 * j + 1 <= behind ? 0xffff0000u : 0u);
+            uint32_t now[ND];
 #pragma unroll
-                for (int d = 0; d < ND; ++d) vf[d][e] = dead ? (bf16)0.f : vf[d][e];
+            for (int d = 0; d < ND; ++d) now[d] = 0;
+            if constexpr (FUSE) {
+                // the token's own key and value take the places that the loads found stale
+                if (own_slot >= 0 && own_slot == page * ps + p % ps) {
+                    const int w = p & 31, r = ((w >> 3) << 2) | (w & 3);
+#pragma unroll
+                    for (int tt = 0; tt < 2; ++tt)
+                        if (((w >> 2) & 1) == tt)
+#pragma unroll
+                            for (int c = 0; c < NC; ++c) {
+                                const bf16x8 k = *(const bf16x8*)(own + c * 32 + qd * 8);
+                                kf[tt][c] = n == r ? k : kf[tt][c];
+                            }
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) own2[j] = (2 * j == behind ? 0xffffu : 0u) | (2 * j + 1 == behind ? 0xffff0000u : 0u);
+#pragma unroll
+                    for (int d = 0; d < ND; ++d) now[d] = __builtin_bit_cast(uint16_t, own[HD + d * 16 + n]) * 0x10001u;
+                }
+            }
+#pragma unroll
+            for (int d = 0; d < ND; ++d) {
+                // (whole vectors: written element by element, clang 22 let other values into the registers of some of them)
+                const u32x4 put = {now[d], now[d], now[d], now[d]};
+                vf[d] = (vf[d] & (keep2 & ~own2)) | (put & own2);
             }
         }
 
@@ -219,10 +282,15 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
 #pragma unroll
         for (int d = 0; d < ND; ++d) {
             o[d] = o[d] * alpha;
-            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[d], pf, o[d], 0, 0, 0);
+            o[d] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, vf[d]), pf, o[d], 0, 0, 0);
         }
+        i += 4;
+        if (i >= re) break;
+        find_block(i);
+        load_block();
     }
 
+    if constexpr (FUSE) __syncthreads();                 // (the own key lies where the records go)
     // the waves' partial results meet in LDS; o[d][i] of lane (n, qd) is O[head n][d*16 + qd*4 + i]
     if (n < QH) {
         float* mine = sm + ((size_t)wave * QH + n) * ROW;
@@ -270,7 +338,9 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
     }
 }
 
-template <int HD>              // HD: the values' width
+// HD: the values' width.  AHEAD: so many splits' elements are asked for together with the maxima and sums, not behind them
+// (past the last split: the last one's again, unused).
+template <int HD, int AHEAD>
 __global__ __launch_bounds__(HD < 64 ? 64 : HD)
 void attn_decode_combine_kernel(const float* __restrict__ part, bf16* __restrict__ out, int H, int n_splits) {
     constexpr int ROW = HD + 2;
@@ -278,6 +348,9 @@ void attn_decode_combine_kernel(const float* __restrict__ part, bf16* __restrict
     __shared__ float linv;
     const int t = blockIdx.x, h = blockIdx.y, c = threadIdx.x;
     const float* rec = part + ((size_t)t * H + h) * n_splits * ROW;
+    float v[AHEAD];
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s) v[s] = rec[(size_t)(s < n_splits ? s : n_splits - 1) * ROW + (c < HD ? c : 0)];
     // the first wave turns the splits' maxima and sums into weights (up to 256 splits, 4 a lane)
     if (c < 64) {
         float ms[4], ls[4];
@@ -304,8 +377,11 @@ void attn_decode_combine_kernel(const float* __restrict__ part, bf16* __restrict
     __syncthreads();
     if (c >= HD) return;                // (narrow values: one wave, not all of its lanes hold an element)
     float acc = 0.f;
+#pragma unroll
+    for (int s = 0; s < AHEAD; ++s)
+        if (s < n_splits) acc += wsh[s] * v[s];
 #pragma unroll 8
-    for (int s = 0; s < n_splits; ++s) acc += wsh[s] * rec[(size_t)s * ROW + c];
+    for (int s = AHEAD; s < n_splits; ++s) acc += wsh[s] * rec[(size_t)s * ROW + c];
     out[((size_t)t * H + h) * HD + c] = (bf16)(acc * linv);
 }
 
@@ -315,9 +391,13 @@ int sp_attn_combine(const float* part, void* out, int T, int H, int hd, int n_sp
     SP_REQUIRE(T >= 0 && H > 0 && H <= 65535 && n_splits >= 1 && n_splits <= 256 && (hd == 32 || hd == 64 || hd == 128),
                "attn_combine: T=%d H=%d hd=%d splits=%d", T, H, hd, n_splits);
     if (T == 0) return 0;
-    if (hd == 128) attn_decode_combine_kernel<128><<<dim3(T, H), 128, 0, st>>>(part, (bf16*)out, H, n_splits);
-    else if (hd == 64) attn_decode_combine_kernel<64><<<dim3(T, H), 64, 0, st>>>(part, (bf16*)out, H, n_splits);
-    else attn_decode_combine_kernel<32><<<dim3(T, H), 64, 0, st>>>(part, (bf16*)out, H, n_splits);
+#define SP_ADC(HDV, A) attn_decode_combine_kernel<HDV, A><<<dim3(T, H), HDV < 64 ? 64 : HDV, 0, st>>>(part, (bf16*)out, H, n_splits)
+#define SP_ADC_HD(HDV) do { if (n_splits <= 8) SP_ADC(HDV, 8); else if (n_splits <= 16) SP_ADC(HDV, 16); else SP_ADC(HDV, 32); } while (0)
+    if (hd == 128) SP_ADC_HD(128);
+    else if (hd == 64) SP_ADC_HD(64);
+    else SP_ADC_HD(32);
+#undef SP_ADC_HD
+#undef SP_ADC
     SP_LAUNCH_CHECK("attn_combine");
     return 0;
 }
@@ -354,8 +434,8 @@ static int attn_decode(const void* q, const void* k_pages, const void* v_pages, 
     if (!sp_vis_has_span(vis)) keep = 0;
     const float sl = scale * 1.4426950408889634f, cr = softcap > 0.f ? scale / softcap : 0.f;
     dim3 grid(n_splits, G, T);
-    const size_t rec = (size_t)4 * (H / G) * (v_dim + 2) * sizeof(float);
-    const size_t sh = rec > (size_t)hd * sizeof(float) ? rec : (size_t)hd * sizeof(float);
+    // the waves' records; before them, in the fused form, the sines and the token's own key and value: always less
+    const size_t sh = (size_t)4 * (H / G) * (v_dim + 2) * sizeof(float);
     const ad_rope ro = rope ? *rope : ad_rope{};
 #define SP_ADK(HDV, VDV, DISTV, FUSEV) attn_decode_kernel<HDV, VDV, DISTV, FUSEV><<<grid, 256, sh, st>>>( \
             (const bf16*)q, (bf16*)k_pages, (bf16*)v_pages, (float*)workspace, (bf16*)out, positions, seq_of_token, block_table, \

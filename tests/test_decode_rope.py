@@ -82,3 +82,32 @@ def test_what_a_query_sees_caps_slopes_and_rows_without_a_place(vis, span, softc
     assert torch.equal(kp2[page], before[0][page]) and torch.equal(vp2[page], before[1][page])
     assert not torch.equal(kp2, before[0])
     assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("hd", [64, 128])
+@pytest.mark.parametrize("n_splits", [1, 2, 9, 17, 40])
+def test_own_key_at_every_place_of_a_block_and_any_number_of_splits(hd, n_splits):
+    """The token's own key and value never pass through memory on their way to the scores: a token at each of the 32 places of a
+    block gives what the two kernels give, bit for bit (without a norm the query is the same), behind one block and behind
+    two; the pages keep NaN where no key has been written; the splits' records are joined 8, 16 or 32 at a time."""
+    lens, H, G, ps = list(range(1, 65)), 6, 2, 32
+    T = len(lens)
+    kv = PagedKV(lens, G, hd, ps, torch.bfloat16)
+    kv.vp[kv.vp == -70.0] = float("nan")
+    kp, vp = ops().kv_operand_order(kv.kp.to(DEV), kv.vp.to(DEV))
+    qkv = rnd(T, (H + 2 * G) * hd, dtype=torch.bfloat16, seed=11)
+    positions = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([kv.tables[s][(n - 1) // ps] * ps + (n - 1) % ps for s, n in enumerate(lens)], dtype=torch.int32, device=DEV)
+    seq, bt = torch.arange(T, dtype=torch.int32, device=DEV), kv.bt.to(DEV)
+    inv = (10000.0 ** (-torch.arange(hd // 2, dtype=torch.float64) / (hd // 2))).float().to(DEV)
+    scratch = torch.empty(ops().attn_decode_workspace(T, H, hd, n_splits) // 4, dtype=torch.float32, device=DEV)
+    q, want, got = (torch.zeros(T, H * hd, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    kp2, vp2 = kp.clone(), vp.clone()
+    ops().rope_kvwrite(qkv, q, kp, vp, positions, slots, inv, H, G, hd, ps, use_rope=True, adjacent=False, use_norm=False, norm_eps=0.0,
+                       use_temp=False, floor_scale=0, attn_scale=0.0, kv_tiled=True)
+    args = (positions, seq, bt, T, H, G, hd, ps, "full", 0, hd ** -0.5, n_splits)
+    ops().attn_decode(q, kp, vp, want, scratch, *args)
+    ops().attn_decode_rope(qkv, kp2, vp2, got, scratch, positions, slots, *args[1:], inv_freq=inv)
+    bits = lambda t: t.view(torch.int16)
+    assert torch.equal(bits(kp), bits(kp2)) and torch.equal(bits(vp), bits(vp2))
+    assert torch.equal(bits(got), bits(want)) and bool(torch.isfinite(want.float()).all())
