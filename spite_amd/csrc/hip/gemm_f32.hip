@@ -12,8 +12,7 @@
 //    2,048 output rows has 1,024 waves in flight; the runs' sums meet in LDS.
 //  gemm_f32_tile: many rows, bound by the MFMAs (256 FLOP a clock and compute unit).  TM (64 or 32) rows of X times 64 rows of
 //    W a workgroup: X through double-buffered LDS, a step ahead, read by all four waves; a wave's 16 rows of W straight into
-//    registers, two steps ahead.  One workgroup a compute unit reaches 45 % of the units' rate, since nothing fills its waits;
-//    several 70 %.
+//    registers, two steps ahead.  One workgroup a compute unit reaches 70 % of the units' rate at K = 2,048, its start and end included.
 //
 // Which one, and its tile: see f32_variant.
 #include "common.h"
@@ -132,79 +131,115 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
 #define F32_TK 64                 // k a step through LDS
 #define F32_LD (F32_TK + 4)       // LDS row: 16 bytes more than a step, so that 16 rows' reads spread over the banks
 
-// The loop over k for a tile whose first LIVE groups of 16 rows hold rows (an expert's last tile is seldom full).  Loads
-// are unconditional, X's a step ahead of its use and W's two (three sets of registers in turn), and X is scaled only when it
-// goes to LDS, so that nothing waits for them before the step's MFMAs; a chain of four MFMAs is spread over the accumulators.
-template <int TM, int NB, int LIVE>
+// The loop over k for a tile whose first LIVE groups of 16 rows hold rows (an expert's last tile is seldom full).  X goes through
+// LDS a step ahead, its operands are read from there a piece of 16 k ahead of their products (read at their use, each piece waited
+// for LDS some 150 of its 256 to 512 cycles of products), and a chain of four MFMAs is spread over the accumulators.  A wave's W lies
+// in sets of registers:
+//  * two, each piece asked for again, two steps on, as soon as its products are issued, and the next step's rows put into LDS before
+//    the last piece's products;
+//  * BURST, groups of few rows, bound by the stream of W from memory: three, a whole step's pieces asked for at once at the start of the
+//    step two before, the rows put into LDS last, since waiting for them is waiting for the W asked for before them.
+// Before and now (us): 200 rows x 2,048 x 3,072 55 / 34, 301 x 3,072 x 2,048 54 / 44, 301 x 32,768 x 2,048 380 / 365, gated 301 x 3,072
+// x 2,048 100 / 78; 16 groups and one of all of 301 rows, gated 2 x 3,072 x 2,048, 271 / 245, and 2,048 x 3,072 144 / 139 (with two sets 150).
+// 128 groups of a few rows of K = 512 are 4 % slower than before (38 / 36): every second step is one of the last.
+template <int TM, int NB, int LIVE, bool BURST>
 __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp, const float* const* xp, const float* sc, int K,
                                               int seg, int lr, int lk, int r, int q, f32x4 (&tot)[TM / 16][NB]) {
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    constexpr int U = F32_TK / 16, XL = TM * F32_TK / 1024;      // steps of 16 k, 16-byte pieces of X a thread
-    f32x4 acc[LIVE][NB], w0[U][NB], w1[U][NB], w2[U][NB], xv[XL];
+    constexpr int U = F32_TK / 16, XL = TM * F32_TK / 1024;      // pieces of 16 k, 16-byte pieces of X a thread
+    constexpr int S = BURST ? 3 : 2;                              // sets of W
+    f32x4 acc[LIVE][NB], w[S][U][NB], xv[XL], x0[LIVE], x1[LIVE];
 #pragma unroll
     for (int m = 0; m < LIVE; ++m)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[m][b] = zero;
-    // k past the end: the last four's address, and zeros instead
-#define F32_W(w, k0) do { \
-    _Pragma("unroll") for (int u = 0; u < U; ++u) { \
-        const int k = (k0) + u * 16 + q * 4, kc = k < K ? k : K - 4; \
-        _Pragma("unroll") for (int b = 0; b < NB; ++b) w[u][b] = *(const f32x4*)(wp[b] + kc); } } while (0)
-#define F32_X(k0) do { \
-    const int kx = (k0) + lk < K ? (k0) + lk : K - 4; \
-    _Pragma("unroll") for (int i = 0; i < XL; ++i) xv[i] = *(const f32x4*)(xp[i] + kx); } while (0)
-#define F32_PUT(buf, k0) do { \
-    _Pragma("unroll") for (int i = 0; i < XL; ++i) \
-        *(f32x4*)(xs + (buf) * (TM * F32_LD) + (lr + i * (TM / XL)) * F32_LD + lk) = (k0) + lk < K ? xv[i] * sc[i] : zero; } while (0)
-    // Step k0 multiplies the set wa with the rows in buffer `buf`; the rows of the next step and W of the step after the
-    // next are asked for first, in this order: waiting for the rows leaves W on its way.
-#define F32_STEP(wa, wc) do { \
-    __syncthreads();                                   /* this step's rows are in LDS, the other buffer is free */ \
-    if (k0 == flush) { \
-        _Pragma("unroll") for (int m = 0; m < LIVE; ++m) \
-        _Pragma("unroll") for (int b = 0; b < NB; ++b) { tot[m][b] += acc[m][b]; acc[m][b] = zero; } \
-        flush += seg; } \
-    F32_X(k0 + F32_TK); \
-    F32_W(wc, k0 + 2 * F32_TK); \
-    __builtin_amdgcn_sched_barrier(0); \
-    const float* xb = xs + buf * (TM * F32_LD); \
-    _Pragma("unroll") for (int u = 0; u < U; ++u) { \
-        if (k0 + u * 16 + 16 > K) { \
-            const bool in = k0 + u * 16 + q * 4 < K; \
-            _Pragma("unroll") for (int b = 0; b < NB; ++b) wa[u][b] = in ? wa[u][b] : zero; } \
-        f32x4 x[LIVE]; \
-        _Pragma("unroll") for (int m = 0; m < LIVE; ++m) x[m] = *(const f32x4*)(xb + (m * 16 + r) * F32_LD + u * 16 + q * 4); \
-        _Pragma("unroll") for (int e = 0; e < 4; ++e) \
-        _Pragma("unroll") for (int m = 0; m < LIVE; ++m) \
-        _Pragma("unroll") for (int b = 0; b < NB; ++b) \
-            acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(wa[u][b][e], x[m][e], acc[m][b], 0, 0, 0); } \
-    F32_PUT(buf ^ 1, k0 + F32_TK); \
-    buf ^= 1; \
-    k0 += F32_TK; } while (0)
-    F32_X(0);
-    F32_W(w0, 0);
-    F32_W(w1, F32_TK);
-    F32_PUT(0, 0);
+    const float* wl[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) wl[b] = wp[b] + q * 4;
+    const float* xl = xs + r * F32_LD + q * 4;
+    float* xw = xs + lr * F32_LD + lk;
     int buf = 0, k0 = 0, flush = seg;
-    while (k0 + 2 * F32_TK < K) {
-        F32_STEP(w0, w2);
-        F32_STEP(w1, w0);
-        F32_STEP(w2, w1);
+    // (whole: every k that the step asks for exists; else k past the end takes the last four's address, and zeros in their place)
+    auto load_w = [&](f32x4 (&w)[NB], int k, bool whole) {
+        const int kc = whole || k + q * 4 < K ? k : K - 4 - q * 4;
+#pragma unroll
+        for (int b = 0; b < NB; ++b) w[b] = *(const f32x4*)(wl[b] + kc);
+    };
+    auto load_x = [&](int k, bool whole) {
+        const int kc = whole || k + lk < K ? k + lk : K - 4;
+#pragma unroll
+        for (int i = 0; i < XL; ++i) xv[i] = *(const f32x4*)(xp[i] + kc);
+    };
+    auto put_x = [&](int to, int k, bool whole) {
+        const bool in = whole || k + lk < K;
+#pragma unroll
+        for (int i = 0; i < XL; ++i) *(f32x4*)(xw + to * (TM * F32_LD) + i * (TM / XL) * F32_LD) = in ? xv[i] * sc[i] : zero;
+    };
+    auto read_x = [&](f32x4 (&x)[LIVE], int u) {
+#pragma unroll
+        for (int m = 0; m < LIVE; ++m) x[m] = *(const f32x4*)(xl + buf * (TM * F32_LD) + m * 16 * F32_LD + u * 16);
+    };
+    auto step = [&](f32x4 (&w)[U][NB], f32x4 (&w2)[U][NB], bool whole) {
+        __syncthreads();                               // this step's rows are in LDS, the other buffer is free
+        if (k0 == flush) {
+#pragma unroll
+            for (int m = 0; m < LIVE; ++m)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) { tot[m][b] += acc[m][b]; acc[m][b] = zero; }
+            flush += seg;
+        }
+        read_x(x0, 0);
+        load_x(k0 + F32_TK, whole);
+        if (BURST)
+#pragma unroll
+            for (int u = 0; u < U; ++u) load_w(w2[u], k0 + 2 * F32_TK + u * 16, whole);
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            f32x4 (&x)[LIVE] = u & 1 ? x1 : x0;
+            if (u + 1 < U) read_x(u & 1 ? x0 : x1, u + 1);
+            else if (!BURST) put_x(buf ^ 1, k0 + F32_TK, whole);
+            if (!whole && k0 + u * 16 + 16 > K) {
+                const bool in = k0 + u * 16 + q * 4 < K;
+#pragma unroll
+                for (int b = 0; b < NB; ++b) w[u][b] = in ? w[u][b] : zero;
+            }
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int e = 0; e < 4; ++e)
+#pragma unroll
+                for (int m = 0; m < LIVE; ++m)
+#pragma unroll
+                    for (int b = 0; b < NB; ++b) acc[m][b] = __builtin_amdgcn_mfma_f32_16x16x4f32(w[u][b][e], x[m][e], acc[m][b], 0, 0, 0);
+            if (!BURST) load_w(w[u], k0 + S * F32_TK + u * 16, whole);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        if (BURST) put_x(buf ^ 1, k0 + F32_TK, whole);
+        buf ^= 1;
+        k0 += F32_TK;
+    };
+    load_x(0, false);
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+        for (int u = 0; u < U; ++u) load_w(w[i][u], i * F32_TK + u * 16, false);
+    put_x(0, 0, false);
+    while (k0 + 2 * S * F32_TK <= K) {
+#pragma unroll
+        for (int i = 0; i < S; ++i) step(w[i], w[(i + 2) % S], true);
     }
-    if (k0 < K) F32_STEP(w0, w2);
-    if (k0 < K) F32_STEP(w1, w0);
+    while (k0 < K) {
+#pragma unroll
+        for (int i = 0; i < S; ++i)
+            if (k0 < K) step(w[i], w[(i + 2) % S], false);
+    }
 #pragma unroll
     for (int m = 0; m < LIVE; ++m)
 #pragma unroll
         for (int b = 0; b < NB; ++b) tot[m][b] += acc[m][b];
-#undef F32_STEP
-#undef F32_W
-#undef F32_X
-#undef F32_PUT
 }
 
-template <int TM, int GLU>
-__global__ __launch_bounds__(256)
+template <int TM, int GLU, bool BURST>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(GLU ? (TM == 64 || BURST ? 2 : 3) : TM == 64 ? 3 : 4)))
 void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, long w_group_stride,
                           float* __restrict__ Y, int ldy, int M, int N, int K, const int* __restrict__ offsets, int n_groups,
                           const int* __restrict__ a_rows, const float* __restrict__ a_scale, const int* __restrict__ y_rows,
@@ -246,13 +281,13 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
     const int rows = row_end - row0, seg = f32_seg(K);
     bool done = false;
     if constexpr (TM == 64) {
-        if (rows > 48) f32_tile_loop<TM, NB, 4>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
-        else if (rows > 32) f32_tile_loop<TM, NB, 3>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+        if (rows > 48) f32_tile_loop<TM, NB, 4, false>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+        else if (rows > 32) f32_tile_loop<TM, NB, 3, false>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
         done = rows > 32;
     }
     if (done) {}
-    else if (rows > 16) f32_tile_loop<TM, NB, 2>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
-    else f32_tile_loop<TM, NB, 1>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+    else if (rows > 16) f32_tile_loop<TM, NB, 2, BURST>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
+    else f32_tile_loop<TM, NB, 1, BURST>(xs, wp, xp, sc, K, seg, lr, lk, r, q, tot);
 #pragma unroll
     for (int m = 0; m < TM / 16; ++m) {
         const int s = row0 + m * 16 + r;
@@ -269,9 +304,12 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
 // 64).  `n_groups` 0: no groups.
 //
 // Both kernels take a time that follows from the most workgroups that a compute unit gets, c: for 2,048 of K, on an MI355X (us), the
-// stream of 16 rows 7 c (gated 11.5 c), tiles of 32 rows 14 + 19.5 c (14 + 47 c), of 64 17 + 36 c (19 + 82 c); the stream gives each
+// stream of 16 rows 7 c (gated 11.5 c), tiles of 32 rows 7 + 19 c (5 + 41 c), of 64 9 + 29 c (10 + 56 c); the stream gives each
 // of its eight waves a run of 64 k and more, so that shorter sums than 512 leave some idle.  The lines lie where 14,900 products (1
-// to 1,500 tokens, up to 128 groups of 1 to 8 a token, K of 128 to 8,192) were timed with every variant:
+// to 1,500 tokens, up to 128 groups of 1 to 8 a token, K of 128 to 8,192) were timed with every variant, with tiles that took
+// 14 + 19.5 c (14 + 47 c) and 17 + 36 c (19 + 82 c), as the figures below have it; with the tiles as they are the choice is 6 % off the
+// best variant on average over 768 products (9 to 1,200 tokens, up to 129 groups, K of 512 to 5,120), most of it where 33 to 64 rows
+// still take the stream (48 rows of 5 groups x 3,072 x 2,048 64 / tiles of 32 33):
 //  * groups of up to eight rows on average: the stream of every group's W, 16 rows a workgroup (16 groups and one of all t rows, 2 x
 //    3,072 x 2,048 gated: t = 16 124, with 32 rows a workgroup 190; t = 64 184 / tiles 207), but tiles of 32 rows where sums are
 //    short and tiles enough (K <= 512 and more than one a compute unit; plain K < 2,048 and more than two: 129 groups x 2,048 x 768,
@@ -313,13 +351,13 @@ int sp_gemm_f32(const float* A, int lda, const float* W, long w_group_stride, fl
 #define SP_F32_ARGS A, lda, W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, act_limit, vec_y
     if (variant < 0) {
         dim3 grid((N + 63) / 64, m_tiles);
-        if (tile == 32) {
-            if (glu) gemm_f32_tile_kernel<32, 1><<<grid, 256, 0, st>>>(SP_F32_ARGS);
-            else gemm_f32_tile_kernel<32, 0><<<grid, 256, 0, st>>>(SP_F32_ARGS);
-        } else {
-            if (glu) gemm_f32_tile_kernel<64, 1><<<grid, 256, 0, st>>>(SP_F32_ARGS);
-            else gemm_f32_tile_kernel<64, 0><<<grid, 256, 0, st>>>(SP_F32_ARGS);
-        }
+#define SP_F32_TILE(TM, GLU) do { if (offsets) gemm_f32_tile_kernel<TM, GLU, true><<<grid, 256, 0, st>>>(SP_F32_ARGS); \
+                                  else gemm_f32_tile_kernel<TM, GLU, false><<<grid, 256, 0, st>>>(SP_F32_ARGS); } while (0)
+        if (tile == 32 && glu) SP_F32_TILE(32, 1);
+        else if (tile == 32) SP_F32_TILE(32, 0);
+        else if (glu) SP_F32_TILE(64, 1);
+        else SP_F32_TILE(64, 0);
+#undef SP_F32_TILE
         SP_LAUNCH_CHECK("gemm_f32_tile");
         return 0;
     }

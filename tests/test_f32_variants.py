@@ -54,3 +54,32 @@ def test_gated_rows_with_both_halves_in_one_operand(M, N, K, groups):
     ops().gemm_generic(a, w, y, M, N, K, glu=True)
     ops().gemm_generic(torch.cat([a, rnd(100, K, seed=3)]), w, many, M + 100, N, K, glu=True)
     assert torch.equal(y, many[:M])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [4, 60, 64, 68, 128, 188, 192, 256, 260, 320, 384, 388, 448, 516, 580, 772])
+@pytest.mark.parametrize("glu", [False, True])
+@pytest.mark.parametrize("M,N", [(90, 200), (75, 33000)])
+def test_tiles_add_up_in_the_streams_order_wherever_the_sum_ends(K, glu, M, N):
+    """Sums that end inside a step, with one, with the steps whose loads would pass the end: a row of a tile (of 32 rows, of
+    64) has the bits that the stream gives it alone, plain and among groups of one to forty rows."""
+    a, w = rnd(M, K), rnd((2 if glu else 1) * N, K, seed=1)
+    whole, one = torch.empty(M, N, device=DEV), torch.empty(1, N, device=DEV)
+    ops().gemm_generic(a, w, whole, M, N, K, glu=glu)
+    for r in (0, 15, 16, 63, 64, M - 1):
+        ops().gemm_generic(a[r:r + 1].contiguous(), w, one, 1, N, K, glu=glu)
+        assert torch.equal(one[0], whole[r])
+    N = min(N, 1024)
+    sizes = [1, 17, 33, 0, 16, 40, 8, 3]
+    offsets = torch.tensor([0] + list(torch.tensor(sizes).cumsum(0)), dtype=torch.int32, device=DEV)
+    n = sum(sizes)
+    x, ws = rnd(n, K, seed=5), rnd(len(sizes), (2 if glu else 1) * N, K, seed=6)
+    y = torch.empty(n, N, device=DEV)
+    ops().gemm_generic(x, ws, y, n, N, K, glu=glu, offsets=offsets, n_groups=len(sizes))
+    at = 0
+    for g, size in enumerate(sizes):
+        for r in {at, at + size - 1} if size else ():
+            alone = torch.empty(1, N, device=DEV)
+            ops().gemm_generic(x[r:r + 1].contiguous(), ws[g].contiguous(), alone, 1, N, K, glu=glu)
+            assert torch.equal(alone[0], y[r])
+        at += size
