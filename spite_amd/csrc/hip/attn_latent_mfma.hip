@@ -3,16 +3,26 @@
 //
 // Because all heads read the same rows, the heads are the kernel's batch: query row t*H + h is
 // one column of a 16-column MFMA tile, so a decoded token alone fills tiles with its heads, and a
-// prompt's portion fills them with (token, head) pairs.  A workgroup takes up to 128 consecutive
+// prompt's portion fills them with (token, head) pairs.  A workgroup of eight waves takes up to 128 consecutive
 // query rows of one request (the list `wg`, built on the host from the step's entries: first row
 // and number of rows), one wave per 16 rows.  All waves walk the same blocks of 32 keys, from the
-// first key that the first row may read to the last row's own position; a block is staged once
-// in LDS for all of them: the rows (the S^T = K Q^T operand, in the order of the tiles' rows), and their first R
-// elements transposed (the O^T = V^T P^T operand).  Every row masks by its own position.
+// first key that the first row may read to the last row's own position.  Every row masks by its own position.
+//
+// A block's rows go straight from the pages to LDS (loads with the lds bit, an eighth of a block a wave), two blocks ahead in
+// three buffers: one barrier a block, no register and no wave waits for them.  They lie there once, row by row, and serve both products:
+//   S^T = K Q^T    reads 16 bytes of a row a lane;
+//   O^T = V^T P^T  reads its operand, the same rows' elements turned, by transposing reads (four rows x 16 columns to 16 lanes).
+// The 16-byte pieces of a row are exchanged by XOR with half its number, so that either read spreads over the banks.
+// A block of rows of 576 takes eight waves 3.0 us, 6,700 cycles: some 2,200 of products, 4,400 and more of reads of LDS (36 KB a
+// wave for the first product, 32 for the second) and the softmax between them, which the waves reach together.  Two tiles of
+// rows a wave would halve the reads, but their output and queries fill the register file (240 spilled).  Before, a block was staged in
+// two layouts, the turned one by 2-byte stores, and prompts had no load in flight: 40 heads of 576 / 512, two prompts of 1,021 and
+// 765 tokens 294 us, now 174; 2,048 tokens 680 / 345; 700 behind a window of 4,096 796 / 485; two tokens of 1,024 keys 25.7 / 20.4, 64 of 500
+// 41.9 / 32.0; rows of 320 and 192 0.43 to 0.88 of the time.
 //
 // Tiles: S^T tile tt (of 2) holds the keys (r/4)*8 + tt*4 + r%4 of the block in its rows r, so the
 // eight scores a lane holds are eight consecutive keys: P^T is the next product's operand without a
-// shuffle.  Scores, maximum, sum and the output are fp32.
+// shuffle.  Scores, maximum (in the exponent's units, base 2), sum and the output are fp32.
 //
 // Few workgroups with many keys (decoded tokens of a few requests over long contexts): the blocks
 // of keys are dealt to `n_splits` workgroups a work item (grid.y), each leaves a record (output not
@@ -20,38 +30,31 @@
 #include "common.h"
 
 #define LM_ROWS 128        // query rows per workgroup at most (8 waves of 16)
-#define LM_PRE 12          // 16-byte pieces of a key's row that a staging thread keeps in registers, per block in flight
-#define LM_KROW_BLOCKS 128 // blocks of keys whose cache rows the staging waves look up ahead of their loop
-#define LM_VT_LD 40        // row stride of the transposed values in LDS (32 keys + 8: no bank conflicts, 16-byte rows)
+#define LM_TABLE 64        // blocks of keys whose cache rows are looked up ahead, a half at a time
+#define LM_BUFS 3
+
+typedef short s16x4 __attribute__((ext_vector_type(4)));
+static __device__ __attribute__((aligned(16))) const unsigned lm_zeros[4] = {0, 0, 0, 0};      // what a row that is not read holds
 
 template <int KQ, int NV>   // Dk <= 32*KQ, R <= 16*NV
-__global__ __launch_bounds__(512)
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KQ > 6 ? 2 : 4)))
 void attn_latent_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kv_pages, bf16* __restrict__ out,
                              const int* __restrict__ positions, const int* __restrict__ seq_of_token,
                              const int* __restrict__ block_table, int max_blocks, const int* __restrict__ wg,
-                             int H, int Dk, int R, int ps, int vis, int span, float scale,
+                             int H, int Dk, int R, int ps, int vis, int span, float scale_log2e,
                              float* __restrict__ part, int n_splits) {
-    extern __shared__ __attribute__((aligned(16))) unsigned char lds_raw[];
-    const int kq = (Dk + 31) >> 5, nv = (R + 15) >> 4;
-    const int ks_ld = kq * 32 + 8;                                  // row stride of the staged rows
-    bf16* Ks = (bf16*)lds_raw;                                      // [32][ks_ld]
-    bf16* Vt = Ks + 32 * ks_ld;                                     // [nv*16][LM_VT_LD]
-    int* kflag = (int*)(Vt + nv * 16 * LM_VT_LD);                   // [32] 1: the key's page was given back
-    int* krow = kflag + 32;                                         // [LM_KROW_BLOCKS * 32] cache rows of the share's keys (staging waves)
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nthreads = blockDim.x;
-    const int row0 = wg[2 * blockIdx.x], nrows = wg[2 * blockIdx.x + 1];
+    constexpr int PP = KQ * 4, BUF = 32 * PP * 16;                  // 16-byte pieces of a staged row; bytes of a block
+    constexpr int XI = (PP / 2 + 7) / 8;                            // loads of a kilobyte a wave and block
+    static_assert(PP % 8 == 0 && PP / 8 % 2 == 1, "an odd number of 128 bytes: neighbouring rows start 32 banks apart");
+    extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
+    int* krow = (int*)(lds + LM_BUFS * BUF);                        // [LM_TABLE * 32] cache rows; -1: page given back, -2: not read
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int c = lane & 15, g4 = lane >> 4;
+    const int item = gridDim.x - 1 - blockIdx.x;                    // an entry's last rows, which read the most keys, start first
+    const int row0 = wg[2 * item], nrows = wg[2 * item + 1];
     const int t_first = row0 / H, t_last = (row0 + nrows - 1) / H;
     const int* bt = block_table + (size_t)seq_of_token[t_first] * max_blocks;
     const int key_lo = sp_first_visible(positions[t_first], vis, span), key_hi = positions[t_last];
-
-    // the staged rows' elements past Dk are zero for good
-    for (int i = tid; i < 32 * (ks_ld - Dk); i += nthreads) {
-        const int key = i / (ks_ld - Dk), f = Dk + i % (ks_ld - Dk);
-        Ks[key * ks_ld + f] = (bf16)0.f;
-    }
-    for (int i = tid; i < (nv * 16 - R) * LM_VT_LD; i += nthreads) Vt[R * LM_VT_LD + i] = (bf16)0.f;
-
-    const int chunks = Dk >> 3;                                     // 16-byte pieces of a row
 
     // this workgroup's share of the blocks of keys
     int blk_first = key_lo >> 5, blk_end = (key_hi >> 5) + 1;
@@ -60,191 +63,165 @@ void attn_latent_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict_
         blk_first += (int)blockIdx.y * per;
         blk_end = blk_first + per < blk_end ? blk_first + per : blk_end;
     }
-    // Waves beyond the ones that hold query rows do all the staging when they can keep a block's
-    // pieces in registers (2 threads a key and wave, PRE pieces a thread) and the share's cache rows
-    // fit their table: they fetch the next two blocks while the others compute on this one.  Their loop
-    // holds no load but the rows' own, so nothing makes them wait for the youngest load; the table
-    // entries of the whole share are looked up before it.
-    constexpr int PRE = KQ <= 6 ? 4 : (KQ <= 10 ? 8 : LM_PRE);      // smaller rows leave the other instantiations their registers
-    const int n_cw = (nrows + 15) >> 4, n_lw = (nthreads >> 6) - n_cw, n_blk = blk_end - blk_first;
-    const bool roles = n_lw * 2 * PRE >= chunks && n_blk <= LM_KROW_BLOCKS && n_blk > 0;
-    if (roles && wave >= n_cw) {
-        const int lt = tid - n_cw * 64, key = lt & 31, piece0 = lt >> 5, piece_step = n_lw * 2;
-        bf16* ks_row = Ks + ((((key >> 2) & 1) << 4) + ((key >> 3) << 2) + (key & 3)) * ks_ld;
-        for (int i = lt; i < n_blk * 32; i += n_lw * 64) {
-            const int j = (blk_first << 5) + i;
-            int r = -2;
-            if (j >= key_lo && j <= key_hi) { const int page = bt[j / ps]; r = page >= 0 ? page * ps + j % ps : -1; }
-            krow[i] = r;
-        }
-        __syncthreads();                                            // (the rows' waves meet it before their loop)
-        bf16x8 preA[PRE], preB[PRE];
-        auto fetch = [&](bf16x8* pre, int r) {
-#pragma unroll
-            for (int u = 0; u < PRE; ++u) {
-                const int pc = piece0 + u * piece_step;
-#pragma unroll
-                for (int e = 0; e < 8; ++e) pre[u][e] = (bf16)0.f;
-                if (r >= 0 && pc < chunks) pre[u] = *(const bf16x8*)(kv_pages + (size_t)r * Dk + (pc << 3));
-            }
-        };
-        auto stage = [&](const bf16x8* pre, int r) {
-            __syncthreads();                                        // the last block's readers are done
-#pragma unroll
-            for (int u = 0; u < PRE; ++u) {
-                const int pc = piece0 + u * piece_step, f = pc << 3;
-                if (pc < chunks) {
-                    *(bf16x8*)(ks_row + f) = pre[u];
-                    if (f < R) {
-#pragma unroll
-                        for (int e = 0; e < 8; ++e) Vt[(f + e) * LM_VT_LD + key] = pre[u][e];
-                    }
-                }
-            }
-            if (lt < 32) kflag[key] = r == -1;
-            __syncthreads();
-        };
-        int rA = krow[key], rB = n_blk > 1 ? krow[32 + key] : -2;
-        fetch(preA, rA);
-        if (n_blk > 1) fetch(preB, rB);
-        for (int b = 0; b < n_blk; b += 2) {
-            stage(preA, rA);
-            if (b + 2 < n_blk) { rA = krow[(b + 2) * 32 + key]; fetch(preA, rA); }   // on its way while the others compute
-            if (b + 1 < n_blk) {
-                stage(preB, rB);
-                if (b + 3 < n_blk) { rB = krow[(b + 3) * 32 + key]; fetch(preB, rB); }
-            }
-        }
-        return;
-    }
+    const int n_blk = blk_end - blk_first;
 
-    const int c = lane & 15, g4 = lane >> 4;
     // this lane's query row: a column of every tile
     const int my = wave * 16 + c;
     const bool row_ok = my < nrows;
     const int row = row0 + (row_ok ? my : 0);
     const int my_p = positions[row / H];
     const int my_lo = sp_first_visible(my_p, vis, span);
-    // what this wave's rows read at all (its first and last row bound it: positions grow with the rows)
-    const int w_first = wave * 16 < nrows ? wave * 16 : 0;
+    // what this wave's rows read at all, and what all of them read (positions grow with the rows)
+    const bool has_rows = wave * 16 < nrows;
     const int w_last = wave * 16 + 15 < nrows ? wave * 16 + 15 : nrows - 1;
-    const int wave_lo = sp_first_visible(positions[(row0 + w_first) / H], vis, span);
-    const int wave_hi = wave * 16 < nrows ? positions[(row0 + w_last) / H] : -1;
+    const int p_first = has_rows ? positions[(row0 + wave * 16) / H] : -1, p_last = has_rows ? positions[(row0 + w_last) / H] : -1;
+    const int wave_lo = sp_first_visible(p_first, vis, span), wave_lo_all = sp_first_visible(p_last, vis, span);
 
     bf16x8 qf[KQ];
 #pragma unroll
     for (int k = 0; k < KQ; ++k) {
         const int f = k * 32 + g4 * 8;
-        bf16x8 z;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) z[e] = (bf16)0.f;
-        qf[k] = (k < kq && f < Dk) ? *(const bf16x8*)(q + (size_t)row * Dk + f) : z;
+        bf16x8 z = {0, 0, 0, 0, 0, 0, 0, 0};
+        if (f < Dk) z = *(const bf16x8*)(q + (size_t)row * Dk + f);
+        qf[k] = z;
     }
+    // (there before the first block is asked for: a wait for them later would be one for the blocks too)
+#pragma unroll
+    for (int k = 0; k < KQ; ++k) asm volatile("" : "+v"(qf[k]));
+
+    // the cache rows of 32 blocks from b0 on, to their half of the table; whether a key of them lies in a page that was given back
+    auto look_up = [&](int b0) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+            const int i = u * 512 + tid, j = ((blk_first + b0) << 5) + i;
+            int r = -2;
+            if (j >= key_lo && j <= key_hi) { const int page = bt[j / ps]; r = page >= 0 ? page * ps + j % ps : -1; }
+            krow[((b0 & (LM_TABLE - 1)) << 5) + i] = r;
+        }
+        __syncthreads();
+    };
+    // this lane's pieces of a block, which key's and which piece of its row: kept in LDS, since the registers are full
+    int* mine = krow + LM_TABLE * 32 + tid;
+#pragma unroll
+    for (int i = 0; i < XI; ++i) {
+        const int at = i * 8 + wave < PP / 2 ? i * 8 + wave : PP / 2 - 1;           // (loads past the block's last: that one again)
+        const int l = at * 64 + lane, r = l / PP, pc = (l % PP) ^ ((r >> 1) & 7);
+        const int key = (((r & 15) >> 2) << 3) + ((r >> 4) << 2) + (r & 3);
+        mine[i * 512] = pc * 8 < Dk ? key | pc << 8 : -1;
+    }
+    const unsigned lds0 = (unsigned)(uintptr_t)(__attribute__((address_space(3))) void*)lds;
+    auto ask = [&](int b, int buf) {
+        const int* tab = krow + ((b & (LM_TABLE - 1)) << 5);
+#pragma unroll
+        for (int i = 0; i < XI; ++i) {
+            const int at = i * 8 + wave < PP / 2 ? i * 8 + wave : PP / 2 - 1;
+            const int what = mine[i * 512], r = what < 0 ? -2 : tab[what & 255];
+            const bf16* src = r >= 0 ? kv_pages + ((size_t)r * Dk + (what >> 8) * 8) : (const bf16*)lm_zeros;
+            const unsigned to = lds0 + buf * BUF + at * 1024;
+            asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off"
+                         :: "v"(src), "s"(__builtin_amdgcn_readfirstlane(to)) : "memory", "m0");
+        }
+    };
+
     float m_run = -INFINITY, l_run = 0.f;
     f32x4 o[NV];
 #pragma unroll
     for (int a = 0; a < NV; ++a) o[a] = f32x4{0.f, 0.f, 0.f, 0.f};
-    // Staging: a thread keeps one key of the block (consecutive lanes take consecutive keys, so the
-    // transposed copy's 2-byte stores fall into consecutive LDS words instead of one bank) and walks
-    // that key's 16-byte pieces.  Where the key's row lies is looked up one block ahead, so the table
-    // entry's way from memory is hidden behind the block before.
-    const int key = tid & 31, piece0 = tid >> 5, piece_step = nthreads >> 5;
-    // LDS row of a key: the 16 rows of S^T tile tt lie together, tile row (key/8)*4 + key%4
-    bf16* ks_row = Ks + ((((key >> 2) & 1) << 4) + ((key >> 3) << 2) + (key & 3)) * ks_ld;
-    auto row_of = [&](int blk0) -> long long {       // first element of the key's cache row; -1: page given back; -2: not read
-        const int j = blk0 + key;
-        if (j < key_lo || j > key_hi) return -2;
-        const int page = bt[j / ps];
-        return page >= 0 ? ((long long)page * ps + j % ps) * Dk : -1;
-    };
-    auto put = [&](int f, const bf16x8& v) {
-        *(bf16x8*)(ks_row + f) = v;
-        if (f < R) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) Vt[(f + e) * LM_VT_LD + key] = v[e];
-        }
-    };
-    if (roles) __syncthreads();                                     // the staging waves have looked up the share's rows
-    long long row_cur = (!roles && blk_first < blk_end) ? row_of(blk_first << 5) : -2;
-    for (int blk0 = blk_first << 5; blk0 < (blk_end << 5); blk0 += 32) {
-      if (roles) {
-        __syncthreads();
-        __syncthreads();                                            // the staging waves have filled the block
-      } else {
-        const long long row_next = blk0 + 32 < (blk_end << 5) ? row_of(blk0 + 32) : -2;
-        __syncthreads();                                            // the last block's readers are done
-        const bf16* src = kv_pages + (row_cur >= 0 ? row_cur : 0);
-        for (int pc = piece0; pc < chunks; pc += 2 * piece_step) {  // two loads in flight before their stores
-            bf16x8 v0, v1;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) { v0[e] = (bf16)0.f; v1[e] = (bf16)0.f; }
-            const bool two = pc + piece_step < chunks;
-            if (row_cur >= 0) {
-                v0 = *(const bf16x8*)(src + (pc << 3));
-                if (two) v1 = *(const bf16x8*)(src + ((pc + piece_step) << 3));
-            }
-            put(pc << 3, v0);
-            if (two) put((pc + piece_step) << 3, v1);
-        }
-        if (tid < 32) kflag[key] = row_cur == -1;
-        row_cur = row_next;
-        __syncthreads();
-      }
-        if (blk0 + 31 < wave_lo || blk0 > wave_hi) continue;        // nothing here for this wave's rows
+    // operands' places in a block: S^T rows c and c + 16, piece 4 k + g4; V^T rows 4 g4 + c / 4 and 16 further on, 8 bytes of piece 2 a + ..
+    const int kx = (c >> 1) & 7, vr = g4 * 4 + (c >> 2), vx = (vr >> 1) & 7;
+    const int kat = c * PP * 16 + ((g4 ^ kx) << 4);                // (pieces 8 n + g4; 8 n + 4 + g4: bit 6 the other way)
+    const int vat = vr * PP * 16 + ((((c >> 1) & 1) ^ (vx & 1)) << 4) + ((c & 1) << 3), vxor = (vx & 6) << 4;
 
-        f32x4 s[2];
-#pragma unroll
-        for (int tt = 0; tt < 2; ++tt) {
-            s[tt] = f32x4{0.f, 0.f, 0.f, 0.f};
-            const bf16* kr = Ks + (tt * 16 + c) * ks_ld + g4 * 8;
-#pragma unroll
-            for (int k = 0; k < KQ; ++k)
-                if (k < kq) s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(kr + k * 32), qf[k], s[tt], 0, 0, 0);
+    if (n_blk > 0) {
+        look_up(0);
+        ask(0, 0);
+        if (n_blk > 1) ask(1, 1);
+    }
+    for (int b = 0, buf = 0; b < n_blk; ++b, buf = buf + 1 < LM_BUFS ? buf + 1 : 0) {
+        if (b + 1 < n_blk) asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(XI) : "memory");
+        else asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)" ::: "memory");
+        __builtin_amdgcn_s_barrier();                               // the block is there, and the one before is no longer read
+        asm volatile("" ::: "memory");
+        if (b + 2 < n_blk) {
+            if (((b + 2) & (LM_TABLE / 2 - 1)) == 0) look_up(b + 2);
+            ask(b + 2, buf ? buf - 1 : LM_BUFS - 1);
         }
+        const int blk0 = (blk_first + b) << 5;
+        if (blk0 + 31 < wave_lo || blk0 > p_last) continue;         // nothing here for this wave's rows
+
+        const unsigned char* kb = lds + buf * BUF;
+        f32x4 s[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
+#pragma unroll
+        for (int k = 0; k < KQ; ++k)
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+                s[tt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(kb + (kat ^ (k & 1) << 6) + (k >> 1) * 128 + tt * 16 * PP * 16), qf[k], s[tt], 0, 0, 0);
+        // the keys' rows, to see whether a page was given back, and masks, where some row does not read the whole block
         float mx = -INFINITY;
-        bool ok[2][4];
+        const int* tab = krow + ((b & (LM_TABLE - 1)) << 5) + g4 * 8;
+        int gone = tab[0];
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
+        for (int i = 1; i < 8; ++i) gone = min(gone, tab[i]);
+        if (blk0 >= wave_lo_all && blk0 + 31 <= p_first && !__any(gone < 0)) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int key = g4 * 8 + tt * 4 + i, j = blk0 + key;
-                ok[tt][i] = row_ok && j >= my_lo && j <= my_p;
-                const float v = ok[tt][i] ? (kflag[key] ? NAN : s[tt][i] * scale) : -INFINITY;
-                s[tt][i] = v;
-                mx = fmaxf(mx, v);
-            }
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) { s[tt][i] *= scale_log2e; mx = fmaxf(mx, s[tt][i]); }
+        } else {
+#pragma unroll
+            for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int j = blk0 + g4 * 8 + tt * 4 + i;
+                    s[tt][i] = row_ok && j >= my_lo && j <= my_p ? (tab[tt * 4 + i] == -1 ? NAN : s[tt][i] * scale_log2e) : -INFINITY;
+                    mx = fmaxf(mx, s[tt][i]);
+                }
+        }
         mx = rows4_max(mx);
         const float m_new = fmaxf(m_run, mx);
-        const float alpha = (m_run == -INFINITY) ? 0.f : __expf(m_run - m_new);
+        const float m_use = m_new == -INFINITY ? 0.f : m_new;       // (a row that has seen no key yet: weights of zero)
+        const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
         float sum = 0.f;
         bf16x8 pf;
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float e = ok[tt][i] ? __expf(s[tt][i] - m_new) : 0.f;
+                const float e = __builtin_amdgcn_exp2f(s[tt][i] - m_use);
                 sum += e;
                 pf[tt * 4 + i] = (bf16)e;
             }
         sum = rows4_sum(sum);
         l_run = l_run * alpha + sum;
         m_run = m_new;
+        if (__any(alpha != 1.f)) {
+#pragma unroll
+            for (int a = 0; a < NV; ++a) o[a] = o[a] * alpha;
+        }
 #pragma unroll
         for (int a = 0; a < NV; ++a) {
-            if (a < nv) {
-                o[a] = o[a] * alpha;
-                o[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(Vt + (a * 16 + c) * LM_VT_LD + g4 * 8), pf, o[a], 0, 0, 0);
-            }
+            const unsigned char* vp = kb + vat + (((a & 7) << 5) ^ vxor) + (a >> 3) * 256;
+            typedef __attribute__((address_space(3))) s16x4* lds4;
+            const s16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)vp);
+            const s16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds4)(vp + 16 * PP * 16));
+            const bf16x8 v = __builtin_bit_cast(bf16x8, __builtin_shufflevector(v0, v1, 0, 1, 2, 3, 4, 5, 6, 7));
+            o[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(v, pf, o[a], 0, 0, 0);
         }
     }
     if (!row_ok) return;
+    if (m_run == -INFINITY && max(my_lo, blk_first << 5) <= min(my_p, (blk_end << 5) - 1)) {
+        // every key that the row reads here has the score -inf: no weights to divide by
+        l_run = NAN;
+#pragma unroll
+        for (int a = 0; a < NV; ++a) o[a] = f32x4{NAN, NAN, NAN, NAN};
+    }
     // o[a][i] of lane (c, g4) is O[row c][a*16 + g4*4 + i]
     if (n_splits > 1) {
         float* rec = part + ((size_t)row * n_splits + blockIdx.y) * (R + 2);
 #pragma unroll
         for (int a = 0; a < NV; ++a) {
             const int col = a * 16 + g4 * 4;
-            if (a < nv && col < R) {
+            if (col < R) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) rec[col + i] = o[a][i];
             }
@@ -257,7 +234,7 @@ void attn_latent_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict_
 #pragma unroll
     for (int a = 0; a < NV; ++a) {
         const int col = a * 16 + g4 * 4;
-        if (a < nv && col < R) {
+        if (col < R) {
             bf16x4 w;
 #pragma unroll
             for (int i = 0; i < 4; ++i) w[i] = (bf16)(o[a][i] * inv);
@@ -269,7 +246,7 @@ void attn_latent_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict_
 // Joins the records [row][split][R + 2] of a split call: one workgroup a query row.
 __global__ __launch_bounds__(256)
 void attn_latent_join_kernel(const float* __restrict__ part, bf16* __restrict__ out, int R, int n_splits) {
-    __shared__ float wsh[1024];          // weight of every split: exp(m_s - M) / L
+    __shared__ float wsh[1024];          // weight of every split: exp2(m_s - M) / L
     __shared__ float red[8];
     const size_t row = blockIdx.x;
     const float* rec = part + row * n_splits * (R + 2);
@@ -291,7 +268,7 @@ void attn_latent_join_kernel(const float* __restrict__ part, bf16* __restrict__ 
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int s = tid + u * 256;
-        const float w = ms[u] == -INFINITY ? 0.f : __expf(ms[u] - M);
+        const float w = ms[u] == -INFINITY ? 0.f : exp2f(ms[u] - M);
         if (s < n_splits) wsh[s] = w;
         L += w * ls[u];
     }
@@ -333,24 +310,14 @@ extern "C" int spite_attn_latent_mfma(const void* q, const void* kv_pages, void*
     SP_REQUIRE(n_splits >= 1 && n_splits <= 1024 && (n_splits == 1 || part), "latent attention: %d splits", n_splits);
     if (n_wg == 0 || max_rows == 0) return 0;
     const int kq = (Dk + 31) / 32, nv = (R + 15) / 16;
-    // a wave for every 16 query rows, and enough waves that staging a block of 32 keys takes a thread
-    // no more than about four 16-byte pieces (waves without rows only stage)
-    int nw = (max_rows + 15) / 16;
-    const int pre = kq <= 6 ? 4 : (kq <= 10 ? 8 : LM_PRE);
-    const int fetch_waves = (Dk / 8 + 2 * pre - 1) / (2 * pre);         // staging waves (see the kernel)
-    if (nw + fetch_waves <= 8) nw += fetch_waves;
-    else {
-        const int stage_waves = (32 * (Dk / 8) + 255) / 256;
-        if (nw < stage_waves) nw = stage_waves < 8 ? stage_waves : 8;
-    }
-    const size_t sh = ((size_t)32 * (kq * 32 + 8) + (size_t)nv * 16 * LM_VT_LD) * sizeof(bf16) + (32 + LM_KROW_BLOCKS * 32) * sizeof(int);
 #define SP_LM(KQV, NVV) do { \
         auto kern = attn_latent_mfma_kernel<KQV, NVV>; \
+        constexpr size_t sh = LM_BUFS * 32 * KQV * 64 + (LM_TABLE * 32 + (KQV * 2 + 7) / 8 * 512) * sizeof(int); \
         static bool allowed = false; \
-        if (sh > 48 * 1024 && !allowed) { hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh); \
+        if (!allowed) { hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh); \
             if (e != hipSuccess) return sp_fail("latent attention: %zu bytes of LDS refused: %s", sh, hipGetErrorString(e)); allowed = true; } \
-        kern<<<dim3(n_wg, n_splits), nw * 64, sh, st>>>((const bf16*)q, (const bf16*)kv_pages, (bf16*)out, positions, seq_of_token, \
-                                        block_table, max_blocks, wg, H, Dk, R, page_size, vis, span, scale, part, n_splits); } while (0)
+        kern<<<dim3(n_wg, n_splits), 512, sh, st>>>((const bf16*)q, (const bf16*)kv_pages, (bf16*)out, positions, seq_of_token, \
+                                        block_table, max_blocks, wg, H, Dk, R, page_size, vis, span, scale * 1.4426950408889634f, part, n_splits); } while (0)
     if (kq <= 6 && nv <= 8) SP_LM(6, 8);
     else if (kq <= 10 && nv <= 16) SP_LM(10, 16);
     else SP_LM(18, 32);

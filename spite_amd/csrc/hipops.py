@@ -1085,11 +1085,12 @@ def latent_workgroups(counts, cu_seqlens, H):
 def latent_splits(n_wg: int, longest: int, Dk: int = 576, R: int = 512) -> int:
     """Into how many workgroups the keys of every work item are best dealt, for ``n_wg`` items whose
     queries read at most ``longest`` keys, in rows of ``Dk`` with a latent of ``R``.  A block of 32 keys takes a workgroup
-    4.6 us and its start about 8, joining the records of 32 splits 6, of 64 10, of 128 16, of 256 25: shares of two blocks up
+    3.0 us and its start about 8, joining the records of 32 splits 6, of 64 10, of 128 16, of 256 25: shares of two blocks up
     to 32 splits, of four beyond (fewer than eight splits only where there are fewer blocks), and about one workgroup a compute unit.  Where a
     unit holds one workgroup, none more: the first one over costs as much time as all of them; narrow rows leave room for
     several a unit.
-    (40 heads on an MI355X, us.  1 item, 1,024 keys: 49 with 4 splits, 23 with 16; 4,096: 51 with 16, 34 with 32; 8,192: 52 with
+    (The lines were timed when a block took 4.6 us; since then two items of 1,024 keys take 20.4 with 32 splits for 25.7, one of 16,384
+    32.8 with 128 for 43.3.  40 heads on an MI355X, us.  1 item, 1,024 keys: 49 with 4 splits, 23 with 16; 4,096: 51 with 16, 34 with 32; 8,192: 52 with
     32, 38 with 64; 16,384: 89 with 32, 56 with 64, 44 with 128; 32,768: 163 with 32, 60 with 128, 49 with 256.  6 items of
     16,384: 94 with 32, 121 with 43.  16 items of 4,096: 59 with 16, 72 with 32.  100 items of 2,048 in rows of 192: 70 with 2,
     53 with 3.)"""
@@ -1100,7 +1101,7 @@ def latent_splits(n_wg: int, longest: int, Dk: int = 576, R: int = 512) -> int:
     if Dk <= 192 and R <= 128:
         room = max(room, min(-(-cus // n_wg), -(-blocks // 8)))
     share = min(max(-(-blocks // 2), min(blocks, 8)), 32)
-    # (no fewer than keep a share within the 4,096 keys whose cache rows the staging waves look up ahead)
+    # (no share of more than 4,096 keys: an end of few workgroups is shorter so)
     return max(1, min(max(share, -(-blocks // 4)), room, 256), min(-(-longest // 4096), 256))
 
 

@@ -291,6 +291,35 @@ def test_latent_attention_matrix_kernel(Hh, Dk, R, ps, vis, span):
     assert float((ref.cpu().double() - c["want"]).abs().max()) < tol
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hh,Dk,R,ps,vis,span", [(2, 576, 512, 64, "full", 0), (3, 320, 256, 24, "window", 2900), (20, 192, 128, 16, "full", 0),
+                                                 (1, 560, 504, 48, "window", 1500), (5, 72, 8, 32, "full", 0)])
+def test_latent_attention_over_many_blocks(Hh, Dk, R, ps, vis, span):
+    """Walks of one block to over a hundred, past every point where the table of cache rows is filled again, in pages that
+    hold no whole number of blocks; and a page that was given back poisons the rows that read it and no other."""
+    from spite_amd.csrc import hipops
+    c = _attention_case(Hh, Dk, R, ps, [1, 9, 2, 1, 3], [3400, 1010, 2020, 0, 1055], vis, span, "bfloat16", Dk + Hh)
+    wg, (n_wg, most) = hipops.latent_workgroups(c["counts"], c["cu"], Hh)
+    tol = 0.02 * float(c["want"].abs().max())
+
+    def run(table, n_splits):
+        out = torch.full((c["T"] * Hh, R), float("nan"), device="cuda:0", dtype=torch.bfloat16)
+        scratch = torch.full((c["T"] * Hh * n_splits * (R + 2),), float("nan"), device="cuda:0") if n_splits > 1 else None
+        hipops.attn_latent_mfma(c["q"], c["pages"], out, c["positions"], c["seq"], table, torch.from_numpy(wg).cuda(), n_wg, most,
+                                c["T"], Hh, Dk, R, vis, span, c["scale"], n_splits=n_splits, scratch=scratch)
+        return out.cpu().double()
+    whole = {n: run(c["table"], n) for n in (1, 2, 7, 40)}
+    for n_splits, out in whole.items():
+        assert float((out - c["want"]).abs().max()) < tol, f"{n_splits} splits"
+    table = c["table"].clone()
+    gone = (1010 - 40) // ps                       # a page just before the second request's new tokens
+    table[1, gone] = -1
+    reads = ((c["seq"] == 1) & (c["positions"] >= gone * ps)).repeat_interleave(Hh).cpu()
+    for n_splits in (1, 7):
+        out = run(table, n_splits)
+        assert bool(torch.isnan(out[reads]).all()) and torch.equal(out[~reads], whole[n_splits][~reads])
+
+
 # ------------------------------------------------------------------------------------------ the model in the engine
 @pytest.fixture(scope="module")
 def models(tmp_path_factory):
