@@ -932,3 +932,27 @@ def test_mfma_loop_runs_and_counts_its_flops():
     assert torch.isfinite(one).all() and float(one.abs().max()) > 0.0 and one.unique().numel() > 1
     assert float((two - 2 * one).abs().max()) <= 1e-4 * float(one.abs().max())
     assert torch.equal(half * 4, one)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 16, 63, 64, 65, 200])
+@pytest.mark.parametrize("N,K", [(1, 8), (3, 16), (16, 24), (127, 32), (128, 40), (130, 56), (260, 64), (1000, 16)])
+@pytest.mark.parametrize("dtype,pad,off", [(torch.float32, 0, 0), (torch.bfloat16, 4, 0), (torch.float32, 3, 1), (torch.bfloat16, 0, 2)])
+def test_gemm_mfma_over_a_short_sum_is_the_tiles_product(M, N, K, dtype, pad, off):
+    """Sums of up to 64 take a kernel of their own: rows of X that lie apart, rows of the result that wide stores take and that
+    they do not, and the bits of the large tiles."""
+    a = rnd(M, 96, dtype=torch.bfloat16)[:, 8:8 + K]
+    w = rnd(N, K, dtype=torch.bfloat16, seed=1)
+    width = N + pad
+    outs = []
+    for shape in (0, 1):
+        room = torch.full((M * width + off,), float("nan"), dtype=dtype, device=DEV)
+        y = room[off:].view(M, width)[:, :N]
+        ops().gemm_mfma(a, w, y, M, N, K, shape=shape)
+        outs.append(room)
+    assert torch.equal(outs[0].view(torch.int16 if dtype == torch.bfloat16 else torch.int32),
+                       outs[1].view(torch.int16 if dtype == torch.bfloat16 else torch.int32))
+    got, want = outs[0][off:].view(M, width)[:, :N].double(), a.double() @ w.double().t()
+    # K products of bfloat16 numbers are exact in fp32; their sum rounds K times, the result once more
+    bound = (K * 2.0 ** -23 + (2.0 ** -8 if dtype == torch.bfloat16 else 0.0)) * (a.double().abs() @ w.double().abs().t())
+    assert bool(((got - want).abs() <= bound + 1e-30).all())
