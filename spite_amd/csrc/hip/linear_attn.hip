@@ -52,14 +52,19 @@ extern "C" int spite_channel_decay(float* z, const float* bias, int T, int width
 // further on for the widest heads; two at 2 dg for heads up to 64): 32 lanes read 512 consecutive bytes of a
 // token's q, k or decay row from LDS in one wide read without bank conflicts.  The tokens' q, k, decay and value slice go
 // through LDS a block of tokens at a time, two buffers: the next block's loads are in flight while this block is computed,
-// and nothing looks at a loaded value before that (what lies outside the head is cleared on the way into LDS).  A whole
+// and nothing looks at a loaded value before that (the places of what lies outside the head are cleared once).  A whole
 // block is one stretch of code: only the state's FMA waits for the token before.  The sums over the key channels are taken
 // for the tokens of a block together (la_sums).  The state tile goes through LDS on the way in and out, so that its rows
 // are read and written 64 bytes at a time.
-// Bound by the reads of q and k from LDS, which every pair of columns makes again (about 190 cycles a token at D = 128 with
-// 8 waves).  1,531 tokens, one request, V = D = 128: 127 us for 16 or 32 heads (208 and 223 with the loads waited for at
-// the head of a block, a sum a token and no read ahead), 106 for heads of 64 (181), 230 for 256 (335); decay per channel:
-// 159 (265).  Half the columns a workgroup where 128 workgroups leave CUs idle gave nothing for heads of 128.
+// Bound by the instructions that a wave issues: at D = 128, 12 a token for the state and 17 around them (the reads from LDS,
+// the sums, the fetches), 185 cycles a token with two waves a SIMD.  So a fetch is set up once and costs a compare, a select
+// and an add a block; k, and what lies outside a head, take no product or select on the way into LDS; and no store is waited
+// for (an asm statement below pins where the loads are waited for: with the loads in branches the compiler also waited at
+// the head of each block, for the block's stores with them).  1,531 tokens, one request, V = D = 128: 114 us for 16 heads
+// and 123 for 32 (128 and 135 before this), decay per channel 146 (160) and 226 for 40 heads (250, 128 registers, so that two
+// workgroups fit a CU: 264 with 134); heads of 64: 96 (104); 800 tokens, 8 heads of 256: 107 (121).  1,000 tokens of fp32,
+// 16 heads: 88 (124).  Tried: two columns a lane, which halves the reads of q and k (168 us with 16 columns a workgroup);
+// half the columns a workgroup where 128 workgroups leave CUs idle (122, 77 for heads of 64); loads two blocks ahead (124).
 // The order of every sum is fixed by D alone: the bits do not depend on how a request's tokens are cut.
 #define LA_VC 16        // value columns a workgroup
 #define LA_NT 512       // threads a workgroup: 16 columns x 32 lanes
@@ -101,125 +106,176 @@ template <int TB> __device__ __forceinline__ float la_sums(float* x, int l) {
 }
 template <int TB> __device__ __forceinline__ int la_owner(int l) { return TB == 16 ? l >> 1 : TB == 8 ? l >> 2 : 0; }
 
+#define LA_OWN(r) (PR >= 4 ? ((r) / 4) * 128 + dg * 4 + ((r) % 4) : dg * PR + (r))    // the thread's r-th key channel
+
+// The workgroup's columns of the state, in and out through LDS (D rows of LA_VC + 1): a thread's PR loads are all asked for
+// before the first is waited for (one
+// after another, a step of single tokens of 8 requests with 16 heads of 128 took 7.4 us for 6.9, of 32 requests 21.3 for 18.7).
+template <int PR> __device__ __forceinline__ void la_state_in(float* S, const float* srow, float* sm, int D, int V, int v0) {
+    const int tid = threadIdx.x, vc = tid / LA_DG, dg = tid % LA_DG, c = tid % LA_VC;
+    float x[PR];
+#pragma unroll
+    for (int u = 0; u < PR; ++u) {
+        const int d = tid / LA_VC + u * (LA_NT / LA_VC);
+        x[u] = srow[d < D && v0 + c < V ? (size_t)d * V + v0 + c : 0];
+    }
+#pragma unroll
+    for (int u = 0; u < PR; ++u) {
+        const int d = tid / LA_VC + u * (LA_NT / LA_VC);
+        sm[d * (LA_VC + 1) + c] = d < D && v0 + c < V ? x[u] : 0.f;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < PR; ++r) S[r] = sm[LA_OWN(r) * (LA_VC + 1) + vc];
+    __syncthreads();
+}
+template <int PR> __device__ __forceinline__ void la_state_out(const float* S, float* srow, float* sm, int D, int V, int v0) {
+    const int tid = threadIdx.x, vc = tid / LA_DG, dg = tid % LA_DG, c = tid % LA_VC;
+#pragma unroll
+    for (int r = 0; r < PR; ++r) sm[LA_OWN(r) * (LA_VC + 1) + vc] = S[r];
+    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < PR; ++u) {
+        const int d = tid / LA_VC + u * (LA_NT / LA_VC);
+        if (d < D && v0 + c < V) srow[(size_t)d * V + v0 + c] = sm[d * (LA_VC + 1) + c];
+    }
+}
+
 // VEC: q, k, v (bfloat16) and the decay rows start on 16 bytes and D and V are multiples of 8: a fetch is
 // 16 bytes.  Otherwise one element.  (Every loop over the arrays below is unrolled and both lambdas are inlined, so that
 // the arrays stay in registers.)
-#define LA_OWN(r) (PR >= 4 ? ((r) / 4) * 128 + dg * 4 + ((r) % 4) : dg * PR + (r))    // the thread's r-th key channel
-// TB: tokens a block: 16 (8 for the widest heads), or 1 for steps of single tokens, whose workgroups then hold
-// little LDS and few registers, so that many are resident and their round trips to memory overlap.
-template <typename T, int RR, bool CH, bool VEC, int TB, bool PRE>
-__global__ __launch_bounds__(LA_NT) __attribute__((amdgpu_waves_per_eu(1, TB == 1 ? 4 : 2)))
+// TB: tokens a block: 16 (8 for the widest heads).
+template <typename T, int RR, bool CH, bool VEC, bool PRE>
+__global__ __launch_bounds__(LA_NT) __attribute__((amdgpu_waves_per_eu(VEC && !(CH && RR == 16) ? 4 : 1, VEC && !(CH && RR == 16) ? 4 : 2)))
 void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int ldq, int ldk, int ldv,
                              const float* __restrict__ decay, const float* __restrict__ head_decay, float q_scale,
                              float* __restrict__ state, const int* __restrict__ cu_seqlens, const int* __restrict__ seq_slots,
                              float* __restrict__ out, int H, int D, int V, int keep, int qk_rep,
                              const float* __restrict__ v_scale, const float* __restrict__ bonus) {
+    constexpr int TB = la_block<RR>::tokens;
     constexpr int Dp = 16 * RR;                     // key channels, padded
     constexpr int PR = RR / 2;                      // key channels a thread
     constexpr int NQ = CH ? 3 : 2;                  // rows of Dp a token: q, k and, per channel, the decay
     constexpr int per = NQ * Dp + LA_VC;
-    // A fetch is one load and no branch around it.  Two lists of fetches a block: A from q, k and the value
-    // slice (elements of type T), B from the decay rows (fp32).
+    // A fetch is one load and no branch around it.  Three lists of fetches a block: q and k, the value slice (elements
+    // of type T) and the decay rows (fp32).
     constexpr int WA = VEC ? 8 : 1, WB = VEC ? 4 : 1;               // elements a fetch
-    constexpr int CA = (2 * Dp + LA_VC) / WA, CB = CH ? Dp / WB : 1; // fetches a token
-    constexpr int UA = (TB * CA + LA_NT - 1) / LA_NT, UB = CH ? (TB * CB + LA_NT - 1) / LA_NT : 0;   // fetches a thread and block
+    constexpr int NQF = TB * Dp / WA, CV = LA_VC / WA, CB = Dp / WB;   // fetches: q's of a block; of v's slice and of the decay a token
+    constexpr int UQ = (2 * NQF + LA_NT - 1) / LA_NT, UB = CH ? (TB * CB + LA_NT - 1) / LA_NT : 0;      // fetches a thread and block
+    static_assert(TB * CV <= LA_NT, "linear_attn_scan: the value slice is one fetch a thread");
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     constexpr int PV = PR < 4 ? PR : 4;             // key channels an LDS read
-    constexpr int LOOK = TB == 1 ? 1 : RR == 16 ? 2 : 4;            // tokens whose rows are on their way from LDS
+    constexpr int LOOK = RR == 16 ? 2 : CH && RR == 8 ? 3 : 4;            // tokens whose rows are on their way from LDS
     typedef float vec __attribute__((ext_vector_type(PV)));
     using RawA = typename std::conditional<VEC, u32x4, T>::type;
     using RawB = typename std::conditional<VEC, f32x4, float>::type;
-    extern __shared__ __attribute__((aligned(16))) float sm[];      // max(2 * TB * per, Dp * 17) floats
+    extern __shared__ __attribute__((aligned(16))) float sm[];      // max(2 * TB * per, Dp * (LA_VC + 1)) floats
     const int e = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * LA_VC;
     const int tid = threadIdx.x, vc = tid / LA_DG, dg = tid % LA_DG;
     const int t_lo = cu_seqlens[e], t_hi = cu_seqlens[e + 1];
     if (t_lo >= t_hi) return;
-    const int vcol = v0 + vc;
-    const bool vok = vcol < V;
-    float* srow = state + ((size_t)seq_slots[e] * H + h) * (size_t)D * V;
-    for (int i = tid; i < D * LA_VC; i += LA_NT) {
-        const int d = i / LA_VC, c = i % LA_VC;
-        sm[d * (LA_VC + 1) + c] = v0 + c < V ? srow[(size_t)d * V + v0 + c] : 0.f;
-    }
-    __syncthreads();
-    float S[PR];
+    const int hq = h / qk_rep;                              // the head of q and k that this head reads
+    // The thread's fetches: where the next block's lie, what one block further is, whether they are part of the head, and
+    // their place in a block's buffer.
+    const T* pq[UQ]; size_t sq[UQ]; int jq[UQ], wq[UQ]; float mq[UQ]; bool iq[UQ];
+    const float* pb[UB > 0 ? UB : 1]; int jb[UB > 0 ? UB : 1], wb[UB > 0 ? UB : 1]; bool ib[UB > 0 ? UB : 1];
+    const int jv0 = tid / CV, cv = (tid % CV) * WA, wv = jv0 * per + NQ * Dp + cv;
+    const bool iv = jv0 < TB && v0 + cv < V;
+    int jv = t_lo + jv0;
+    const T *pv = v + (size_t)jv * ldv + h * V + v0 + cv, *some = q + (size_t)t_lo * ldq + hq * D;   // (some: for fetches outside the head or past the last token)
 #pragma unroll
-    for (int r = 0; r < PR; ++r) {
-        const int d = LA_OWN(r);
-        S[r] = d < D ? sm[d * (LA_VC + 1) + vc] : 0.f;
+    for (int u = 0; u < UQ; ++u) {
+        const int x = tid + u * LA_NT, part = x / NQF, j = x % NQF / (Dp / WA), d = x % (Dp / WA) * WA;
+        const int ld = part ? ldk : ldq;
+        iq[u] = part < 2 && d < D;
+        jq[u] = t_lo + j; wq[u] = j * per + part * Dp + d; mq[u] = part ? 1.f : q_scale; sq[u] = (size_t)TB * ld;
+        pq[u] = (part ? k : q) + (size_t)(t_lo + j) * ld + hq * D + d;
     }
-    __syncthreads();
+#pragma unroll
+    for (int u = 0; u < UB; ++u) {
+        const int x = tid + u * LA_NT, j = x / CB, d = (x % CB) * WB;
+        ib[u] = j < TB && d < D;
+        jb[u] = t_lo + j; wb[u] = j * per + 2 * Dp + d;
+        pb[u] = decay + ((size_t)(t_lo + j) * H + h) * D + d;
+    }
+    RawA nq[UQ], nv;
+    float fv = 1.f;                                          // the factor on the value fetch
+    RawB nb[UB > 0 ? UB : 1];
+    auto ask = [&]() __attribute__((always_inline)) {        // asks for the next block in order
+#pragma unroll
+        for (int u = 0; u < UQ; ++u) {
+            nq[u] = *(const RawA*)(iq[u] && jq[u] < t_hi ? pq[u] : some);
+            pq[u] += sq[u]; jq[u] += TB;
+        }
+        const bool ok = iv && jv < t_hi;
+        nv = *(const RawA*)(ok ? pv : some);
+        if (v_scale) fv = v_scale[(size_t)(ok ? jv : t_lo) * H + h];
+        pv += (size_t)TB * ldv; jv += TB;
+#pragma unroll
+        for (int u = 0; u < UB; ++u) {
+            nb[u] = *(const RawB*)(ib[u] && jb[u] < t_hi ? pb[u] : decay);
+            pb[u] += (size_t)TB * H * D; jb[u] += TB;
+        }
+    };
+    ask();                                                  // (beside the state's own loads)
+    float* srow = state + ((size_t)seq_slots[e] * H + h) * (size_t)D * V;
+    float S[PR];
+    la_state_in<PR>(S, srow, sm, D, V, v0);
+    if (D < Dp || v0 + LA_VC > V) {                            // what lies outside the head is never written: clear it once
+        for (int i = tid; i < 2 * TB * per; i += LA_NT) sm[i] = 0.f;
+        __syncthreads();
+    }
     const float hd = CH ? 1.f : head_decay[h];
-    const int hq = h / qk_rep, Hq = H / qk_rep;             // the head of q and k that this head reads
-    (void)Hq;
     float ub[PRE ? PR : 1];
     if constexpr (PRE) {
 #pragma unroll
         for (int r = 0; r < PR; ++r) { const int d = LA_OWN(r); ub[r] = d < D ? bonus[(size_t)h * D + d] : 0.f; }
     }
-    RawA na[UA];
-    float ns[UA];                                            // the factor on a fetch's elements
-    RawB nb[UB > 0 ? UB : 1];
+    const int own = la_owner<TB>(dg);                        // the token of a block whose result the thread stores
+    const bool stores = dg % (LA_DG / TB) == 0 && v0 + vc < V;
+    float* po = out + ((size_t)(t_lo + own) * H + h) * V + v0 + vc;
     // Turn `it` computes block `it` from buffer it & 1 while block it + 1 is on its way into the other one;
     // turn -1 only fetches.
     const int n_blocks = (t_hi - t_lo + TB - 1) / TB;
     for (int it = -1; it < n_blocks; ++it) {
-        const int t0 = t_lo + it * TB, tn = t0 + TB;                // this block's first token, the next block's
+        const int t0 = t_lo + it * TB;                              // this block's first token
         const bool more = it + 1 < n_blocks;
-        if (more) {
+        float accs[TB];
+        const float* cur = sm + (it & 1) * (TB * per);
+        const int n_tok = t_hi - t0 < TB ? t_hi - t0 : TB;
+        // A whole block is one stretch of code, its tokens' rows read LOOK tokens ahead of their use (the barriers keep
+        // the compiler from moving the reads back to it): only the state's FMA waits for the token before.
+        vec q4[LOOK][PR / PV], k4[LOOK][PR / PV], a4[CH ? LOOK : 1][PR / PV];
+        float vv[LOOK];
+        auto read = [&](int j) {
+            const float* row = cur + j * per;
+            vv[j % LOOK] = row[NQ * Dp + vc];
 #pragma unroll
-            for (int u = 0; u < UA; ++u) {
-                const int x = tid + u * LA_NT, j = x / CA, e0 = (x % CA) * WA, part = e0 / Dp, d = e0 % Dp;
-                // q and k: channel d of the head; the value slice: column v0 + e0 - 2 Dp
-                const T* base = part == 0 ? q : part == 1 ? k : v;
-                const int ld = part == 0 ? ldq : part == 1 ? ldk : ldv;
-                const int col = part < 2 ? hq * D + d : h * V + v0 + (e0 - 2 * Dp);
-                const bool ok = j < TB && tn + j < t_hi && (part < 2 ? d < D : v0 + (e0 - 2 * Dp) < V);
-                na[u] = *(const RawA*)(base + (size_t)(ok ? tn + j : t_lo) * ld + (ok ? col : 0));
-                ns[u] = part == 0 ? q_scale : (part == 2 && v_scale) ? v_scale[(size_t)(ok ? tn + j : t_lo) * H + h] : 1.f;
+            for (int r = 0; r < PR; r += PV) {
+                q4[j % LOOK][r / PV] = *(const vec*)(row + LA_OWN(r));
+                k4[j % LOOK][r / PV] = *(const vec*)(row + Dp + LA_OWN(r));
+                if constexpr (CH) a4[j % LOOK][r / PV] = *(const vec*)(row + 2 * Dp + LA_OWN(r));
             }
+        };
+        auto token = [&](int j) {                               // the state moves on; the thread's part of the result
+            accs[j] = 0.f;
 #pragma unroll
-            for (int u = 0; u < UB; ++u) {
-                const int x = tid + u * LA_NT, j = x / CB, d = (x % CB) * WB;
-                const bool ok = j < TB && tn + j < t_hi && d < D;
-                nb[u] = *(const RawB*)(decay + ((size_t)(ok ? tn + j : t_lo) * H + h) * D + (ok ? d : 0));
+            for (int r = 0; r < PR; ++r) {
+                float a = hd;
+                if constexpr (CH) a = a4[j % LOOK][r / PV][r % PV];
+                const float qr = q4[j % LOOK][r / PV][r % PV], kv = k4[j % LOOK][r / PV][r % PV] * vv[j % LOOK];
+                if (PRE) accs[j] = fmaf(fmaf(ub[PRE ? r : 0], kv, S[r]), qr, accs[j]);
+                S[r] = fmaf(a, S[r], kv);
+                if (!PRE) accs[j] = fmaf(S[r], qr, accs[j]);
             }
-        }
-        float mine = 0.f;                                           // one token's result (la_owner)
+        };
         if (it >= 0) {
-            const float* cur = sm + (it & 1) * (TB * per);
-            const int n_tok = t_hi - t0 < TB ? t_hi - t0 : TB;
-            float accs[TB];
-            // A whole block is one stretch of code, its tokens' rows read LOOK tokens ahead of their use (the barriers keep
-            // the compiler from moving the reads back to it): only the state's FMA waits for the token before.
-            vec q4[LOOK][PR / PV], k4[LOOK][PR / PV], a4[CH ? LOOK : 1][PR / PV];
-            float vv[LOOK];
-            auto read = [&](int j) {
-                const float* row = cur + j * per;
-                vv[j % LOOK] = row[NQ * Dp + vc];
 #pragma unroll
-                for (int r = 0; r < PR; r += PV) {
-                    q4[j % LOOK][r / PV] = *(const vec*)(row + LA_OWN(r));
-                    k4[j % LOOK][r / PV] = *(const vec*)(row + Dp + LA_OWN(r));
-                    if constexpr (CH) a4[j % LOOK][r / PV] = *(const vec*)(row + 2 * Dp + LA_OWN(r));
-                }
-            };
-            auto token = [&](int j) {                               // the state moves on; the thread's part of the result
-                accs[j] = 0.f;
-#pragma unroll
-                for (int r = 0; r < PR; ++r) {
-                    float a = hd;
-                    if constexpr (CH) a = a4[j % LOOK][r / PV][r % PV];
-                    const float qr = q4[j % LOOK][r / PV][r % PV], kv = k4[j % LOOK][r / PV][r % PV] * vv[j % LOOK];
-                    if (PRE) accs[j] = fmaf(fmaf(ub[PRE ? r : 0], kv, S[r]), qr, accs[j]);
-                    S[r] = fmaf(a, S[r], kv);
-                    if (!PRE) accs[j] = fmaf(S[r], qr, accs[j]);
-                }
-            };
+            for (int j = 0; j < LOOK; ++j) read(j);
+            __builtin_amdgcn_sched_barrier(0x7);
+            ask();
             if (n_tok == TB) {
-#pragma unroll
-                for (int j = 0; j < LOOK; ++j) read(j);
 #pragma unroll
                 for (int j = 0; j < TB; ++j) {
                     __builtin_amdgcn_sched_barrier(0x7);
@@ -234,14 +290,137 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
                     if (j < n_tok) { read(j); token(j); }
                 }
             }
-            mine = la_sums<TB>(accs, dg);
         }
+        // The loads are waited for here, whatever the branches below do: what the compiler holds for pending at the head of the
+        // loop it waits for there, and for this block's stores with it.
+#pragma unroll
+        for (int u = 0; u < UQ; ++u) asm volatile("" : "+v"(nq[u]));
+        asm volatile("" : "+v"(nv), "+v"(fv));
+#pragma unroll
+        for (int u = 0; u < UB; ++u) asm volatile("" : "+v"(nb[u]));
         if (more) {
             float* buf = sm + ((it + 1) & 1) * (TB * per);
+            auto put = [&](float* dst, const RawA& got, float m) __attribute__((always_inline)) {
+                if constexpr (VEC) {
+                    const u32x4 w = got;
+                    f32x4 lo, hi;
+                    lo.x = __builtin_bit_cast(float, w.x << 16) * m, lo.y = __builtin_bit_cast(float, w.x & 0xffff0000u) * m;
+                    lo.z = __builtin_bit_cast(float, w.y << 16) * m, lo.w = __builtin_bit_cast(float, w.y & 0xffff0000u) * m;
+                    hi.x = __builtin_bit_cast(float, w.z << 16) * m, hi.y = __builtin_bit_cast(float, w.z & 0xffff0000u) * m;
+                    hi.z = __builtin_bit_cast(float, w.w << 16) * m, hi.w = __builtin_bit_cast(float, w.w & 0xffff0000u) * m;
+                    *(f32x4*)dst = lo;
+                    *(f32x4*)(dst + 4) = hi;
+                } else dst[0] = to_f32<T>(got) * m;
+            };
+#pragma unroll
+            for (int u = 0; u < UQ; ++u) if (iq[u]) put(buf + wq[u], nq[u], u * LA_NT >= NQF ? 1.f : mq[u]);   // (known for k: no product)
+            if (iv) put(buf + wv, nv, fv);
+#pragma unroll
+            for (int u = 0; u < UB; ++u) if (ib[u]) *(RawB*)(buf + wb[u]) = nb[u];
+        }
+        if (it < 0) { __syncthreads(); continue; }
+        const float mine = la_sums<TB>(accs, dg);
+        // the block's results leave after the next block's rows are in LDS: waiting for those loads does not wait for these stores
+        if (stores && t0 + own < t_hi) *po = mine;
+        po += (size_t)TB * H * V;
+        __syncthreads();
+    }
+    if (keep) la_state_out<PR>(S, srow, sm, D, V, v0);
+}
+
+// Steps of single tokens: workgroups that hold little LDS and few registers, so that many are resident and their round
+// trips to memory overlap (the kernel above with blocks of one token holds up to 77 registers against 52 and was 2 to 16
+// per cent slower).  The same sums in the same order; an entry of more tokens is right too, a token at a time.
+template <typename T, int RR, bool CH, bool VEC, bool PRE>
+__global__ __launch_bounds__(LA_NT) __attribute__((amdgpu_waves_per_eu(1, 4)))
+void linear_attn_single_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int ldq, int ldk, int ldv,
+                             const float* __restrict__ decay, const float* __restrict__ head_decay, float q_scale,
+                             float* __restrict__ state, const int* __restrict__ cu_seqlens, const int* __restrict__ seq_slots,
+                             float* __restrict__ out, int H, int D, int V, int keep, int qk_rep,
+                             const float* __restrict__ v_scale, const float* __restrict__ bonus) {
+    constexpr int Dp = 16 * RR;                     // key channels, padded
+    constexpr int PR = RR / 2;                      // key channels a thread
+    constexpr int NQ = CH ? 3 : 2;                  // rows of Dp a token: q, k and, per channel, the decay
+    constexpr int per = NQ * Dp + LA_VC;
+    // Two lists of fetches: A from q, k and the value slice (elements of type T), B from the decay rows (fp32).
+    constexpr int WA = VEC ? 8 : 1, WB = VEC ? 4 : 1;               // elements a fetch
+    constexpr int CA = (2 * Dp + LA_VC) / WA, CB = CH ? Dp / WB : 1; // fetches a token
+    constexpr int UA = (CA + LA_NT - 1) / LA_NT, UB = CH ? (CB + LA_NT - 1) / LA_NT : 0;     // fetches a thread
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    constexpr int PV = PR < 4 ? PR : 4;             // key channels an LDS read
+    typedef float vec __attribute__((ext_vector_type(PV)));
+    using RawA = typename std::conditional<VEC, u32x4, T>::type;
+    using RawB = typename std::conditional<VEC, f32x4, float>::type;
+    extern __shared__ __attribute__((aligned(16))) float sm[];      // max(2 * per, Dp * (LA_VC + 1)) floats
+    const int e = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * LA_VC;
+    const int tid = threadIdx.x, vc = tid / LA_DG, dg = tid % LA_DG;
+    const int t_lo = cu_seqlens[e], t_hi = cu_seqlens[e + 1];
+    if (t_lo >= t_hi) return;
+    const int vcol = v0 + vc;
+    const bool vok = vcol < V;
+    float* srow = state + ((size_t)seq_slots[e] * H + h) * (size_t)D * V;
+    float S[PR];
+    la_state_in<PR>(S, srow, sm, D, V, v0);
+    const float hd = CH ? 1.f : head_decay[h];
+    const int hq = h / qk_rep;
+    float ub[PRE ? PR : 1];
+    if constexpr (PRE) {
+#pragma unroll
+        for (int r = 0; r < PR; ++r) { const int d = LA_OWN(r); ub[r] = d < D ? bonus[(size_t)h * D + d] : 0.f; }
+    }
+    RawA na[UA];
+    float ns[UA];                                            // the factor on a fetch's elements
+    RawB nb[UB > 0 ? UB : 1];
+    for (int t = t_lo - 1; t < t_hi; ++t) {                 // (turn t_lo - 1 only fetches)
+        const int tn = t + 1;
+        const bool more = tn < t_hi;
+        if (more) {
+#pragma unroll
+            for (int u = 0; u < UA; ++u) {
+                const int x = tid + u * LA_NT, j = x / CA, e0 = (x % CA) * WA, part = e0 / Dp, d = e0 % Dp;
+                // q and k: channel d of the head; the value slice: column v0 + e0 - 2 Dp
+                const T* base = part == 0 ? q : part == 1 ? k : v;
+                const int ld = part == 0 ? ldq : part == 1 ? ldk : ldv;
+                const int col = part < 2 ? hq * D + d : h * V + v0 + (e0 - 2 * Dp);
+                const bool ok = j < 1 && tn + j < t_hi && (part < 2 ? d < D : v0 + (e0 - 2 * Dp) < V);
+                na[u] = *(const RawA*)(base + (size_t)(ok ? tn + j : t_lo) * ld + (ok ? col : 0));
+                ns[u] = part == 0 ? q_scale : (part == 2 && v_scale) ? v_scale[(size_t)(ok ? tn + j : t_lo) * H + h] : 1.f;
+            }
+#pragma unroll
+            for (int u = 0; u < UB; ++u) {
+                const int x = tid + u * LA_NT, j = x / CB, d = (x % CB) * WB;
+                const bool ok = j < 1 && tn + j < t_hi && d < D;
+                nb[u] = *(const RawB*)(decay + ((size_t)(ok ? tn + j : t_lo) * H + h) * D + (ok ? d : 0));
+            }
+        }
+        float mine = 0.f;
+        if (t >= t_lo) {
+            const float* row = sm + ((t - t_lo) & 1) * per;
+            const float vv = row[NQ * Dp + vc];
+#pragma unroll
+            for (int r = 0; r < PR; r += PV) {
+                const vec q4 = *(const vec*)(row + LA_OWN(r)), k4 = *(const vec*)(row + Dp + LA_OWN(r));
+                vec a4;
+                if constexpr (CH) a4 = *(const vec*)(row + 2 * Dp + LA_OWN(r));
+#pragma unroll
+                for (int x = 0; x < PV; ++x) {
+                    float a = hd;
+                    if constexpr (CH) a = a4[x];
+                    const float kv = k4[x] * vv;
+                    if (PRE) mine = fmaf(fmaf(ub[PRE ? r + x : 0], kv, S[r + x]), q4[x], mine);
+                    S[r + x] = fmaf(a, S[r + x], kv);
+                    if (!PRE) mine = fmaf(S[r + x], q4[x], mine);
+                }
+            }
+            mine = la_sums<1>(&mine, dg);
+        }
+        if (more) {
+            float* buf = sm + ((tn - t_lo) & 1) * per;
 #pragma unroll
             for (int u = 0; u < UA; ++u) {
                 const int x = tid + u * LA_NT, j = x / CA, e0 = (x % CA) * WA, part = e0 / Dp;
-                if (j < TB && tn + j < t_hi) {
+                if (j < 1 && tn + j < t_hi) {
                     float* dst = buf + j * per + (part < 2 ? e0 : e0 + (NQ - 2) * Dp);
                     const float m = ns[u];
                     const bool in = ((part < 2) & (e0 % Dp < D)) | ((part >= 2) & (v0 + (e0 - 2 * Dp) < V));
@@ -261,30 +440,15 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
                 const int x = tid + u * LA_NT, j = x / CB, d = (x % CB) * WB;
-                if (j < TB && tn + j < t_hi) {
+                if (j < 1 && tn + j < t_hi) {
                     *(RawB*)(buf + j * per + 2 * Dp + d) = d < D ? nb[u] : RawB{};
                 }
             }
         }
-        // the block's results leave after the next block's rows are in LDS: waiting for those loads does not wait for these stores
-        if (it >= 0 && dg % (LA_DG / TB) == 0) {
-            const int t = t0 + la_owner<TB>(dg);
-            if (t < t_hi && vok) out[((size_t)t * H + h) * V + vcol] = mine;
-        }
+        if (t >= t_lo && dg == 0 && vok) out[((size_t)t * H + h) * V + vcol] = mine;
         __syncthreads();
     }
-    if (keep) {
-#pragma unroll
-        for (int r = 0; r < PR; ++r) {
-            const int d = LA_OWN(r);
-            if (d < D) sm[d * (LA_VC + 1) + vc] = S[r];
-        }
-        __syncthreads();
-        for (int i = tid; i < D * LA_VC; i += LA_NT) {
-            const int d = i / LA_VC, c = i % LA_VC;
-            if (v0 + c < V) srow[(size_t)d * V + v0 + c] = sm[d * (LA_VC + 1) + c];
-        }
-    }
+    if (keep) la_state_out<PR>(S, srow, sm, D, V, v0);
 }
 #undef LA_OWN
 
@@ -293,34 +457,31 @@ struct la_args {
     float* state; const int *cu_seqlens, *seq_slots; float* out; int H, D, V, keep, qk_rep; const float *v_scale, *bonus;
 };
 
-template <typename T, int RR, bool CH, bool VEC, int TB, bool PRE = false>
-static void la_launch(const la_args& a) {
+template <typename T, int RR, bool CH, bool VEC, bool PRE>
+static void la_launch(const la_args& a, bool single) {
+    const int TB = single ? 1 : la_block<RR>::tokens;
     constexpr int Dp = 16 * RR, per = (CH ? 3 : 2) * Dp + LA_VC;
-    constexpr size_t blocks = (size_t)2 * TB * per, tile = (size_t)Dp * (LA_VC + 1);
-    constexpr size_t bytes = (blocks > tile ? blocks : tile) * sizeof(float);
-    static_assert(bytes <= 64 * 1024, "linear_attn_scan: the token blocks must fit the default LDS limit");
-    linear_attn_scan_kernel<T, RR, CH, VEC, TB, PRE><<<a.grid, LA_NT, bytes, a.st>>>(
+    constexpr size_t tile = (size_t)Dp * (LA_VC + 1);
+    static_assert(sizeof(float) * 2 * la_block<RR>::tokens * per <= 64 * 1024, "linear_attn_scan: the token blocks must fit the default LDS limit");
+    const size_t blocks = (size_t)2 * TB * per, bytes = (blocks > tile ? blocks : tile) * sizeof(float);
+    auto* kernel = single ? linear_attn_single_kernel<T, RR, CH, VEC, PRE> : linear_attn_scan_kernel<T, RR, CH, VEC, PRE>;
+    kernel<<<a.grid, LA_NT, bytes, a.st>>>(
         (const T*)a.q, (const T*)a.k, (const T*)a.v, a.ldq, a.ldk, a.ldv, a.decay, a.head_decay, a.q_scale, a.state, a.cu_seqlens,
         a.seq_slots, a.out, a.H, a.D, a.V, a.keep, a.qk_rep, a.v_scale, a.bonus);
 }
 
 template <typename T, bool VEC, int RR>
-static void la_pick_block(const la_args& a, bool single) {
-    constexpr int TB = la_block<RR>::tokens;
-    const bool ch = a.decay != nullptr;
-    if (a.bonus) {                                  // (the caller has made sure that a bonus comes with a decay per channel)
-        if (single) la_launch<T, RR, true, VEC, 1, true>(a); else la_launch<T, RR, true, VEC, TB, true>(a);
-        return;
-    }
-    if (single) { if (ch) la_launch<T, RR, true, VEC, 1>(a); else la_launch<T, RR, false, VEC, 1>(a); }
-    else { if (ch) la_launch<T, RR, true, VEC, TB>(a); else la_launch<T, RR, false, VEC, TB>(a); }
+static void la_pick_decay(const la_args& a, bool single) {
+    if (a.bonus) la_launch<T, RR, true, VEC, true>(a, single);      // (the caller has made sure that a bonus comes with a decay per channel)
+    else if (a.decay) la_launch<T, RR, true, VEC, false>(a, single);
+    else la_launch<T, RR, false, VEC, false>(a, single);
 }
 
 template <typename T, bool VEC>
 static void la_pick(const la_args& a, bool single) {
-    if (a.D <= 64) la_pick_block<T, VEC, 4>(a, single);
-    else if (a.D <= 128) la_pick_block<T, VEC, 8>(a, single);
-    else la_pick_block<T, VEC, 16>(a, single);
+    if (a.D <= 64) la_pick_decay<T, VEC, 4>(a, single);
+    else if (a.D <= 128) la_pick_decay<T, VEC, 8>(a, single);
+    else la_pick_decay<T, VEC, 16>(a, single);
 }
 
 extern "C" int spite_linear_attn_scan(const void* q, const void* k, const void* v, int ldq, int ldk, int ldv, int dtype,

@@ -32,3 +32,31 @@ def test_blocks_of_tokens_match_single_tokens(kind, H, D, V, dtype, lens):
             hipops.linear_attn_scan(q[t:t + 1], k[t:t + 1], v[t:t + 1], single[t:t + 1], s_single, one, slots[i:i + 1], 1, H, D, V,
                                     longest=1, **cut)
     assert torch.equal(whole, single) and torch.equal(s_whole, s_single)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["channel", "head"])
+@pytest.mark.parametrize("D,V,dtype", [(6, 10, torch.float32), (24, 40, torch.bfloat16), (72, 24, torch.bfloat16), (130, 20, torch.bfloat16)])
+@pytest.mark.parametrize("T", [1, 16, 37])
+def test_a_head_takes_nothing_from_its_neighbours(kind, D, V, dtype, T):
+    """Heads that fill no whole row of lanes: what lies beside a head in q, k, v and the decay, and beyond the last token, is
+    not a number, and neither the head's results nor its state may differ from those of a batch that holds only numbers."""
+    from spite_amd.csrc import hipops
+    torch.manual_seed(D * T)
+    H, pad = 3, 20
+    numbers = (torch.randn(T + pad, H * (2 * D + V), device="cuda") * 0.5).to(dtype)
+    decay = torch.rand(T + pad, H * D, device="cuda")
+    start = torch.randn(1, H, D, V, device="cuda")
+    cu, slot = torch.tensor([0, T], dtype=torch.int32, device="cuda"), torch.zeros(1, dtype=torch.int32, device="cuda")
+    got = []
+    for spoil in (False, True):
+        row, a = numbers.clone(), decay.clone()
+        if spoil:                                   # heads 0 and 2, and every row past the request's last
+            for part, w in ((row[:, :H * D], D), (row[:, H * D:2 * H * D], D), (row[:, 2 * H * D:], V), (a, D)):
+                part[:, :w] = part[:, 2 * w:] = float("nan")
+                part[T:] = float("nan")
+        opt = dict(decay=a[:T]) if kind == "channel" else dict(head_decay=torch.full((H,), 0.75, device="cuda"))
+        out, state = torch.zeros(T, H * V, device="cuda"), start.clone()
+        hipops.linear_attn_scan(row[:T, :H * D], row[:T, H * D:2 * H * D], row[:T, 2 * H * D:], out, state, cu, slot, 1, H, D, V, **opt)
+        got.append((out[:, V:2 * V].clone(), state[:, 1].clone()))
+    assert torch.isfinite(got[0][0]).all() and torch.equal(got[0][0], got[1][0]) and torch.equal(got[0][1], got[1][1])
