@@ -22,7 +22,8 @@
 //
 // Tiles: S^T tile tt (of 2) holds the keys (r/4)*8 + tt*4 + r%4 of the block in its rows r, so the
 // eight scores a lane holds are eight consecutive keys: P^T is the next product's operand without a
-// shuffle.  Scores, maximum (in the exponent's units, base 2), sum and the output are fp32.
+// shuffle.  Scores, maximum, sum and the output are fp32; a score less the maximum goes into the exponent's units, base 2, and
+// not the score: rounded there, scores of some thousands would each be off by more than their difference is.
 //
 // Few workgroups with many keys (decoded tokens of a few requests over long contexts): the blocks
 // of keys are dealt to `n_splits` workgroups a work item (grid.y), each leaves a record (output not
@@ -36,12 +37,18 @@
 typedef short s16x4 __attribute__((ext_vector_type(4)));
 static __device__ __attribute__((aligned(16))) const unsigned lm_zeros[4] = {0, 0, 0, 0};      // what a row that is not read holds
 
+// A scaled score, rounded: the maximum is taken off it afterwards, not in the same operation, with masks or without.
+static __device__ __forceinline__ float lm_scaled(float s, float scale) {
+#pragma clang fp contract(off)
+    return s * scale;
+}
+
 template <int KQ, int NV>   // Dk <= 32*KQ, R <= 16*NV
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(KQ > 6 ? 2 : 4)))
 void attn_latent_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict__ kv_pages, bf16* __restrict__ out,
                              const int* __restrict__ positions, const int* __restrict__ seq_of_token,
                              const int* __restrict__ block_table, int max_blocks, const int* __restrict__ wg,
-                             int H, int Dk, int R, int ps, int vis, int span, float scale_log2e,
+                             int H, int Dk, int R, int ps, int vis, int span, float scale,
                              float* __restrict__ part, int n_splits) {
     constexpr int PP = KQ * 4, BUF = 32 * PP * 16;                  // 16-byte pieces of a staged row; bytes of a block
     constexpr int XI = (PP / 2 + 7) / 8;                            // loads of a kilobyte a wave and block
@@ -166,28 +173,28 @@ void attn_latent_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict_
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) { s[tt][i] *= scale_log2e; mx = fmaxf(mx, s[tt][i]); }
+                for (int i = 0; i < 4; ++i) { s[tt][i] = lm_scaled(s[tt][i], scale); mx = fmaxf(mx, s[tt][i]); }
         } else {
 #pragma unroll
             for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
                 for (int i = 0; i < 4; ++i) {
                     const int j = blk0 + g4 * 8 + tt * 4 + i;
-                    s[tt][i] = row_ok && j >= my_lo && j <= my_p ? (tab[tt * 4 + i] == -1 ? NAN : s[tt][i] * scale_log2e) : -INFINITY;
+                    s[tt][i] = row_ok && j >= my_lo && j <= my_p ? (tab[tt * 4 + i] == -1 ? NAN : lm_scaled(s[tt][i], scale)) : -INFINITY;
                     mx = fmaxf(mx, s[tt][i]);
                 }
         }
         mx = rows4_max(mx);
         const float m_new = fmaxf(m_run, mx);
         const float m_use = m_new == -INFINITY ? 0.f : m_new;       // (a row that has seen no key yet: weights of zero)
-        const float alpha = __builtin_amdgcn_exp2f(m_run - m_use);
+        const float alpha = __expf(m_run - m_use);
         float sum = 0.f;
         bf16x8 pf;
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const float e = __builtin_amdgcn_exp2f(s[tt][i] - m_use);
+                const float e = __expf(s[tt][i] - m_use);
                 sum += e;
                 pf[tt * 4 + i] = (bf16)e;
             }
@@ -246,7 +253,7 @@ void attn_latent_mfma_kernel(const bf16* __restrict__ q, const bf16* __restrict_
 // Joins the records [row][split][R + 2] of a split call: one workgroup a query row.
 __global__ __launch_bounds__(256)
 void attn_latent_join_kernel(const float* __restrict__ part, bf16* __restrict__ out, int R, int n_splits) {
-    __shared__ float wsh[1024];          // weight of every split: exp2(m_s - M) / L
+    __shared__ float wsh[1024];          // weight of every split: exp(m_s - M) / L
     __shared__ float red[8];
     const size_t row = blockIdx.x;
     const float* rec = part + row * n_splits * (R + 2);
@@ -268,7 +275,7 @@ void attn_latent_join_kernel(const float* __restrict__ part, bf16* __restrict__ 
 #pragma unroll
     for (int u = 0; u < 4; ++u) {
         const int s = tid + u * 256;
-        const float w = ms[u] == -INFINITY ? 0.f : exp2f(ms[u] - M);
+        const float w = ms[u] == -INFINITY ? 0.f : __expf(ms[u] - M);
         if (s < n_splits) wsh[s] = w;
         L += w * ls[u];
     }
@@ -317,7 +324,7 @@ extern "C" int spite_attn_latent_mfma(const void* q, const void* kv_pages, void*
         if (!allowed) { hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh); \
             if (e != hipSuccess) return sp_fail("latent attention: %zu bytes of LDS refused: %s", sh, hipGetErrorString(e)); allowed = true; } \
         kern<<<dim3(n_wg, n_splits), 512, sh, st>>>((const bf16*)q, (const bf16*)kv_pages, (bf16*)out, positions, seq_of_token, \
-                                        block_table, max_blocks, wg, H, Dk, R, page_size, vis, span, scale * 1.4426950408889634f, part, n_splits); } while (0)
+                                        block_table, max_blocks, wg, H, Dk, R, page_size, vis, span, scale, part, n_splits); } while (0)
     if (kq <= 6 && nv <= 8) SP_LM(6, 8);
     else if (kq <= 10 && nv <= 16) SP_LM(10, 16);
     else SP_LM(18, 32);

@@ -320,6 +320,35 @@ def test_latent_attention_over_many_blocks(Hh, Dk, R, ps, vis, span):
         assert bool(torch.isnan(out[reads]).all()) and torch.equal(out[~reads], whole[n_splits][~reads])
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("Hh,Dk,R", [(3, 96, 64), (2, 320, 256), (2, 576, 512)])
+@pytest.mark.parametrize("n_splits", [1, 3])
+def test_latent_attention_weighs_large_scores_by_their_difference(Hh, Dk, R, n_splits):
+    """Scores of 1,024 * 1,024 and some quarters more or less, each a number of fp32: a weight is exp(score - maximum), whose exponent
+    is the exact difference.  Whatever is rounded at the scores' own size is off by some hundredths, several times what follows from
+    bfloat16: a weight and the result rounded once, 2^-8 of it at most; the sums' own rounding is some 2^-20."""
+    from spite_amd.csrc import hipops
+    n, ps = 200, 32
+    g = torch.Generator().manual_seed(Dk)
+    kv = torch.randn(n, Dk, generator=g).bfloat16()
+    kv[:, 0], kv[:, 1] = 1024.0, (torch.randint(-12, 13, (n,), generator=g) * 0.25).bfloat16()
+    q = torch.zeros(Hh, Dk)
+    q[:, 0], q[:, 1] = 1024.0, torch.tensor([1.0, -1.0, 2.0])[:Hh]
+    pages = torch.zeros(-(-n // ps), 1, ps, Dk, dtype=torch.bfloat16)
+    pages.view(-1, Dk)[:n] = kv
+    weights = torch.softmax(q.double() @ kv.double().t(), 1)
+    want, size = weights @ kv[:, :R].double(), weights @ kv[:, :R].double().abs()
+    dev = "cuda:0"
+    wg, (n_wg, most) = hipops.latent_workgroups([1], [0, 1], Hh)
+    table = torch.arange(pages.shape[0], dtype=torch.int32).view(1, -1).to(dev)
+    out = torch.empty(Hh, R, dtype=torch.bfloat16, device=dev)
+    scratch = torch.empty(Hh * n_splits * (R + 2), device=dev) if n_splits > 1 else None
+    hipops.attn_latent_mfma(q.bfloat16().to(dev), pages.to(dev), out, torch.tensor([n - 1], dtype=torch.int32, device=dev),
+                            torch.zeros(1, dtype=torch.int32, device=dev), table, torch.from_numpy(wg).to(dev), n_wg, most, 1, Hh, Dk, R,
+                            "full", 0, 1.0, n_splits=n_splits, scratch=scratch)
+    assert bool(((out.cpu().double() - want).abs() <= 2.0 ** -8 * (size + want.abs()) + 2.0 ** -18 * size).all())
+
+
 # ------------------------------------------------------------------------------------------ the model in the engine
 @pytest.fixture(scope="module")
 def models(tmp_path_factory):
