@@ -48,7 +48,7 @@ extern "C" int spite_channel_decay(float* z, const float* bias, int T, int width
 // ------------------------------------------------------------------ the recurrence, token by token
 // A workgroup of 512 threads takes 16 value columns of one head of one entry of the step and walks the
 // entry's tokens in order.  Thread (vc, dg) = (tid / 32, tid % 32) holds, in registers, the state's elements
-// S[d][v0 + vc] and S[d][v0 + vc + 8] for D / 32 key channels d (four consecutive ones at 4 dg, and again 128
+// S[d][v0 + vc] for D / 32 key channels d (four consecutive ones at 4 dg, and again 128
 // further on for the widest heads; two at 2 dg for heads up to 64): 32 lanes read 512 consecutive bytes of a
 // token's q, k or decay row from LDS in one wide read without bank conflicts.  The tokens' q, k, decay and value slice go
 // through LDS a block of tokens at a time, two buffers: the next block's loads are in flight while this block is computed,
@@ -57,14 +57,19 @@ extern "C" int spite_channel_decay(float* z, const float* bias, int T, int width
 // for the tokens of a block together (la_sums).  The state tile goes through LDS on the way in and out, so that its rows
 // are read and written 64 bytes at a time.
 // Bound by the instructions that a wave issues: at D = 128, 12 a token for the state and 17 around them (the reads from LDS,
-// the sums, the fetches), 185 cycles a token with two waves a SIMD.  So a fetch is set up once and costs a compare, a select
-// and an add a block; k, and what lies outside a head, take no product or select on the way into LDS; and no store is waited
-// for (an asm statement below pins where the loads are waited for: with the loads in branches the compiler also waited at
-// the head of each block, for the block's stores with them).  1,531 tokens, one request, V = D = 128: 114 us for 16 heads
-// and 123 for 32 (128 and 135 before this), decay per channel 146 (160) and 226 for 40 heads (250, 128 registers, so that two
-// workgroups fit a CU: 264 with 134); heads of 64: 96 (104); 800 tokens, 8 heads of 256: 107 (121).  1,000 tokens of fp32,
-// 16 heads: 88 (124).  Tried: two columns a lane, which halves the reads of q and k (168 us with 16 columns a workgroup);
-// half the columns a workgroup where 128 workgroups leave CUs idle (122, 77 for heads of 64); loads two blocks ahead (124).
+// the sums, the fetches), 180 cycles a token with two waves a SIMD.  So a fetch is set up once and costs a compare, a select
+// and an add a block; k, and what lies outside a head, take no product or select on the way into LDS, tokens past the last none at all;
+// and no store is waited for (an asm statement below pins where the loads are waited for: with the loads in branches the compiler
+// also waited at the head of each block, for the block's stores with them).  At the start, what is the same for a
+// workgroup is asked for at once, then the state, then the first tokens.  128 registers, so that two workgroups fit a CU, for
+// the widest heads too (their rows are read one token ahead where there is a decay per channel).
+// us, and in brackets before a fetch was set up once: 1,531 tokens, one request, V = D = 128: 107 for 16 heads
+// and 108 for 32 (126 and 127), decay per channel 135 (159) and 218 for 40 heads (248); heads of 64: 93 (104);
+// 800 tokens, 8 heads of 256: 102 (122), decay per channel 124 (146); 3 requests of 700 tokens, 40 heads of 256 with a decay
+// per channel: 363 (406; 453 with 153 registers); 32 of 17 tokens, 16 heads: 64 (83; 102).  1,000 tokens of fp32,
+// 16 heads: 83 (121).  Tried: two columns a lane, which halves the reads of q and k (168 us with 16 columns a workgroup);
+// half the columns a workgroup where 128 workgroups leave CUs idle (122, 77 for heads of 64); loads two blocks ahead (124); addresses
+// from one scalar base and 32-bit offsets (fp32 5 to 14 % slower, short entries no faster).
 // The order of every sum is fixed by D alone: the bits do not depend on how a request's tokens are cut.
 #define LA_VC 16        // value columns a workgroup
 #define LA_NT 512       // threads a workgroup: 16 columns x 32 lanes
@@ -110,15 +115,17 @@ template <int TB> __device__ __forceinline__ int la_owner(int l) { return TB == 
 
 // The workgroup's columns of the state, in and out through LDS (D rows of LA_VC + 1): a thread's PR loads are all asked for
 // before the first is waited for (one
-// after another, a step of single tokens of 8 requests with 16 heads of 128 took 7.4 us for 6.9, of 32 requests 21.3 for 18.7).
-template <int PR> __device__ __forceinline__ void la_state_in(float* S, const float* srow, float* sm, int D, int V, int v0) {
-    const int tid = threadIdx.x, vc = tid / LA_DG, dg = tid % LA_DG, c = tid % LA_VC;
-    float x[PR];
+// after another, a step of single tokens of 8 requests with 16 heads of 128 took 7.5 us for 7.0, of 32 requests 21.3 for 18.4).
+template <int PR> __device__ __forceinline__ void la_state_ask(float* x, const float* srow, int D, int V, int v0) {
+    const int tid = threadIdx.x, c = tid % LA_VC;
 #pragma unroll
     for (int u = 0; u < PR; ++u) {
         const int d = tid / LA_VC + u * (LA_NT / LA_VC);
         x[u] = srow[d < D && v0 + c < V ? (size_t)d * V + v0 + c : 0];
     }
+}
+template <int PR> __device__ __forceinline__ void la_state_in(float* S, const float* x, float* sm, int D, int V, int v0) {
+    const int tid = threadIdx.x, vc = tid / LA_DG, dg = tid % LA_DG, c = tid % LA_VC;
 #pragma unroll
     for (int u = 0; u < PR; ++u) {
         const int d = tid / LA_VC + u * (LA_NT / LA_VC);
@@ -146,7 +153,7 @@ template <int PR> __device__ __forceinline__ void la_state_out(const float* S, f
 // the arrays stay in registers.)
 // TB: tokens a block: 16 (8 for the widest heads).
 template <typename T, int RR, bool CH, bool VEC, bool PRE>
-__global__ __launch_bounds__(LA_NT) __attribute__((amdgpu_waves_per_eu(VEC && !(CH && RR == 16) ? 4 : 1, VEC && !(CH && RR == 16) ? 4 : 2)))
+__global__ __launch_bounds__(LA_NT) __attribute__((amdgpu_waves_per_eu(VEC ? 4 : 1, VEC ? 4 : 2)))
 void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int ldq, int ldk, int ldv,
                              const float* __restrict__ decay, const float* __restrict__ head_decay, float q_scale,
                              float* __restrict__ state, const int* __restrict__ cu_seqlens, const int* __restrict__ seq_slots,
@@ -166,16 +173,25 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
     typedef float f32x4 __attribute__((ext_vector_type(4)));
     constexpr int PV = PR < 4 ? PR : 4;             // key channels an LDS read
-    constexpr int LOOK = RR == 16 ? 2 : CH && RR == 8 ? 3 : 4;            // tokens whose rows are on their way from LDS
+    constexpr int LOOK = RR == 16 ? (CH && VEC ? 1 : 2) : CH && RR == 8 ? 3 : 4;            // tokens whose rows are on their way from LDS
     typedef float vec __attribute__((ext_vector_type(PV)));
     using RawA = typename std::conditional<VEC, u32x4, T>::type;
     using RawB = typename std::conditional<VEC, f32x4, float>::type;
     extern __shared__ __attribute__((aligned(16))) float sm[];      // max(2 * TB * per, Dp * (LA_VC + 1)) floats
     const int e = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * LA_VC;
     const int tid = threadIdx.x, vc = tid / LA_DG, dg = tid % LA_DG;
-    const int t_lo = cu_seqlens[e], t_hi = cu_seqlens[e + 1];
+    // (all that is the same for the workgroup at once: left where they are used, these loads are five more waits in a row,
+    // half a microsecond that an entry of few tokens cannot hide)
+    asm volatile("" :: "s"(q), "s"(k), "s"(v), "s"(decay), "s"(state), "s"(out), "s"(v_scale), "s"(H), "s"(D), "s"(V), "s"(keep), "s"(qk_rep),
+                 "s"(ldq), "s"(ldk), "s"(ldv), "s"(q_scale));
+    int t_lo = cu_seqlens[e], t_hi = cu_seqlens[e + 1], slot = seq_slots[e];
+    float hd = CH ? 1.f : head_decay[h];
+    asm volatile("" : "+s"(t_lo), "+s"(t_hi), "+s"(slot), "+s"(hd));
     if (t_lo >= t_hi) return;
-    const int hq = h / qk_rep;                              // the head of q and k that this head reads
+    float* srow = state + ((size_t)slot * H + h) * (size_t)D * V;
+    float S[PR], x[PR];
+    la_state_ask<PR>(x, srow, D, V, v0);                    // (on its way while the fetches are set up)
+    const int hq = qk_rep == 1 ? h : h / qk_rep;            // the head of q and k that this head reads
     // The thread's fetches: where the next block's lie, what one block further is, whether they are part of the head, and
     // their place in a block's buffer.
     const T* pq[UQ]; size_t sq[UQ]; int jq[UQ], wq[UQ]; float mq[UQ]; bool iq[UQ];
@@ -201,32 +217,41 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
     }
     RawA nq[UQ], nv;
     float fv = 1.f;                                          // the factor on the value fetch
+    asm volatile("" : "+v"(fv));                             // (written here: behind a load it would wait for it)
     RawB nb[UB > 0 ? UB : 1];
+    bool gq[UQ], gv = false, gb[UB > 0 ? UB : 1];            // which of the fetches asked for last there are
     auto ask = [&]() __attribute__((always_inline)) {        // asks for the next block in order
 #pragma unroll
         for (int u = 0; u < UQ; ++u) {
-            nq[u] = *(const RawA*)(iq[u] && jq[u] < t_hi ? pq[u] : some);
+            const bool ok = iq[u] && jq[u] < t_hi;
+            gq[u] = VEC ? ok : iq[u];
+            nq[u] = *(const RawA*)(ok ? pq[u] : some);
             pq[u] += sq[u]; jq[u] += TB;
         }
-        const bool ok = iv && jv < t_hi;
-        nv = *(const RawA*)(ok ? pv : some);
-        if (v_scale) fv = v_scale[(size_t)(ok ? jv : t_lo) * H + h];
+        gv = iv && jv < t_hi;
+        nv = *(const RawA*)(gv ? pv : some);
+        if (v_scale) fv = v_scale[(size_t)(gv ? jv : t_lo) * H + h];
         pv += (size_t)TB * ldv; jv += TB;
 #pragma unroll
         for (int u = 0; u < UB; ++u) {
-            nb[u] = *(const RawB*)(ib[u] && jb[u] < t_hi ? pb[u] : decay);
+            const bool ok = ib[u] && jb[u] < t_hi;
+            gb[u] = VEC ? ok : ib[u];
+            nb[u] = *(const RawB*)(ok ? pb[u] : decay);
             pb[u] += (size_t)TB * H * D; jb[u] += TB;
         }
     };
-    ask();                                                  // (beside the state's own loads)
-    float* srow = state + ((size_t)seq_slots[e] * H + h) * (size_t)D * V;
-    float S[PR];
-    la_state_in<PR>(S, srow, sm, D, V, v0);
-    if (D < Dp || v0 + LA_VC > V) {                            // what lies outside the head is never written: clear it once
-        for (int i = tid; i < 2 * TB * per; i += LA_NT) sm[i] = 0.f;
-        __syncthreads();
+    ask();
+    la_state_in<PR>(S, x, sm, D, V, v0);
+    if (D < Dp || v0 + LA_VC > V) {                            // the places of what lies outside the head, in both buffers: never written again
+        auto clear = [&](int at, int n) __attribute__((always_inline)) {
+            for (int i = 0; i < n; ++i) sm[at + i] = sm[TB * per + at + i] = 0.f;
+        };
+#pragma unroll
+        for (int u = 0; u < UQ; ++u) if (!iq[u] && tid + u * LA_NT < 2 * NQF) clear(wq[u], WA);
+        if (jv0 < TB && !iv) clear(wv, WA);
+#pragma unroll
+        for (int u = 0; u < UB; ++u) if (!ib[u] && tid + u * LA_NT < TB * CB) clear(wb[u], WB);
     }
-    const float hd = CH ? 1.f : head_decay[h];
     float ub[PRE ? PR : 1];
     if constexpr (PRE) {
 #pragma unroll
@@ -274,8 +299,9 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
 #pragma unroll
             for (int j = 0; j < LOOK; ++j) read(j);
             __builtin_amdgcn_sched_barrier(0x7);
-            ask();
+            if (!VEC) ask();
             if (n_tok == TB) {
+                if (VEC) ask();
 #pragma unroll
                 for (int j = 0; j < TB; ++j) {
                     __builtin_amdgcn_sched_barrier(0x7);
@@ -283,7 +309,7 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
                     if (j + LOOK < TB) read(j + LOOK);
                 }
                 __builtin_amdgcn_sched_barrier(0x7);
-            } else {
+            } else {                                            // (the last block: nothing left to ask for)
 #pragma unroll
                 for (int j = 0; j < TB; ++j) {
                     accs[j] = 0.f;
@@ -313,10 +339,10 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
                 } else dst[0] = to_f32<T>(got) * m;
             };
 #pragma unroll
-            for (int u = 0; u < UQ; ++u) if (iq[u]) put(buf + wq[u], nq[u], u * LA_NT >= NQF ? 1.f : mq[u]);   // (known for k: no product)
-            if (iv) put(buf + wv, nv, fv);
+            for (int u = 0; u < UQ; ++u) if (gq[u]) put(buf + wq[u], nq[u], u * LA_NT >= NQF ? 1.f : mq[u]);   // (known for k: no product)
+            if (gv) put(buf + wv, nv, fv);
 #pragma unroll
-            for (int u = 0; u < UB; ++u) if (ib[u]) *(RawB*)(buf + wb[u]) = nb[u];
+            for (int u = 0; u < UB; ++u) if (gb[u]) *(RawB*)(buf + wb[u]) = nb[u];
         }
         if (it < 0) { __syncthreads(); continue; }
         const float mine = la_sums<TB>(accs, dg);
@@ -329,8 +355,8 @@ void linear_attn_scan_kernel(const T* __restrict__ q, const T* __restrict__ k, c
 }
 
 // Steps of single tokens: workgroups that hold little LDS and few registers, so that many are resident and their round
-// trips to memory overlap (the kernel above with blocks of one token holds up to 77 registers against 52 and was 2 to 16
-// per cent slower).  The same sums in the same order; an entry of more tokens is right too, a token at a time.
+// trips to memory overlap (the scan, 32 requests of a token, 16 heads of 128: 26.7 us for 18.4).  The same sums in the same order; an
+// entry of more tokens is right too, a token at a time.
 template <typename T, int RR, bool CH, bool VEC, bool PRE>
 __global__ __launch_bounds__(LA_NT) __attribute__((amdgpu_waves_per_eu(1, 4)))
 void linear_attn_single_kernel(const T* __restrict__ q, const T* __restrict__ k, const T* __restrict__ v, int ldq, int ldk, int ldv,
@@ -361,7 +387,9 @@ void linear_attn_single_kernel(const T* __restrict__ q, const T* __restrict__ k,
     const bool vok = vcol < V;
     float* srow = state + ((size_t)seq_slots[e] * H + h) * (size_t)D * V;
     float S[PR];
-    la_state_in<PR>(S, srow, sm, D, V, v0);
+    float x[PR];
+    la_state_ask<PR>(x, srow, D, V, v0);
+    la_state_in<PR>(S, x, sm, D, V, v0);
     const float hd = CH ? 1.f : head_decay[h];
     const int hq = h / qk_rep;
     float ub[PRE ? PR : 1];
@@ -378,20 +406,20 @@ void linear_attn_single_kernel(const T* __restrict__ q, const T* __restrict__ k,
         if (more) {
 #pragma unroll
             for (int u = 0; u < UA; ++u) {
-                const int x = tid + u * LA_NT, j = x / CA, e0 = (x % CA) * WA, part = e0 / Dp, d = e0 % Dp;
+                const int e0 = (tid + u * LA_NT) * WA, part = e0 / Dp, d = e0 % Dp;
                 // q and k: channel d of the head; the value slice: column v0 + e0 - 2 Dp
                 const T* base = part == 0 ? q : part == 1 ? k : v;
                 const int ld = part == 0 ? ldq : part == 1 ? ldk : ldv;
                 const int col = part < 2 ? hq * D + d : h * V + v0 + (e0 - 2 * Dp);
-                const bool ok = j < 1 && tn + j < t_hi && (part < 2 ? d < D : v0 + (e0 - 2 * Dp) < V);
-                na[u] = *(const RawA*)(base + (size_t)(ok ? tn + j : t_lo) * ld + (ok ? col : 0));
-                ns[u] = part == 0 ? q_scale : (part == 2 && v_scale) ? v_scale[(size_t)(ok ? tn + j : t_lo) * H + h] : 1.f;
+                const bool ok = e0 < CA * WA && (part < 2 ? d < D : v0 + (e0 - 2 * Dp) < V);
+                na[u] = *(const RawA*)(base + (size_t)(ok ? tn : t_lo) * ld + (ok ? col : 0));
+                ns[u] = part == 0 ? q_scale : (part == 2 && v_scale) ? v_scale[(size_t)(ok ? tn : t_lo) * H + h] : 1.f;
             }
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
-                const int x = tid + u * LA_NT, j = x / CB, d = (x % CB) * WB;
-                const bool ok = j < 1 && tn + j < t_hi && d < D;
-                nb[u] = *(const RawB*)(decay + ((size_t)(ok ? tn + j : t_lo) * H + h) * D + (ok ? d : 0));
+                const int d = (tid + u * LA_NT) * WB;
+                const bool ok = d < D;
+                nb[u] = *(const RawB*)(decay + ((size_t)(ok ? tn : t_lo) * H + h) * D + (ok ? d : 0));
             }
         }
         float mine = 0.f;
@@ -419,9 +447,9 @@ void linear_attn_single_kernel(const T* __restrict__ q, const T* __restrict__ k,
             float* buf = sm + ((tn - t_lo) & 1) * per;
 #pragma unroll
             for (int u = 0; u < UA; ++u) {
-                const int x = tid + u * LA_NT, j = x / CA, e0 = (x % CA) * WA, part = e0 / Dp;
-                if (j < 1 && tn + j < t_hi) {
-                    float* dst = buf + j * per + (part < 2 ? e0 : e0 + (NQ - 2) * Dp);
+                const int e0 = (tid + u * LA_NT) * WA, part = e0 / Dp;
+                if (e0 < CA * WA) {
+                    float* dst = buf + (part < 2 ? e0 : e0 + (NQ - 2) * Dp);
                     const float m = ns[u];
                     const bool in = ((part < 2) & (e0 % Dp < D)) | ((part >= 2) & (v0 + (e0 - 2 * Dp) < V));
                     const RawA got = in ? na[u] : RawA{};
@@ -439,10 +467,8 @@ void linear_attn_single_kernel(const T* __restrict__ q, const T* __restrict__ k,
             }
 #pragma unroll
             for (int u = 0; u < UB; ++u) {
-                const int x = tid + u * LA_NT, j = x / CB, d = (x % CB) * WB;
-                if (j < 1 && tn + j < t_hi) {
-                    *(RawB*)(buf + j * per + 2 * Dp + d) = d < D ? nb[u] : RawB{};
-                }
+                const int d = (tid + u * LA_NT) * WB;
+                if (d < Dp) *(RawB*)(buf + 2 * Dp + d) = d < D ? nb[u] : RawB{};
             }
         }
         if (t >= t_lo && dg == 0 && vok) out[((size_t)t * H + h) * V + vcol] = mine;
@@ -450,38 +476,165 @@ void linear_attn_single_kernel(const T* __restrict__ q, const T* __restrict__ k,
     }
     if (keep) la_state_out<PR>(S, srow, sm, D, V, v0);
 }
+
+// Heads of up to 64 where instructions and not round trips are what a workgroup waits for (the rule is in spite_linear_attn_scan): one
+// fetch a thread covers q, k and the value slice of a block of 16 tokens, its address is found again for each block, what lies outside a head
+// goes to LDS as zeros: some 40 instructions less than the scan before the first token, and fewer loads a block.  bfloat16 in pieces of
+// 16 bytes.  The same sums in the same order.
+template <bool CH, bool PRE>
+__global__ __launch_bounds__(LA_NT) __attribute__((amdgpu_waves_per_eu(1, 2)))
+void linear_attn_blocks_kernel(const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v, int ldq, int ldk, int ldv,
+                               const float* __restrict__ decay, const float* __restrict__ head_decay, float q_scale,
+                               float* __restrict__ state, const int* __restrict__ cu_seqlens, const int* __restrict__ seq_slots,
+                               float* __restrict__ out, int H, int D, int V, int keep, int qk_rep,
+                               const float* __restrict__ v_scale, const float* __restrict__ bonus) {
+    constexpr int TB = 16, Dp = 64, PR = 2, LOOK = 4;               // tokens a block; key channels, padded, and a thread's; tokens read ahead
+    constexpr int NQ = CH ? 3 : 2, per = NQ * Dp + LA_VC;           // rows of Dp a token, its floats in LDS
+    constexpr int CA = (2 * Dp + LA_VC) / 8, CB = Dp / 4;           // fetches a token: q, k and the value slice; the decay
+    static_assert(TB * CA <= LA_NT && TB * CB <= LA_NT && la_block<4>::tokens == TB, "linear_attn_blocks: a fetch of each kind a thread");
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    typedef float f32x4 __attribute__((ext_vector_type(4)));
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    extern __shared__ __attribute__((aligned(16))) float sm[];      // 2 * TB * per floats
+    const int e = blockIdx.x, h = blockIdx.y, v0 = blockIdx.z * LA_VC;
+    const int tid = threadIdx.x, vc = tid / LA_DG, dg = tid % LA_DG;
+    const int t_lo = cu_seqlens[e], t_hi = cu_seqlens[e + 1];
+    if (t_lo >= t_hi) return;
+    float* srow = state + ((size_t)seq_slots[e] * H + h) * (size_t)D * V;
+    float S[PR], x[PR];
+    la_state_ask<PR>(x, srow, D, V, v0);
+    la_state_in<PR>(S, x, sm, D, V, v0);
+    const float hd = CH ? 1.f : head_decay[h];
+    float ub[PR];
+    if constexpr (PRE) {
+#pragma unroll
+        for (int r = 0; r < PR; ++r) { const int d = LA_OWN(r); ub[r] = d < D ? bonus[(size_t)h * D + d] : 0.f; }
+    }
+    // the thread's fetches: token ja of a block and elements ea .. + 7 of its row of q, k and value slice; token jb and channels db .. + 3
+    const int ja = tid / CA, ea = tid % CA * 8, part = ea / Dp, hq = h / qk_rep;
+    const bf16* base = part == 0 ? q : part == 1 ? k : v;
+    const int ld = part == 0 ? ldq : part == 1 ? ldk : ldv, col = part < 2 ? hq * D + ea % Dp : h * V + v0 + (ea - 2 * Dp);
+    const bool in = part < 2 ? ea % Dp < D : v0 + (ea - 2 * Dp) < V;
+    const int jb = tid / CB, db = tid % CB * 4;
+    u32x4 na;
+    f32x4 nb;
+    float ns;                                                // the factor on the fetch's elements
+    const int n_blocks = (t_hi - t_lo + TB - 1) / TB;
+    for (int it = -1; it < n_blocks; ++it) {                 // (turns as in the scan)
+        const int t0 = t_lo + it * TB, tn = t0 + TB;                // this block's first token, the next block's
+        const bool more = it + 1 < n_blocks;
+        if (more) {
+            const bool ok = ja < TB && tn + ja < t_hi && in;
+            na = *(const u32x4*)(base + (size_t)(ok ? tn + ja : t_lo) * ld + (ok ? col : 0));
+            ns = part == 0 ? q_scale : (part == 2 && v_scale) ? v_scale[(size_t)(ok ? tn + ja : t_lo) * H + h] : 1.f;
+            if constexpr (CH) {
+                const bool okb = jb < TB && tn + jb < t_hi && db < D;
+                nb = *(const f32x4*)(decay + ((size_t)(okb ? tn + jb : t_lo) * H + h) * D + (okb ? db : 0));
+            }
+        }
+        float mine = 0.f;                                           // one token's result (la_owner)
+        if (it >= 0) {
+            const float* cur = sm + (it & 1) * (TB * per);
+            const int n_tok = t_hi - t0 < TB ? t_hi - t0 : TB;
+            float accs[TB], vv[LOOK];
+            f32x2 q2[LOOK], k2[LOOK], a2[CH ? LOOK : 1];
+            auto read = [&](int j) {
+                const float* row = cur + j * per;
+                vv[j % LOOK] = row[NQ * Dp + vc];
+                q2[j % LOOK] = *(const f32x2*)(row + LA_OWN(0));
+                k2[j % LOOK] = *(const f32x2*)(row + Dp + LA_OWN(0));
+                if constexpr (CH) a2[j % LOOK] = *(const f32x2*)(row + 2 * Dp + LA_OWN(0));
+            };
+            auto token = [&](int j) {
+                accs[j] = 0.f;
+#pragma unroll
+                for (int r = 0; r < PR; ++r) {
+                    float a = hd;
+                    if constexpr (CH) a = a2[j % LOOK][r];
+                    const float qr = q2[j % LOOK][r], kv = k2[j % LOOK][r] * vv[j % LOOK];
+                    if (PRE) accs[j] = fmaf(fmaf(ub[r], kv, S[r]), qr, accs[j]);
+                    S[r] = fmaf(a, S[r], kv);
+                    if (!PRE) accs[j] = fmaf(S[r], qr, accs[j]);
+                }
+            };
+            if (n_tok == TB) {
+#pragma unroll
+                for (int j = 0; j < LOOK; ++j) read(j);
+#pragma unroll
+                for (int j = 0; j < TB; ++j) {
+                    __builtin_amdgcn_sched_barrier(0x7);
+                    token(j);
+                    if (j + LOOK < TB) read(j + LOOK);
+                }
+                __builtin_amdgcn_sched_barrier(0x7);
+            } else {
+#pragma unroll
+                for (int j = 0; j < TB; ++j) {
+                    accs[j] = 0.f;
+                    if (j < n_tok) { read(j); token(j); }
+                }
+            }
+            mine = la_sums<TB>(accs, dg);
+        }
+        if (more) {
+            float* buf = sm + ((it + 1) & 1) * (TB * per);
+            if (ja < TB && tn + ja < t_hi) {
+                float* dst = buf + ja * per + (part < 2 ? ea : ea + (NQ - 2) * Dp);
+                const u32x4 w = in ? na : u32x4{0, 0, 0, 0};
+                f32x4 lo, hi;
+                lo.x = __builtin_bit_cast(float, w.x << 16) * ns, lo.y = __builtin_bit_cast(float, w.x & 0xffff0000u) * ns;
+                lo.z = __builtin_bit_cast(float, w.y << 16) * ns, lo.w = __builtin_bit_cast(float, w.y & 0xffff0000u) * ns;
+                hi.x = __builtin_bit_cast(float, w.z << 16) * ns, hi.y = __builtin_bit_cast(float, w.z & 0xffff0000u) * ns;
+                hi.z = __builtin_bit_cast(float, w.w << 16) * ns, hi.w = __builtin_bit_cast(float, w.w & 0xffff0000u) * ns;
+                *(f32x4*)dst = lo;
+                *(f32x4*)(dst + 4) = hi;
+            }
+            if constexpr (CH) {
+                if (jb < TB && tn + jb < t_hi) *(f32x4*)(buf + jb * per + 2 * Dp + db) = db < D ? nb : f32x4{0.f, 0.f, 0.f, 0.f};
+            }
+        }
+        if (it >= 0 && dg % (LA_DG / TB) == 0) {
+            const int t = t0 + la_owner<TB>(dg);
+            if (t < t_hi && v0 + vc < V) out[((size_t)t * H + h) * V + v0 + vc] = mine;
+        }
+        __syncthreads();
+    }
+    if (keep) la_state_out<PR>(S, srow, sm, D, V, v0);
+}
 #undef LA_OWN
 
+enum la_form { LA_SCAN, LA_BLOCKS, LA_SINGLE };
 struct la_args {
     dim3 grid; hipStream_t st; const void *q, *k, *v; int ldq, ldk, ldv; const float *decay, *head_decay; float q_scale;
     float* state; const int *cu_seqlens, *seq_slots; float* out; int H, D, V, keep, qk_rep; const float *v_scale, *bonus;
 };
 
 template <typename T, int RR, bool CH, bool VEC, bool PRE>
-static void la_launch(const la_args& a, bool single) {
-    const int TB = single ? 1 : la_block<RR>::tokens;
+static void la_launch(const la_args& a, la_form form) {
+    const int TB = form == LA_SINGLE ? 1 : la_block<RR>::tokens;
     constexpr int Dp = 16 * RR, per = (CH ? 3 : 2) * Dp + LA_VC;
     constexpr size_t tile = (size_t)Dp * (LA_VC + 1);
     static_assert(sizeof(float) * 2 * la_block<RR>::tokens * per <= 64 * 1024, "linear_attn_scan: the token blocks must fit the default LDS limit");
     const size_t blocks = (size_t)2 * TB * per, bytes = (blocks > tile ? blocks : tile) * sizeof(float);
-    auto* kernel = single ? linear_attn_single_kernel<T, RR, CH, VEC, PRE> : linear_attn_scan_kernel<T, RR, CH, VEC, PRE>;
+    auto* kernel = form == LA_SINGLE ? linear_attn_single_kernel<T, RR, CH, VEC, PRE> : linear_attn_scan_kernel<T, RR, CH, VEC, PRE>;
+    if constexpr (RR == 4 && VEC) if (form == LA_BLOCKS) kernel = linear_attn_blocks_kernel<CH, PRE>;
     kernel<<<a.grid, LA_NT, bytes, a.st>>>(
         (const T*)a.q, (const T*)a.k, (const T*)a.v, a.ldq, a.ldk, a.ldv, a.decay, a.head_decay, a.q_scale, a.state, a.cu_seqlens,
         a.seq_slots, a.out, a.H, a.D, a.V, a.keep, a.qk_rep, a.v_scale, a.bonus);
 }
 
 template <typename T, bool VEC, int RR>
-static void la_pick_decay(const la_args& a, bool single) {
-    if (a.bonus) la_launch<T, RR, true, VEC, true>(a, single);      // (the caller has made sure that a bonus comes with a decay per channel)
-    else if (a.decay) la_launch<T, RR, true, VEC, false>(a, single);
-    else la_launch<T, RR, false, VEC, false>(a, single);
+static void la_pick_decay(const la_args& a, la_form form) {
+    if (a.bonus) la_launch<T, RR, true, VEC, true>(a, form);      // (the caller has made sure that a bonus comes with a decay per channel)
+    else if (a.decay) la_launch<T, RR, true, VEC, false>(a, form);
+    else la_launch<T, RR, false, VEC, false>(a, form);
 }
 
 template <typename T, bool VEC>
-static void la_pick(const la_args& a, bool single) {
-    if (a.D <= 64) la_pick_decay<T, VEC, 4>(a, single);
-    else if (a.D <= 128) la_pick_decay<T, VEC, 8>(a, single);
-    else la_pick_decay<T, VEC, 16>(a, single);
+static void la_pick(const la_args& a, la_form form) {
+    if (a.D <= 64) la_pick_decay<T, VEC, 4>(a, form);
+    else if (a.D <= 128) la_pick_decay<T, VEC, 8>(a, form);
+    else la_pick_decay<T, VEC, 16>(a, form);
 }
 
 extern "C" int spite_linear_attn_scan(const void* q, const void* k, const void* v, int ldq, int ldk, int ldv, int dtype,
@@ -504,10 +657,17 @@ extern "C" int spite_linear_attn_scan(const void* q, const void* k, const void* 
     auto on16 = [](const void* p) { return ((uintptr_t)p & 15) == 0; };
     const bool vec = dtype == SP_BF16 && D % 8 == 0 && V % 8 == 0 && ldq % 8 == 0 && ldk % 8 == 0 && ldv % 8 == 0
                      && on16(q) && on16(k) && on16(v) && on16(decay);
-    const bool single = longest == 1;               // (0: not known)
-    if (dtype == SP_F32) la_pick<float, false>(a, single);
-    else if (vec) la_pick<bf16, true>(a, single);
-    else la_pick<bf16, false>(a, single);
+    // Which kernel (the same bits from each): single tokens their own; heads of up to 64 in blocks where instructions and not
+    // round trips are what a workgroup waits for: with a decay per head and more than two workgroups a compute unit (16 requests, 40
+    // heads of 64, us with the scan / in blocks: 5 tokens 15.8 / 13.5, 33 26.9 / 24.8, 500 242 / 233; but 4 requests, 16 heads, 256
+    // workgroups, 500 tokens 34.3 / 38.3), and for heads of less than 64, which the scan pads, with no more tokens than a
+    // block (8 requests, 16 heads of 32, a decay per channel, 5 tokens: 5.8 / 5.2).
+    const long groups = (long)n_seqs * H * ((V + LA_VC - 1) / LA_VC);
+    const bool blocks = D <= 64 && ((!decay && groups > 2L * sp_cu_count()) || (D < 64 && longest > 0 && longest <= la_block<4>::tokens));
+    const la_form form = longest == 1 ? LA_SINGLE : vec && blocks ? LA_BLOCKS : LA_SCAN;      // (longest 0: not known)
+    if (dtype == SP_F32) la_pick<float, false>(a, form);
+    else if (vec) la_pick<bf16, true>(a, form);
+    else la_pick<bf16, false>(a, form);
     SP_LAUNCH_CHECK("linear_attn_scan");
     return 0;
 }
