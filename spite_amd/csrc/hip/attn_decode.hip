@@ -78,8 +78,8 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
     const int re = (rb + per < nblk) ? rb + per : nblk;
 
     const bf16x8 zero8 = {0, 0, 0, 0, 0, 0, 0, 0};
-    // Block i of the split, its page and first key, and its keys and values on their way.
-    int key0 = 0, page = 0;
+    // Block i of the split, its first key, where that lies in its page, and its keys and values on their way.
+    int key0 = 0, off0 = 0, page = 0;
     bf16x8 kf[2][NC];
     u32x4 vf[ND];                    // (pairs of values: they are masked as such)
 #pragma unroll
@@ -88,14 +88,16 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
     for (int d = 0; d < ND; ++d) vf[d] = u32x4{0, 0, 0, 0};
     auto find_block = [&](int i) {
         key0 = (i < b_kept ? i : b_first + (i - b_kept)) * 32;
-        page = bt[key0 / ps];
+        const int at = key0 / ps;
+        off0 = key0 - at * ps;
+        page = bt[at];
     };
-    auto load_block = [&]() {
+    auto load_block = [&](int l) {
         const size_t pg = (size_t)(page < 0 ? 0 : page) * G + g;
-        const int blk = key0 % ps >> 5;                              // the block of 32 keys inside the page
-        const bf16* kbase = k_pages + pg * ps * HD + (size_t)blk * 2 * NC * 512 + lane * 8;
+        const int blk = off0 >> 5;                                   // the block of 32 keys inside the page
+        const bf16* kbase = k_pages + pg * ps * HD + (size_t)blk * 2 * NC * 512 + l * 8;
         // (value heads may be fewer than key heads: key head g reads value head g % Gv)
-        const bf16* vbase = v_pages + ((size_t)(page < 0 ? 0 : page) * Gv + g % Gv) * VD * ps + (size_t)blk * ND * 512 + lane * 8;
+        const bf16* vbase = v_pages + ((size_t)(page < 0 ? 0 : page) * Gv + g % Gv) * VD * ps + (size_t)blk * ND * 512 + l * 8;
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
@@ -107,32 +109,31 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
     int i = rb + wave;
     bf16x8 qf[NC];
     // the fused form's own key and value, for the wave that reads their block
-    bf16* own = (bf16*)(sm + HD);                        // [HD] rotated key, [VD] value, behind the sines
+    bf16* own = (bf16*)(sm + (size_t)4 * QH * ROW);      // [HD] rotated key, [VD] value, behind the records
     int own_slot = -1;
     if constexpr (FUSE) {
-        // Everything that is read is asked for before the sines and the barrier, the first block of keys and values too
-        // (the token's own key in it is a stale one, replaced in registers below): one trip to memory where there were four in a row.
-        // With the join's loads taken together, a layer's attention in us before and now (40 heads over 8): 8 tokens of 4,096 keys
-        // 29.7 / 27.8, 16 of 1,211 22.9 / 20.2, 32 of 300 13.8 / 12.7, 64 of 1,000 51.2 / 48.7, one of 14,000 19.8 / 18.4; one of 1,000
-        // and fewer 9.2 / 9.3, most of it the sines and the query's norm.
+        // Everything that is read is asked for before the sines and the barrier, the frequency first and the first block of keys and values last
+        // (the token's own key in it is a stale one, replaced in registers below), in no branch: loads behind a branch that may not
+        // have been taken are waited for with those in it.  A wave without a block asks for 16 bytes of another's pieces.
+        // A layer's attention, 40 heads over 8, in us: before anything was asked for ahead / with every load waited for before the block's / now:
+        // one token of 40 keys 6.3 / 6.6 / 6.0, of 100 6.5 / 6.9 / 6.5, of 1,000 9.4 / 9.6 / 9.2, of 4,096 11.5 / 11.1 / 10.6; 8 of 4,096
+        // 29.0 / 27.0 / 26.5, 16 of 64 6.3 / 6.8 / 6.2, 16 of 1,211 22.5 / 19.9 / 19.5, 64 of 1,000 50.4 / 47.8 / 47.5; 0.93 of the first over
+        // 92 sizes.  What is left in a short context is the sines, the query's norm and instructions fetched for a single use.
         const bf16* row = q + (size_t)t * (H + 2 * G) * HD;
+        const int slot = *(const __attribute__((address_space(4))) int*)(uintptr_t)(rope.slot_map + t);
+        find_block(i < re ? i : re - 1);
+        float freq = (rope.inv_freq ? rope.inv_freq : (const float*)row)[threadIdx.x & (HD / 2 - 1)];      // (without a rotation: not used)
         const bf16* qr = row + (size_t)(g * QH + (n < QH ? n : 0)) * HD + qd * 8;
         bf16x8 qlo[NC / 2], qhi[NC / 2];
 #pragma unroll
         for (int c = 0; c < NC / 2; ++c) { qlo[c] = *(const bf16x8*)(qr + c * 32); qhi[c] = *(const bf16x8*)(qr + c * 32 + HD / 2); }
-        const bool mine = rb < re && re == nblk;         // (one workgroup of the splits has the last block)
-        const int slot = rope.slot_map[t];
         const bf16* kr = row + (size_t)(H + g) * HD + (HD == 64 ? lane & 31 : lane);
         const bf16* vr = row + (size_t)(H + G + g) * HD + lane;
-        bf16 kx = kr[0], ky = kr[HD / 2], v0 = vr[0], v1 = vr[VD - 64];
+        const bf16 kx = kr[0], ky = kr[HD / 2], v0 = vr[0], v1 = vr[VD - 64];
         float* cs = sm;                                  // [HD / 2] pairs (cosine, sine)
-        float freq = rope.inv_freq ? rope.inv_freq[threadIdx.x & (HD / 2 - 1)] : 0.f;
-        if (i < re) find_block(i);
-        // these are there before the long loads go out: a wait for them would be one for those too
-#pragma unroll
-        for (int c = 0; c < NC / 2; ++c) asm volatile("" : "+v"(qlo[c]), "+v"(qhi[c]));
-        asm volatile("" : "+v"(kx), "+v"(ky), "+v"(v0), "+v"(v1), "+v"(freq), "+s"(page));
-        if (i < re) load_block();
+        __builtin_amdgcn_sched_barrier(0);
+        load_block(i < re ? lane : 0);
+        asm volatile("" : "+v"(freq));                   // (not asked for behind the block's loads, in the branch that needs it)
         if (threadIdx.x < HD / 2) {
             float sn = 0.f, c = 1.f;
             if (rope.inv_freq) sincosf((float)p * freq, &sn, &c);
@@ -140,10 +141,33 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
             cs[2 * threadIdx.x + 1] = sn;
         }
         __syncthreads();
-        if (mine && slot >= 0) {
+        if (i < re) {
+            // the queries: element c * 32 + qd * 8 + e turns with the one HD / 2 further on, which this lane holds as well
+            float x[NC][8], ss = 0.f;
+#pragma unroll
+            for (int c = 0; c < NC / 2; ++c) {
+#pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const f32x4 two = *(const f32x4*)(cs + 2 * (c * 32 + qd * 8 + (e & 6)));
+                    sp_rotate((float)qlo[c][e], (float)qhi[c][e], two[2 * (e & 1)], two[2 * (e & 1) + 1], x[c][e], x[c + NC / 2][e]);
+                    ss += x[c][e] * x[c][e] + x[c + NC / 2][e] * x[c + NC / 2][e];
+                }
+            }
+            ss = rows4_sum(ss);
+            float scale = rope.norm_eps > 0.f ? 1.0f / sqrtf(ss / (float)HD + rope.norm_eps) : 1.0f;
+            if (rope.floor_scale > 0) scale *= logf((float)((p + 1) / rope.floor_scale) + 1.0f) * rope.attn_scale + 1.0f;
+#pragma unroll
+            for (int c = 0; c < NC; ++c)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qf[c][e] = n < QH ? (bf16)(x[c][e] * scale) : (bf16)0.f;
+        } else {
+#pragma unroll
+            for (int c = 0; c < NC; ++c) qf[c] = zero8;
+        }
+        if (rb < re && re == nblk && slot >= 0) {        // (one workgroup of the splits has the last block; its last two waves, which have the fewest)
             own_slot = slot;
             const int at = slot / ps, off = slot % ps;
-            if (wave == 0) {
+            if (wave == 3) {
                 bf16* kp = k_pages + ((size_t)at * G + g) * ps * HD;
                 float a = 0.f, b = 0.f;
                 if (lane < HD / 2) sp_rotate((float)kx, (float)ky, cs[2 * lane], cs[2 * lane + 1], a, b);
@@ -155,7 +179,7 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
                     kp[sp_k_index(off, lane, HD, true)] = (bf16)(a * scale);
                     kp[sp_k_index(off, lane + HD / 2, HD, true)] = (bf16)(b * scale);
                 }
-            } else if (wave == 1) {
+            } else if (wave == 2) {
                 bf16* vp = v_pages + ((size_t)at * G + g) * ps * VD;
                 own[HD + lane] = v0;
                 vp[sp_v_index(lane, off, VD, ps, true)] = v0;
@@ -165,30 +189,12 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
                 }
             }
         }
-        // the queries: element c * 32 + qd * 8 + e turns with the one HD / 2 further on, which this lane holds as well
-        float x[NC][8], ss = 0.f;
-#pragma unroll
-        for (int c = 0; c < NC / 2; ++c) {
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const f32x4 two = *(const f32x4*)(cs + 2 * (c * 32 + qd * 8 + (e & 6)));
-                sp_rotate((float)qlo[c][e], (float)qhi[c][e], two[2 * (e & 1)], two[2 * (e & 1) + 1], x[c][e], x[c + NC / 2][e]);
-                ss += x[c][e] * x[c][e] + x[c + NC / 2][e] * x[c + NC / 2][e];
-            }
-        }
-        ss = rows4_sum(ss);
-        float scale = rope.norm_eps > 0.f ? 1.0f / sqrtf(ss / (float)HD + rope.norm_eps) : 1.0f;
-        if (rope.floor_scale > 0) scale *= logf((float)((p + 1) / rope.floor_scale) + 1.0f) * rope.attn_scale + 1.0f;
-#pragma unroll
-        for (int c = 0; c < NC; ++c)
-#pragma unroll
-            for (int e = 0; e < 8; ++e) qf[c][e] = n < QH ? (bf16)(x[c][e] * scale) : (bf16)0.f;
         __syncthreads();                                 // the own key and value are in LDS
     } else {
 #pragma unroll
         for (int c = 0; c < NC; ++c)
             qf[c] = n < QH ? *(const bf16x8*)(q + ((size_t)t * H + g * QH + n) * HD + c * 32 + qd * 8) : zero8;
-        if (i < re) { find_block(i); load_block(); }
+        if (i < re) { find_block(i); load_block(lane); }
     }
 
     float m_run = -INFINITY, l_run = 0.f;
@@ -200,42 +206,46 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
     for (int d = 0; d < ND; ++d) o[d] = f32x4{0.f, 0.f, 0.f, 0.f};
 
     if (i < re) for (;;) {
-        if (FUSE ? key0 + 31 >= p : key0 + 31 > p) {
+        const int k0 = key0, o0 = off0, pg0 = page;
+        if (!FUSE && i + 4 < re) find_block(i + 4);      // (its table entry is there by the time it is needed; in the fused form no faster)
+        if (FUSE ? k0 + 31 >= p : k0 + 31 > p) {
             // The block that holds the query's own key: the rows behind it still hold what the
             // page's last owner left, and a probability of zero times a value that is not finite
-            // is not zero; those values are taken as zero (this lane's keys are key0 + qd*8 + e).
+            // is not zero; those values are taken as zero (this lane's keys are k0 + qd*8 + e).
             // Masks of two values each: few instructions, as every one of this kernel is fetched for a single use.
-            const int behind = p - (key0 + qd * 8);                  // elements e > behind are past the query
-            u32x4 keep2, own2 = {0, 0, 0, 0};
+            const int behind = p - (k0 + qd * 8);                  // elements e > behind are past the query
+            u32x4 keep2;
 #pragma unroll
             for (int j = 0; j < 4; ++j) keep2[j] = (2 * j <= behind ? 0xffffu : 0u) | (2 * j + 1 <= behind ? 0xffff0000u : 0u);
-            uint32_t now[ND];
-#pragma unroll
-            for (int d = 0; d < ND; ++d) now[d] = 0;
             if constexpr (FUSE) {
-                // the token's own key and value take the places that the loads found stale
-                if (own_slot >= 0 && own_slot == page * ps + p % ps) {
-                    const int w = p & 31, r = ((w >> 3) << 2) | (w & 3);
+                // the token's own key and value take the places that the loads found stale, by masks of bits: no branch (LDS holds
+                // some bits where there are none, and the masks are zero)
+                const int w = p & 31;
+                const bool there = own_slot >= 0 && own_slot == pg0 * ps + o0 + w;
+                const bool row_is = there && n == (((w >> 3) << 2) | (w & 3));
+                u32x4 own2;
 #pragma unroll
-                    for (int tt = 0; tt < 2; ++tt)
-                        if (((w >> 2) & 1) == tt)
+                for (int j = 0; j < 4; ++j) own2[j] = there ? (2 * j == behind ? 0xffffu : 0u) | (2 * j + 1 == behind ? 0xffff0000u : 0u) : 0u;
 #pragma unroll
-                            for (int c = 0; c < NC; ++c) {
-                                const bf16x8 k = *(const bf16x8*)(own + c * 32 + qd * 8);
-                                kf[tt][c] = n == r ? k : kf[tt][c];
-                            }
+                for (int c = 0; c < NC; ++c) {
+                    const u32x4 k = *(const u32x4*)(own + c * 32 + qd * 8);
 #pragma unroll
-                    for (int j = 0; j < 4; ++j) own2[j] = (2 * j == behind ? 0xffffu : 0u) | (2 * j + 1 == behind ? 0xffff0000u : 0u);
+                    for (int tt = 0; tt < 2; ++tt) {
+                        const uint32_t m = row_is && ((w >> 2) & 1) == tt ? ~0u : 0u;
+                        const u32x4 m4 = {m, m, m, m};
+                        kf[tt][c] = __builtin_bit_cast(bf16x8, (k & m4) | (__builtin_bit_cast(u32x4, kf[tt][c]) & ~m4));
+                    }
+                }
 #pragma unroll
-                    for (int d = 0; d < ND; ++d) now[d] = __builtin_bit_cast(uint16_t, own[HD + d * 16 + n]) * 0x10001u;
+                for (int d = 0; d < ND; ++d) {
+                    const uint32_t v = __builtin_bit_cast(uint16_t, own[HD + d * 16 + n]), vv = v | v << 16;
+                    const u32x4 put = {vv, vv, vv, vv};
+                    vf[d] = (put & own2) | (vf[d] & ~own2);
                 }
             }
+            // (whole vectors: written element by element, clang 22 let other values into the registers of some of them)
 #pragma unroll
-            for (int d = 0; d < ND; ++d) {
-                // (whole vectors: written element by element, clang 22 let other values into the registers of some of them)
-                const u32x4 put = {now[d], now[d], now[d], now[d]};
-                vf[d] = (vf[d] & (keep2 & ~own2)) | (put & own2);
-            }
+            for (int d = 0; d < ND; ++d) vf[d] = vf[d] & keep2;
         }
 
         f32x4 s[2];
@@ -248,18 +258,18 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
         }
         float mx = -INFINITY;
         bool ok[2][4];
-        const bool near = DIST && key0 + 31 > p - (n_dist - 1);      // some key of the block is nearer than the table's end
+        const bool near = DIST && k0 + 31 > p - (n_dist - 1);      // some key of the block is nearer than the table's end
 #pragma unroll
         for (int tt = 0; tt < 2; ++tt)
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int j = key0 + qd * 8 + tt * 4 + i;
+                const int j = k0 + qd * 8 + tt * 4 + i;
                 ok[tt][i] = sp_visible(j, p, lo, keep);
                 float raw = s[tt][i] + slope * (float)(j - p);
                 if (DIST) raw += near ? tab[min(max(p - j, 0), n_dist - 1)] * inv_scale : far_bias;
                 // a cap on the scores: cap * tanh(score * scale / cap), with cap_ratio = scale / cap
                 if (cap_ratio > 0.f) raw = tanhf(raw * cap_ratio) / cap_ratio;
-                const float v = ok[tt][i] ? (page < 0 ? NAN : raw * scale_log2e) : -INFINITY;
+                const float v = ok[tt][i] ? (pg0 < 0 ? NAN : raw * scale_log2e) : -INFINITY;
                 s[tt][i] = v;
                 mx = fmaxf(mx, v);
             }
@@ -286,11 +296,10 @@ void attn_decode_kernel(const bf16* __restrict__ q, bf16* k_pages,
         }
         i += 4;
         if (i >= re) break;
-        find_block(i);
-        load_block();
+        if (FUSE) find_block(i);
+        load_block(lane);
     }
 
-    if constexpr (FUSE) __syncthreads();                 // (the own key lies where the records go)
     // the waves' partial results meet in LDS; o[d][i] of lane (n, qd) is O[head n][d*16 + qd*4 + i]
     if (n < QH) {
         float* mine = sm + ((size_t)wave * QH + n) * ROW;
@@ -434,8 +443,8 @@ static int attn_decode(const void* q, const void* k_pages, const void* v_pages, 
     if (!sp_vis_has_span(vis)) keep = 0;
     const float sl = scale * 1.4426950408889634f, cr = softcap > 0.f ? scale / softcap : 0.f;
     dim3 grid(n_splits, G, T);
-    // the waves' records; before them, in the fused form, the sines and the token's own key and value: always less
-    const size_t sh = (size_t)4 * (H / G) * (v_dim + 2) * sizeof(float);
+    // the waves' records (before them, in the fused form, the sines: always less) and, there, the token's own key and value
+    const size_t sh = (size_t)4 * (H / G) * (v_dim + 2) * sizeof(float) + (rope ? (hd + v_dim) * sizeof(bf16) : 0);
     const ad_rope ro = rope ? *rope : ad_rope{};
 #define SP_ADK(HDV, VDV, DISTV, FUSEV) attn_decode_kernel<HDV, VDV, DISTV, FUSEV><<<grid, 256, sh, st>>>( \
             (const bf16*)q, (bf16*)k_pages, (bf16*)v_pages, (float*)workspace, (bf16*)out, positions, seq_of_token, block_table, \

@@ -581,9 +581,10 @@ def attn_decode_splits(heads: int, longest: int) -> int:
 
 def attn_decode_rope_suits(heads: int) -> bool:
     """Whether rotation and cache write are better done inside the decode attention of ``heads`` (tokens times kv heads): up to
-    two workgroups a compute unit, where they cost a launch less, about 2 us.  Beyond, every further workgroup that a unit
-    takes up waits for its sines and its query's norm before it asks for keys (4,096 workgroups of 256 keys: 115 us against 108
-    in two kernels; 1,536 of 4,096: 313 against 305)."""
+    two workgroups a compute unit, where they cost a launch less, about 2 us (40 heads over 8 on an MI355X, us, inside and in two
+    kernels: 64 tokens of 300 keys 17.4 and 22.3, of 1,000 47.5 and 51.6).  Beyond, it depends on the contexts, which the rule does not know: every
+    workgroup has its sines and its query's norm to do, and long contexts lose by that what short ones gain by the launch (128 tokens of 300
+    keys 32.3 and 38.0, of 2,000 174.6 and 173.5; 192 of 4,096 513 and 495; 300 of 1,000 220 and 217; 512 of 256 108.9 and 108.9)."""
     return heads <= 2 * cu_count()
 
 

@@ -111,3 +111,31 @@ def test_own_key_at_every_place_of_a_block_and_any_number_of_splits(hd, n_splits
     bits = lambda t: t.view(torch.int16)
     assert torch.equal(bits(kp), bits(kp2)) and torch.equal(bits(vp), bits(vp2))
     assert torch.equal(bits(got), bits(want)) and bool(torch.isfinite(want.float()).all())
+
+
+@pytest.mark.parametrize("H,G,hd", [(4, 4, 64), (4, 4, 128), (16, 1, 128)])
+@pytest.mark.parametrize("vis,span", [("full", 0), ("window", 40), ("chunk", 48)])
+@pytest.mark.parametrize("n_splits", [1, 3, 64])
+def test_waves_and_splits_without_a_block(H, G, hd, vis, span, n_splits):
+    """One to sixteen query heads a kv head (the records' room), contexts of one block and of five, splits that have none: the two
+    kernels' bits, and pages whose other places hold NaN."""
+    lens, ps = [1, 2, 31, 32, 33, 64, 65, 97, 129, 160], 64
+    T = len(lens)
+    kv = PagedKV(lens, G, hd, ps, torch.bfloat16)
+    kv.vp[kv.vp == -70.0] = float("nan")
+    kp, vp = ops().kv_operand_order(kv.kp.to(DEV), kv.vp.to(DEV))
+    qkv = rnd(T, (H + 2 * G) * hd, dtype=torch.bfloat16, seed=5)
+    positions = torch.tensor([n - 1 for n in lens], dtype=torch.int32, device=DEV)
+    slots = torch.tensor([kv.tables[s][(n - 1) // ps] * ps + (n - 1) % ps for s, n in enumerate(lens)], dtype=torch.int32, device=DEV)
+    seq, bt = torch.arange(T, dtype=torch.int32, device=DEV), kv.bt.to(DEV)
+    scratch = torch.empty(ops().attn_decode_workspace(T, H, hd, n_splits) // 4, dtype=torch.float32, device=DEV)
+    q, want, got = (torch.zeros(T, H * hd, dtype=torch.bfloat16, device=DEV) for _ in range(3))
+    kp2, vp2 = kp.clone(), vp.clone()
+    ops().rope_kvwrite(qkv, q, kp, vp, positions, slots, None, H, G, hd, ps, use_rope=False, adjacent=False, use_norm=False, norm_eps=0.0,
+                       use_temp=False, floor_scale=0, attn_scale=0.0, kv_tiled=True)
+    args = (positions, seq, bt, T, H, G, hd, ps, vis, span, hd ** -0.5, n_splits)
+    ops().attn_decode(q, kp, vp, want, scratch, *args)
+    ops().attn_decode_rope(qkv, kp2, vp2, got, scratch, positions, slots, *args[1:])
+    bits = lambda t: t.view(torch.int16)
+    assert torch.equal(bits(kp), bits(kp2)) and torch.equal(bits(vp), bits(vp2))
+    assert torch.equal(bits(got), bits(want)) and bool(torch.isfinite(want.float()).all())
