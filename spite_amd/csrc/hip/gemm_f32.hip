@@ -141,7 +141,9 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
 //    step two before, the rows put into LDS last, since waiting for them is waiting for the W asked for before them.
 // Before and now (us): 200 rows x 2,048 x 3,072 55 / 34, 301 x 3,072 x 2,048 54 / 44, 301 x 32,768 x 2,048 380 / 365, gated 301 x 3,072
 // x 2,048 100 / 78; 16 groups and one of all of 301 rows, gated 2 x 3,072 x 2,048, 271 / 245, and 2,048 x 3,072 144 / 139 (with two sets 150).
-// 128 groups of a few rows of K = 512 are 4 % slower than before (38 / 36): every second step is one of the last.
+// Groups' last steps, whose loads would pass the end, are not in the whole steps' loop nor guarded one by one (they were, and short sums spent
+// most of their time there: 128 groups and one of all of 150 rows, 2,048 x 512, 73 us before / 76 with guards / 68 now; 800 rows of 128
+// groups x 768 x 512 38.7 / 41.5 / 38.6).  64 groups of a few rows x 2,048 x 3,072 take 3 % more than before (317 / 308), at 5.1 TB/s of W.
 template <int TM, int NB, int LIVE, bool BURST>
 __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp, const float* const* xp, const float* sc, int K,
                                               int seg, int lr, int lk, int r, int q, f32x4 (&tot)[TM / 16][NB]) {
@@ -223,10 +225,18 @@ __device__ __forceinline__ void f32_tile_loop(float* xs, const float* const* wp,
 #pragma unroll
         for (int u = 0; u < U; ++u) load_w(w[i][u], i * F32_TK + u * 16, false);
     put_x(0, 0, false);
-    while (k0 + 2 * S * F32_TK <= K) {
+    while (k0 + (S + 2) * F32_TK <= K) {
 #pragma unroll
         for (int i = 0; i < S; ++i) step(w[i], w[(i + 2) % S], true);
     }
+    if constexpr (BURST) {
+        while (k0 + 2 * F32_TK < K) {
+#pragma unroll
+            for (int i = 0; i < S; ++i) step(w[i], w[(i + 2) % S], false);
+        }
+        if (k0 < K) step(w[0], w[2 % S], false);
+        if (k0 < K) step(w[1], w[0], false);
+    } else
     while (k0 < K) {
 #pragma unroll
         for (int i = 0; i < S; ++i)
