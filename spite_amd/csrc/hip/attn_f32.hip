@@ -223,8 +223,11 @@ int sp_attn_f32(const float* q, const float* k_pages, const float* v_pages, floa
     if (hd % 16 || hd > 128 || page_size % 4 || ((uintptr_t)q | (uintptr_t)k_pages | (uintptr_t)v_pages) % 16) return 1;
     // Waves for no more tiles than a query sees, lanes for no more of the head than there is: 3,000 tokens of a prompt, 4 heads
     // of 16 behind a window of 64 keys, 23 us (46 with eight waves and heads padded to 64, 60 for the plain kernel); of 16 heads of 128
-    // over 4, 190.  Windows of a few keys as well (1,000 tokens, 16 heads of 128 over 4, windows of one and eight keys: 37 and 42 us, the
-    // plain kernel's wave a row 48 and 97; over 16, one key, 65 and 64; one token of 16 heads 4.7 and 11.0).
+    // over 4, 190.  Windows of up to eight keys only where two heads share a workgroup's loads and the head fills its lanes (1,000 tokens, 16
+    // heads of 128 over 4, windows of one and eight keys: 37 and 42 us, the plain kernel's wave a row 48 and 97; 0.45 to 0.9 over
+    // heads of 16 to 64 and 128); else the plain kernel's, which makes no tile of 32 keys for each head (700 tokens, two keys:
+    // 40 heads of 128 over 8 94 / 109, 12 of 96 over 4 23 / 34, 6 of 80 over 2 12 / 20).  By the layer alone: a token's bits do not depend on the step.
+    if (sp_vis_has_span(vis) && span <= 8 && !(H / G % 2 == 0 && (hd <= 64 || hd == 128))) return 1;
     const long tiles = sp_vis_has_span(vis) ? ((long)span + 30) / 32 + 1 : 8;      // that a query sees at most
     const int waves = tiles <= 2 ? 2 : tiles <= 4 ? 4 : 8, nq = af_heads(T, H, H / G, hd, waves);
 #define AF_GO(NI, W, NQ) attn_f32_kernel<NI, W, NQ><<<dim3(T, H / NQ), 64 * W, 0, st>>>(q, k_pages, v_pages, out, positions, seq_of_token, block_table, \

@@ -51,3 +51,11 @@ def test_keys_of_a_page_that_was_given_back_poison_every_query_that_sees_them(H,
     ops().attn_generic(q, kv.kp.to(DEV), kv.vp.to(DEV), out, pos, seq, bt.to(DEV), T, H, G, hd, ps, "full", 0, hd ** -0.5)
     sees = pos >= first * ps
     assert bool(torch.isnan(out[sees]).all()) and bool(torch.isfinite(out[~sees]).all())
+
+
+@pytest.mark.parametrize("H,G,hd", [(5, 1, 128), (12, 4, 96), (6, 2, 80), (4, 4, 64), (8, 2, 128), (4, 2, 48)])
+@pytest.mark.parametrize("vis,span", [("window", 1), ("window", 8), ("chunk", 8), ("window", 9)])
+def test_windows_of_a_few_keys(H, G, hd, vis, span):
+    """Which kernel takes them depends on the layer alone: a token has the same bits alone and among many, on both sides of the lines."""
+    over_tiles(H, G, hd, 32, vis, span)
+    test_a_token_has_the_same_bits_alone_and_among_many(H, G, hd, vis, span)
