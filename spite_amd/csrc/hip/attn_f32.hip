@@ -171,30 +171,37 @@ void attn_f32_kernel(const float* __restrict__ q, const float* __restrict__ k_pa
         if (lane == 0) { ml_sh[wave][nq][0] = m[nq]; ml_sh[wave][nq][1] = l[nq]; }
     }
     __syncthreads();
-    // a wave's weight exp(its maximum - the largest), and one over the sum: by as many threads as there are
-    if (threadIdx.x < NQ) {
-        const int nq = threadIdx.x;
+    // a wave's weight exp(its maximum - the largest), and one over the sum: of one head by every thread for itself, of more by as many
+    // threads as there are heads (one barrier more: 32 tokens, 4 heads of 16, 4.8 us with it, 4.6 without)
+    auto weights = [&](int nq, float* f) {
         float mm = ml_sh[0][nq][0];
 #pragma unroll
         for (int w = 1; w < W; ++w) mm = fmaxf(mm, ml_sh[w][nq][0]);
         float ll = 0.f;
 #pragma unroll
         for (int w = 0; w < W; ++w) {
-            const float f = ml_sh[w][nq][0] == -INFINITY ? 0.f : expf(ml_sh[w][nq][0] - mm);
-            ll = fmaf(ml_sh[w][nq][1], f, ll);
-            f_sh[nq][w] = f;
+            f[w] = ml_sh[w][nq][0] == -INFINITY ? 0.f : expf(ml_sh[w][nq][0] - mm);
+            ll = fmaf(ml_sh[w][nq][1], f[w], ll);
         }
-        f_sh[nq][W] = 1.0f / fmaxf(ll, 1e-30f);
+        f[W] = 1.0f / fmaxf(ll, 1e-30f);
+    };
+    if constexpr (NQ > 1) {
+        if (threadIdx.x < NQ) weights(threadIdx.x, f_sh[threadIdx.x]);
+        __syncthreads();
     }
-    __syncthreads();
     for (int c = threadIdx.x; c < NQ * NI * 16; c += 64 * W) {
         const int nq = c / (NI * 16), e = c % (NI * 16);
         if (e >= hd) continue;
+        float f[W + 1];
+        if constexpr (NQ == 1) weights(0, f);
+        else
+#pragma unroll
+            for (int w = 0; w <= W; ++w) f[w] = f_sh[nq][w];
         float a = 0.f;
 #pragma unroll
         for (int w = 0; w < W; ++w)
-            if (ml_sh[w][nq][1] != 0.f) a = fmaf(o_sh[w][nq][e], f_sh[nq][w], a);
-        out[((size_t)t * H + h0 + nq) * hd + e] = a * f_sh[nq][W];
+            if (ml_sh[w][nq][1] != 0.f) a = fmaf(o_sh[w][nq][e], f[w], a);
+        out[((size_t)t * H + h0 + nq) * hd + e] = a * f[W];
     }
 }
 
