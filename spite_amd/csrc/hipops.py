@@ -1083,10 +1083,11 @@ def latent_workgroups(counts, cu_seqlens, H):
     return np.asarray(out, dtype=np.int32), (len(out) // 2, most)
 
 
-def latent_splits(n_wg: int, longest: int, Dk: int = 576, R: int = 512) -> int:
+def latent_splits(n_wg: int, longest: int, Dk: int = 576, R: int = 512, rows: int = 0) -> int:
     """Into how many workgroups the keys of every work item are best dealt, for ``n_wg`` items whose
-    queries read at most ``longest`` keys, in rows of ``Dk`` with a latent of ``R``.  A block of 32 keys takes a workgroup
-    3.0 us and its start about 8, joining the records of 32 splits 6, of 64 10, of 128 16, of 256 25: shares of two blocks up
+    queries read at most ``longest`` keys, in rows of ``Dk`` with a latent of ``R``; ``rows``: the items' query rows in all (0: as many as
+    they may have).  A block of 32 keys takes a workgroup 3.0 us (rows of 576; narrower ones less) and its start about 8, joining the
+    records of 32 splits 6, of 64 10, of 128 16, of 256 25: shares of two blocks up
     to 32 splits, of four beyond (fewer than eight splits only where there are fewer blocks), and about one workgroup a compute unit.  Where a
     unit holds one workgroup, none more: the first one over costs as much time as all of them; narrow rows leave room for
     several a unit.
@@ -1094,16 +1095,31 @@ def latent_splits(n_wg: int, longest: int, Dk: int = 576, R: int = 512) -> int:
     32.8 with 128 for 43.3.  40 heads on an MI355X, us.  1 item, 1,024 keys: 49 with 4 splits, 23 with 16; 4,096: 51 with 16, 34 with 32; 8,192: 52 with
     32, 38 with 64; 16,384: 89 with 32, 56 with 64, 44 with 128; 32,768: 163 with 32, 60 with 128, 49 with 256.  6 items of
     16,384: 94 with 32, 121 with 43.  16 items of 4,096: 59 with 16, 72 with 32.  100 items of 2,048 in rows of 192: 70 with 2,
-    53 with 3.)"""
+    53 with 3.)
+
+    Many items with more than 4,096 keys: up to a split for every 4,096, as many as take the fewest rounds over the compute
+    units, the records' way to memory and back counted (199 sizes of 64 to 640 items, 2,500 to 32,768 keys, up to 8 splits, each timed with
+    1, 2, 3, 4 and more: 5 % off the best on average; always a split for every 4,096 keys, as it was, 8 %, never 15 %.  40 heads, us:
+    700 tokens behind a window of 4,096, 219 items, 429 with 1 and 486 with 2; 2,048 at 15,000 keys, 640 items, 4,043 with 2, 4,701 with
+    8; 300 tokens of a request each at 16,300 keys 2,852 with 1, 1,864 with 4).  Narrow rows, several workgroups a unit, and contexts
+    beyond, which were not timed: a split for every 4,096."""
     if n_wg <= 0:
         return 1
     blocks, cus = -(-longest // 32), cu_count()
     room = max(1, cus // n_wg)
-    if Dk <= 192 and R <= 128:
+    narrow = Dk <= 192 and R <= 128
+    if narrow:
         room = max(room, min(-(-cus // n_wg), -(-blocks // 8)))
     share = min(max(-(-blocks // 2), min(blocks, 8)), 32)
-    # (no share of more than 4,096 keys: an end of few workgroups is shorter so)
-    return max(1, min(max(share, -(-blocks // 4)), room, 256), min(-(-longest // 4096), 256))
+    n = max(1, min(max(share, -(-blocks // 4)), room, 256))
+    most = min(-(-longest // 4096), 256)
+    if most <= n or narrow or longest > 32768:
+        return max(n, most)
+    records = (rows or n_wg * LATENT_WG_ROWS) * (R + 2) * 8 / 4e6      # us a split, written and read at 4 TB/s
+
+    def us(k):
+        return -(-n_wg * k // cus) * (3.0 * Dk / 576 * -(-blocks // k) + 8.0) + (6.0 + k * records if k > 1 else 0.0)
+    return min(range(n, most + 1), key=us)
 
 
 def attn_latent_mfma(q, kv_pages, out, positions, seq_of_token, block_table, wg, n_wg, max_rows, T, H, Dk, R, vis, span, scale,

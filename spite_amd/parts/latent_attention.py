@@ -166,7 +166,7 @@ class LatentAttention(Mixer):
             longest = cache.block_table.shape[1] * cache.page_size
             if self.visibility != "full":
                 longest = min(longest, self.span + ctx.max_count + 31)
-            n_splits = hipops.latent_splits(n_wg, longest, Dk, R)
+            n_splits = hipops.latent_splits(n_wg, longest, Dk, R, T * H)
             scratch = ws.take((T * H * n_splits * (R + 2),), torch.float32) if n_splits > 1 else None
             hipops.attn_latent_mfma(qa, cache.k_pages, o_lat, ctx.positions, ctx.seq_of_token, cache.block_table,
                                     wg, n_wg, most, T, H, Dk, R, self.visibility, self.span, self.scale,

@@ -48,6 +48,20 @@ def test_latent_splits_beyond_a_window_and_for_many_items():
         assert latent_splits(n, 2048, 192, 128) == -(-256 // n) and latent_splits(n, 2048) == 256 // n
 
 
+def test_latent_splits_of_many_items_with_long_contexts():
+    """Sizes that were timed with every count of splits: one round of the compute units stays one, what overflows it is dealt so that
+    the rounds come out even, and records cost their way to memory; never more than a split for every 4,096 keys."""
+    from spite_amd.csrc.hipops import latent_splits
+    assert [latent_splits(n, 4827, rows=40 * 700) for n in (157, 219, 250)] == [1, 1, 1]            # (2 before: 13 % more)
+    assert latent_splits(469, 5627, rows=60000) == 1 and latent_splits(94, 16384, rows=12000) == 2
+    assert [latent_splits(n, 16384, rows=40 * n) for n in (110, 130, 200, 256, 300, 500, 640)] == [2, 3, 1, 1, 4, 1, 2]
+    assert latent_splits(640, 32768, rows=81920) == 2
+    for n in range(1, 700, 3):
+        for longest in (64, 4096, 4128, 9000, 32768, 50000):
+            assert 1 <= latent_splits(n, longest) <= 256
+            assert latent_splits(n, longest) <= max(256 // n, -(-longest // 4096)) or n < 2
+
+
 def test_decode_attention_splits():
     """Where the rule's lines lie, at sizes that were timed with every count of splits."""
     from spite_amd.csrc.hipops import attn_decode_splits
