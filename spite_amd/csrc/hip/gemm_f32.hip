@@ -315,23 +315,26 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
 //
 // Both kernels take a time that follows from the most workgroups that a compute unit gets, c: for 2,048 of K, on an MI355X (us), the
 // stream of 16 rows 7 c (gated 11.5 c), tiles of 32 rows 7 + 19 c (5 + 41 c), of 64 9 + 29 c (10 + 56 c); the stream gives each
-// of its eight waves a run of 64 k and more, so that shorter sums than 512 leave some idle.  The lines lie where 14,900 products (1
-// to 1,500 tokens, up to 128 groups of 1 to 8 a token, K of 128 to 8,192) were timed with every variant, with tiles that took
-// 14 + 19.5 c (14 + 47 c) and 17 + 36 c (19 + 82 c), as the figures below have it; with the tiles as they are the choice is 6 % off the
-// best variant on average over 768 products (9 to 1,200 tokens, up to 129 groups, K of 512 to 5,120), most of it where 33 to 64 rows
-// still take the stream (48 rows of 5 groups x 3,072 x 2,048 64 / tiles of 32 33):
+// of its eight waves a run of 64 k and more, so that shorter sums than 512 leave some idle.  Most lines lie where 14,900 products (1
+// to 1,500 tokens, up to 128 groups of 1 to 8 a token, K of 128 to 8,192) were timed with every variant when tiles took
+// 14 + 19.5 c (14 + 47 c) and 17 + 36 c (19 + 82 c); those of 17 to 64 rows, and the figures here, are of the tiles as they are (1,428
+// products, 9 to 1,200 tokens, up to 129 groups, K of 512 to 5,120: the choice is 4 % off the best variant on average, 17 to 64 rows 1 in
+// groups and 4 without, where the lines before were 70 and 18 off; groups of few rows 6 to 9, which tiles have gained most on):
 //  * groups of up to eight rows on average: the stream of every group's W, 16 rows a workgroup (16 groups and one of all t rows, 2 x
-//    3,072 x 2,048 gated: t = 16 124, with 32 rows a workgroup 190; t = 64 184 / tiles 207), but tiles of 32 rows where sums are
-//    short and tiles enough (K <= 512 and more than one a compute unit; plain K < 2,048 and more than two: 129 groups x 2,048 x 768,
-//    535 rows, 151 / stream 233; 128 x 4,096 x 1,536, 885 rows, 567 / 794; at K = 2,048 either is as fast).  A group that holds most of
-//    the rows has its W read once every 16 of them, which the rule does not know (128 groups of one row a token and one of all, 2,048 x
-//    2,048: gated t = 451 881 / 887, but plain t = 318 449 / 380).
-//  * no groups: the stream up to 64 rows, unless W is tall enough for two workgroups of tiles a compute unit (32,768 x 2,048: 9 rows
-//    54 with the stream, 48 with tiles of 32; 16: 64 / 49; 64: 198 / 98; 8 51 / 52; 3,072 x 2,048 stays, 64 rows 26 / 35).
-//  * more rows: tiles of 32 up to three of them a compute unit, gated two, with groups two and a quarter (3,072 x 2,048, 100 rows: 35
-//    / 53, 301: 54 / 60; 16,384 x 3,072, 186 rows, over the line, 215 / 191; gated 16,384 x 4,096, 78 rows, 346 / 255; gated, 8
-//    groups and one of all x 512 x 2,048, t = 212, 105 / 172), and where groups hold up to 20 rows, plain ones 160 (17 groups, 2 x
-//    3,072 x 2,048, t = 150 214 / 237, t = 200, over the line, 264 / 247); none past 128 a compute unit, more than was timed.
+//    3,072 x 2,048 gated: t = 17 114, with 32 rows a workgroup 170, tiles 131; t = 64 184 / tiles 171), but tiles of 32 rows where sums are
+//    short and tiles enough (K <= 512 and more than one a compute unit; plain K < 2,048 and more than two: 129 groups x 4,096 x 1,536,
+//    400 rows, 465 / stream 634; 2,048 x 2,048 stays, 500 rows, 396 / tiles 344).
+//  * 17 to 64 rows, no groups or larger ones: over three to seven groups the stream, 16 rows a workgroup, up to four of them a compute unit
+//    (c of 2.8: 5 groups, 48 rows x 2,048 x 2,048, 25.5, tiles of 32 28.9, 64 rows a workgroup 48; over the line: x 3,072 x 2,048, 4.1,
+//    36 / 30 / 63, gated 59 / 51 / 100; 64 rows, gated 6,144 x 768, 9.8, 48 / 38 / 103).  Over one or two and without groups three and a half,
+//    where W is taller than a workgroup of any rows a unit (64 rows x 5,120 x 5,120, c = 5, 96 / 55 / 106; 52 x 4,096 x 1,536 stays, 18 / 20);
+//    below, 16 rows up to one workgroup a unit (64 x 1,024 x 1,024 7.9, all rows in one 13.8), then as many rows a workgroup as there are, which
+//    reads W once (33 x 3,072 x 2,048 19.3, with 16 rows 21.6).  W of fewer than 256 columns over groups was not timed and has the rows it had.
+//  * up to 16 rows: the stream, unless W is tall enough for two workgroups of tiles a compute unit (32,768 x 2,048: 9 rows
+//    55 with the stream, 46 with tiles of 32).
+//  * more rows: tiles of 32 up to three of them a compute unit, gated two, with groups two and a quarter (3,072 x 2,048, 101 rows: 26
+//    / 43, 301, near the line, 45 / 45; gated, 380, over it, 119 / 148), and where groups hold up to 20 rows, plain ones 160 (17 groups, 2 x
+//    3,072 x 2,048, t = 150 177 / 174, t = 301, over the line, 238 / 230); none past 128 a compute unit, more than was timed.
 //  * eight columns: up to a workgroup of sixteen a compute unit, up to three for K of 2,048 and more (3,072 x 2,048, two groups of a
 //    row 23.9 / 27.3; 5 rows x 6,144 x 768, over the line, 16.9 / 15.3).
 static int f32_variant(int M, int N, int K, int n_groups, int glu) {
@@ -340,6 +343,11 @@ static int f32_variant(int M, int N, int K, int n_groups, int glu) {
     const bool few = n_groups && M > 16 && M <= 8L * n_groups;
     const bool short_sum = (K <= 512 && live * cols > cus) || (!glu && K < 2048 && live * cols > 2 * cus);
     if (few && !short_sum && M / 16L + n_groups <= 65535) return halves ? 8 : 16;      // (the grid's limit)
+    if (!few && M > 16 && M <= 64 && (!n_groups || N >= 256)) {
+        const double c = ((N + 15) / 16) * (n_groups ? M / 16.0 + 0.5 * live : (M + 15) / 16) / cus;      // workgroups of 16 rows a compute unit
+        if (n_groups > 2 ? c > 4.0 : c > 3.5 && (N + 15) / 16 > cus) return -32;
+        if (n_groups > 2 || c <= 1.0) return 16;
+    }
     if (!few && M <= 64 && (n_groups || M <= 8 || cols * ((M + 31) / 32) < 2 * cus)) return M > 32 ? 64 : M > 16 ? 32 : halves ? 8 : 16;
     const double tiles = (n_groups ? M / 32.0 + 0.5 * live : (M + 31) / 32) * cols / cus;         // of 32 rows, a compute unit
     if (tiles <= (!glu ? 3.0 : n_groups ? 2.25 : 2.0) || (!n_groups && M <= 64)) return -32;

@@ -23,6 +23,17 @@ def test_lines_lie_where_both_sides_were_timed():
     assert [at(1, 6144, k, 0, 1) for k in (512, 2047, 2048)] == [16, 16, 8] and at(1, 4096, 128, 0, 1) == 8 and at(1, 4100, 2048, 0, 1) == 16
 
 
+def test_lines_of_17_to_64_rows():
+    """Both sides timed with the tiles as they are: the stream of 16 rows up to four workgroups a compute unit, without groups three and
+    a half and below one; then tiles of 32 (48 rows of 5 groups x 3,072 x 2,048: 30 us, 64 rows a workgroup of the stream 63)."""
+    from spite_amd.csrc.hipops import lib
+    at = lib().spite_gemm_f32_choice
+    assert [at(48, n, 2048, 5, 0) for n in (1024, 2048, 3072)] == [16, 16, -32] and [at(m, 3072, 2048, 5, 1) for m in (40, 48, 64)] == [16, -32, -32]
+    assert [at(m, 5120, 5120, 3, 0) for m in (25, 34, 64)] == [16, -32, -32] and at(64, 6144, 768, 5, 1) == -32 and at(64, 768, 512, 5, 0) == 16
+    assert [at(m, 1024, 1024, 0, 0) for m in (17, 64)] == [16, 16] and [at(m, 5120, 5120, 0, 0) for m in (32, 33, 64)] == [32, -32, -32]
+    assert [at(m, 3072, 2048, 0, 0) for m in (17, 33, 64)] == [32, 64, 64] and at(64, 200, 2048, 5, 0) == 64
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("M,groups", [(200, 40), (70, 5), (300, 5), (40, 3)])
 @pytest.mark.parametrize("N,K,glu", [(80, 292, False), (80, 292, True), (16400, 36, False)])
