@@ -73,7 +73,7 @@ def test_gated_rows_with_both_halves_in_one_operand(M, N, K, groups):
 @pytest.mark.parametrize("M,N", [(90, 200), (75, 33000)])
 def test_tiles_add_up_in_the_streams_order_wherever_the_sum_ends(K, glu, M, N):
     """Sums that end inside a step, with one, with the steps whose loads would pass the end: a row of a tile (of 32 rows, of
-    64) has the bits that the stream gives it alone, plain and among groups of one to forty rows."""
+    64) has the bits that the stream gives it alone, and a row of a tile of 32 among groups of one to forty rows."""
     a, w = rnd(M, K), rnd((2 if glu else 1) * N, K, seed=1)
     whole, one = torch.empty(M, N, device=DEV), torch.empty(1, N, device=DEV)
     ops().gemm_generic(a, w, whole, M, N, K, glu=glu)
@@ -93,4 +93,26 @@ def test_tiles_add_up_in_the_streams_order_wherever_the_sum_ends(K, glu, M, N):
             alone = torch.empty(1, N, device=DEV)
             ops().gemm_generic(x[r:r + 1].contiguous(), ws[g].contiguous(), alone, 1, N, K, glu=glu)
             assert torch.equal(alone[0], y[r])
+        at += size
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("K", [4, 60, 64, 68, 128, 188, 192, 256, 260, 320, 384, 388, 448, 516, 580, 772])
+@pytest.mark.parametrize("glu,N,sizes", [(True, 3000, [1, 17, 33, 0, 49, 64, 40, 60, 65]), (False, 2100, [1, 17, 33, 49, 1000])])
+def test_groups_in_tiles_of_64_rows_wherever_the_sum_ends(K, glu, N, sizes):
+    """Tiles of 64 rows over groups: one to four live quarters, both loops over k, sums that end anywhere in a step; the choice is
+    asserted, so that the case stays on the kernel that it is for.  A row has the bits that the stream gives it alone."""
+    from spite_amd.csrc.hipops import lib
+    n, ng = sum(sizes), len(sizes)
+    assert lib().spite_gemm_f32_choice(n, N, K, ng, int(glu)) == -64
+    offsets = torch.tensor([0] + list(torch.tensor(sizes).cumsum(0)), dtype=torch.int32, device=DEV)
+    x, ws = rnd(n, K, seed=5), rnd(ng, (2 if glu else 1) * N, K, seed=6)
+    y = torch.empty(n, N, device=DEV)
+    ops().gemm_generic(x, ws, y, n, N, K, glu=glu, offsets=offsets, n_groups=ng)
+    at = 0
+    for g, size in enumerate(sizes):
+        for r in {at, at + size // 2, at + size - 1} if size else ():
+            alone = torch.empty(1, N, device=DEV)
+            ops().gemm_generic(x[r:r + 1].contiguous(), ws[g].contiguous(), alone, 1, N, K, glu=glu)
+            assert torch.equal(alone[0], y[r]), (g, r - at)
         at += size
