@@ -163,6 +163,138 @@ void gemm_skinny_kernel(const bf16* __restrict__ X, int ldx, const bf16* __restr
     }
 }
 
+// The same for W in operand order over groups of up to 16 rows, and for one or two rows, with the loads of a wave's next block on
+// their way while a block is multiplied.  In the kernel above every load stands behind a condition, so that each product waits for all
+// that were asked for; many waves make up for that where the stream is long, a short one waits for memory block by block.  Here
+// each number of blocks that may be left has a piece of its own without conditions; all arguments are read at once, and what a
+// result's place depends on before the stream, not behind it.  The same bits.  Not for three and more rows without groups nor for
+// tables of 2^27 elements: those gain by the other kernel's fewer loads in flight (8 x 5,120 x 5,120 13.1 us, by this one 14.6; 1 x
+// 32,768 x 5,120 52.7 / 54.3).
+// us in a chain of launches in a graph, the kernel above and this one: 1 x 3,072 x 2,048 4.45 / 4.14, 1 x 2,048 x 2,048 4.05 / 3.86, two groups of
+// one row x 2,048 x 3,072 7.16 / 6.66 and 2 x 3,072 x 2,048 gated 11.60 / 11.02, 2 x 8,192 x 5,120 53.8 / 52.7; nine groups of 8 rows x 2 x 8,192 x
+// 5,120 225.3 / 224.3, 33 of 1 to 32 rows 720.4 / 719.1.  An empty kernel takes 1.7.
+#include <type_traits>
+
+// A buffer of 2 GiB from p on, p the same in every lane.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t sk_buffer(const void* p) {
+    const uint64_t a = (uint64_t)(uintptr_t)p;
+    const uint64_t u = ((uint64_t)(uint32_t)__builtin_amdgcn_readfirstlane((int)(a >> 32)) << 32) | (uint32_t)__builtin_amdgcn_readfirstlane((int)a);
+    return __builtin_amdgcn_make_buffer_rsrc((void*)(uintptr_t)u, 0, 0x7fffffff, 0x00020000);
+}
+
+template <int R, int NW, bool GLU, typename TY>
+__global__ __launch_bounds__(NW * 64)
+void gemm_skinny_piped_kernel(const bf16* __restrict__ X, int ldx, const bf16* __restrict__ W, long w_group_stride,
+                              TY* __restrict__ Y, int ldy, int M, int N, int K,
+                              const int* __restrict__ offsets, int n_groups, const int* __restrict__ a_rows,
+                              const float* __restrict__ a_scale, const int* __restrict__ y_rows, int act, float act_limit) {
+    constexpr int RA = GLU ? 2 * R : R;        // A tiles per wave
+    constexpr int J = RA * 4, JO = R * 4;      // partial sums and results per lane position (gate and up fold into one)
+    extern __shared__ float red[];             // [NW][J][64]
+    asm volatile("" :: "s"(X), "s"(ldx), "s"(W), "s"(w_group_stride), "s"(Y), "s"(ldy), "s"(M), "s"(N), "s"(K), "s"(offsets), "s"(n_groups),
+                 "s"(a_rows), "s"(a_scale), "s"(y_rows), "s"(act), "s"(act_limit));
+    int g = 0, row0, row_end = M;
+    if (offsets) {
+        if (!sp_find_tile(offsets, n_groups, 16, blockIdx.y, g, row0, row_end)) return;
+    } else {
+        row0 = blockIdx.y * 16;
+        if (row0 >= M) return;
+    }
+    const int n0 = blockIdx.x * (16 * R);
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int r = lane & 15, q = lane >> 4;
+    const bool live = row0 + r < row_end;
+    const int slot = live ? row0 + r : row_end - 1;        // slots past the group: its last slot
+    const int x_at = a_rows ? a_rows[slot] : slot;
+    float out_scale = a_scale ? a_scale[slot] : 1.0f;
+    int out_row = y_rows ? y_rows[slot] : slot;
+
+    const bf16* Wg = W + (size_t)g * w_group_stride + (size_t)n0 * K;
+    const __amdgpu_buffer_rsrc_t wbuf = sk_buffer(Wg), ubuf = sk_buffer(Wg + (size_t)(GLU ? N : 0) * K);
+    int band[R];                               // a band of 16 rows; bands past N read the last one again, what that gives is not stored
+#pragma unroll
+    for (int a = 0; a < R; ++a) band[a] = __builtin_amdgcn_readfirstlane((n0 / 16 + a < N / 16 ? a : N / 16 - 1 - n0 / 16) * K * 32);
+    const int wlane = lane * 16, blocks = K / 64;
+    const int n_blk = blocks > wave ? (blocks - wave + NW - 1) / NW : 0;      // the wave's blocks: wave, wave + NW, ..
+    const bf16* xp = nullptr;
+    bf16x8 w[2][RA][2], x[2][2];
+    auto load_w = [&](bf16x8 (&w)[RA][2], int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int a = 0; a < RA; ++a) {
+                const int at = __builtin_amdgcn_readfirstlane(band[a % R] + ((wave + i * NW) * 2 + s) * 1024);
+                w[a][s] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(a < R ? wbuf : ubuf, wlane, at, 2));   // (2: non-temporal)
+            }
+    };
+    auto load_x = [&](bf16x8 (&x)[2], int i) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s) x[s] = *(const bf16x8*)(xp + (wave + i * NW) * 64 + s * 32);
+    };
+    f32x4 acc[RA];
+#pragma unroll
+    for (int a = 0; a < RA; ++a) acc[a] = f32x4{0.f, 0.f, 0.f, 0.f};
+    auto mul = [&](int j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int s = 0; s < 2; ++s)
+#pragma unroll
+            for (int a = 0; a < RA; ++a) acc[a] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j][a][s], x[j][s], acc[a], 0, 0, 0);
+    };
+    auto start = [&](auto n) __attribute__((always_inline)) {       // W first: the rows of X may wait for the row list
+#pragma unroll
+        for (int j = 0; j < n.value; ++j) load_w(w[j], j);
+        __builtin_amdgcn_sched_barrier(0);
+        xp = X + (size_t)x_at * ldx + q * 8;
+#pragma unroll
+        for (int j = 0; j < n.value; ++j) load_x(x[j], j);
+    };
+    auto next = [&](int j, int i) __attribute__((always_inline)) { load_w(w[j], i); load_x(x[j], i); };
+    if (n_blk >= 2) {
+        start(std::integral_constant<int, 2>());
+        int i = 0;
+        for (; i + 4 <= n_blk; i += 2) {
+            mul(0);
+            next(0, i + 2);
+            mul(1);
+            next(1, i + 3);
+        }
+        if (i + 2 == n_blk) {
+            mul(0);
+            mul(1);
+        } else {
+            mul(0);
+            next(0, i + 2);
+            mul(1);
+            mul(0);
+        }
+    } else if (n_blk == 1) {
+        start(std::integral_constant<int, 1>());
+        mul(0);
+    }
+    // partial sums of the waves meet in LDS: red[wave][j][lane]
+#pragma unroll
+    for (int a = 0; a < RA; ++a)
+#pragma unroll
+        for (int i = 0; i < 4; ++i) red[(wave * J + a * 4 + i) * 64 + lane] = acc[a][i];
+    asm volatile("" : "+v"(out_scale), "+v"(out_row));     // (here at the latest, not behind the barrier)
+    __syncthreads();
+    // acc[a][i] of lane (r, q) is the element (row n0 + a*16 + q*4 + i, slot row0 + r): a wave sums one of them, the others have none
+    static_assert(JO <= NW, "a wave sums one result of a lane");
+    if (wave >= JO) return;
+    const int n = n0 + (wave >> 2) * 16 + q * 4 + (wave & 3);
+    if (n >= N || !live) return;
+    float v = 0.f, u = 0.f;
+#pragma unroll
+    for (int i = 0; i < NW; ++i) {
+        v += red[(i * J + wave) * 64 + lane];
+        if (GLU) u += red[(i * J + wave + JO) * 64 + lane];
+    }
+    if (a_scale) { v *= out_scale; u *= out_scale; }
+    if (GLU) v = sp_gated(v, u, act, act_limit, true);
+    else if (act < 0) v = sp_unary(v, -act, true);
+    Y[(size_t)out_row * ldy + n] = from_f32<TY>(v);
+}
+
 // The activation of the product that the calling thread is launching: the gate's code, or minus the
 // code of a plain product's own activation (set by the entry point).
 static thread_local int g_skinny_act = 0;
@@ -182,8 +314,11 @@ static int launch_skinny(const void* X, int ldx, const void* W, long wgs, void* 
     SP_REQUIRE(m_tiles <= 65535, "gemm_skinny: too many row tiles (%d)", m_tiles);
     dim3 grid((N + 16 * R - 1) / (16 * R), m_tiles);
     const size_t sh = (size_t)NW * (glu ? 2 : 1) * R * G * 4 * 64 * sizeof(float);
+    constexpr bool can = G == 1 && S == 2 && R * 4 <= NW;
+    const bool piped = can && tiled && K % 64 == 0 && (offsets || (M <= 2 && (size_t)N * K < ((size_t)1 << 27)));
 #define SP_SK(GLUV, TY) do { \
-        auto kern = tiled ? gemm_skinny_kernel<R, G, S, NW, GLUV, true, TY> : gemm_skinny_kernel<R, G, S, NW, GLUV, false, TY>; \
+        auto kern = piped ? gemm_skinny_piped_kernel<can ? R : 1, can ? NW : 4, GLUV, TY> : \
+            tiled ? gemm_skinny_kernel<R, G, S, NW, GLUV, true, TY> : gemm_skinny_kernel<R, G, S, NW, GLUV, false, TY>; \
         if (sh > 48 * 1024) { hipError_t e = hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)sh); \
             if (e != hipSuccess) return sp_fail("gemm_skinny: cannot get %zu bytes of LDS: %s", sh, hipGetErrorString(e)); } \
         kern<<<grid, NW * 64, sh, st>>>((const bf16*)X, ldx, (const bf16*)W, wgs, (TY*)Y, ldy, M, N, K, offsets, \
@@ -261,6 +396,7 @@ extern "C" int spite_gemm_skinny(const void* X, int ldx, const void* W, long w_g
     SP_REQUIRE(y_dtype == SP_BF16 || y_dtype == SP_F32, "gemm_skinny: output dtype %d", y_dtype);
     SP_REQUIRE(!offsets || n_groups > 0, "gemm_skinny: grouped call without groups");
     SP_REQUIRE(!w_tiled || (K % 32 == 0 && N % 16 == 0), "gemm_skinny: operand order needs K=%d a multiple of 32 and N=%d of 16", K, N);
+    SP_REQUIRE(K < (1 << 24), "gemm_skinny: K=%d is beyond the loads' 32-bit offsets", K);
     if (M == 0) return 0;
 #define SP_ARGS X, ldx, W, w_group_stride, Y, y_dtype, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, w_tiled, live_groups, st
     if (variant == 0) variant = skinny_variant(M, N, K, offsets ? n_groups : 0, live_groups, glu != 0, max_rows);
