@@ -64,18 +64,6 @@ __device__ __forceinline__ float wave_max(float v) {
     return v;
 }
 
-// The sum over the lanes up to and with this one, by moves within the vector registers (through LDS, as shuffles go, each of the six
-// steps is a wait).
-__device__ __forceinline__ int sp_wave_scan(int x) {
-    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);      // from one lane below within 16, two, four, eight
-    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
-    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);     // lane 15 to row 1, 47 to row 3
-    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);     // lane 31 to rows 2 and 3
-    return x;
-}
-
 // Which group and which rows the row tile `mt` of a grouped product covers.  Groups are walked
 // in order, group e bringing ceil((offsets[e+1] - offsets[e]) / MT) tiles of MT rows.  A wave
 // looks at 64 groups at a time (a prefix sum over its lanes), so that hundreds of groups cost a
@@ -90,10 +78,47 @@ __device__ __forceinline__ bool sp_find_tile(const int* offsets, int n_groups, i
         int b = 0, en = 0;
         if (e < n_groups) { b = offsets[e]; en = offsets[e + 1]; }
         const int nt = (en - b + MT - 1) / MT;
-        const int incl = sp_wave_scan(nt), total = __builtin_amdgcn_readlane(incl, 63);
+        int incl = nt;
+#pragma unroll
+        for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
+        const int total = __shfl(incl, 63, 64);
         if (mt < base + total) {
             const bool mine = mt >= base + incl - nt && mt < base + incl;
-            // the same in every lane: read from its lane, in scalar registers
+            const int src = __ffsll((unsigned long long)__ballot(mine)) - 1;
+            // the same in every lane: say so, to keep them in scalar registers
+            g = __builtin_amdgcn_readfirstlane(c + src);
+            row0 = __builtin_amdgcn_readfirstlane(__shfl(b, src, 64) + (mt - base - __shfl(incl - nt, src, 64)) * MT);
+            row_end = __builtin_amdgcn_readfirstlane(__shfl(en, src, 64));
+            return true;
+        }
+        base += total;
+    }
+    return false;
+}
+
+// The sum over the lanes up to and with this one, by moves within the vector registers (through LDS, as shuffles go, each of the six
+// steps is a wait).
+__device__ __forceinline__ int sp_wave_scan(int x) {
+    x += __builtin_amdgcn_update_dpp(0, x, 0x111, 0xf, 0xf, true);      // from one lane below within 16, two, four, eight
+    x += __builtin_amdgcn_update_dpp(0, x, 0x112, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x114, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x118, 0xf, 0xf, true);
+    x += __builtin_amdgcn_update_dpp(0, x, 0x142, 0xa, 0xf, false);     // lane 15 to row 1, 47 to row 3
+    x += __builtin_amdgcn_update_dpp(0, x, 0x143, 0xc, 0xf, false);     // lane 31 to rows 2 and 3
+    return x;
+}
+
+// The same by the scan above, for kernels of few rows, whose start is a good part of their time: 0.2 to 0.4 us less.  (Not in the other's
+// place everywhere: with its results in scalar registers the fp32 tiles spill, 145 -> 157 us.)
+__device__ __forceinline__ bool sp_find_tile_scalar(const int* offsets, int n_groups, int MT, int mt, int& g, int& row0, int& row_end) {
+    const int lane = threadIdx.x & 63;
+    int base = 0;
+    for (int c = 0; c < n_groups; c += 64) {
+        int b = 0, en = 0;
+        if (c + lane < n_groups) { b = offsets[c + lane]; en = offsets[c + lane + 1]; }
+        const int nt = (en - b + MT - 1) / MT, incl = sp_wave_scan(nt), total = __builtin_amdgcn_readlane(incl, 63);
+        if (mt < base + total) {
+            const bool mine = mt >= base + incl - nt && mt < base + incl;
             const int src = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(mine)) - 1);
             g = c + src;
             row0 = __builtin_amdgcn_readlane(b, src) + (mt - base - __builtin_amdgcn_readlane(incl - nt, src)) * MT;

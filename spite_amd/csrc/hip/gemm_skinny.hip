@@ -195,7 +195,7 @@ void gemm_skinny_piped_kernel(const bf16* __restrict__ X, int ldx, const bf16* _
                  "s"(a_rows), "s"(a_scale), "s"(y_rows), "s"(act), "s"(act_limit));
     int g = 0, row0, row_end = M;
     if (offsets) {
-        if (!sp_find_tile(offsets, n_groups, 16, blockIdx.y, g, row0, row_end)) return;
+        if (!sp_find_tile_scalar(offsets, n_groups, 16, blockIdx.y, g, row0, row_end)) return;
     } else {
         row0 = blockIdx.y * 16;
         if (row0 >= M) return;
