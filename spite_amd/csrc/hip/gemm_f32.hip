@@ -9,7 +9,10 @@
 //
 //  gemm_f32_rows: few rows.  Bound by the stream of W (one row of X makes 0.5 FLOP a byte).  A workgroup takes 16
 //    rows of W (GLU: 16 of each half) and gives one run of k to each of its eight waves, so that a product with
-//    2,048 output rows has 1,024 waves in flight; the runs' sums meet in LDS.
+//    2,048 output rows has 1,024 waves in flight; the runs' sums meet in LDS.  A wave's next 32 k are on their way while 32 are multiplied, so
+//    that a wave needs 54 registers and three and four workgroups fit a compute unit (us, with 128 k asked for behind conditions and waited for
+//    together / now: 1 row x 3,072 x 2,048 8.4 / 7.5, x 32,768 54.8 / 50.6, two groups of a row gated 2 x 3,072 x 2,048 24.4 / 19.1, 17 groups
+//    of 16 rows and of one 107.5 / 97.7, 64 x 3,072 x 2,048 25.8 / 23.8).
 //  gemm_f32_tile: many rows, bound by the MFMAs (256 FLOP a clock and compute unit).  TM (64 or 32) rows of X times 64 rows of
 //    W a workgroup: X through double-buffered LDS, a step ahead, read by all four waves; a wave's 16 rows of W straight into
 //    registers, two steps ahead.  One workgroup a compute unit reaches 70 % of the units' rate at K = 2,048, its start and end included.
@@ -48,9 +51,11 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
                           int act, float act_limit, int vec_y) {
     constexpr int NB = GLU && !HALVES ? 2 : 1;
     __shared__ f32x4 red[8][MT * NB][64];
+    asm volatile("" :: "s"(A), "s"(lda), "s"(W), "s"(w_group_stride), "s"(Y), "s"(ldy), "s"(M), "s"(N), "s"(K), "s"(offsets), "s"(n_groups), "s"(a_rows),
+                 "s"(a_scale), "s"(y_rows), "s"(act), "s"(act_limit), "s"(vec_y));      // (every argument at once)
     int g = 0, row0 = 0, row_end = M;
     if (offsets) {
-        if (!sp_find_tile(offsets, n_groups, MT * 16, blockIdx.y, g, row0, row_end)) return;
+        if (!sp_find_tile_scalar(offsets, n_groups, MT * 16, blockIdx.y, g, row0, row_end)) return;
     } else {
         row0 = blockIdx.y * (MT * 16);
     }
@@ -80,26 +85,63 @@ void gemm_f32_rows_kernel(const float* __restrict__ A, int lda, const float* __r
     for (int m = 0; m < MT; ++m)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[m][b] = {0.f, 0.f, 0.f, 0.f};
-    constexpr int U = MT == 4 ? 4 : 8;                  // steps of 16 k whose loads are in flight together (registers)
-    for (int k0 = k_lo; k0 < k_hi; k0 += 16 * U) {
-        f32x4 w[U][NB], x[U][MT];
+    constexpr int U = 2, KU = 16 * U;                   // steps of 16 k a piece (four: one or two rows 3 to 6 % slower, tall tables 3 % faster)
+    f32x4 w[2][U][NB], x[2][U][MT];
+    auto load = [&](int to, int k0) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             const int k = k0 + u * 16 + q * 4;
-            const bool in = k < k_hi;                  // K is a multiple of 4, a run's end of 4
 #pragma unroll
-            for (int b = 0; b < NB; ++b) w[u][b] = in ? *(const f32x4*)(wp[b] + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int b = 0; b < NB; ++b) w[to][u][b] = *(const f32x4*)(wp[b] + k);
 #pragma unroll
-            for (int m = 0; m < MT; ++m) x[u][m] = in ? *(const f32x4*)(xp[m] + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int m = 0; m < MT; ++m) x[to][u][m] = *(const f32x4*)(xp[m] + k);
         }
+    };
+    auto mul = [&](int to) __attribute__((always_inline)) {
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
             for (int m = 0; m < MT; ++m) {
-                const f32x4 xs = x[u][m] * sc[m];
+                const f32x4 xs = x[to][u][m] * sc[m];
 #pragma unroll
-                for (int b = 0; b < NB; ++b) f32_step(acc[m][b], w[u][b], xs);
+                for (int b = 0; b < NB; ++b) f32_step(acc[m][b], w[to][u][b], xs);
             }
+    };
+    // A piece is multiplied while the next one is on its way.  No load stands behind a condition, where the compiler would wait at the
+    // next product for every load there may be.
+    const int whole = k_hi > k_lo ? (k_hi - k_lo) / KU : 0;
+    if (whole >= 2) {
+        load(0, k_lo);
+        load(1, k_lo + KU);
+        int i = 0;
+        for (; i + 4 <= whole; i += 2) {
+            mul(0);
+            load(0, k_lo + (i + 2) * KU);
+            mul(1);
+            load(1, k_lo + (i + 3) * KU);
+        }
+        mul(0);
+        if (i + 2 == whole) mul(1);
+        else {
+            load(0, k_lo + (i + 2) * KU);
+            mul(1);
+            mul(0);
+        }
+    } else if (whole == 1) {
+        load(0, k_lo);
+        mul(0);
+    }
+    if (k_lo + whole * KU < k_hi) {                    // the run's end: zeros past it (K is a multiple of 4, a run's end of 4)
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+            const int k = k_lo + whole * KU + u * 16 + q * 4;
+            const bool in = k < k_hi;
+#pragma unroll
+            for (int b = 0; b < NB; ++b) w[0][u][b] = in ? *(const f32x4*)(wp[b] + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int m = 0; m < MT; ++m) x[0][u][m] = in ? *(const f32x4*)(xp[m] + k) : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+        mul(0);
     }
 #pragma unroll
     for (int m = 0; m < MT; ++m)
