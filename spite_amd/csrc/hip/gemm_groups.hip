@@ -5,8 +5,9 @@
 // of one height for all multiplies padding for the small groups and reads W again for the large ones; here every group
 // takes as few tiles as `cap` rows (128 or 160) allow, all of the height, in units of 16 rows, that then covers it.
 //
-// A workgroup of NW waves (eight or four) owns 64 * NW rows of W (GLU: 32 * NW gate rows and the matching up rows) and one tile
-// of 16 * NB rows of X; a wave owns 64 rows of W and every row of X: 4 x NB accumulator tiles.
+// A workgroup of NW waves (eight or four) owns 16 * A * NW rows of W (GLU: half of them gate rows, the others the matching up rows) and
+// one tile of 16 * NB rows of X; a wave owns A bands of 16 rows of W and every row of X: A x NB accumulator tiles.  A is four, or five for
+// plain products whose tiles of 320 columns fit the chip where those of 256 and 512 do not (one wave a SIMD, its accumulators in AGPRs).
 //  * W never touches LDS: S rotating sets of operand registers (six up to 96 rows, four above), each asked for again as soon as
 //    its products are issued, S - 1 half steps of 32 k ahead.  A group of one tile reads its W once: non-temporal loads.
 //  * X goes straight to LDS (buffer loads with the lds bit), four buffers of 64 k, asked for three steps ahead: no register
@@ -15,8 +16,8 @@
 //  * Rows past the group and steps past K (K is cut into rounds of S / 2 steps of 64) are loads beyond the buffer's end, which
 //    give zeros: no branch in the loop, and products of zeros cost the matrix units less power, which is what bounds the
 //    clock here.
-//  * Workgroups go to the eight XCDs in turn; XCD x takes the x-th eighth of the tiles, the row tile running fastest, so that
-//    those which run at a time share what they read.
+//  * Workgroups go to the eight XCDs in turn, an eighth of the tiles each, in an order by which those that run at a time share what they
+//    read (gemm_groups_kernel).
 // The sum over k runs in the order of gemm_tiled and gemm_lds: the same bits.
 //
 // Measured on an MI355X against gemm_tiled's best tile (us; 16 experts of which a token takes `top`, beside them one or two
@@ -42,11 +43,11 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t gg_buffer(const void* p) {
 }
 
 // One tile: rows row0 .. of the group g whose rows end at row_end, columns of the result from n0 on.
-template <int NW, int NB, int S, bool GLU, typename TY, bool NTW>
+template <int NW, int A, int NB, int S, bool GLU, typename TY, bool NTW>
 __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, int g, int row0, int row_end, int n0, int u_first, int nu, TY* Y) {
     constexpr int XB = 16 * NB * 128;                            // bytes of a step of X
     constexpr int XI = (2 * NB + NW - 1) / NW;                   // load instructions a wave: a step of X (eight rows each)
-    constexpr int TG = GLU ? 2 : 4;                              // bands that name distinct columns
+    constexpr int TG = GLU ? A / 2 : A;                          // bands that name distinct columns
     static_assert(S % 2 == 0, "whole steps a round");
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int r = lane & 15, q = lane >> 4, N = p.N, kt = 2 * nu;
@@ -60,9 +61,9 @@ __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, in
         xoff[i] = (p.a_rows ? p.a_rows[at] : at) * p.ldx * 2 + (((lane & 7) ^ ((row >> 1) & 7)) * 16);
         if (s >= row_end) xoff[i] = GG_PAST;
     }
-    int wband[4];
+    int wband[A];
 #pragma unroll
-    for (int a = 0; a < 4; ++a) {
+    for (int a = 0; a < A; ++a) {
         int band = n0 / 16 + wave * TG + a % TG;
         band = band < N / 16 ? band : N / 16 - 1;                // bands past N read the last one again
         if (GLU && a >= TG) band += N / 16;
@@ -75,19 +76,19 @@ __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, in
 #pragma unroll
         for (int i = 0; i < XI; ++i) sp_load_lds(xbuf, xoff[i] | past, __builtin_amdgcn_readfirstlane(k0), lds0 + (u & 3) * XB + xblk[i] * 1024);
     };
-    auto load_w = [&](bf16x8 (&ws)[4], int t) {
+    auto load_w = [&](bf16x8 (&ws)[A], int t) {
         const int at = (t < kt ? t : 0) * 1024, past = t < kt ? 0 : GG_PAST;
 #pragma unroll
-        for (int a = 0; a < 4; ++a)          // (2: non-temporal)
+        for (int a = 0; a < A; ++a)          // (2: non-temporal)
             ws[a] = __builtin_bit_cast(bf16x8, __builtin_amdgcn_raw_buffer_load_b128(wbuf, wlane | past, wband[a] + at, NTW ? 2 : 0));
     };
-    f32x4 acc[4][NB];          // [W band a][slot tile b]
+    f32x4 acc[A][NB];          // [W band a][slot tile b]
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+    for (int a = 0; a < A; ++a)
 #pragma unroll
         for (int b = 0; b < NB; ++b) acc[a][b] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int swz = (r >> 1) & 7, xl0 = r * 128 + ((q ^ swz) * 16), xl1 = r * 128 + (((4 + q) ^ swz) * 16);
-    auto mul = [&](bf16x8 (&ws)[4], int buf, int kk) {
+    auto mul = [&](bf16x8 (&ws)[A], int buf, int kk) {
         const unsigned char* xs = lds + buf * XB + (kk ? xl1 : xl0);
         constexpr int NX = NB == 9 ? 3 : 4;                      // slot tiles read from LDS at a time
 #pragma unroll
@@ -97,7 +98,7 @@ __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, in
             for (int b = 0; b < NX; ++b)
                 if (b0 + b < NB) xf[b] = *(const bf16x8*)(xs + (b0 + b) * 2048);
 #pragma unroll
-            for (int a = 0; a < 4; ++a)
+            for (int a = 0; a < A; ++a)
 #pragma unroll
                 for (int b = 0; b < NX; ++b)
                     if (b0 + b < NB)
@@ -108,19 +109,20 @@ __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, in
     // left (every wave has passed the barrier behind it).  Before the barrier each wave waits until its own loads of X for
     // step u + 1 are there: younger than those are two steps of X and the W asked for since, three steps of eight loads or,
     // with fewer sets, at least the sets of the start and one step.
-    constexpr int PENDING = 2 * XI + (8 + 4 * S < 24 ? 8 + 4 * S : 24);
+    constexpr int PENDING = 2 * XI + (2 + S < 6 ? 2 + S : 6) * A;
+    static_assert(PENDING < 64, "a wait for more loads than the counter holds");
 #define GG_MEET(pending) do { \
         asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" :: "n"(pending) : "memory"); \
         __builtin_amdgcn_s_barrier(); \
         __builtin_amdgcn_sched_barrier(0); } while (0)
-    bf16x8 w[S][4];
+    bf16x8 w[S][A];
     load_x(0);
     load_x(1);
     load_x(2);
 #pragma unroll
     for (int s = 0; s < S; ++s) load_w(w[s], s);
-    GG_MEET(2 * XI + 4 * S);
-    auto step = [&](bf16x8 (&wa)[4], bf16x8 (&wb)[4], int u) {
+    GG_MEET(2 * XI + A * S);
+    auto step = [&](bf16x8 (&wa)[A], bf16x8 (&wb)[A], int u) {
         load_x(u + 3);
         __builtin_amdgcn_sched_barrier(0);
         mul(wa, u & 3, 0);
@@ -153,7 +155,7 @@ __device__ __forceinline__ void gg_tile(const gg_args& p, unsigned char* lds, in
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
                 v[i] = acc[a][b][i] * sc;
-                if constexpr (GLU) v[i] = sp_gated(v[i], acc[a + 2][b][i] * sc, SP_ACT_SILU, 0.f, true);
+                if constexpr (GLU) v[i] = sp_gated(v[i], acc[a + TG][b][i] * sc, SP_ACT_SILU, 0.f, true);
             }
             if constexpr (sizeof(TY) == 2) {
                 bf16x4 o;
@@ -175,8 +177,8 @@ __device__ __host__ __forceinline__ int gg_group_tiles(int rows, int cap, int& n
     return tiles;
 }
 
-template <int NW, bool GLU, typename TY>
-__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(2, 2)))
+template <int NW, int A, bool GLU, typename TY>
+__global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(A == 4 ? 2 : 1, A == 4 ? 2 : 1)))
 void gemm_groups_kernel(gg_args p) {
     extern __shared__ __attribute__((aligned(1024))) unsigned char lds[];
     // The groups' tiles, 64 groups at a time: a prefix sum over the lanes (one after another the loads of the offsets cost half a
@@ -185,67 +187,133 @@ void gemm_groups_kernel(gg_args p) {
     // more than its eighth, and two tiles met on one compute unit while others had none (126 rows of 4 of 4 experts and of one more x 2 x
     // 5,120 x 16,384 gated, 200 tiles of four waves, 506 -> 292 us; 1,483 of 8 of 32 x 768 x 16,384, eight waves, 846 -> 483; over 559 sizes 0.96).
     const int lane = threadIdx.x & 63;
-    int b = 0, e = 0, h = 0, nt = 0, incl = 0, all = 0;
-    auto scan = [&](int c) {
-        b = e = 0;
-        if (c + lane < p.n_groups) { b = p.offsets[c + lane]; e = p.offsets[c + lane + 1]; }
-        nt = incl = gg_group_tiles(e - b, p.cap, h);
+    int b = 0, e = 0, h = 0, nt = 0;                     // the lane's group: its rows, their tiles and these tiles' height
+    int g = -1, row0 = 0, row_end = 0, nb = 8, tiles = 1, col = 0;
+    if constexpr (NW == 8) {                             // row tiles of all groups run fastest
+        int incl = 0, all = 0;
+        auto scan = [&](int c) {
+            b = e = 0;
+            if (c + lane < p.n_groups) { b = p.offsets[c + lane]; e = p.offsets[c + lane + 1]; }
+            nt = incl = gg_group_tiles(e - b, p.cap, h);
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
-        return __builtin_amdgcn_readlane(incl, 63);
-    };
-    for (int c = 0; c < p.n_groups; c += 64) all += scan(c);
-    const int units = all * p.n_tiles, per_xcd = (units + 7) / 8;
-    const int unit = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
-    if ((int)(blockIdx.x / 8) >= per_xcd || unit >= units) return;
-    const int mt = __builtin_amdgcn_readfirstlane(unit % all);
-    int g = -1, row0 = 0, row_end = 0, nb = 8, tiles = 0, base = 0;
-    for (int c = 0; c < p.n_groups; c += 64) {
-        const int total = p.n_groups <= 64 ? all : scan(c);
-        if (mt < base + total) {
-            const bool mine = mt >= base + incl - nt && mt < base + incl;
-            const int src = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(mine)) - 1);
-            g = c + src;
-            nb = __builtin_amdgcn_readlane(h, src);
-            tiles = __builtin_amdgcn_readlane(nt, src);
-            row_end = __builtin_amdgcn_readlane(e, src);
-            row0 = __builtin_amdgcn_readlane(b, src) + (mt - base - __builtin_amdgcn_readlane(incl - nt, src)) * 16 * nb;
-            break;
+            for (int o = 1; o < 64; o <<= 1) { const int v = __shfl_up(incl, o, 64); if (lane >= o) incl += v; }
+            return __builtin_amdgcn_readlane(incl, 63);
+        };
+        for (int c = 0; c < p.n_groups; c += 64) all += scan(c);
+        const int units = all * p.n_tiles, per_xcd = (units + 7) / 8;
+        const int unit = (blockIdx.x % 8) * per_xcd + blockIdx.x / 8;
+        if ((int)(blockIdx.x / 8) >= per_xcd || unit >= units) return;
+        const int mt = __builtin_amdgcn_readfirstlane(unit % all);
+        int base = 0;
+        for (int c = 0; c < p.n_groups; c += 64) {
+            const int total = p.n_groups <= 64 ? all : scan(c);
+            if (mt < base + total) {
+                const bool mine = mt >= base + incl - nt && mt < base + incl;
+                const int src = __builtin_amdgcn_readfirstlane(__ffsll((unsigned long long)__ballot(mine)) - 1);
+                g = c + src;
+                nb = __builtin_amdgcn_readlane(h, src);
+                tiles = __builtin_amdgcn_readlane(nt, src);
+                row_end = __builtin_amdgcn_readlane(e, src);
+                row0 = __builtin_amdgcn_readlane(b, src) + (mt - base - __builtin_amdgcn_readlane(incl - nt, src)) * 16 * nb;
+                break;
+            }
+            base += total;
         }
-        base += total;
+        col = __builtin_amdgcn_readfirstlane(unit / all);
+    } else {
+        // (Not with eight waves: a gated product beside a shared expert lost 3 to 5 %.)
+        //  * groups of up to four tiles and no more than twice the average (experts): all columns of a group go to one XCD, row tiles of a column
+        //    next to each other, so that what runs there at a time reads the group's rows of X once from memory and its W once;
+        //  * larger ones (a shared expert): row tiles of all of them running fastest, an eighth of the columns an XCD.
+        // An XCD has an eighth of either kind, in turn: the first wait for the stream of W, the second for the matrix units.  (1,531 rows of 4 of
+        // 16 experts and of two more x 2,048 x 1,024 59.7 -> 53.6 us, 2 x 1,024 x 2,048 gated 93.4 -> 89.8; one tile of 320 columns a compute unit, 2,048
+        // rows x 5,120 x 8,192, 242 -> 223, with 1.38 GB read instead of 1.61.)
+        int few = 0, many = 0, limit = 0;      // tiles of either kind up to and with the lane's group; the first kind's most
+        auto look = [&](int c) {
+            b = e = 0;
+            if (c + lane < p.n_groups) { b = p.offsets[c + lane]; e = p.offsets[c + lane + 1]; }
+            nt = gg_group_tiles(e - b, p.cap, h);
+        };
+        auto scan = [&](int c) {
+            if (c > 0 || p.n_groups > 64) look(c);
+            few = sp_wave_scan(nt <= limit ? nt : 0);
+            many = sp_wave_scan(nt <= limit ? 0 : nt);
+        };
+        int all = 0, live = 0;
+        for (int c = 0; c < p.n_groups; c += 64) {
+            look(c);
+            all += __builtin_amdgcn_readlane(sp_wave_scan(nt), 63);
+            live += __popcll(__ballot(nt > 0));
+        }
+        if (all == 0) return;
+        limit = min(4, 2 * all / live);
+        int all_few = 0, all_many = 0;
+        for (int c = 0; c < p.n_groups; c += 64) {
+            scan(c);
+            all_few += __builtin_amdgcn_readlane(few, 63);
+            all_many += __builtin_amdgcn_readlane(many, 63);
+        }
+        const int xcd = blockIdx.x % 8, at = blockIdx.x / 8;     // the XCD's workgroups in turn
+        const int units_few = all_few * p.n_tiles, units_many = all_many * p.n_tiles, per_few = (units_few + 7) / 8, per_many = (units_many + 7) / 8;
+        const int n_few = min(max(units_few - xcd * per_few, 0), per_few), n_all = n_few + min(max(units_many - xcd * per_many, 0), per_many);
+        if (at >= n_all) return;
+        const int before = __builtin_amdgcn_readfirstlane((int)((long)at * n_few / n_all));
+        const bool is_few = __builtin_amdgcn_readfirstlane((int)((long)(at + 1) * n_few / n_all)) > before;
+        const int unit = is_few ? xcd * per_few + before : xcd * per_many + at - before;
+        const int mt = is_few ? 0 : __builtin_amdgcn_readfirstlane(unit % all_many);
+        int base = 0;
+        for (int c = 0; c < p.n_groups; c += 64) {
+            if (p.n_groups > 64) scan(c);
+            const int first = base + (is_few ? few - (nt <= limit ? nt : 0) : many - (nt <= limit ? 0 : nt));      // tiles of its kind before the lane's group
+            const bool mine = (nt <= limit) == is_few && (is_few ? unit >= first * p.n_tiles && unit < (first + nt) * p.n_tiles : mt >= first && mt < first + nt);
+            const unsigned long long who = __ballot(mine);
+            if (who) {
+                const int src = __builtin_amdgcn_readfirstlane(__ffsll(who) - 1);
+                const int first_tile = __builtin_amdgcn_readlane(first, src);
+                g = c + src;
+                nb = __builtin_amdgcn_readlane(h, src);
+                tiles = __builtin_amdgcn_readlane(nt, src);
+                row_end = __builtin_amdgcn_readlane(e, src);
+                const int j = unit - first_tile * p.n_tiles;
+                col = __builtin_amdgcn_readfirstlane(is_few ? j / tiles : unit / all_many);
+                row0 = __builtin_amdgcn_readlane(b, src) + (is_few ? __builtin_amdgcn_readfirstlane(j % tiles) : mt - first_tile) * 16 * nb;
+                break;
+            }
+            base += __builtin_amdgcn_readlane(is_few ? few : many, 63);
+        }
     }
     if (g < 0) return;
-    const int n0 = __builtin_amdgcn_readfirstlane(unit / all) * (GLU ? 32 * NW : 64 * NW);
-#define GG_TILE(NB, S, NT) gg_tile<NW, NB, S, GLU, TY, NT>(p, lds, g, row0, row_end, n0, 0, p.K / 64, (TY*)p.Y)
+    const int n0 = col * (GLU ? 8 : 16) * A * NW;
+#define GG_TILE(NB, S, NT) gg_tile<NW, A, NB, S, GLU, TY, NT>(p, lds, g, row0, row_end, n0, 0, p.K / 64, (TY*)p.Y)
 #define GG_TILES(NT) switch (nb) { \
         case 2: GG_TILE(2, 6, NT); break; \
         case 4: GG_TILE(4, 6, NT); break; \
         case 5: GG_TILE(5, 6, NT); break; \
         case 6: GG_TILE(6, 6, NT); break; \
-        case 7: GG_TILE(7, 4, NT); break; \
-        case 8: GG_TILE(8, 4, NT); break; \
-        case 9: GG_TILE(9, 4, NT); break; \
-        default: GG_TILE(10, 4, NT); }
+        case 7: GG_TILE(7, A == 5 ? 6 : 4, NT); break; \
+        case 8: GG_TILE(8, A == 5 ? 6 : 4, NT); break; \
+        case 9: GG_TILE(9, A == 5 ? 6 : 4, NT); break; \
+        default: GG_TILE(10, A == 5 ? 6 : 4, NT); }
     if (tiles == 1) GG_TILES(true) else GG_TILES(false)
 #undef GG_TILES
 #undef GG_TILE
 }
 
-template <int NW, bool GLU, typename TY>
+template <int NW, int A, bool GLU, typename TY>
 static int gg_launch(gg_args p, hipStream_t st) {
-    const int cols = (GLU ? 32 : 64) * NW;
+    const int cols = (GLU ? 8 : 16) * A * NW;
     p.n_tiles = (p.N + cols - 1) / cols;
     // row tiles: a group of r rows has ceil(r / cap): at most r / cap + 1
     p.m_tiles = p.M / p.cap + (p.n_groups < p.M ? p.n_groups : p.M);
     SP_REQUIRE((long)p.m_tiles * p.n_tiles < (1L << 30), "gemm_groups: too many tiles");
-    const int grid = (p.m_tiles * p.n_tiles + 7) / 8 * 8;
+    const int grid = ((p.m_tiles * p.n_tiles + 7) / 8 + 1) * 8;      // (an eighth of either kind, rounded up)
     static bool allowed = false;
     if (!allowed) {
-        hipError_t e = hipFuncSetAttribute((const void*)gemm_groups_kernel<NW, GLU, TY>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 160 * 128);
+        hipError_t e = hipFuncSetAttribute((const void*)gemm_groups_kernel<NW, A, GLU, TY>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 160 * 128);
         SP_REQUIRE(e == hipSuccess, "gemm_groups: 80 KB of LDS refused: %s", hipGetErrorString(e));
         allowed = true;
     }
-    gemm_groups_kernel<NW, GLU, TY><<<grid, NW * 64, (size_t)4 * p.cap * 128, st>>>(p);
+    gemm_groups_kernel<NW, A, GLU, TY><<<grid, NW * 64, (size_t)4 * p.cap * 128, st>>>(p);
     SP_LAUNCH_CHECK("gemm_groups");
     return 0;
 }
@@ -271,7 +339,7 @@ void gemm_runs_kernel(gg_args p, int runs) {
     // (quotients: in scalar registers again)
     const int mt = __builtin_amdgcn_readfirstlane(unit % p.m_tiles), n0 = __builtin_amdgcn_readfirstlane(tile / runs) * 256;
     const int each = __builtin_amdgcn_readfirstlane((all + runs - 1) / runs), first = __builtin_amdgcn_readfirstlane(ks) * each;
-    gg_tile<4, NB, S, false, TY, true>(p, lds, 0, mt * 16 * NB, p.M, n0, first, all - first < each ? all - first : each,
+    gg_tile<4, 4, NB, S, false, TY, true>(p, lds, 0, mt * 16 * NB, p.M, n0, first, all - first < each ? all - first : each,
                                        (TY*)p.Y + (size_t)ks * p.M * p.N);
 }
 
@@ -356,7 +424,7 @@ extern "C" int spite_gemm_runs_choice(int M, int N, int K, double* us) {
     return best;
 }
 
-// Arguments as spite_gemm_lds's (`x_rows`: how many rows X has); `waves` 4 or 8, `cap` 128 or 160.  Gated with silu
+// Arguments as spite_gemm_lds's (`x_rows`: how many rows X has); `waves` 4 or 8, or 5 for four waves of 80 columns (plain only), `cap` 128 or 160.  Gated with silu
 // (`glu` SP_ACT_SILU) or plain (0); rows of Y that 16-byte stores can take.
 extern "C" int spite_gemm_groups(const void* X, int ldx, const void* W, long w_group_stride, void* Y, int y_dtype, int ldy, int M,
                                  int N, int K, const int* offsets, int n_groups, const int* a_rows, const float* a_scale,
@@ -368,19 +436,20 @@ extern "C" int spite_gemm_groups(const void* X, int ldx, const void* W, long w_g
     SP_REQUIRE(ldy % 4 == 0 && ((uintptr_t)Y & 15) == 0, "gemm_groups: rows of Y must be 16-byte aligned");
     SP_REQUIRE(y_dtype == SP_BF16 || y_dtype == SP_F32, "gemm_groups: output dtype %d", y_dtype);
     SP_REQUIRE(glu == 0 || glu == SP_ACT_SILU, "gemm_groups: activation code %d", glu);
-    SP_REQUIRE((waves == 4 || waves == 8) && (cap == 128 || cap == 160), "gemm_groups: %d waves, tiles of %d rows", waves, cap);
+    SP_REQUIRE(((waves == 4 || waves == 8) && (cap == 128 || cap == 160)) || (waves == 5 && !glu && (cap == 128 || cap == 160)), "gemm_groups: %d waves, tiles of %d rows", waves, cap);
     SP_REQUIRE(x_rows > 0 && (a_rows || x_rows >= M), "gemm_groups: %d rows of X", x_rows);
     // the loads' offsets are 32-bit: rows of X and a group's W
     SP_REQUIRE((size_t)x_rows * ldx * 2 < ((size_t)1 << 31) && (size_t)(glu ? 2 : 1) * N * K * 2 < ((size_t)1 << 31),
                "gemm_groups: operands of 2 GiB and more (%d rows of X, N=%d K=%d)", x_rows, N, K);
     if (M == 0) return 0;
     const gg_args p{(const bf16*)X, ldx, (const bf16*)W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, 0, 0, cap};
+    if (waves == 5) return y_dtype == SP_BF16 ? gg_launch<4, 5, false, bf16>(p, st) : gg_launch<4, 5, false, float>(p, st);
     if (waves == 8) {
-        if (glu) return y_dtype == SP_BF16 ? gg_launch<8, true, bf16>(p, st) : gg_launch<8, true, float>(p, st);
-        return y_dtype == SP_BF16 ? gg_launch<8, false, bf16>(p, st) : gg_launch<8, false, float>(p, st);
+        if (glu) return y_dtype == SP_BF16 ? gg_launch<8, 4, true, bf16>(p, st) : gg_launch<8, 4, true, float>(p, st);
+        return y_dtype == SP_BF16 ? gg_launch<8, 4, false, bf16>(p, st) : gg_launch<8, 4, false, float>(p, st);
     }
-    if (glu) return y_dtype == SP_BF16 ? gg_launch<4, true, bf16>(p, st) : gg_launch<4, true, float>(p, st);
-    return y_dtype == SP_BF16 ? gg_launch<4, false, bf16>(p, st) : gg_launch<4, false, float>(p, st);
+    if (glu) return y_dtype == SP_BF16 ? gg_launch<4, 4, true, bf16>(p, st) : gg_launch<4, 4, true, float>(p, st);
+    return y_dtype == SP_BF16 ? gg_launch<4, 4, false, bf16>(p, st) : gg_launch<4, 4, false, float>(p, st);
 }
 
 // What a product over groups takes, in us: `routed` groups that hold `mean` rows each on average (sizes taken as normal about it)
@@ -395,7 +464,8 @@ extern "C" int spite_gemm_groups(const void* X, int ldx, const void* W, long w_g
 // Fitted to 3,600 products (4 to 128 groups of 1 to 8 a token, 65 to 6,000 tokens, N of 512 to 8,192, K of 512 to 16,384, gated in
 // bfloat16 and plain in fp32), each timed with every kernel: 7 to 9 % off (gemm_lds 11), much of it alike for all of one size.
 struct gg_fit { int rows, cols; double start, tile, w, x, tbs, power, part, alone, gated, out, aligned; };
-static const gg_fit GG_FITS[8] = {       // gemm_groups with four waves and tiles of up to 128 and 160 rows, and eight; gemm_tiled's three; gemm_lds
+// (The last two, four waves of 80 columns, are fitted to 205 plain products of 8 to 64 experts: 5 % off.)
+static const gg_fit GG_FITS[10] = {      // gemm_groups with four waves and tiles of up to 128 and 160 rows, and eight; gemm_tiled's three; gemm_lds; four waves of 80 columns
     {128, 256, 7.15, 2.46, 73.6, 6.2, 9, 1.3, 0.32, 0.444, 0.957, 4.77, 1.03},
     {160, 256, 6.86, 3.15, 86.8, 6.28, 8.58, 1.49, 0.334, 0.45, 0.962, 4.54, 1.02},
     {128, 512, 3.56, 7.1, 99, 2.34, 9, 1.56, 0.784, 0.892, 0.971, 6.32, 1.06},
@@ -403,10 +473,12 @@ static const gg_fit GG_FITS[8] = {       // gemm_groups with four waves and tile
     {128, 512, 6.34, 6.22, 74.1, 6.16, 9, 1.67, 0.654, 0.821, 1.01, 5.73, 0.992},
     {160, 512, 11.1, 5.39, 80.7, 6.63, 7.06, 2.33, 0.659, 0.792, 1.02, 5.3, 1},
     {64, 512, 1.25, 6.7, 72.8, 6.27, 8.59, 1.65, 0.896, 0.922, 1.02, 2, 0.987},
-    {256, 256, 2.24, 12.1, 12.9, 12.9, 7.19, 1.47, 0.75, 0.827, 0.979, 6.65, 1.01}
+    {256, 256, 2.24, 12.1, 12.9, 12.9, 7.19, 1.47, 0.75, 0.827, 0.979, 6.65, 1.01},
+    {128, 320, 6.37, 2.26, 57.5, 5.01, 8.93, 1.89, 0.786, 0.827, 1, 4.83, 1.04},
+    {160, 320, 5.88, 2.12, 63.2, 4.83, 7.89, 2.62, 0.828, 0.851, 1, 4.49, 1.03}
 };
 static int gg_fit_tiles(int kind, int rows, int& nb) {
-    if (kind < 4) return gg_group_tiles(rows, GG_FITS[kind].rows, nb);
+    if (kind < 4 || kind >= 8) return gg_group_tiles(rows, GG_FITS[kind].rows, nb);
     const int height = GG_FITS[kind].rows, tiles = (rows + height - 1) / height;
     nb = height / 16;
     if (kind == 7) {                     // as gemm_lds takes them
@@ -420,14 +492,16 @@ static double gg_estimate(int kind, int tokens, int routed, double mean, int who
     const gg_fit& f = GG_FITS[kind];
     const double share = mean / tokens < 1.0 ? mean / tokens : 1.0, sd = sqrt(tokens * share * (1.0 - share));
     double n = 0.0, sum = 0.0;
-    int most = 2, nb;
+    int most = 2, least = 1 << 30, nb;
     for (double z : Z) {
         const int rows = (int)(mean + z * sd + 0.5);
         if (rows <= 0) continue;
         const int t = gg_fit_tiles(kind, rows, nb);
         n += t; sum += (double)t * nb;
         most = nb > most ? nb : most;
+        least = t < least ? t : least;
     }
+    const double over = n / 11.0 - least, more = over > 0.0 && over < 1.0 ? over : 0.0;      // how likely a group's further tile is
     n *= routed / 11.0; sum *= routed / 11.0;
     if (whole) {
         const int t = gg_fit_tiles(kind, tokens, nb);
@@ -438,8 +512,9 @@ static double gg_estimate(int kind, int tokens, int routed, double mean, int who
     const long cols = (N + f.cols / (glu ? 2 : 1) - 1) / (f.cols / (glu ? 2 : 1));
     const double rows = (double)routed * mean + (double)whole * tokens, cus = sp_cu_count();
     double u;                            // rounds of tiles
-    if (kind < 4) {
-        u = ceil(n * cols / 8.0) / (cus / 8.0 * (kind < 2 ? 2.0 : 1.0));
+    if (kind < 4 || kind >= 8) {
+        // (80 columns a wave: a tile more than one a compute unit costs a round, so a standard deviation of tiles more than to be expected has to fit)
+        u = ceil((n + (kind < 4 ? 0.0 : sqrt(routed * more * (1.0 - more)))) * cols / 8.0) / (cus / 8.0 * (kind < 2 ? 2.0 : 1.0));
     } else {
         const long real = n > 1.0 ? (long)(n + 0.5) : 1, groups = routed + whole;
         long launched = (long)(rows / f.rows) + (groups < (long)rows ? groups : (long)rows), most_tiles = 0;
@@ -480,4 +555,23 @@ extern "C" int spite_gemm_groups_choice(int tokens, int routed, double mean, int
     if (*us < 0.98 * other) return best;
     *us = other;
     return 0;
+}
+
+// The same for a plain product by tiles of four waves of 80 columns (waves code 5), against whichever of the others would run: 0, or 5 * 256 +
+// cap where they are estimated 5 % faster.  A plain product back has few columns: 5,120 make ten tiles of 512 for each of 16 experts, 160 for
+// 256 compute units, and 320 of 256, of which 64 units have two; sixteen of 320 are one each.  Of 276 products (8 to 64 experts, 65 to 4,000
+// tokens, N of 2,048 to 8,192, K of 1,024 to 16,384) 35 take them: 9 % faster on average (16 experts, 5,120 x 8,192: 2,048 tokens 273 / 237 us,
+// 1,547 236 / 219; x 4,096, 2,077 tokens 158 / 118), four of them 2 % and more slower (3, 6, 9 and 29 %, where a group's further tile came that
+// was not to be expected).
+extern "C" int spite_gemm_groups_wide_choice(int tokens, int routed, double mean, int whole, int N, int K, int shape, int lds) {
+    double us;
+    spite_gemm_groups_choice(tokens, routed, mean, whole, N, K, 0, shape, lds, &us);
+    if (us <= 0.0) return 0;
+    int best = 0;
+    us *= 0.95;
+    for (int kind = 8; kind < 10; ++kind) {
+        const double t = gg_estimate(kind, tokens, routed, mean, whole, N, K, 0);
+        if (t < us) { best = 5 * 256 + GG_FITS[kind].rows; us = t; }
+    }
+    return best;
 }

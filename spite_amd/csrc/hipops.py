@@ -126,6 +126,8 @@ def lib():
         l.spite_gemm_skinny_variant.restype = c_int
         l.spite_gemm_groups_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I, I, I, P]
         l.spite_gemm_groups_choice.restype = c_int
+        l.spite_gemm_groups_wide_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I, I]
+        l.spite_gemm_groups_wide_choice.restype = c_int
         l.spite_gemm_f32_variant.argtypes = [I, I, I]
         l.spite_gemm_f32_variant.restype = c_int
         l.spite_gemm_f32_choice.argtypes = [I] * 5
@@ -803,6 +805,13 @@ def gemm_groups_choice(tokens: int, routed: int, mean: float, whole: int, N: int
     return gemm_groups_estimate(tokens, routed, mean, whole, N, K, glu, shape, lds)[0]
 
 
+def gemm_groups_wide_choice(tokens: int, routed: int, mean: float, whole: int, N: int, K: int, shape: int = 0, lds: bool = False):
+    """(5, cap) for ``gemm_groups`` where a plain product's tiles of 320 columns are estimated faster than what ``gemm_groups_choice``
+    leaves, or None (arguments as there)."""
+    code = lib().spite_gemm_groups_wide_choice(tokens, routed, mean, whole, N, K, int(shape), int(bool(lds)))
+    return divmod(code, 256) if code else None
+
+
 def gemm_groups_ok(a, y, M, N, K, glu) -> bool:
     """Whether ``gemm_groups`` takes these operands: 32-bit offsets into the rows of ``a`` and a group of W, rows of ``y`` that
     16-byte stores can take, silu or no gate."""
@@ -811,7 +820,7 @@ def gemm_groups_ok(a, y, M, N, K, glu) -> bool:
 
 def gemm_groups(a, w, y, M, N, K, *, offsets, n_groups, a_rows=None, a_scale=None, y_rows=None, glu=False, waves=8, cap=128):
     """Tiled bf16 product over groups, each in tiles of the height that suits it (see gemm_groups.hip); arguments as gemm_generic,
-    ``glu`` with silu.  ``waves`` (4 or 8) and ``cap`` (128 or 160): see ``gemm_groups_choice``."""
+    ``glu`` with silu.  ``waves`` (4 or 8; 5: four of 80 columns, plain only) and ``cap`` (128 or 160): see ``gemm_groups_choice``."""
     rows_w = _gemm_checks(a, w, y, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, "gemm_groups")
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise KernelError(f"gemm_groups: bfloat16 operands only, got {a.dtype} and {w.dtype}")

@@ -205,7 +205,9 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
                                              *_group_tiles(M, n_groups, most, group_rows, N, bool(glu))))
             if offsets is not None and M > 0 and act is None and hipops.gemm_groups_ok(x, y, M, N, K, glu):
                 mean, whole = _routed_and_whole(M, n_groups, most, group_rows)
-                choice = hipops.gemm_groups_choice(most, n_groups - whole, float(mean), whole, N, K, bool(glu), tile_shape, lds)
+                sizes = (most, n_groups - whole, float(mean), whole, N, K)
+                choice = (None if glu else hipops.gemm_groups_wide_choice(*sizes, tile_shape, lds)) or \
+                    hipops.gemm_groups_choice(*sizes, bool(glu), tile_shape, lds)
                 if choice is not None:
                     hipops.gemm_groups(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
                                        y_rows=y_rows, glu=bool(glu), waves=choice[0], cap=choice[1])
