@@ -315,7 +315,7 @@ static int launch_skinny(const void* X, int ldx, const void* W, long wgs, void* 
     dim3 grid((N + 16 * R - 1) / (16 * R), m_tiles);
     const size_t sh = (size_t)NW * (glu ? 2 : 1) * R * G * 4 * 64 * sizeof(float);
     constexpr bool can = G == 1 && S == 2 && R * 4 <= NW;
-    const bool piped = can && tiled && K % 64 == 0 && (offsets || (M <= 2 && (size_t)N * K < ((size_t)1 << 27)));
+    const bool piped = can && tiled && K % 64 == 0 && K < (1 << 24) && (offsets ||      /* (the loads' offsets are 32-bit) */ (M <= 2 && (size_t)N * K < ((size_t)1 << 27)));
 #define SP_SK(GLUV, TY) do { \
         auto kern = piped ? gemm_skinny_piped_kernel<can ? R : 1, can ? NW : 4, GLUV, TY> : \
             tiled ? gemm_skinny_kernel<R, G, S, NW, GLUV, true, TY> : gemm_skinny_kernel<R, G, S, NW, GLUV, false, TY>; \
@@ -396,7 +396,6 @@ extern "C" int spite_gemm_skinny(const void* X, int ldx, const void* W, long w_g
     SP_REQUIRE(y_dtype == SP_BF16 || y_dtype == SP_F32, "gemm_skinny: output dtype %d", y_dtype);
     SP_REQUIRE(!offsets || n_groups > 0, "gemm_skinny: grouped call without groups");
     SP_REQUIRE(!w_tiled || (K % 32 == 0 && N % 16 == 0), "gemm_skinny: operand order needs K=%d a multiple of 32 and N=%d of 16", K, N);
-    SP_REQUIRE(K < (1 << 24), "gemm_skinny: K=%d is beyond the loads' 32-bit offsets", K);
     if (M == 0) return 0;
 #define SP_ARGS X, ldx, W, w_group_stride, Y, y_dtype, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, w_tiled, live_groups, st
     if (variant == 0) variant = skinny_variant(M, N, K, offsets ? n_groups : 0, live_groups, glu != 0, max_rows);
