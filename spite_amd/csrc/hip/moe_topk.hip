@@ -22,6 +22,24 @@
 
 #define TOPK_MAX_PER_LANE 8      // up to 512 experts
 
+// The largest and the smallest of a wave's values, by moves within the vector registers, the same in every lane.  (By six steps of shuffles of
+// value, expert and score an expert that is taken was a chain of 0.6 us; us before and now, with the row list: one token, 4 of 16 experts 5.2 /
+// 3.6, 2 of 16 3.7 / 2.9; 8 tokens, 8 of 128 11.2 / 8.2, 8 of 512 16.9 / 13.6; 1,531, 4 of 16 10.2 / 8.5.)
+#define SP_TOPK_STEP(op, ctrl, rows) x = op(x, __builtin_bit_cast(decltype(x), __builtin_amdgcn_update_dpp(__builtin_bit_cast(int, x), __builtin_bit_cast(int, x), ctrl, rows, 0xf, false)))
+#define SP_TOPK_STEPS(op) /* from one lane below within 16, two, four, eight; rows 0 and 2 to 1 and 3; row 1 to 2 and 3 */ \
+    SP_TOPK_STEP(op, 0x111, 0xf); SP_TOPK_STEP(op, 0x112, 0xf); SP_TOPK_STEP(op, 0x114, 0xf); SP_TOPK_STEP(op, 0x118, 0xf); \
+    SP_TOPK_STEP(op, 0x142, 0xa); SP_TOPK_STEP(op, 0x143, 0xc)
+__device__ __forceinline__ float topk_max(float x) {
+    SP_TOPK_STEPS(fmaxf);
+    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, x), 63));
+}
+__device__ __forceinline__ int topk_min(int x) {
+    SP_TOPK_STEPS(min);
+    return __builtin_amdgcn_readlane(x, 63);
+}
+#undef SP_TOPK_STEPS
+#undef SP_TOPK_STEP
+
 // One token's choice by one wave: lane j < min(top, 64) gets the j-th taken expert and its weight, and everything is
 // written to expert[] and weight[].  NU: experts a lane, so that 64 * NU >= E.
 template <int NU>
@@ -94,11 +112,16 @@ __device__ __forceinline__ int topk_of_token(const float* __restrict__ logits, c
             const int e = lane + u * 64;
             if (e < E && (c[u] > best || (c[u] == best && e < be))) { best = c[u]; be = e; bs = s[u]; }
         }
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) {
-            const float ob = __shfl_xor(best, o, 64); const int oe = __shfl_xor(be, o, 64); const float os = __shfl_xor(bs, o, 64);
-            if (ob > best || (ob == best && oe < be)) { best = ob; be = oe; bs = os; }
+        // the lanes that hold the largest value, and of them the lowest expert (one lane but for ties)
+        const float most = topk_max(best);
+        unsigned long long who = __ballot(best == most && be != 0x7fffffff);      // (a lane without an expert has that one)
+        if (NU > 1 && (who & (who - 1))) {
+            const int lowest = topk_min(best == most ? be : 0x7fffffff);          // (every lane's)
+            who = __ballot(best == most && be == lowest);
         }
+        const int src = __ffsll(who) - 1;
+        be = __builtin_amdgcn_readlane(be, src);
+        bs = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(bs), src));
         // a taken expert leaves the contest: its mark lies below every score
 #pragma unroll
         for (int u = 0; u < NU; ++u) if (lane + u * 64 == be) c[u] = -INFINITY;
@@ -136,8 +159,8 @@ void router_topk_kernel(const float* __restrict__ logits, const float* __restric
 
 // The choice and the row list of the grouped products (moe_plan with a fan of `top` and `shared` groups that every token
 // visits) of a step of a few tokens by one workgroup, a wave a token: two kernels become one.  Both are a chain of
-// latencies: the logits' load, then six steps of shuffles for every expert that is taken.  Measured on an
-// MI355X, one launch against two, us: 1 token, 1 of 16 experts 3.1 / 4.0, 4 of 64 5.1 / 6.0; 8 tokens, 2 of 16 4.5 / 5.7, 8 of
+// latencies: the logits' load, then a maximum over the wave for every expert that is taken.  Measured on an
+// MI355X when that was six steps of shuffles, one launch against two, us: 1 token, 1 of 16 experts 3.1 / 4.0, 4 of 64 5.1 / 6.0; 8 tokens, 2 of 16 4.5 / 5.7, 8 of
 // 128 11.0 / 11.7, 8 of 512 17.7 / 18.4.  No second token a wave: its choice would wait for the first one's, which
 // router_topk's further workgroups do not (16 tokens, 8 of 64 17.8 / 12.9; 64 tokens, 8 of 128 72 / 16; 512 tokens, 1 of 16
 // 95 / 9.7).  The entries' experts stay in LDS in between; ranks are counted as moe_plan_kernel counts them.
