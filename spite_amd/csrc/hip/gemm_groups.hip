@@ -189,7 +189,7 @@ void gemm_groups_kernel(gg_args p) {
     const int lane = threadIdx.x & 63;
     int b = 0, e = 0, h = 0, nt = 0;                     // the lane's group: its rows, their tiles and these tiles' height
     int g = -1, row0 = 0, row_end = 0, nb = 8, tiles = 1, col = 0;
-    if constexpr (NW == 8) {                             // row tiles of all groups run fastest
+    if constexpr (A == 4) {                              // row tiles of all groups run fastest
         int incl = 0, all = 0;
         auto scan = [&](int c) {
             b = e = 0;
@@ -221,13 +221,17 @@ void gemm_groups_kernel(gg_args p) {
         }
         col = __builtin_amdgcn_readfirstlane(unit / all);
     } else {
-        // (Not with eight waves: a gated product beside a shared expert lost 3 to 5 %.)
+        // (Not with 64 columns a wave.  With eight waves a gated product beside a shared expert lost 3 to 5 %.  With four, products in a row
+        // are 2 to 3 % faster by it, but within a step, where the rows of X come from the product before or by a row list, they are not: 1,531 rows
+        // of 4 of 16 experts and of two more x 2 x 1,024 x 2,048 gated 91.2 us, by this order 94.8, x 2,048 x 1,024 66.3 / 65.8, latent
+        // attention's over its heads 49.7 / 50.9; and where the fullest group has 1.6 times the average an XCD waits for another: 903 rows of 8
+        // experts x 2 x 3,072 x 1,024 32 / 38.)
         //  * groups of up to four tiles and no more than twice the average (experts): all columns of a group go to one XCD, row tiles of a column
         //    next to each other, so that what runs there at a time reads the group's rows of X once from memory and its W once;
         //  * larger ones (a shared expert): row tiles of all of them running fastest, an eighth of the columns an XCD.
-        // An XCD has an eighth of either kind, in turn: the first wait for the stream of W, the second for the matrix units.  (1,531 rows of 4 of
-        // 16 experts and of two more x 2,048 x 1,024 59.7 -> 53.6 us, 2 x 1,024 x 2,048 gated 93.4 -> 89.8; one tile of 320 columns a compute unit, 2,048
-        // rows x 5,120 x 8,192, 242 -> 223, with 1.38 GB read instead of 1.61.)
+        // An XCD has an eighth of either kind, in turn: the first wait for the stream of W, the second for the matrix units.  (One tile a
+        // compute unit, 2,048 rows of 16 experts x 5,120 x 8,192, 242 -> 223 us, with 1.38 GB read instead of 1.61; 36 products of 8 to 128 experts
+        // 5 % faster on average.)
         int few = 0, many = 0, limit = 0;      // tiles of either kind up to and with the lane's group; the first kind's most
         auto look = [&](int c) {
             b = e = 0;

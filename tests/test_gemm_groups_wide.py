@@ -1,5 +1,5 @@
-"""The product over groups in tiles of 320 columns, and the order in which four waves' tiles go to the XCDs: every height, groups of up to
-four tiles and larger ones, among many groups; bit for bit against the tiled product."""
+"""The product over groups in tiles of 320 columns, whose groups go to the XCDs by their tiles, beside four waves' tiles of 256, whose do not: every
+height, groups of up to four tiles and larger ones, among many groups; bit for bit against the tiled product."""
 import pytest
 import torch
 
