@@ -177,6 +177,9 @@ __device__ __host__ __forceinline__ int gg_group_tiles(int rows, int cap, int& n
     return tiles;
 }
 
+// Groups from which on four waves' tiles of 64 columns go to the XCDs by group too.
+#define GG_BY_GROUP 64
+
 template <int NW, int A, bool GLU, typename TY>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(A == 4 ? 2 : 1, A == 4 ? 2 : 1)))
 void gemm_groups_kernel(gg_args p) {
@@ -189,7 +192,7 @@ void gemm_groups_kernel(gg_args p) {
     const int lane = threadIdx.x & 63;
     int b = 0, e = 0, h = 0, nt = 0;                     // the lane's group: its rows, their tiles and these tiles' height
     int g = -1, row0 = 0, row_end = 0, nb = 8, tiles = 1, col = 0;
-    if constexpr (A == 4) {                              // row tiles of all groups run fastest
+    if (A == 4 && (NW == 8 || p.n_groups < GG_BY_GROUP)) {     // row tiles of all groups run fastest
         int incl = 0, all = 0;
         auto scan = [&](int c) {
             b = e = 0;
@@ -221,11 +224,12 @@ void gemm_groups_kernel(gg_args p) {
         }
         col = __builtin_amdgcn_readfirstlane(unit / all);
     } else {
-        // (Not with 64 columns a wave.  With eight waves a gated product beside a shared expert lost 3 to 5 %.  With four, products in a row
-        // are 2 to 3 % faster by it, but within a step, where the rows of X come from the product before or by a row list, they are not: 1,531 rows
-        // of 4 of 16 experts and of two more x 2 x 1,024 x 2,048 gated 91.2 us, by this order 94.8, x 2,048 x 1,024 66.3 / 65.8, latent
-        // attention's over its heads 49.7 / 50.9; and where the fullest group has 1.6 times the average an XCD waits for another: 903 rows of 8
-        // experts x 2 x 3,072 x 1,024 32 / 38.)
+        // (80 columns a wave, or four waves and 64 groups and more.  With eight waves a gated product beside a shared expert lost 3 to 5 %.  With
+        // four and fewer groups, products in a row are 2 to 3 % faster by it, but within a step, where the rows of X come from the product before or
+        // by a row list, they are not: 1,531 rows of 4 of 16 experts and of two more x 2 x 1,024 x 2,048 gated 91.2 us, by this order 94.8, x 2,048 x
+        // 1,024 66.3 / 65.8, latent attention's over its heads 49.7 / 50.9; and where the fullest of a few groups has 1.6 times the average an XCD
+        // waits for another: 903 rows of 8 experts x 2 x 3,072 x 1,024 32 / 38.  Over 64 and more the XCDs' shares even out: nine products, rows spread
+        // by chance and by lognormal loads of 0.2 to 0.8, 4 % faster on average, none slower; serving 128 experts, a step 44.4 ms / 43.6.)
         //  * groups of up to four tiles and no more than twice the average (experts): all columns of a group go to one XCD, row tiles of a column
         //    next to each other, so that what runs there at a time reads the group's rows of X once from memory and its W once;
         //  * larger ones (a shared expert): row tiles of all of them running fastest, an eighth of the columns an XCD.

@@ -1,4 +1,4 @@
-"""The product over groups in tiles of 320 columns, whose groups go to the XCDs by their tiles, beside four waves' tiles of 256, whose do not: every
+"""The product over groups in tiles of 320 columns, and the order in which these and four waves' tiles over many groups go to the XCDs: every
 height, groups of up to four tiles and larger ones, among many groups; bit for bit against the tiled product."""
 import pytest
 import torch
@@ -28,7 +28,7 @@ def test_every_height_row_lists_and_scales(out_dtype, N, K, cap):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("waves", [4, 5])
-@pytest.mark.parametrize("rows", [[512, 513, 0, 700, 1], [3] * 70 + [900] + [129] * 60, [1300, 600], [0] * 63 + [641, 2, 640], [20] * 9])
+@pytest.mark.parametrize("rows", [[512, 513, 0, 700, 1], [3] * 70 + [900] + [129] * 60, [1300, 600], [0] * 63 + [641, 2, 640], [20] * 9, [30] * 62 + [200], [30] * 63 + [200]])
 def test_small_and_large_groups_among_each_other(waves, rows):
     M, N, K, G = sum(rows), 1296, 128, len(rows)
     a, w = rnd(M, K, dtype=torch.bfloat16), ops().operand_order(rnd(G, N, K, dtype=torch.bfloat16, seed=1))
