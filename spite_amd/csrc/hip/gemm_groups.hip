@@ -32,6 +32,7 @@ struct gg_args {
     const bf16* X; int ldx; const bf16* W; long w_group_stride; void* Y; int ldy, M, N, K;
     const int* offsets; int n_groups; const int* a_rows; const float* a_scale; const int* y_rows;
     int m_tiles, n_tiles, cap;
+    int per_xcd; int* others;              // tiles an XCD may have, and where the groups go that have more (see gemm_groups_kernel)
 };
 #define GG_PAST ((int)0x80000000)      // an offset beyond every buffer's end: loads give zeros
 
@@ -253,8 +254,7 @@ void gemm_groups_kernel(gg_args p) {
             all += __builtin_amdgcn_readlane(sp_wave_scan(nt), 63);
             live += __popcll(__ballot(nt > 0));
         }
-        if (all == 0) return;
-        limit = min(4, 2 * all / live);
+        limit = all ? min(4, 2 * all / live) : 0;
         int all_few = 0, all_many = 0;
         for (int c = 0; c < p.n_groups; c += 64) {
             scan(c);
@@ -264,6 +264,15 @@ void gemm_groups_kernel(gg_args p) {
         const int xcd = blockIdx.x % 8, at = blockIdx.x / 8;     // the XCD's workgroups in turn
         const int units_few = all_few * p.n_tiles, units_many = all_many * p.n_tiles, per_few = (units_few + 7) / 8, per_many = (units_many + 7) / 8;
         const int n_few = min(max(units_few - xcd * per_few, 0), per_few), n_all = n_few + min(max(units_many - xcd * per_many, 0), per_many);
+        if (p.others) {
+            // The host knows the groups' sizes on average alone, and a tile more than fits the rounds that it reckoned with costs a round (a tile
+            // of 320 columns has a compute unit to itself).  So the tiles that there are decide: where they do not fit, this launch does
+            // nothing and leaves the groups to the product behind it, which walks `others`, empty groups otherwise.
+            const bool fits = per_few + per_many <= p.per_xcd;
+            if (blockIdx.x == 0)
+                for (int i = threadIdx.x; i <= p.n_groups; i += NW * 64) p.others[i] = fits ? 0 : p.offsets[i];
+            if (!fits) return;
+        }
         if (at >= n_all) return;
         const int before = __builtin_amdgcn_readfirstlane((int)((long)at * n_few / n_all));
         const bool is_few = __builtin_amdgcn_readfirstlane((int)((long)(at + 1) * n_few / n_all)) > before;
@@ -314,7 +323,8 @@ static int gg_launch(gg_args p, hipStream_t st) {
     // row tiles: a group of r rows has ceil(r / cap): at most r / cap + 1
     p.m_tiles = p.M / p.cap + (p.n_groups < p.M ? p.n_groups : p.M);
     SP_REQUIRE((long)p.m_tiles * p.n_tiles < (1L << 30), "gemm_groups: too many tiles");
-    const int grid = ((p.m_tiles * p.n_tiles + 7) / 8 + 1) * 8;      // (an eighth of either kind, rounded up)
+    int grid = ((p.m_tiles * p.n_tiles + 7) / 8 + 1) * 8;      // (an eighth of either kind, rounded up)
+    if (p.others && grid > 8 * p.per_xcd) grid = 8 * p.per_xcd;
     static bool allowed = false;
     if (!allowed) {
         hipError_t e = hipFuncSetAttribute((const void*)gemm_groups_kernel<NW, A, GLU, TY>, hipFuncAttributeMaxDynamicSharedMemorySize, 4 * 160 * 128);
@@ -397,7 +407,7 @@ extern "C" int spite_gemm_runs(const void* X, int ldx, const void* W, void* Y, i
     SP_REQUIRE(runs == 1 ? ldy % 4 == 0 && ((uintptr_t)Y & 15) == 0 : part && ((uintptr_t)part & 15) == 0, "gemm_runs: rows of the result must be 16-byte aligned");
     // the loads' offsets are 32-bit
     SP_REQUIRE((size_t)M * ldx * 2 < ((size_t)1 << 31) && (size_t)N * K * 2 < ((size_t)1 << 31), "gemm_runs: operands of 2 GiB and more (M=%d N=%d K=%d)", M, N, K);
-    gg_args p{(const bf16*)X, ldx, (const bf16*)W, 0, Y, ldy, M, N, K, nullptr, 1, nullptr, nullptr, nullptr, 0, 0, 0};
+    gg_args p{(const bf16*)X, ldx, (const bf16*)W, 0, Y, ldy, M, N, K, nullptr, 1, nullptr, nullptr, nullptr, 0, 0, 0, 0, nullptr};
     if (runs == 1) return y_dtype == SP_BF16 ? gr_launch_nb<bf16>(p, 1, nb, st) : gr_launch_nb<float>(p, 1, nb, st);
     p.Y = part;
     p.ldy = N;
@@ -433,10 +443,11 @@ extern "C" int spite_gemm_runs_choice(int M, int N, int K, double* us) {
 }
 
 // Arguments as spite_gemm_lds's (`x_rows`: how many rows X has); `waves` 4 or 8, or 5 for four waves of 80 columns (plain only), `cap` 128 or 160.  Gated with silu
-// (`glu` SP_ACT_SILU) or plain (0); rows of Y that 16-byte stores can take.
+// (`glu` SP_ACT_SILU) or plain (0); rows of Y that 16-byte stores can take.  `others` (with waves 5; n_groups + 1 offsets, or none): only where
+// the groups' tiles fit `rounds` of a tile a compute unit, others then all 0; else nothing is computed and others is a copy of offsets.
 extern "C" int spite_gemm_groups(const void* X, int ldx, const void* W, long w_group_stride, void* Y, int y_dtype, int ldy, int M,
                                  int N, int K, const int* offsets, int n_groups, const int* a_rows, const float* a_scale,
-                                 const int* y_rows, int glu, int waves, int cap, int x_rows, hipStream_t st) {
+                                 const int* y_rows, int glu, int waves, int cap, int x_rows, int rounds, int* others, hipStream_t st) {
     SP_REQUIRE(M >= 0 && N > 0 && K > 0 && ldx >= K && ldy >= N, "gemm_groups: bad sizes M=%d N=%d K=%d", M, N, K);
     SP_REQUIRE(offsets && n_groups > 0, "gemm_groups: no groups");
     SP_REQUIRE(K % 64 == 0 && N % 16 == 0, "gemm_groups: operand order needs K=%d a multiple of 64 and N=%d of 16", K, N);
@@ -446,11 +457,12 @@ extern "C" int spite_gemm_groups(const void* X, int ldx, const void* W, long w_g
     SP_REQUIRE(glu == 0 || glu == SP_ACT_SILU, "gemm_groups: activation code %d", glu);
     SP_REQUIRE(((waves == 4 || waves == 8) && (cap == 128 || cap == 160)) || (waves == 5 && !glu && (cap == 128 || cap == 160)), "gemm_groups: %d waves, tiles of %d rows", waves, cap);
     SP_REQUIRE(x_rows > 0 && (a_rows || x_rows >= M), "gemm_groups: %d rows of X", x_rows);
+    SP_REQUIRE(!others || (waves == 5 && rounds > 0 && rounds < (1 << 16) && others != offsets), "gemm_groups: %d rounds of tiles for others, with %d waves", rounds, waves);
     // the loads' offsets are 32-bit: rows of X and a group's W
     SP_REQUIRE((size_t)x_rows * ldx * 2 < ((size_t)1 << 31) && (size_t)(glu ? 2 : 1) * N * K * 2 < ((size_t)1 << 31),
                "gemm_groups: operands of 2 GiB and more (%d rows of X, N=%d K=%d)", x_rows, N, K);
     if (M == 0) return 0;
-    const gg_args p{(const bf16*)X, ldx, (const bf16*)W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, 0, 0, cap};
+    const gg_args p{(const bf16*)X, ldx, (const bf16*)W, w_group_stride, Y, ldy, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, 0, 0, cap, rounds * (sp_cu_count() / 8), others};
     if (waves == 5) return y_dtype == SP_BF16 ? gg_launch<4, 5, false, bf16>(p, st) : gg_launch<4, 5, false, float>(p, st);
     if (waves == 8) {
         if (glu) return y_dtype == SP_BF16 ? gg_launch<8, 4, true, bf16>(p, st) : gg_launch<8, 4, true, float>(p, st);
@@ -495,21 +507,19 @@ static int gg_fit_tiles(int kind, int rows, int& nb) {
     }
     return tiles;
 }
-static double gg_estimate(int kind, int tokens, int routed, double mean, int whole, int N, int K, int glu) {
+static double gg_estimate(int kind, int tokens, int routed, double mean, int whole, int N, int K, int glu, int rounds = 0) {
     static const double Z[11] = {-1.6, -1.0, -0.67, -0.43, -0.2, 0.0, 0.2, 0.43, 0.67, 1.0, 1.6};
     const gg_fit& f = GG_FITS[kind];
     const double share = mean / tokens < 1.0 ? mean / tokens : 1.0, sd = sqrt(tokens * share * (1.0 - share));
     double n = 0.0, sum = 0.0;
-    int most = 2, least = 1 << 30, nb;
+    int most = 2, nb;
     for (double z : Z) {
         const int rows = (int)(mean + z * sd + 0.5);
         if (rows <= 0) continue;
         const int t = gg_fit_tiles(kind, rows, nb);
         n += t; sum += (double)t * nb;
         most = nb > most ? nb : most;
-        least = t < least ? t : least;
     }
-    const double over = n / 11.0 - least, more = over > 0.0 && over < 1.0 ? over : 0.0;      // how likely a group's further tile is
     n *= routed / 11.0; sum *= routed / 11.0;
     if (whole) {
         const int t = gg_fit_tiles(kind, tokens, nb);
@@ -521,8 +531,8 @@ static double gg_estimate(int kind, int tokens, int routed, double mean, int who
     const double rows = (double)routed * mean + (double)whole * tokens, cus = sp_cu_count();
     double u;                            // rounds of tiles
     if (kind < 4 || kind >= 8) {
-        // (80 columns a wave: a tile more than one a compute unit costs a round, so a standard deviation of tiles more than to be expected has to fit)
-        u = ceil((n + (kind < 4 ? 0.0 : sqrt(routed * more * (1.0 - more)))) * cols / 8.0) / (cus / 8.0 * (kind < 2 ? 2.0 : 1.0));
+        u = ceil(n * cols / 8.0) / (cus / 8.0 * (kind < 2 ? 2.0 : 1.0));
+        if (rounds) u = fmin(fmax(u, rounds - 1 + cols / cus), rounds);      // (one tile of a group more than fits the rounds before, at the least)
     } else {
         const long real = n > 1.0 ? (long)(n + 0.5) : 1, groups = routed + whole;
         long launched = (long)(rows / f.rows) + (groups < (long)rows ? groups : (long)rows), most_tiles = 0;
@@ -565,21 +575,50 @@ extern "C" int spite_gemm_groups_choice(int tokens, int routed, double mean, int
     return 0;
 }
 
+// How likely the tiles of `cap` rows of all groups are no more than `budget`: a group's rows taken as normal, and the sum of their tiles too.
+static double gg_chance(int cap, int tokens, int routed, double mean, int whole, long budget) {
+    const double share = mean / tokens < 1.0 ? mean / tokens : 1.0, sd = sqrt(tokens * share * (1.0 - share)) + 1e-9;
+    double m = 0.0, sq = 0.0;                // a group's tiles, and their square: the sums over k of P(more than k tiles) and of 2 k + 1 times that
+    for (int k = 0; (double)k * cap <= tokens; ++k) {
+        const double more = 0.5 * erfc(((double)k * cap + 0.5 - mean) / (sd * M_SQRT2));
+        if (more < 1e-12) break;
+        m += more; sq += (2 * k + 1) * more;
+    }
+    const double sum = routed * m + (double)whole * ((tokens + cap - 1) / cap), spread = sqrt(routed * (sq - m * m > 0.0 ? sq - m * m : 0.0)) + 1e-9;
+    return 0.5 * erfc((sum - (budget + 0.5)) / (spread * M_SQRT2));
+}
+
 // The same for a plain product by tiles of four waves of 80 columns (waves code 5), against whichever of the others would run: 0, or 5 * 256 +
-// cap where they are estimated 5 % faster.  A plain product back has few columns: 5,120 make ten tiles of 512 for each of 16 experts, 160 for
-// 256 compute units, and 320 of 256, of which 64 units have two; sixteen of 320 are one each.  Of 276 products (8 to 64 experts, 65 to 4,000
-// tokens, N of 2,048 to 8,192, K of 1,024 to 16,384) 35 take them: 9 % faster on average (16 experts, 5,120 x 8,192: 2,048 tokens 273 / 237 us,
-// 1,547 236 / 219; x 4,096, 2,077 tokens 158 / 118), four of them 2 % and more slower (3, 6, 9 and 29 %, where a group's further tile came that
-// was not to be expected).
-extern "C" int spite_gemm_groups_wide_choice(int tokens, int routed, double mean, int whole, int N, int K, int shape, int lds) {
+// cap, and in `rounds` those of a tile a compute unit that the groups' tiles have to fit.  A plain product back has few columns: 5,120 make ten
+// tiles of 512 for each of 16 experts, 160 for 256 compute units, and 320 of 256, of which 64 units have two; sixteen of 320 are one each, but
+// with one expert of more than `cap` rows they are 272, in two rounds: 2,048 rows x 5,120 x 8,192 273 us by tiles of 512 columns, 237 by one round of
+// these, 350 by two.  Routers do not spread their rows as evenly as chance would, which the estimate cannot know, so that the device decides
+// by the tiles that there are (gemm_groups_kernel).  Of the two launches one finds nothing to do: 2 to 4 us, which products
+// of 120 us and more make up for where the tiles can be expected to fit.  (79 products of 8 to 128 experts that are
+// taken, rows spread as by chance / by lognormal loads of 0.2 / 0.4 / 0.8 besides: 0.90 / 0.94 / 0.96 / 0.97 of what ran otherwise on average, four of
+// the 316 times more than 3 % slower, the worst 13; without the device's decision 0.90 / 0.97 / 0.98 / 1.02, 63 times, 65.  16 experts, 5,120 x
+// 8,192, 2,048 rows by chance, the fullest expert 143, 445 / 244; unevenly, 186 to 353, 288 / 290, 299 / 302, 282 / 283.)
+extern "C" int spite_gemm_groups_wide_choice(int tokens, int routed, double mean, int whole, int N, int K, int shape, int lds, int* rounds) {
     double us;
+    *rounds = 0;
     spite_gemm_groups_choice(tokens, routed, mean, whole, N, K, 0, shape, lds, &us);
-    if (us <= 0.0) return 0;
+    if (us < 120.0) return 0;
     int best = 0;
-    us *= 0.95;
+    double least = 0.95 * us;
+    const long cols = (N + 319) / 320, cus = sp_cu_count();
     for (int kind = 8; kind < 10; ++kind) {
-        const double t = gg_estimate(kind, tokens, routed, mean, whole, N, K, 0);
-        if (t < us) { best = 5 * 256 + GG_FITS[kind].rows; us = t; }
+        const int cap = GG_FITS[kind].rows;
+        int r = 1;
+        double chance;
+        while ((chance = gg_chance(cap, tokens, routed, mean, whole, r * cus / cols)) < 0.5) ++r;
+        const double t = chance * gg_estimate(kind, tokens, routed, mean, whole, N, K, 0, r) + (1.0 - chance) * us + 3.0;
+        if (t < least) {
+            best = 5 * 256 + cap;
+            *rounds = r;
+            // the taller tiles: where groups are of one shorter tile on average, for those that are not (the others' are the same); else
+            // theirs differ more in height, and have to be the faster ones
+            least = fmin(0.95 * us, (mean <= cap ? 1.02 : 0.98) * t);
+        }
     }
     return best;
 }

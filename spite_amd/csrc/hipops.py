@@ -69,7 +69,7 @@ def lib():
             "spite_attn_decode": [P, P, P, P, P, P, P, P, I, I, I, I, I, I, I, I, F, F, P, I, I, P, I, I, P, I, P],
             "spite_gemm_mfma": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
             "spite_gemm_lds": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, I, P],
-            "spite_gemm_groups": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, I, I, I, P],
+            "spite_gemm_groups": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, I, I, I, I, P, P],
             "spite_gemm_runs": [P, I, P, P, I, I, I, I, I, I, I, P, P],
             "spite_gemm_runs_choice": [I, I, I, P],
             "spite_gemm_tiled": [P, I, P, L, P, I, I, I, I, I, P, I, P, P, P, I, F, I, P],
@@ -126,7 +126,7 @@ def lib():
         l.spite_gemm_skinny_variant.restype = c_int
         l.spite_gemm_groups_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I, I, I, P]
         l.spite_gemm_groups_choice.restype = c_int
-        l.spite_gemm_groups_wide_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I, I]
+        l.spite_gemm_groups_wide_choice.argtypes = [I, I, ctypes.c_double, I, I, I, I, I, P]
         l.spite_gemm_groups_wide_choice.restype = c_int
         l.spite_gemm_f32_variant.argtypes = [I, I, I]
         l.spite_gemm_f32_variant.restype = c_int
@@ -805,11 +805,18 @@ def gemm_groups_choice(tokens: int, routed: int, mean: float, whole: int, N: int
     return gemm_groups_estimate(tokens, routed, mean, whole, N, K, glu, shape, lds)[0]
 
 
+@functools.lru_cache(maxsize=4096)
+def gemm_groups_wide_estimate(tokens: int, routed: int, mean: float, whole: int, N: int, K: int, shape: int = 0, lds: bool = False):
+    """((5, cap), the rounds that the groups' tiles have to fit) for ``gemm_groups`` where a plain product's tiles of 320 columns are
+    estimated faster than what ``gemm_groups_choice`` leaves, or (None, 0) (arguments as there)."""
+    rounds = ctypes.c_int()
+    code = lib().spite_gemm_groups_wide_choice(tokens, routed, mean, whole, N, K, int(shape), int(bool(lds)), ctypes.addressof(rounds))
+    return (divmod(code, 256) if code else None), rounds.value
+
+
 def gemm_groups_wide_choice(tokens: int, routed: int, mean: float, whole: int, N: int, K: int, shape: int = 0, lds: bool = False):
-    """(5, cap) for ``gemm_groups`` where a plain product's tiles of 320 columns are estimated faster than what ``gemm_groups_choice``
-    leaves, or None (arguments as there)."""
-    code = lib().spite_gemm_groups_wide_choice(tokens, routed, mean, whole, N, K, int(shape), int(bool(lds)))
-    return divmod(code, 256) if code else None
+    """The choice of ``gemm_groups_wide_estimate``."""
+    return gemm_groups_wide_estimate(tokens, routed, mean, whole, N, K, shape, lds)[0]
 
 
 def gemm_groups_ok(a, y, M, N, K, glu) -> bool:
@@ -818,17 +825,22 @@ def gemm_groups_ok(a, y, M, N, K, glu) -> bool:
     return glu in (0, 1) and gemm_lds_ok(a, None, M, N, K, glu) and y.stride(0) % 4 == 0 and y.data_ptr() % 16 == 0
 
 
-def gemm_groups(a, w, y, M, N, K, *, offsets, n_groups, a_rows=None, a_scale=None, y_rows=None, glu=False, waves=8, cap=128):
+def gemm_groups(a, w, y, M, N, K, *, offsets, n_groups, a_rows=None, a_scale=None, y_rows=None, glu=False, waves=8, cap=128,
+                rounds=0, others=None):
     """Tiled bf16 product over groups, each in tiles of the height that suits it (see gemm_groups.hip); arguments as gemm_generic,
-    ``glu`` with silu.  ``waves`` (4 or 8; 5: four of 80 columns, plain only) and ``cap`` (128 or 160): see ``gemm_groups_choice``."""
+    ``glu`` with silu.  ``waves`` (4 or 8; 5: four of 80 columns, plain only) and ``cap`` (128 or 160): see ``gemm_groups_choice``.
+    ``others`` (int32, n_groups + 1 offsets; with ``waves`` 5): the product is made only where the groups' tiles fit ``rounds`` of
+    one a compute unit, and ``others`` receives the offsets that are left to another product, all 0 or ``offsets``."""
     rows_w = _gemm_checks(a, w, y, M, N, K, offsets, n_groups, a_rows, a_scale, y_rows, glu, "gemm_groups")
     if a.dtype != torch.bfloat16 or w.dtype != torch.bfloat16:
         raise KernelError(f"gemm_groups: bfloat16 operands only, got {a.dtype} and {w.dtype}")
+    if others is not None and (others.numel() < n_groups + 1 or M <= 0):
+        raise KernelError(f"gemm_groups: {others.numel()} offsets for what is left of {n_groups} groups and {M} rows")
     _check(lib().spite_gemm_groups(
         _ptr_rows(a, "a"), a.stride(0), _ptr(w, "w"), rows_w * K, _ptr_rows(y, "y"), dtype_code(y.dtype), y.stride(0),
         M, N, K, _ptr(offsets, "offsets", torch.int32), n_groups, _ptr(a_rows, "a_rows", torch.int32, True),
         _ptr(a_scale, "a_scale", torch.float32, True), _ptr(y_rows, "y_rows", torch.int32, True), int(bool(glu)),
-        int(waves), int(cap), a.shape[0], _stream()), "gemm_groups")
+        int(waves), int(cap), a.shape[0], int(rounds), _ptr(others, "others", torch.int32, True), _stream()), "gemm_groups")
 
 
 def attn_prefill_splits(counts, H, G, max_keys) -> int:

@@ -206,8 +206,13 @@ def linear(x, w, y, *, glu=False, offsets=None, n_groups=1, a_rows=None, a_scale
             if offsets is not None and M > 0 and act is None and hipops.gemm_groups_ok(x, y, M, N, K, glu):
                 mean, whole = _routed_and_whole(M, n_groups, most, group_rows)
                 sizes = (most, n_groups - whole, float(mean), whole, N, K)
-                choice = (None if glu else hipops.gemm_groups_wide_choice(*sizes, tile_shape, lds)) or \
-                    hipops.gemm_groups_choice(*sizes, bool(glu), tile_shape, lds)
+                wide, rounds = (None, 0) if glu else hipops.gemm_groups_wide_estimate(*sizes, tile_shape, lds)
+                if wide is not None:         # (where the groups are not as even as hoped for, they go to the product that follows)
+                    others = _scratch(ws, (n_groups + 1,), torch.int32, x.device)
+                    hipops.gemm_groups(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
+                                       y_rows=y_rows, waves=wide[0], cap=wide[1], rounds=rounds, others=others)
+                    offsets = others
+                choice = hipops.gemm_groups_choice(*sizes, bool(glu), tile_shape, lds)
                 if choice is not None:
                     hipops.gemm_groups(x, w, y, M, N, K, offsets=offsets, n_groups=n_groups, a_rows=a_rows, a_scale=a_scale,
                                        y_rows=y_rows, glu=bool(glu), waves=choice[0], cap=choice[1])
