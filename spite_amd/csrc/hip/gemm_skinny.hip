@@ -163,14 +163,15 @@ void gemm_skinny_kernel(const bf16* __restrict__ X, int ldx, const bf16* __restr
     }
 }
 
-// The same for W in operand order over groups of up to 16 rows, and for one or two rows, with the loads of a wave's next block on
-// their way while a block is multiplied.  In the kernel above every load stands behind a condition, so that each product waits for all
-// that were asked for; many waves make up for that where the stream is long, a short one waits for memory block by block.  Here
+// The same for W in operand order over groups of up to 16 rows, and for one or two rows without a gate, with the loads of a wave's next
+// block on their way while a block is multiplied.  In the kernel above every load stands behind a condition, so that each product waits for
+// all that were asked for; many waves make up for that where the stream is long, a short one waits for memory block by block.  Here
 // each number of blocks that may be left has a piece of its own without conditions; all arguments are read at once, and what a
 // result's place depends on before the stream, not behind it.  The same bits.  Not for three and more rows without groups nor for
 // tables of 2^27 elements: those gain by the other kernel's fewer loads in flight (8 x 5,120 x 5,120 13.1 us, by this one 14.6; 1 x
-// 32,768 x 5,120 52.7 / 54.3).
-// us in a chain of launches in a graph, the kernel above and this one: 1 x 3,072 x 2,048 4.45 / 4.14, 1 x 2,048 x 2,048 4.05 / 3.86, two groups of
+// 32,768 x 5,120 52.7 / 54.3); nor for one or two rows with a gate (1 x 2 x 2,048 x 2,816 7.15 / 7.62, x 5,120 x 8,192 29.0 / 30.3; 75 sizes the same
+// on average), nor, 32 rows of W a workgroup, for sums of more than 5,120 (5,120 x 8,192 15.9 / 16.3, 4,096 x 6,144 11.5 / 12.1).
+// us in a chain of launches in a graph, the kernel above and this one: 1 x 3,072 x 2,048 4.45 / 4.14, 1 x 2,048 x 2,048 4.23 / 3.98, two groups of
 // one row x 2,048 x 3,072 7.16 / 6.66 and 2 x 3,072 x 2,048 gated 11.60 / 11.02, 2 x 8,192 x 5,120 53.8 / 52.7; nine groups of 8 rows x 2 x 8,192 x
 // 5,120 225.3 / 224.3, 33 of 1 to 32 rows 720.4 / 719.1.  An empty kernel takes 1.7.
 #include <type_traits>
@@ -258,15 +259,13 @@ void gemm_skinny_piped_kernel(const bf16* __restrict__ X, int ldx, const bf16* _
             mul(1);
             next(1, i + 3);
         }
-        if (i + 2 == n_blk) {
-            mul(0);
-            mul(1);
-        } else {
-            mul(0);
-            next(0, i + 2);
-            mul(1);
-            mul(0);
-        }
+        // Two blocks are left, or three.  (In a branch for each, what the other one reads stayed in registers, and the third block's loads waited for one
+        // after another: 1 x 2 x 2,048 x 1,536 6.1 us.)
+        const bool third = i + 2 < n_blk;
+        mul(0);
+        if (third) next(0, i + 2);
+        mul(1);
+        if (third) mul(0);
     } else if (n_blk == 1) {
         start(std::integral_constant<int, 1>());
         mul(0);
@@ -315,7 +314,9 @@ static int launch_skinny(const void* X, int ldx, const void* W, long wgs, void* 
     dim3 grid((N + 16 * R - 1) / (16 * R), m_tiles);
     const size_t sh = (size_t)NW * (glu ? 2 : 1) * R * G * 4 * 64 * sizeof(float);
     constexpr bool can = G == 1 && S == 2 && R * 4 <= NW;
-    const bool piped = can && tiled && K % 64 == 0 && K < (1 << 24) && (offsets ||      /* (the loads' offsets are 32-bit) */ (M <= 2 && (size_t)N * K < ((size_t)1 << 27)));
+    // (32-bit offsets of the loads; plain products that the kernel's comment names)
+    const bool piped = can && tiled && K % 64 == 0 && K < (1 << 24) &&
+        (offsets || (!glu && M <= 2 && (size_t)N * K < ((size_t)1 << 27) && (R == 1 || K <= 5120)));
 #define SP_SK(GLUV, TY) do { \
         auto kern = piped ? gemm_skinny_piped_kernel<can ? R : 1, can ? NW : 4, GLUV, TY> : \
             tiled ? gemm_skinny_kernel<R, G, S, NW, GLUV, true, TY> : gemm_skinny_kernel<R, G, S, NW, GLUV, false, TY>; \
