@@ -29,7 +29,7 @@
 //       with one group per head walks rows that lie token by token.
 // Angles, rotation and norm are fp32; sine and cosine are the accurate routines.
 #define LAT_PAIRS 256
-template <typename T>
+template <typename T, bool PAST>      // PAST: more pairs than the table holds
 __global__ __launch_bounds__(256)
 void latent_prepare_kernel(const T* __restrict__ qd, int ldq, const T* __restrict__ dkv_all, int ld_dkv, T* __restrict__ qa, T* __restrict__ kv_pages,
                            const int* __restrict__ positions, const int* __restrict__ slot_map,
@@ -39,7 +39,10 @@ void latent_prepare_kernel(const T* __restrict__ qd, int ldq, const T* __restric
                            const T* __restrict__ cq_raw, int ld_cq, const float* __restrict__ w_cq, T* __restrict__ cq_out, int Q) {
     // The angles' sines and cosines once a token, in LDS (pairs past the table are turned by their own), beside the norms' sums: one
     // barrier, and then every pair of every head by a thread.  Each element by a thread with a sine and a cosine of its own took, for 40
-    // heads of 64 beside a latent of 512, two tokens 7.1 us and 1,786 17.0; this 4.3 and 10.7 (three heads of 30, five tokens 3.4 / 3.6).
+    // heads of 64 beside a latent of 512, two tokens 7.2 us and 1,786 16.6; this 3.7 and 8.9 (eight heads 4.0 / 3.3 and 7.3 / 5.6).  Pairs past the
+    // table are another kernel's: their sine and cosine in every loop, which hardly any size needs, doubled the code, and 1,786 tokens of few heads were
+    // up to 29 % slower by it than without a table (eight heads, fp32, beside a query latent of 1,536: 11.9 us, 14.4, now 10.8).
+    static_assert(LAT_PAIRS == 256, "a pair of the table a thread");
     __shared__ float red[8], sin_of[LAT_PAIRS], cos_of[LAT_PAIRS];
     const int t = blockIdx.x, tid = threadIdx.x;
     const int Dk = R + r, hw = n + r, pairs = rot_dims >> 1;
@@ -51,14 +54,14 @@ void latent_prepare_kernel(const T* __restrict__ qd, int ldq, const T* __restric
     float sq_c = 0.f, sq = 0.f;
     if (cq_out) for (int e = tid; e < Q; e += 256) { const float x = to_f32<T>(cq[e]); sq_c += x * x; }
     if (own) for (int e = tid; e < R; e += 256) { const float x = to_f32<T>(dkv[e]); sq += x * x; }
-    for (int i = tid; i < pairs && i < LAT_PAIRS; i += 256) sincosf(pos * inv_freq[i], &sin_of[i], &cos_of[i]);
+    if (tid < pairs) sincosf(pos * inv_freq[tid], &sin_of[tid], &cos_of[tid]);
     sq_c = wave_sum(sq_c);
     sq = wave_sum(sq);
     if ((tid & 63) == 0) { red[tid >> 6] = sq_c; red[4 + (tid >> 6)] = sq; }
     __syncthreads();
     auto turn = [&](const T* from, T* to, int i) __attribute__((always_inline)) {      // pair i
         float sn, cs;
-        if (i < LAT_PAIRS) { sn = sin_of[i]; cs = cos_of[i]; }
+        if (!PAST || i < LAT_PAIRS) { sn = sin_of[i]; cs = cos_of[i]; }
         else sincosf(pos * inv_freq[i], &sn, &cs);
         const float u = to_f32<T>(from[2 * i]), v = to_f32<T>(from[2 * i + 1]);
         to[2 * i] = from_f32<T>(fmaf(u, cs, -(v * sn)));
@@ -104,13 +107,13 @@ extern "C" int spite_latent_prepare(const void* qd, int ldq, const void* dkv, in
     SP_REQUIRE(!own || (dkv && kv_pages && slot_map && w_norm && eps > 0.f), "latent_prepare: the cache row needs pages, slots and the norm");
     SP_REQUIRE((long)T * H < (1L << 31), "latent_prepare: too many rows");
     if (T == 0) return 0;
-    if (dtype == SP_F32)
-        latent_prepare_kernel<float><<<T, 256, 0, st>>>((const float*)qd, ldq, (const float*)dkv, ld_dkv, (float*)qa, (float*)kv_pages, positions, slot_map,
-            inv_freq, w_norm, eps, H, n, r, R, rot_dims, own, rows_th, offsets_h, T, (const float*)cq_raw, ld_cq, w_cq, (float*)cq_out, Q);
-    else if (dtype == SP_BF16)
-        latent_prepare_kernel<bf16><<<T, 256, 0, st>>>((const bf16*)qd, ldq, (const bf16*)dkv, ld_dkv, (bf16*)qa, (bf16*)kv_pages, positions, slot_map,
-            inv_freq, w_norm, eps, H, n, r, R, rot_dims, own, rows_th, offsets_h, T, (const bf16*)cq_raw, ld_cq, w_cq, (bf16*)cq_out, Q);
+#define SP_LP(TY, PAST) latent_prepare_kernel<TY, PAST><<<T, 256, 0, st>>>((const TY*)qd, ldq, (const TY*)dkv, ld_dkv, (TY*)qa, (TY*)kv_pages, positions, slot_map, \
+        inv_freq, w_norm, eps, H, n, r, R, rot_dims, own, rows_th, offsets_h, T, (const TY*)cq_raw, ld_cq, w_cq, (TY*)cq_out, Q)
+    const bool past = rot_dims / 2 > LAT_PAIRS;
+    if (dtype == SP_F32) { if (past) SP_LP(float, true); else SP_LP(float, false); }
+    else if (dtype == SP_BF16) { if (past) SP_LP(bf16, true); else SP_LP(bf16, false); }
     else return sp_fail("latent_prepare: unknown dtype %d", dtype);
+#undef SP_LP
     SP_LAUNCH_CHECK("latent_prepare");
     return 0;
 }
