@@ -361,7 +361,10 @@ void gemm_f32_tile_kernel(const float* __restrict__ A, int lda, const float* __r
 // to 1,500 tokens, up to 128 groups of 1 to 8 a token, K of 128 to 8,192) were timed with every variant when tiles took
 // 14 + 19.5 c (14 + 47 c) and 17 + 36 c (19 + 82 c); those of 17 to 64 rows, and the figures here, are of the tiles as they are (1,428
 // products, 9 to 1,200 tokens, up to 129 groups, K of 512 to 5,120: the choice is 4 % off the best variant on average, 17 to 64 rows 1 in
-// groups and 4 without, where the lines before were 70 and 18 off; groups of few rows 6 to 9, which tiles have gained most on):
+// groups and 4 without, where the lines before were 70 and 18 off; groups of few rows 6 to 9, which tiles have gained most on).  The stream has become 8 to 22 % faster since (see the top); by 260 products with
+// every variant as it is the choice is off the best by 1.5 % for groups of few rows, 4 up to 16 rows (gated: sixteen columns a workgroup
+// instead of eight), 5 and 7 at 17 to 64 without groups and with, and 16 to 18 beyond, where narrow W, which leaves tiles too few, would be
+// the stream's (4 groups, 119 rows x 256 x 1,024 17.1 us, by the stream 6.8):
 //  * groups of up to eight rows on average: the stream of every group's W, 16 rows a workgroup (16 groups and one of all t rows, 2 x
 //    3,072 x 2,048 gated: t = 17 114, with 32 rows a workgroup 170, tiles 131; t = 64 184 / tiles 171), but tiles of 32 rows where sums are
 //    short and tiles enough (K <= 512 and more than one a compute unit; plain K < 2,048 and more than two: 129 groups x 4,096 x 1,536,

@@ -343,6 +343,9 @@ static int launch_skinny(const void* X, int ldx, const void* W, long wgs, void* 
 // variant 8, 6.6 against 6.3 TB/s; seven groups 169.6 against 173.4), and so do one or two rows times a table of
 // 2^27 elements and up, if those are four a compute unit (variant 5 / 8: 16,384 x 8,192 41.7 / 44.4, 26,496 x 5,120
 // 42.8 / 46.2, 65,536 x 2,048 40.9 / 42.2; fewer: 14,736 x 10,432 50.2 / 46.9).
+// The lines lie where the kernel that asks for all loads together was timed, which groups and one or two rows without a gate now leave to
+// the piped one: over 103 such products and gated ones of one and two rows the choice is 1.3 % off the best of the three variants on average, two
+// of them, gated 2 x 4,096 x 2,048 and 5,120, by 20 % and more (16 rows of W a workgroup 7.9 us, 32 9.5).
 static int skinny_variant(int M, int N, int K, int n_groups, int live_groups, bool glu, int max_rows) {
     const long cus = sp_cu_count();
     const size_t nk = (size_t)N * K;

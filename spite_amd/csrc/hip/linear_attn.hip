@@ -812,7 +812,9 @@ void gated_group_norm_wide_kernel(const float* __restrict__ o, const TO* __restr
 
 // The same without a gate before the sum or a skip, for groups of up to 256 * V: a thread keeps its elements, and what it loads (the row, the
 // gate and the weights) is asked for at once, where the kernel above waits for memory in each of its loops, twice.  The same elements a thread
-// and the same order of sums: the same bits.  us, above and here: one row of 2,048 5.2 / 3.3, of 5,120 10.0 / 5.1, of 8,192 14.1 / 6.9; 1,531 rows of 2,048 9.2 / 7.0.
+// and the same order of sums: the same bits.  us, above and here: one row of 2,048 5.2 / 3.3, of 5,120 10.0 / 5.1, of 8,192 14.1 / 6.9;
+// 1,531 rows of 2,048 9.2 / 7.0.  Elements a thread come in steps of 8, 20 and 32: what a group has less is its last element again, from the cache
+// (one row of 512 3.2 / 2.6, of 2,304 4.3 / 3.2, of 5,632 7.2 / 4.1; 1,531 of 512 5.3 / 4.7, of 2,304 8.1 / 7.0; of 18 widths none is slower).
 template <typename TO, int V>
 __global__ __launch_bounds__(256)
 void gated_group_norm_rows_kernel(const float* __restrict__ o, const TO* __restrict__ gate, int ldg, const float* __restrict__ w,

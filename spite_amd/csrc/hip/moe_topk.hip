@@ -160,10 +160,10 @@ void router_topk_kernel(const float* __restrict__ logits, const float* __restric
 // The choice and the row list of the grouped products (moe_plan with a fan of `top` and `shared` groups that every token
 // visits) of a step of a few tokens by one workgroup, a wave a token: two kernels become one.  Both are a chain of
 // latencies: the logits' load, then a maximum over the wave for every expert that is taken.  Measured on an
-// MI355X when that was six steps of shuffles, one launch against two, us: 1 token, 1 of 16 experts 3.1 / 4.0, 4 of 64 5.1 / 6.0; 8 tokens, 2 of 16 4.5 / 5.7, 8 of
-// 128 11.0 / 11.7, 8 of 512 17.7 / 18.4.  No second token a wave: its choice would wait for the first one's, which
-// router_topk's further workgroups do not (16 tokens, 8 of 64 17.8 / 12.9; 64 tokens, 8 of 128 72 / 16; 512 tokens, 1 of 16
-// 95 / 9.7).  The entries' experts stay in LDS in between; ranks are counted as moe_plan_kernel counts them.
+// MI355X, one launch against two, us: 1 token, 1 of 16 experts 2.4 / 3.5, 4 of 64 3.3 / 4.4; 8 tokens, 2 of 16 3.4 / 4.6, 8 of
+// 128 7.5 / 8.6, 8 of 512 12.6 / 14.6.  No second token a wave: its choice would wait for the first one's, which
+// router_topk's further workgroups do not (when the maximum was six steps of shuffles: 16 tokens, 8 of 64 17.8 / 12.9; 64 tokens, 8 of 128 72 /
+// 16; 512 tokens, 1 of 16 95 / 9.7).  The entries' experts stay in LDS in between; ranks are counted as moe_plan_kernel counts them.
 #define RP_NT 512
 #define RP_MAX (RP_NT / 64 * 64)       // entries: a token a wave, up to 64 experts each; a thread ranks one
 template <int NU>
