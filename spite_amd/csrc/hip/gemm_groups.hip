@@ -594,7 +594,7 @@ static double gg_chance(int cap, int tokens, int routed, double mean, int whole,
 // tiles of 512 for each of 16 experts, 160 for 256 compute units, and 320 of 256, of which 64 units have two; sixteen of 320 are one each, but
 // with one expert of more than `cap` rows they are 272, in two rounds: 2,048 rows x 5,120 x 8,192 273 us by tiles of 512 columns, 237 by one round of
 // these, 350 by two.  Routers do not spread their rows as evenly as chance would, which the estimate cannot know, so that the device decides
-// by the tiles that there are (gemm_groups_kernel).  Of the two launches one finds nothing to do: 2 to 4 us, which products
+// by the tiles that there are (gemm_groups_kernel).  Of the two launches one finds nothing to do: 2 to 5 us, which products
 // of 120 us and more make up for where the tiles can be expected to fit.  (79 products of 8 to 128 experts that are
 // taken, rows spread as by chance / by lognormal loads of 0.2 / 0.4 / 0.8 besides: 0.90 / 0.94 / 0.96 / 0.97 of what ran otherwise on average, four of
 // the 316 times more than 3 % slower, the worst 13; without the device's decision 0.90 / 0.97 / 0.98 / 1.02, 63 times, 65.  16 experts, 5,120 x
